@@ -16,6 +16,7 @@
 //                          position.
 #include "int4_kernels.hpp"
 #include "persist.hpp"
+#include "prefill.hpp"
 #include "sampler_kernels.hpp"
 
 #include <climits>
@@ -482,6 +483,8 @@ struct llama2_decoder {
     l2::PersistLayer* persist_layers = nullptr;
     void* persist_scratch = nullptr;
     l2::PersistArgs pa{};
+    // buffers of the batched prompt (fused decoders)
+    l2::PrefillWorkspace prefill;
 };
 
 using namespace l2;
@@ -762,8 +765,24 @@ int launch_step(llama2_decoder* d, int kind, int position)
     return LLAMA2_OK;
 }
 
+// The prompt's tokens from `position` on are known before the first step (positions below n_prompt); all
+// but the last of them go through the layers in batches, the last one is an ordinary step, so the state
+// after it is that of a decode step.  Advances position and steps past the batch.
+int run_prompt(llama2_decoder* d, int& position, int& steps, int n_prompt)
+{
+    const long long known = static_cast<long long>(n_prompt) - position;
+    const int batch = static_cast<int>(known < steps ? known : steps) - 1;
+    if (batch < kPrefillMinRows)
+        return LLAMA2_OK;
+    L2_TRY(prefill_run(d->prefill, d->cfg, d->layers.data(), d->w, d->s, position, batch));
+    position += batch;
+    steps -= batch;
+    return LLAMA2_OK;
+}
+
 void release(llama2_decoder* d)
 {
+    prefill_destroy(d->prefill);
     for (auto& kind : d->graphs)
         for (hipGraphExec_t g : kind)
             if (g)
@@ -960,6 +979,10 @@ int llama2_decode_create(llama2_decoder** decoder, const llama2_config* config,
             release(d);
             return hip_fail(e, "llama2_decode_create: scratch allocation");
         }
+        if (const int rc = prefill_create(d->prefill, c)) {
+            release(d);
+            return rc;
+        }
         if (variant >= 0) {
             const int rc = persist_setup(d);
             if (rc != LLAMA2_OK) {
@@ -1092,6 +1115,7 @@ int llama2_decode_run_sampled(llama2_decoder* d, int position, int steps, int n_
         }
         d->sampled_temperature = temperature, d->sampled_top_p = top_p, d->sampled_seed = seed;
     }
+    L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)
         L2_TRY(launch_step(d, llama2_decoder::kGraphStepSampled, position + i));
@@ -1112,6 +1136,7 @@ int llama2_decode_run(llama2_decoder* d, int position, int steps, int n_prompt)
         }
         return LLAMA2_OK;
     }
+    L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)
         L2_TRY(launch_step(d, llama2_decoder::kGraphStep, position + i));

@@ -1,0 +1,702 @@
+// The layers of Transformer.Forward (src/Transformer.cs:158-183) for many known tokens at once.
+//
+// A prompt's tokens are all there before the first step, and only their key and value rows matter to
+// what follows (the step of the last prompt token, which produces the first logits anyone reads, is an
+// ordinary decode step).  Taken one by one each token reads all the weights, 3.6 GB for Llama-2-7B; here up
+// to kPrefillMaxRows tokens share one reading and the matrix products run on the matrix cores:
+//   norm (+ embedding) | QKV + RoPE + cache rows | causal attention | o-proj + residual | norm |
+//   SwiGLU | down-proj + residual: 7 launches per layer and batch.
+//
+// Arithmetic, module by module as in the decode step: fp16 between the modules, exact integer weights
+// (n - z) in fp16, fp32 sums of their products with the fp16 inputs over a quantisation group of 128,
+// the group's scale applied in fp32, fp32 sums over the groups; scores rounded to fp16, softmax
+// statistics and probabilities in fp32.  The order of the sums is not that of the decode step.
+//
+// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 21.0 ms;
+// 13B, 74 tokens behind 600 rows: 151 -> 11 ms.
+#include "int4_kernels.hpp"
+#include "prefill.hpp"
+
+#include <cmath>
+
+namespace l2 {
+
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef float f16v_t __attribute__((ext_vector_type(16)));
+
+constexpr int kTile = 32;         // rows of a token tile, columns of a weight tile (v_mfma_f32_32x32x16_f16)
+constexpr int kGroup = 128;       // quantisation group along K
+constexpr int kFragBytes = 1024;  // one operand fragment: 64 lanes of 16 bytes
+constexpr int kBlockBytes = 8 * kFragBytes; // a token tile times a group
+
+// Fragment order of an activation matrix [m][k]: the lane (k / 64 % 2) * 32 + m % 32 of fragment
+// (m / 32, k / 128, k / 8 % 8) holds 8 consecutive k, in the order in which the weights' nibbles come out of
+// a word (0 4 1 5 2 6 3 7).  The word of weights that goes with them is word k / 8 of its row, so a lane's 8
+// words of a group are 32 contiguous bytes, and every fragment is one fully coalesced load.
+__device__ __forceinline__ uint32_t frag_offset(int m, int k, int groups)
+{
+    return static_cast<uint32_t>(((m >> 5) * groups + (k >> 7)) * 8 + ((k >> 3) & 7)) * kFragBytes +
+           ((((k >> 6) & 1) << 5) + (m & 31)) * 16;
+}
+
+__device__ __forceinline__ u32x4 frag_order(u32x4 v) // 8 consecutive values -> 0 4 1 5 2 6 3 7
+{
+    u32x4 o;
+    o[0] = (v[0] & 0xFFFFu) | (v[2] << 16);
+    o[1] = (v[0] >> 16) | (v[2] & 0xFFFF0000u);
+    o[2] = (v[1] & 0xFFFFu) | (v[3] << 16);
+    o[3] = (v[1] >> 16) | (v[3] & 0xFFFF0000u);
+    return o;
+}
+
+// ---------------------------------------------------------------- RoPE angles
+__global__ __launch_bounds__(256) void prefill_rope_kernel(float* tab, int position, int count, float theta)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x, row = i >> 6;
+    if (row >= count)
+        return;
+    float c, s;
+    rope_cos_sin(c, s, i & 63, kRopeHeadSize, position + row, theta);
+    tab[2 * i] = c;
+    tab[2 * i + 1] = s;
+}
+
+// ---------------------------------------------------------------- RMSNorm into fragment order
+struct NormArgs {
+    uint16_t* x; // [rows][K]
+    const uint16_t* gamma;
+    uint16_t* xf;
+    const uint16_t* embedding; // non-null: the row comes from the table and is also written to x
+    const int* tokens;         // of the first row
+    int vocab, K;
+    float eps;
+};
+
+// One row per workgroup of 256 threads; the same sums as the decode step's RMSNorm (block256_sum).
+template <int PIECES>
+__global__ __launch_bounds__(256) void prefill_norm_kernel(NormArgs a)
+{
+    __shared__ float red4[4];
+    const int m = blockIdx.x;
+    uint16_t* row = a.x + static_cast<size_t>(m) * a.K;
+    const uint16_t* src = row;
+    if (a.embedding) {
+        int token = a.tokens[m];
+        token = token < 0 ? 0 : (token >= a.vocab ? a.vocab - 1 : token); // never read outside the table
+        src = a.embedding + static_cast<size_t>(token) * a.K;
+    }
+    VecPieces<PIECES> p, g;
+    p.load(src, a.K);
+    g.load(a.gamma, a.K);
+    if (a.embedding) {
+        const __amdgpu_buffer_rsrc_t ro = make_rsrc(row, a.K * 2);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            __builtin_amdgcn_raw_buffer_store_b128(p.v[i], ro, (threadIdx.x + i * 256) * 16, 0, 0);
+    }
+    const float ss = block256_sum(p.sum_squares(), red4);
+    p.scale(1.0f / sqrtf(ss / static_cast<float>(a.K) + a.eps), g);
+    const int groups = a.K / kGroup;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int k = (threadIdx.x + i * 256) * 8;
+        if (k < a.K)
+            *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(a.xf) + frag_offset(m, k, groups)) = frag_order(p.v[i]);
+    }
+}
+
+// ---------------------------------------------------------------- int4 matrix product
+enum PrefillEpi { EPI_QKV, EPI_RESIDUAL, EPI_SWIGLU };
+
+struct GemmArgs {
+    QW m[3];
+    const uint16_t* xf;
+    uint32_t xf_bytes;
+    int groups, N, ws, ss, zs; // N: rows of one tensor
+    int M, mblocks, pairs;
+    uint16_t* out[3]; // QKV: q, key-cache rows, value-cache rows of this batch; RESIDUAL: x; SWIGLU: hf
+    int out_groups;   // SWIGLU: groups of hf
+    const float* rope;
+};
+
+// 8 nibbles of a word as fp16 n - z, exact: n sits in the mantissa of 1024 + n (bits 0-3 of a half) or
+// 1024 + 16 n (bits 4-7).
+__device__ __forceinline__ h8_t dequant(uint32_t w, h2_t zlo /* 1024 + z */, h2_t zhi /* -(64 + z) */)
+{
+    const h2_t sixteenth = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
+    const uint32_t w8 = w >> 8;
+    const h2_t a = as_h2((w & 0x000F000Fu) | 0x64006400u) - zlo;
+    const h2_t b = __builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | 0x64006400u), sixteenth, zhi);
+    const h2_t c = as_h2((w8 & 0x000F000Fu) | 0x64006400u) - zlo;
+    const h2_t d = __builtin_elementwise_fma(as_h2((w8 & 0x00F000F0u) | 0x64006400u), sixteenth, zhi);
+    return h8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
+
+__device__ __forceinline__ f16v_t mfma(h8_t a, h8_t b, f16v_t c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// A workgroup owns MT token tiles and two weight tiles of 32 rows whose results belong together (the two
+// halves of a RoPE pair, gate and up, or neighbours); its WK wavefronts share the groups of K among them
+// and add up through LDS at the end.
+template <int MT, int WK, int EPI>
+__global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs a)
+{
+    __shared__ float red[WK][2][16][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5, l31 = lane & 31;
+    // The token blocks of one pair of weight tiles run on one XCD, next to each other in time: its L2
+    // serves the weights to all but the first.
+    const int slot = blockIdx.x >> 3;
+    const int pair = (slot / a.mblocks) * 8 + (blockIdx.x & 7), mb = slot % a.mblocks;
+    if (pair >= a.pairs)
+        return;
+    int t0, t1, r0, r1; // tensors and first rows of the two tiles
+    if (EPI == EPI_QKV) {
+        const int per = a.N >> 6, t = pair / per, r = pair - t * per;
+        t0 = t1 = t;
+        r0 = (r >> 1) * kRopeHeadSize + (r & 1) * kTile;
+        r1 = r0 + 64;
+    } else if (EPI == EPI_SWIGLU) {
+        t0 = 0, t1 = 1;
+        r0 = r1 = pair * kTile;
+    } else {
+        t0 = t1 = 0;
+        r0 = pair * 2 * kTile;
+        r1 = r0 + kTile;
+    }
+    const int row0 = r0 + l31 < a.N ? r0 + l31 : a.N - 1, row1 = r1 + l31 < a.N ? r1 + l31 : a.N - 1;
+
+    // Reads past the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet
+    // zeros of the input.
+    const QW q0 = a.m[t0], q1 = a.m[t1];
+    const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(q0.w, static_cast<uint32_t>(a.N) * a.ws * 4),
+                                 rw1 = make_rsrc(q1.w, static_cast<uint32_t>(a.N) * a.ws * 4),
+                                 rz0 = make_rsrc(q0.z, static_cast<uint32_t>(a.N) * a.zs * 4),
+                                 rz1 = make_rsrc(q1.z, static_cast<uint32_t>(a.N) * a.zs * 4),
+                                 rs0 = make_rsrc(q0.s, static_cast<uint32_t>(a.N) * a.ss * 2),
+                                 rs1 = make_rsrc(q1.s, static_cast<uint32_t>(a.N) * a.ss * 2),
+                                 rx = make_rsrc(a.xf, a.xf_bytes);
+    const int wo0 = row0 * a.ws * 4 + h * 32, wo1 = row1 * a.ws * 4 + h * 32;
+    const int zo0 = row0 * a.zs * 4, zo1 = row1 * a.zs * 4, so0 = row0 * a.ss * 2, so1 = row1 * a.ss * 2;
+    const int xo = lane * 16;
+
+    const int g_begin = a.groups * wave / WK, g_end = a.groups * (wave + 1) / WK;
+    const int mt0 = mb * MT;
+
+    struct Raw {
+        u32x4 w[2][2];
+        uint32_t z[2];
+        uint16_t s[2];
+    };
+    auto load_raw = [&](Raw& r, int g) {
+        r.w[0][0] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0, g * 64, 0);
+        r.w[0][1] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0 + 16, g * 64, 0);
+        r.w[1][0] = __builtin_amdgcn_raw_buffer_load_b128(rw1, wo1, g * 64, 0);
+        r.w[1][1] = __builtin_amdgcn_raw_buffer_load_b128(rw1, wo1 + 16, g * 64, 0);
+        r.z[0] = __builtin_amdgcn_raw_buffer_load_b32(rz0, zo0, (g >> 3) * 4, 0);
+        r.z[1] = __builtin_amdgcn_raw_buffer_load_b32(rz1, zo1, (g >> 3) * 4, 0);
+        r.s[0] = __builtin_amdgcn_raw_buffer_load_b16(rs0, so0, g * 2, 0);
+        r.s[1] = __builtin_amdgcn_raw_buffer_load_b16(rs1, so1, g * 2, 0);
+    };
+    auto load_x = [&](u32x4 (&x)[8], int mt, int g) {
+        const int base = ((mt0 + mt) * a.groups + g) * kBlockBytes;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            x[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo + j * kFragBytes, base, 0);
+    };
+
+    f16v_t acc[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                acc[mt][t][i] = 0.0f;
+
+    if (g_begin < g_end) {
+        Raw cur;
+        u32x4 x[8];
+        load_raw(cur, g_begin);
+        load_x(x, 0, g_begin);
+        for (int g = g_begin; g < g_end; ++g) {
+            const int gn = g + 1 < g_end ? g + 1 : g;
+            Raw nxt;
+            load_raw(nxt, gn);
+            h8_t wf[2][8];
+            float sc[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float z = static_cast<float>((cur.z[t] >> ((g & 7) * 4)) & 0xFu);
+                const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
+                const h2_t zlo = {lo, lo}, zhi = {hi, hi};
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    wf[t][j] = dequant(cur.w[t][j >> 2][j & 3], zlo, zhi);
+                sc[t] = half_bits_to_float(cur.s[t]);
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                u32x4 xn[8];
+                load_x(xn, mt + 1 < MT ? mt + 1 : 0, mt + 1 < MT ? g : gn);
+                f16v_t p0 = {}, p1 = {};
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const h8_t xa = __builtin_bit_cast(h8_t, x[j]);
+                    p0 = mfma(xa, wf[0][j], p0);
+                    p1 = mfma(xa, wf[1][j], p1);
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    acc[mt][0][i] = __builtin_fmaf(p0[i], sc[0], acc[mt][0][i]);
+                    acc[mt][1][i] = __builtin_fmaf(p1[i], sc[1], acc[mt][1][i]);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    x[j] = xn[j];
+            }
+            cur = nxt;
+        }
+    }
+
+    constexpr int SHARE = 16 / WK; // accumulator registers a wavefront adds up per tile
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        if (mt)
+            __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                red[wave][t][i][lane] = acc[mt][t][i];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < SHARE; ++u) {
+            const int i = wave * SHARE + u;
+            float v0 = 0.0f, v1 = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WK; ++w) {
+                v0 += red[w][0][i][lane];
+                v1 += red[w][1][i][lane];
+            }
+            const int m = (mt0 + mt) * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (m >= a.M)
+                continue;
+            if (EPI == EPI_QKV) {
+                // q and k are rounded to fp16 before RoPE reads them (native/rope_kernel.cu:14-26)
+                uint16_t b0 = float_to_half_bits(v0), b1 = float_to_half_bits(v1);
+                if (t0 < 2) {
+                    const int idx = (r0 & 63) + l31;
+                    const float* cs = a.rope + (static_cast<size_t>(m) * 64 + idx) * 2;
+                    rope_rotate(b0, b1, half_bits_to_float(b0), half_bits_to_float(b1), cs[0], cs[1]);
+                }
+                uint16_t* o = a.out[t0] + static_cast<size_t>(m) * a.N;
+                o[r0 + l31] = b0;
+                o[r1 + l31] = b1;
+            } else if (EPI == EPI_RESIDUAL) {
+                uint16_t* o = a.out[0] + static_cast<size_t>(m) * a.N;
+                o[r0 + l31] = float_to_half_bits(v0 + half_bits_to_float(o[r0 + l31]));
+                o[r1 + l31] = float_to_half_bits(v1 + half_bits_to_float(o[r1 + l31]));
+            } else {
+                const int n = r0 + l31;
+                if (n < a.N) {
+                    float v = v0;
+                    v *= 1.0f / (1.0f + expf(-v)); // native/mat_vec_kernel.cu:219-221
+                    v *= v1;
+                    const int e = n & 7;
+                    *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(a.out[0]) + frag_offset(m, n, a.out_groups) +
+                                                 2 * ((e & 3) * 2 + (e >> 2))) = float_to_half_bits(v);
+                }
+            }
+        }
+    }
+}
+
+template <int EPI>
+int launch_gemm(const char* name, GemmArgs a)
+{
+    // token tiles in blocks of equal size, at most 4
+    const int tiles = ceil_div(a.M, kTile);
+    a.mblocks = ceil_div(tiles, 4);
+    const int mt = ceil_div(tiles, a.mblocks);
+    a.mblocks = ceil_div(tiles, mt);
+    const dim3 grid(ceil_div(a.pairs, 8) * 8 * a.mblocks);
+    const hipStream_t st = ctx().stream;
+    switch (mt) {
+    case 1: hipLaunchKernelGGL((prefill_gemm_kernel<1, 8, EPI>), grid, dim3(512), 0, st, a); break;
+    case 2: hipLaunchKernelGGL((prefill_gemm_kernel<2, 8, EPI>), grid, dim3(512), 0, st, a); break;
+    case 3: hipLaunchKernelGGL((prefill_gemm_kernel<3, 4, EPI>), grid, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((prefill_gemm_kernel<4, 4, EPI>), grid, dim3(256), 0, st, a); break;
+    }
+    L2_LAUNCH_CHECK(name);
+    return LLAMA2_OK;
+}
+
+// ---------------------------------------------------------------- causal attention
+struct PrefillAttnArgs {
+    const uint16_t* q; // [rows][dim], rotated
+    const uint16_t* kcache;
+    const uint16_t* vcache; // layer base, rows of `dim`
+    uint16_t* xf;
+    int position, M, dim, n_heads;
+    float scale;
+};
+
+constexpr int kAttnT = 64;        // timesteps per pass
+constexpr int kKStride = 256 + 16; // bytes of a key row in LDS: 8 lanes x 16 bytes of consecutive rows hit all banks
+constexpr int kVStride = 128 + 16; // bytes of a row of 64 timesteps of one output element
+constexpr float kProbScale = 16384.0f;
+
+__device__ __forceinline__ int v_row_offset(int d) { return d * kVStride + (d >> 3) * 16; }
+
+// The 16 timesteps t0 .. t0 + 15 of one operand step, one product each, kept only by the queries that
+// attend it (lane half u / 8 holds timestep t0 + u % 8 / 4 * 8 + u / 8 * 4 + u % 4 as element u % 8).
+__device__ __forceinline__ void one_by_one(f16v_t (&o)[4], h8_t hi, h8_t lo, const char* v, int l31, int hl, int t0, int limit)
+{
+    for (int u = 0; u < 16; ++u) {
+        const bool keep = t0 + ((u & 7) >> 2) * 8 + (u >> 3) * 4 + (u & 3) <= limit;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            u32x4 w = *reinterpret_cast<const u32x4*>(v + v_row_offset(d * 32 + l31));
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                w[k] &= hl == (u >> 3) && k == ((u & 7) >> 1) ? ((u & 1) ? 0xFFFF0000u : 0x0000FFFFu) : 0u;
+            const h8_t vf = __builtin_bit_cast(h8_t, w);
+            f16v_t c = mfma(vf, hi, f16v_t{});
+            c = mfma(vf, lo, c);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                o[d][i] = keep ? o[d][i] + c[i] : o[d][i];
+        }
+    }
+}
+
+// One wavefront per tile of 32 queries of a head, NW tiles per workgroup share the key and value rows in
+// LDS.  Scores are computed transposed (rows: timesteps, columns: queries), so that a lane holds 32
+// timesteps of ONE query and its probabilities are already the second operand of the product with the
+// transposed values.  Probabilities keep fp32's precision: each is scaled by 2^14 and split into two fp16
+// numbers that go through the matrix cores one after the other (22 bits; below 2^-17 an absolute 2^-39).
+template <int NW>
+__global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a)
+{
+    __shared__ __align__(16) char ks[kAttnT * kKStride];
+    __shared__ __align__(16) char vs[kRopeHeadSize * kVStride + 16 * 16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hl = lane >> 5, l31 = lane & 31;
+    const int head = blockIdx.y;
+    const int qb = gridDim.x - 1 - blockIdx.x; // the longest blocks first
+    const int tile = qb * NW + wave;
+    const int m = tile * kTile + l31;
+    const int rows = a.position + a.M; // valid cache rows
+    const int last_q = (qb * NW + NW) * kTile < a.M ? (qb * NW + NW) * kTile : a.M;
+    const int t_end = a.position + last_q; // timesteps any query of the workgroup attends
+    const int limit = a.position + m;      // last timestep of this lane's query
+    const int wave_limit = a.position + tile * kTile + kTile - 1;
+
+    h8_t qf[8];
+    {
+        const int mq = m < a.M ? m : a.M - 1;
+        const uint16_t* q = a.q + static_cast<size_t>(mq) * a.dim + head * kRopeHeadSize + hl * 64;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            qf[j] = *reinterpret_cast<const h8_t*>(q + j * 8);
+    }
+    const uint32_t cache_bytes = static_cast<uint32_t>(rows) * a.dim * 2; // < 2^31: checked on the host
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.kcache, cache_bytes), rv = make_rsrc(a.vcache, cache_bytes);
+
+    f16v_t o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+        o[d] = f16v_t{};
+    float mx = -INFINITY, sum = 0.0f;
+
+    constexpr int KP = kAttnT * 16 / (NW * 64); // 16-byte pieces of the key rows per thread
+    constexpr int VP = 256 / (NW * 64);         // blocks of 4 timesteps x 8 elements per thread
+    u32x4 kr[KP], vr[VP][4];
+    auto request = [&](int tb) {
+#pragma unroll
+        for (int i = 0; i < KP; ++i) {
+            const int e = threadIdx.x + i * NW * 64;
+            kr[i] = __builtin_amdgcn_raw_buffer_load_b128(
+                rk, ((tb + (e >> 4)) * a.dim + head * kRopeHeadSize + (e & 15) * 8) * 2, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < VP; ++i) {
+            const int e = threadIdx.x + i * NW * 64, u = e >> 4;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                vr[i][r] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rv, ((tb + 4 * u + r) * a.dim + head * kRopeHeadSize + (e & 15) * 8) * 2, 0, 0);
+        }
+    };
+    request(0);
+    for (int tb = 0; tb < t_end; tb += kAttnT) {
+        __syncthreads(); // the previous pass has been read
+#pragma unroll
+        for (int i = 0; i < KP; ++i) {
+            const int e = threadIdx.x + i * NW * 64;
+            *reinterpret_cast<u32x4*>(ks + (e >> 4) * kKStride + (e & 15) * 16) = kr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < VP; ++i) {
+            const int e = threadIdx.x + i * NW * 64, u = e >> 4, d0 = (e & 15) * 8;
+            // unit u: timesteps 4u .. 4u + 3, i.e. block a = (u >> 1) & 3 and half u & 1 of tile u >> 3
+            const int at = (u >> 3) * 64 + (u & 1) * 32 + ((u >> 1) & 3) * 8;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t a0 = vr[i][0][k], a1 = vr[i][1][k], a2 = vr[i][2][k], a3 = vr[i][3][k];
+                const u32x2 even = {(a0 & 0xFFFFu) | (a1 << 16), (a2 & 0xFFFFu) | (a3 << 16)};
+                const u32x2 odd = {(a0 >> 16) | (a1 & 0xFFFF0000u), (a2 >> 16) | (a3 & 0xFFFF0000u)};
+                *reinterpret_cast<u32x2*>(vs + v_row_offset(d0 + 2 * k) + at) = even;
+                *reinterpret_cast<u32x2*>(vs + v_row_offset(d0 + 2 * k + 1) + at) = odd;
+            }
+        }
+        __syncthreads();
+        if (tb + kAttnT < t_end)
+            request(tb + kAttnT);
+        if (tb > wave_limit)
+            continue; // this tile attends nothing here (the barriers are the same for all wavefronts)
+
+        // Where some queries do not attend some of these timesteps, an infinite or NaN value must not reach
+        // them through a probability of 0.
+        bool careful = false;
+        if (tb + kAttnT - 1 > a.position + tile * kTile) {
+            uint32_t bad = 0;
+            for (int d = 0; d < 4; ++d)
+                for (int u = 0; u < 4; ++u) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(vs + v_row_offset(d * 32 + l31) + (u >> 1) * 64 +
+                                                                    hl * 32 + (u & 1) * 16);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        bad |= (v[k] & 0x7C007C00u) + 0x04000400u; // bits 15 and 31: all exponent bits set
+                }
+            careful = __any((bad & 0x80008000u) != 0);
+        }
+
+        f16v_t s[2] = {};
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt) {
+                const h8_t kf = *reinterpret_cast<const h8_t*>(ks + (tt * 32 + l31) * kKStride + hl * 128 + j * 16);
+                s[tt] = mfma(kf, qf[j], s[tt]);
+            }
+        float bm = -INFINITY;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int t = tb + tt * 32 + 8 * (i >> 2) + 4 * hl + (i & 3);
+                const float v = half_bits_to_float(float_to_half_bits(s[tt][i] * a.scale)); // native/mat_vec_kernel.cu:71-74
+                s[tt][i] = t <= limit ? v : -INFINITY;
+                bm = fmaxf(bm, s[tt][i]);
+            }
+        bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
+        const float nm = fmaxf(mx, bm); // finite: timestep 0 is in the first pass
+        const float alpha = expf(mx - nm);
+        mx = nm;
+        sum *= alpha;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                o[d][i] *= alpha;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                h8_t hi, lo;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float p = expf(s[tt][8 * j + i] - mx);
+                    sum += p;
+                    const float ps = p * kProbScale;
+                    hi[i] = static_cast<_Float16>(ps);
+                    lo[i] = static_cast<_Float16>(ps - static_cast<float>(hi[i]));
+                }
+                if (careful) {
+                    one_by_one(o, hi, lo, vs + tt * 64 + hl * 32 + j * 16, l31, hl, tb + tt * 32 + j * 16, limit);
+                    continue;
+                }
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const h8_t vf =
+                        *reinterpret_cast<const h8_t*>(vs + v_row_offset(d * 32 + l31) + tt * 64 + hl * 32 + j * 16);
+                    o[d] = mfma(vf, hi, o[d]);
+                    o[d] = mfma(vf, lo, o[d]);
+                }
+            }
+    }
+    sum += __shfl_xor(sum, 32, 64);
+    const float inv = 1.0f / kProbScale;
+    if (tile * kTile >= a.M) // the whole wavefront
+        return;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) { // blocks of 8 outputs, two at a time: the lower half of the lanes stores the first
+            uint32_t w[2][2];
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const int i = (2 * p + b) * 4 + 2 * k;
+                    w[b][k] = static_cast<uint32_t>(float_to_half_bits(o[d][i] * inv / sum)) |
+                              static_cast<uint32_t>(float_to_half_bits(o[d][i + 1] * inv / sum)) << 16;
+                }
+            uint32_t lo[2], hi[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const uint32_t got = __shfl_xor(static_cast<int>(hl ? w[0][k] : w[1][k]), 32, 64);
+                lo[k] = hl ? got : w[0][k];
+                hi[k] = hl ? w[1][k] : got;
+            }
+            const u32x4 out = {(lo[0] & 0xFFFFu) | (hi[0] << 16), (lo[0] >> 16) | (hi[0] & 0xFFFF0000u),
+                               (lo[1] & 0xFFFFu) | (hi[1] << 16), (lo[1] >> 16) | (hi[1] & 0xFFFF0000u)};
+            const int k0 = head * kRopeHeadSize + (d * 4 + 2 * p + hl) * 8;
+            if (m < a.M)
+                *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(a.xf) + frag_offset(m, k0, a.n_heads)) = out;
+        }
+}
+
+int launch_prefill_attn(const PrefillAttnArgs& a)
+{
+    const int tiles = ceil_div(a.M, kTile);
+    const hipStream_t st = ctx().stream;
+    if (ceil_div(tiles, 4) * a.n_heads >= ctx().num_cus)
+        hipLaunchKernelGGL((prefill_attn_kernel<4>), dim3(ceil_div(tiles, 4), a.n_heads), dim3(256), 0, st, a);
+    else if (ceil_div(tiles, 2) * a.n_heads >= ctx().num_cus)
+        hipLaunchKernelGGL((prefill_attn_kernel<2>), dim3(ceil_div(tiles, 2), a.n_heads), dim3(128), 0, st, a);
+    else
+        hipLaunchKernelGGL((prefill_attn_kernel<1>), dim3(tiles, a.n_heads), dim3(64), 0, st, a);
+    L2_LAUNCH_CHECK("prefill attention");
+    return LLAMA2_OK;
+}
+
+int launch_prefill_norm(const NormArgs& a, int M)
+{
+    const dim3 grid(M), block(256);
+    const hipStream_t st = ctx().stream;
+    switch (ceil_div(a.K, 2048)) {
+    case 1: hipLaunchKernelGGL((prefill_norm_kernel<1>), grid, block, 0, st, a); break;
+    case 2: hipLaunchKernelGGL((prefill_norm_kernel<2>), grid, block, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((prefill_norm_kernel<3>), grid, block, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((prefill_norm_kernel<4>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((prefill_norm_kernel<8>), grid, block, 0, st, a); break;
+    }
+    L2_LAUNCH_CHECK("prefill norm");
+    return LLAMA2_OK;
+}
+
+static size_t up256(size_t n) { return (n + 255) / 256 * 256; }
+
+int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
+{
+    const int rows = ceil_div(cfg.seq_len < kPrefillMaxRows ? cfg.seq_len : kPrefillMaxRows, kTile) * kTile;
+    const size_t vec = up256(static_cast<size_t>(rows) * cfg.dim * 2);
+    const size_t hid = up256(static_cast<size_t>(rows) * ceil_div(cfg.hidden_dim, kGroup) * kGroup * 2);
+    const size_t rope = static_cast<size_t>(rows) * 128 * sizeof(float);
+    const size_t total = 3 * vec + hid + rope;
+    L2_HIP(hipMalloc(&ws.base, total));
+    char* p = static_cast<char*>(ws.base);
+    ws.x = reinterpret_cast<uint16_t*>(p);
+    ws.q = reinterpret_cast<uint16_t*>(p + vec);
+    ws.xf = reinterpret_cast<uint16_t*>(p + 2 * vec);
+    ws.hf = reinterpret_cast<uint16_t*>(p + 3 * vec);
+    ws.rope = reinterpret_cast<float*>(p + 3 * vec + hid);
+    ws.rows = rows;
+    // hf beyond hidden_dim is never written and must read as zero
+    L2_HIP(hipMemsetAsync(ws.base, 0, total, ctx().stream));
+    L2_HIP(hipStreamSynchronize(ctx().stream));
+    return LLAMA2_OK;
+}
+
+void prefill_destroy(PrefillWorkspace& ws)
+{
+    if (ws.base)
+        (void)hipFree(ws.base);
+    ws = PrefillWorkspace{};
+}
+
+#define L2_TRY(expr)          \
+    do {                      \
+        int rc_ = (expr);     \
+        if (rc_ != LLAMA2_OK) \
+            return rc_;       \
+    } while (0)
+
+static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, const llama2_layer_weights* layers,
+                         const llama2_transformer_weights& w, const llama2_run_state& s, int position, int M)
+{
+    const int dim = c.dim, hidden = c.hidden_dim;
+    const int ss = ceil_div(dim, 128), wsz = ceil_div(dim, 32) * 4, zs = ceil_div(ss, 8);
+    const int hss = ceil_div(hidden, 128), hws = ceil_div(hidden, 32) * 4, hzs = ceil_div(hss, 8);
+    const uint32_t xf_bytes = static_cast<uint32_t>(ws.rows) * ss * kGroup * 2;
+    const uint32_t hf_bytes = static_cast<uint32_t>(ws.rows) * hss * kGroup * 2;
+    auto qw = [](const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; };
+    hipLaunchKernelGGL(prefill_rope_kernel, dim3(ceil_div(M * 64, 256)), dim3(256), 0, ctx().stream, ws.rope, position,
+                       M, c.rope_theta);
+    L2_LAUNCH_CHECK("prefill rope");
+    for (int i = 0; i < c.n_layers; ++i) {
+        const llama2_layer_weights& L = layers[i];
+        const size_t layer_offset = static_cast<size_t>(i) * c.seq_len * dim;
+        const size_t row = layer_offset + static_cast<size_t>(position) * dim;
+        NormArgs n{};
+        n.x = ws.x, n.gamma = L.rms_attention, n.xf = ws.xf, n.K = dim, n.eps = 1e-5f;
+        if (i == 0)
+            n.embedding = w.token_embedding_table, n.tokens = s.tokens + position, n.vocab = c.vocab_size;
+        L2_TRY(launch_prefill_norm(n, M));
+        {
+            GemmArgs a{};
+            a.m[0] = qw(L.query), a.m[1] = qw(L.key), a.m[2] = qw(L.value);
+            a.out[0] = ws.q, a.out[1] = s.key_cache + row, a.out[2] = s.value_cache + row;
+            a.xf = ws.xf, a.xf_bytes = xf_bytes, a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M;
+            a.pairs = 3 * (dim / 64), a.rope = ws.rope;
+            L2_TRY(launch_gemm<EPI_QKV>("prefill qkv", a));
+        }
+        if (i == c.n_layers - 1)
+            break; // the batch's tokens leave nothing but their cache rows
+        {
+            PrefillAttnArgs a{};
+            a.q = ws.q, a.kcache = s.key_cache + layer_offset, a.vcache = s.value_cache + layer_offset, a.xf = ws.xf;
+            a.position = position, a.M = M, a.dim = dim, a.n_heads = c.n_heads;
+            a.scale = 1.0f / sqrtf(static_cast<float>(kRopeHeadSize));
+            L2_TRY(launch_prefill_attn(a));
+        }
+        {
+            GemmArgs a{};
+            a.m[0] = qw(L.output), a.out[0] = ws.x, a.xf = ws.xf, a.xf_bytes = xf_bytes;
+            a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M, a.pairs = dim / 64;
+            L2_TRY(launch_gemm<EPI_RESIDUAL>("prefill o-proj", a));
+        }
+        n.gamma = L.rms_feed_forward, n.embedding = nullptr;
+        L2_TRY(launch_prefill_norm(n, M));
+        {
+            GemmArgs a{};
+            a.m[0] = qw(L.gate), a.m[1] = qw(L.up), a.out[0] = ws.hf, a.xf = ws.xf, a.xf_bytes = xf_bytes;
+            a.groups = ss, a.N = hidden, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M, a.pairs = ceil_div(hidden, kTile);
+            a.out_groups = hss;
+            L2_TRY(launch_gemm<EPI_SWIGLU>("prefill swiglu", a));
+        }
+        {
+            GemmArgs a{};
+            a.m[0] = qw(L.down), a.out[0] = ws.x, a.xf = ws.hf, a.xf_bytes = hf_bytes;
+            a.groups = hss, a.N = dim, a.ws = hws, a.ss = hss, a.zs = hzs, a.M = M, a.pairs = dim / 64;
+            L2_TRY(launch_gemm<EPI_RESIDUAL>("prefill down-proj", a));
+        }
+    }
+    return LLAMA2_OK;
+}
+
+int prefill_run(const PrefillWorkspace& ws, const llama2_config& cfg, const llama2_layer_weights* layers,
+                const llama2_transformer_weights& w, const llama2_run_state& s, int position, int count)
+{
+    const int batches = ceil_div(count, ws.rows), rows = ceil_div(count, batches);
+    for (int done = 0; done < count; done += rows)
+        L2_TRY(prefill_batch(ws, cfg, layers, w, s, position + done, rows < count - done ? rows : count - done));
+    return LLAMA2_OK;
+}
+
+} // namespace l2

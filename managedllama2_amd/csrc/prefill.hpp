@@ -1,0 +1,34 @@
+// Prompt tokens in batches: host interface (prefill.hip).
+#pragma once
+
+#include <cstddef>
+#include <cstdint>
+
+#include "../../include/llama2_hip.h"
+
+namespace l2 {
+
+constexpr int kPrefillMaxRows = 1024; // tokens per batch; longer prompts go through in batches of equal size
+// Fewer known tokens take the decode step one by one: up to half of a matrix tile would be padding, and the
+// short prompts keep the decode step's sums bit for bit.
+constexpr int kPrefillMinRows = 16;
+
+struct PrefillWorkspace {
+    uint16_t* x = nullptr;    // residual stream, [rows][dim]
+    uint16_t* q = nullptr;    // rotated queries, [rows][dim]
+    uint16_t* xf = nullptr;   // normalised input / attention output in fragment order
+    uint16_t* hf = nullptr;   // SwiGLU output in fragment order
+    float* rope = nullptr;    // (cos, sin) of 64 angles per row
+    void* base = nullptr;     // the one allocation behind all of them
+    int rows = 0;             // capacity, a multiple of 32
+};
+
+// Sizes `ws` for batches of up to min(seq_len, kPrefillMaxRows) tokens and allocates it.
+int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg);
+void prefill_destroy(PrefillWorkspace& ws);
+// The layers of Transformer.Forward for the `count` tokens at positions position .. position + count - 1,
+// which are known: fills their rows of the key and value caches (nothing else of the run state).
+int prefill_run(const PrefillWorkspace& ws, const llama2_config& cfg, const llama2_layer_weights* layers,
+                const llama2_transformer_weights& w, const llama2_run_state& s, int position, int count);
+
+} // namespace l2

@@ -1,0 +1,144 @@
+"""The batched prompt of the device-resident loop (prefill.hip) against the fp64 oracle, token by token.
+
+llama2_decode_run sends all but the last of the known tokens through the layers in batches when there are
+at least 16 of them; their only results are rows of the key and value caches, which every later step
+attends, so the caches and the first logits are compared.  Both paths round the same quantities to fp16 and
+sum in fp32, in other orders, so over a whole cache (thousands of values) their 2-norm distances from the
+oracle are two samples of the same error: the batch may be 1.5 times as far off as single steps, plus a tenth
+of an fp16 rounding (1e-4) where both are nearly exact.  Where single steps are the reference, the bound is
+the end-to-end bound of the small models in test_gpu_transformer.py."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_util import assert_close_normwise
+from managedllama2_amd import capi, synth
+from managedllama2_amd.transformer import Transformer
+
+pytestmark = pytest.mark.gpu
+FUSED_GRAPH = capi.DECODE_FUSED | capi.DECODE_GRAPH
+TOL = 1e-2
+
+
+def config(dim, hidden, layers, seq_len):
+    return dict(dim=dim, hidden_dim=hidden, n_layers=layers, n_heads=dim // 128, n_kv_heads=dim // 128, vocab_size=512,
+                seq_len=seq_len, rope_theta=10000.0)
+
+
+def caches(t, cfg, n):
+    shape = (cfg["n_layers"], cfg["seq_len"], cfg["dim"])
+    return [b.to_host().reshape(shape)[:, :n] for b in (t.runstate.keyCache, t.runstate.valueCache)]
+
+
+def step_by_step(cfg, model, prompt, first, history=None):
+    """The same positions through single steps (what the loop did for fewer known tokens)."""
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    if history:
+        t.runstate.keyCache.copy_to_device(history[0])
+        t.runstate.valueCache.copy_to_device(history[1])
+    t.runstate.tokens.copy_to_device(prompt, first)
+    for pos in range(first, first + len(prompt)):
+        t.Forward(pos, pos + 1)
+    return t
+
+
+# batch = known - 1: around the tile of 32 tokens and the block of 128; hidden sizes that are no multiple of a tile
+# or of a group; the largest goes through in two batches
+@pytest.mark.parametrize("dim,hidden,known", [(256, 640, 16), (256, 640, 17), (256, 328, 33), (384, 1000, 34),
+                                              (256, 640, 65), (512, 1408, 97), (128, 136, 129), (256, 640, 130),
+                                              (384, 1000, 258), (256, 328, 1060)])
+def test_prompt_fills_the_caches(oracle, dim, hidden, known):
+    cfg = config(dim, hidden, 2, known + 3)
+    model = synth.random_model(cfg, seed=61, rms_random=True)
+    prompt = synth.rng_for(801, known).integers(3, 512, known).astype(np.int32)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run", t._decoder, 0, known, known)
+    ref = step_by_step(cfg, model, prompt, 0)
+    hm = oracle.HostModel(cfg, model)
+    hm.tokens[:known] = prompt
+    for pos in range(known):
+        hm.forward(pos, pos + 1)
+    shape = (cfg["n_layers"], cfg["seq_len"], dim)
+    for name, g, s, w in zip("kv", caches(t, cfg, known), caches(ref, cfg, known), (hm.key_cache, hm.value_cache)):
+        want = w.reshape(shape)[:, :known].astype(np.float64)
+        for layer in range(cfg["n_layers"]):
+            batch, steps = (float(np.linalg.norm(v[layer] - want[layer]) / np.linalg.norm(want[layer])) for v in (g, s))
+            print(name, layer, "batch %.2e steps %.2e" % (batch, steps))
+            assert batch <= 1.5 * steps + 1e-4, (name, layer, batch, steps)
+    token = int(t.runstate.tokens.to_host(1, known)[0])
+    assert token == int(np.argmax(t.runstate.logits.to_host()))
+    assert np.array_equal(t.runstate.tokens.to_host(known), prompt)
+    for tr in (t, ref):
+        tr.close()
+
+
+@pytest.mark.parametrize("first,known", [(1, 17), (63, 40), (200, 131)])
+def test_prompt_behind_a_history(first, known):
+    cfg = config(256, 640, 2, first + known + 2)
+    model = synth.random_model(cfg, seed=62)
+    rng = synth.rng_for(802, first)
+    n = cfg["n_layers"] * cfg["seq_len"] * cfg["dim"]
+    history = synth.normal_f16(rng, n), synth.normal_f16(rng, n)
+    prompt = rng.integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, first, history)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.keyCache.copy_to_device(history[0])
+    t.runstate.valueCache.copy_to_device(history[1])
+    t.runstate.tokens.copy_to_device(prompt, first)
+    # a prompt that reaches beyond the steps asked for: every step of the call is known, nothing is generated
+    capi.call("llama2_decode_run", t._decoder, first, known, first + known + 5)
+    for g, w in zip(caches(t, cfg, first + known), caches(ref, cfg, first + known)):
+        assert np.array_equal(g[:, :first].view(np.uint16), w[:, :first].view(np.uint16))
+        assert_close_normwise(g.ravel(), w.ravel().astype(np.float64), "cache", TOL)
+    assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
+    for tr in (t, ref):
+        tr.close()
+
+
+def test_overflowing_token_reaches_only_later_positions():
+    """One token whose embedding overflows to infinities: the rows of the positions before it stay finite."""
+    cfg = config(256, 640, 3, 96)
+    model = synth.random_model(cfg, seed=63)
+    embedding = model["embedding"].reshape(512, 256)
+    embedding[7] = np.float16(np.inf)
+    prompt = synth.rng_for(803).integers(8, 512, 90).astype(np.int32)
+    bad = 45
+    prompt[bad] = 7
+    ref = step_by_step(cfg, model, prompt, 0)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run", t._decoder, 0, 90, 90)
+    for g, w in zip(caches(t, cfg, 90), caches(ref, cfg, 90)):
+        assert np.array_equal(np.isfinite(g), np.isfinite(w))
+        assert np.all(np.isfinite(g[:, :bad])) and not np.any(np.isfinite(g[1:, bad:]))
+        assert_close_normwise(g[:, :bad].ravel(), w[:, :bad].ravel().astype(np.float64), "cache", TOL)
+    for tr in (t, ref):
+        tr.close()
+
+
+def test_captured_prompt_replays():
+    """The whole prompt as a graph of the caller's: every replay gives the caches of the eager call."""
+    cfg = config(256, 640, 2, 64)
+    model = synth.random_model(cfg, seed=64)
+    prompt = synth.rng_for(804).integers(3, 512, 50).astype(np.int32)
+    t = Transformer(dict(cfg), model, mode=capi.DECODE_FUSED)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run", t._decoder, 0, 52, 50)
+    want = caches(t, cfg, 52), t.runstate.tokens.to_host(53)
+    g = C.c_void_p()
+    capi.call("llama2_graph_begin_capture")
+    capi.call("llama2_decode_run", t._decoder, 0, 52, 50)
+    capi.call("llama2_graph_end_capture", C.byref(g))
+    for rep in range(3):
+        capi.call("llama2_memset", t.runstate.keyCache.ptr, 0, 2 * 64 * 256 * 2)
+        capi.call("llama2_memset", t.runstate.valueCache.ptr, 0, 2 * 64 * 256 * 2)
+        t.runstate.tokens.copy_to_device(np.concatenate([prompt, np.zeros(3, np.int32)]))
+        capi.call("llama2_graph_launch", g)
+        assert np.array_equal(t.runstate.tokens.to_host(53), want[1]), rep
+        for a, b in zip(caches(t, cfg, 52), want[0]):
+            assert np.array_equal(a.view(np.uint16), b.view(np.uint16)), rep
+        t.Forward(51, 52)  # the decoder's own path between the replays
+    capi.call("llama2_graph_destroy", g)
+    t.close()

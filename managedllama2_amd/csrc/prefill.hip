@@ -68,11 +68,15 @@ struct NormArgs {
     uint16_t* xf;
     const uint16_t* embedding; // non-null: the row comes from the table and is also written to x
     const int* tokens;         // of the first row
+    const float* parts; // non-null: x += the sum of n_parts fp32 results [part][part_rows][K] of the product before
+    int n_parts, part_rows;
     int vocab, K;
     float eps;
 };
 
-// One row per workgroup of 256 threads; the same sums as the decode step's RMSNorm (block256_sum).
+// One row per workgroup of 256 threads; the same sums as the decode step's RMSNorm (block256_sum).  The
+// residual product before it leaves fp32 sums over pieces of K; they are added here, in order, and
+// rounded to fp16 once, so that product can be split over as many workgroups as the GPU holds.
 template <int PIECES>
 __global__ __launch_bounds__(256) void prefill_norm_kernel(NormArgs a)
 {
@@ -88,7 +92,28 @@ __global__ __launch_bounds__(256) void prefill_norm_kernel(NormArgs a)
     VecPieces<PIECES> p, g;
     p.load(src, a.K);
     g.load(a.gamma, a.K);
-    if (a.embedding) {
+    if (a.parts) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int k = (threadIdx.x + i * 256) * 8;
+            if (k >= a.K)
+                continue;
+            float sum[8] = {};
+            for (int t = 0; t < a.n_parts; ++t) {
+                const float* q = a.parts + (static_cast<size_t>(t) * a.part_rows + m) * a.K + k;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    sum[e] += q[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const h2_t x = as_h2(p.v[i][e]);
+                p.v[i][e] = static_cast<uint32_t>(float_to_half_bits(sum[2 * e] + static_cast<float>(x[0]))) |
+                            static_cast<uint32_t>(float_to_half_bits(sum[2 * e + 1] + static_cast<float>(x[1]))) << 16;
+            }
+        }
+    }
+    if (a.embedding || a.parts) {
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(row, a.K * 2);
 #pragma unroll
         for (int i = 0; i < PIECES; ++i)
@@ -106,16 +131,18 @@ __global__ __launch_bounds__(256) void prefill_norm_kernel(NormArgs a)
 }
 
 // ---------------------------------------------------------------- int4 matrix product
-enum PrefillEpi { EPI_QKV, EPI_RESIDUAL, EPI_SWIGLU };
+enum PrefillEpi { EPI_QKV, EPI_PARTIAL, EPI_SWIGLU };
 
 struct GemmArgs {
     QW m[3];
     const uint16_t* xf;
     uint32_t xf_bytes;
     int groups, N, ws, ss, zs; // N: rows of one tensor
-    int M, mblocks, pairs;
-    uint16_t* out[3]; // QKV: q, key-cache rows, value-cache rows of this batch; RESIDUAL: x; SWIGLU: hf
-    int out_groups;   // SWIGLU: groups of hf
+    int M, mblocks, nblocks, splits;
+    uint16_t* out[3]; // QKV: q, key-cache rows, value-cache rows of this batch; SWIGLU: hf
+    float* parts;     // PARTIAL: [splits][part_rows][N]
+    int part_rows;
+    int out_groups; // SWIGLU: groups of hf
     const float* rope;
 };
 
@@ -125,10 +152,12 @@ __device__ __forceinline__ h8_t dequant(uint32_t w, h2_t zlo /* 1024 + z */, h2_
 {
     const h2_t sixteenth = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
     const uint32_t w8 = w >> 8;
-    const h2_t a = as_h2((w & 0x000F000Fu) | 0x64006400u) - zlo;
-    const h2_t b = __builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | 0x64006400u), sixteenth, zhi);
-    const h2_t c = as_h2((w8 & 0x000F000Fu) | 0x64006400u) - zlo;
-    const h2_t d = __builtin_elementwise_fma(as_h2((w8 & 0x00F000F0u) | 0x64006400u), sixteenth, zhi);
+    uint32_t magic = 0x64006400u; // in a vector register: (w & mask) | magic is one instruction then
+    asm("" : "+v"(magic));
+    const h2_t a = as_h2((w & 0x000F000Fu) | magic) - zlo;
+    const h2_t b = __builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | magic), sixteenth, zhi);
+    const h2_t c = as_h2((w8 & 0x000F000Fu) | magic) - zlo;
+    const h2_t d = __builtin_elementwise_fma(as_h2((w8 & 0x00F000F0u) | magic), sixteenth, zhi);
     return h8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
@@ -137,21 +166,45 @@ __device__ __forceinline__ f16v_t mfma(h8_t a, h8_t b, f16v_t c)
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-// A workgroup owns MT token tiles and two weight tiles of 32 rows whose results belong together (the two
-// halves of a RoPE pair, gate and up, or neighbours); its WK wavefronts share the groups of K among them
-// and add up through LDS at the end.
-template <int MT, int WK, int EPI>
-__global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs a)
+// 64 lanes x 16 bytes from a buffer straight into LDS at `lds` + 16 lane (`lds`, `soff` uniform).  Written
+// as assembly because the compiler, told that LDS is written, waits for it before any later LDS read,
+// also of the other half of a ring; there is no destination register, and the caller waits (vmcnt)
+// before the barrier that publishes the data.
+__device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, int voff, int soff)
 {
-    __shared__ float red[WK][2][16][64];
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory", "m0");
+}
+
+// A workgroup owns MT token tiles and WN pairs of weight tiles of 32 rows; the two tiles of a pair hold
+// results that belong together (the two halves of a RoPE pair, gate and up, or neighbours) and stay in one
+// wavefront.  WK wavefronts share the groups of K and add up through LDS at the end; the launch may split
+// K further (EPI_PARTIAL).
+//
+// What bounds it: a wavefront's MT x 16 products of a group take MT x 512 cycles of its matrix core, the
+// dequantisation and the scaling about half as many of its vector unit.  Everything the next group needs has to
+// arrive meanwhile, and loads return in order, so a fragment requested behind a weight from HBM waits
+// for that weight.  Hence the activations go to LDS (each fragment once per workgroup instead of once
+// per wavefront) a whole group ahead, the weights to registers two groups ahead, and there is one wait
+// per group.
+template <int MT, int WN, int WK, int EPI>
+__global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(GemmArgs a)
+{
+    constexpr int kStage = WK * MT * kBlockBytes;
+    constexpr int kRed = WK * WN * 2 * 16 * 64 * 4;
+    __shared__ __align__(1024) char lds[2 * kStage > kRed ? 2 * kStage : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = wave % WN, wk = wave / WN;
     const int h = lane >> 5, l31 = lane & 31;
-    // The token blocks of one pair of weight tiles run on one XCD, next to each other in time: its L2
+    // The token blocks of one block of weights run on one XCD, next to each other in time: its L2
     // serves the weights to all but the first.
     const int slot = blockIdx.x >> 3;
-    const int pair = (slot / a.mblocks) * 8 + (blockIdx.x & 7), mb = slot % a.mblocks;
-    if (pair >= a.pairs)
+    const int unit = (slot / a.mblocks) * 8 + (blockIdx.x & 7), mb = slot % a.mblocks;
+    if (unit >= a.nblocks * a.splits)
         return;
+    const int nb = unit / a.splits, split = unit - nb * a.splits, pair = nb * WN + wn;
     int t0, t1, r0, r1; // tensors and first rows of the two tiles
     if (EPI == EPI_QKV) {
         const int per = a.N >> 6, t = pair / per, r = pair - t * per;
@@ -171,25 +224,31 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
     // Reads past the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet
     // zeros of the input.
     const QW q0 = a.m[t0], q1 = a.m[t1];
-    const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(q0.w, static_cast<uint32_t>(a.N) * a.ws * 4),
-                                 rw1 = make_rsrc(q1.w, static_cast<uint32_t>(a.N) * a.ws * 4),
-                                 rz0 = make_rsrc(q0.z, static_cast<uint32_t>(a.N) * a.zs * 4),
-                                 rz1 = make_rsrc(q1.z, static_cast<uint32_t>(a.N) * a.zs * 4),
-                                 rs0 = make_rsrc(q0.s, static_cast<uint32_t>(a.N) * a.ss * 2),
-                                 rs1 = make_rsrc(q1.s, static_cast<uint32_t>(a.N) * a.ss * 2),
-                                 rx = make_rsrc(a.xf, a.xf_bytes);
+    const uint32_t wbytes = static_cast<uint32_t>(a.N) * a.ws * 4, zbytes = static_cast<uint32_t>(a.N) * a.zs * 4,
+                   sbytes = static_cast<uint32_t>(a.N) * a.ss * 2;
+    const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(uniform_ptr(q0.w), wbytes), rw1 = make_rsrc(uniform_ptr(q1.w), wbytes),
+                                 rz0 = make_rsrc(uniform_ptr(q0.z), zbytes), rz1 = make_rsrc(uniform_ptr(q1.z), zbytes),
+                                 rs0 = make_rsrc(uniform_ptr(q0.s), sbytes), rs1 = make_rsrc(uniform_ptr(q1.s), sbytes);
+    const unsigned long long xp = reinterpret_cast<unsigned long long>(a.xf);
+    const u32x4 rx = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(xp))),
+                      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(xp >> 32))), a.xf_bytes,
+                      0x00020000u};
     const int wo0 = row0 * a.ws * 4 + h * 32, wo1 = row1 * a.ws * 4 + h * 32;
     const int zo0 = row0 * a.zs * 4, zo1 = row1 * a.zs * 4, so0 = row0 * a.ss * 2, so1 = row1 * a.ss * 2;
-    const int xo = lane * 16;
-
-    const int g_begin = a.groups * wave / WK, g_end = a.groups * (wave + 1) / WK;
-    const int mt0 = mb * MT;
+    const int mt0 = mb * MT, last_tile = (a.M - 1) / kTile;
+    const int g_begin = a.groups * split / a.splits, g_end = a.groups * (split + 1) / a.splits;
+    const int steps = (g_end - g_begin + WK - 1) / WK;
+    auto group_of = [&](int step) { // a group that does not exist is loaded as the last one and not used
+        const int g = g_begin + step * WK + wk;
+        return g < g_end ? g : g_end - 1;
+    };
 
     struct Raw {
         u32x4 w[2][2];
         uint32_t z[2];
         uint16_t s[2];
     };
+    constexpr int kRawLoads = 8;
     auto load_raw = [&](Raw& r, int g) {
         r.w[0][0] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0, g * 64, 0);
         r.w[0][1] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0 + 16, g * 64, 0);
@@ -200,11 +259,21 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
         r.s[0] = __builtin_amdgcn_raw_buffer_load_b16(rs0, so0, g * 2, 0);
         r.s[1] = __builtin_amdgcn_raw_buffer_load_b16(rs1, so1, g * 2, 0);
     };
-    auto load_x = [&](u32x4 (&x)[8], int mt, int g) {
-        const int base = ((mt0 + mt) * a.groups + g) * kBlockBytes;
+    const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
+        static_cast<int>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)));
+    auto load_x = [&](int step) { // this wavefront's share of the fragments of its WK group
+        const int g = group_of(step);
+        const uint32_t dst = lds_base + (step & 1) * kStage + wk * MT * kBlockBytes;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            x[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo + j * kFragBytes, base, 0);
+        for (int mt = 0; mt < MT; ++mt) {
+            const int tile = mt0 + mt <= last_tile ? mt0 + mt : last_tile; // the last block may have tiles to spare
+#pragma unroll
+            for (int j = 0; j < 8 / WN; ++j) {
+                const int f = wn * (8 / WN) + j;
+                load_to_lds(rx, dst + mt * kBlockBytes + f * kFragBytes, lane * 16,
+                            (tile * a.groups + g) * kBlockBytes + f * kFragBytes);
+            }
+        }
     };
 
     f16v_t acc[MT][2];
@@ -216,35 +285,43 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
             for (int i = 0; i < 16; ++i)
                 acc[mt][t][i] = 0.0f;
 
-    if (g_begin < g_end) {
-        Raw cur;
-        u32x4 x[8];
-        load_raw(cur, g_begin);
-        load_x(x, 0, g_begin);
-        for (int g = g_begin; g < g_end; ++g) {
-            const int gn = g + 1 < g_end ? g + 1 : g;
-            Raw nxt;
-            load_raw(nxt, gn);
-            h8_t wf[2][8];
-            float sc[2];
+    Raw cur, next;
+    load_raw(cur, group_of(0));
+    load_x(0);
+    load_raw(next, group_of(1));
+    static_assert(kRawLoads == 8, "the waits below");
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    __syncthreads();
+    for (int step = 0; step < steps; ++step) {
+        const int g = g_begin + step * WK + wk;
+        h8_t wf[2][8];
+        float sc[2];
+        const int zsh = (group_of(step) & 7) * 4;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const float z = static_cast<float>((cur.z[t] >> ((g & 7) * 4)) & 0xFu);
-                const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
-                const h2_t zlo = {lo, lo}, zhi = {hi, hi};
+        for (int t = 0; t < 2; ++t) {
+            const float z = static_cast<float>((cur.z[t] >> zsh) & 0xFu);
+            const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
+            const h2_t zlo = {lo, lo}, zhi = {hi, hi};
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    wf[t][j] = dequant(cur.w[t][j >> 2][j & 3], zlo, zhi);
-                sc[t] = half_bits_to_float(cur.s[t]);
-            }
+            for (int j = 0; j < 8; ++j)
+                wf[t][j] = dequant(cur.w[t][j >> 2][j & 3], zlo, zhi);
+            sc[t] = half_bits_to_float(cur.s[t]);
+        }
+        // the weights are taken before anything new is requested: the compiler's own wait for them counts
+        // the loads it knows, and would otherwise wait for the fragments as well
+        __builtin_amdgcn_sched_barrier(0);
+        cur = next;
+        load_x(step + 1);
+        load_raw(next, group_of(step + 2));
+        __builtin_amdgcn_sched_barrier(0);
+        if (g < g_end) {
+            const char* xs = lds + (step & 1) * kStage + wk * MT * kBlockBytes + lane * 16;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                u32x4 xn[8];
-                load_x(xn, mt + 1 < MT ? mt + 1 : 0, mt + 1 < MT ? g : gn);
                 f16v_t p0 = {}, p1 = {};
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const h8_t xa = __builtin_bit_cast(h8_t, x[j]);
+                    const h8_t xa = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes + j * kFragBytes);
                     p0 = mfma(xa, wf[0][j], p0);
                     p1 = mfma(xa, wf[1][j], p1);
                 }
@@ -253,15 +330,18 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
                     acc[mt][0][i] = __builtin_fmaf(p0[i], sc[0], acc[mt][0][i]);
                     acc[mt][1][i] = __builtin_fmaf(p1[i], sc[1], acc[mt][1][i]);
                 }
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    x[j] = xn[j];
             }
-            cur = nxt;
         }
+        // the fragments of the next step are there, only its successor's weights are still on their way
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        __syncthreads();
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing may still write LDS
+    __syncthreads();
 
     constexpr int SHARE = 16 / WK; // accumulator registers a wavefront adds up per tile
+    float* red = reinterpret_cast<float*>(lds);
+    auto red_at = [&](int w, int t, int i) { return red + (((w * WN + wn) * 2 + t) * 16 + i) * 64 + lane; };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (mt)
@@ -270,16 +350,16 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                red[wave][t][i][lane] = acc[mt][t][i];
+                *red_at(wk, t, i) = acc[mt][t][i];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < SHARE; ++u) {
-            const int i = wave * SHARE + u;
+            const int i = wk * SHARE + u;
             float v0 = 0.0f, v1 = 0.0f;
 #pragma unroll
             for (int w = 0; w < WK; ++w) {
-                v0 += red[w][0][i][lane];
-                v1 += red[w][1][i][lane];
+                v0 += *red_at(w, 0, i);
+                v1 += *red_at(w, 1, i);
             }
             const int m = (mt0 + mt) * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
             if (m >= a.M)
@@ -295,10 +375,10 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
                 uint16_t* o = a.out[t0] + static_cast<size_t>(m) * a.N;
                 o[r0 + l31] = b0;
                 o[r1 + l31] = b1;
-            } else if (EPI == EPI_RESIDUAL) {
-                uint16_t* o = a.out[0] + static_cast<size_t>(m) * a.N;
-                o[r0 + l31] = float_to_half_bits(v0 + half_bits_to_float(o[r0 + l31]));
-                o[r1 + l31] = float_to_half_bits(v1 + half_bits_to_float(o[r1 + l31]));
+            } else if (EPI == EPI_PARTIAL) {
+                float* o = a.parts + (static_cast<size_t>(split) * a.part_rows + m) * a.N;
+                o[r0 + l31] = v0;
+                o[r1 + l31] = v1;
             } else {
                 const int n = r0 + l31;
                 if (n < a.N) {
@@ -314,22 +394,46 @@ __global__ __launch_bounds__(WK * 64, WK / 4) void prefill_gemm_kernel(GemmArgs 
     }
 }
 
-template <int EPI>
-int launch_gemm(const char* name, GemmArgs a)
+// Two token tiles per workgroup (one for batches of one tile).
+static int token_blocks(int M) { return M <= kTile ? 1 : ceil_div(M, 2 * kTile); }
+
+constexpr int kMaxSplits = 8;
+
+// Pieces of K of a residual product: as many as it takes to give every compute unit a workgroup, each
+// with at least 4 groups.
+static int residual_splits(int M, int N, int groups)
 {
-    // token tiles in blocks of equal size, at most 4
-    const int tiles = ceil_div(a.M, kTile);
-    a.mblocks = ceil_div(tiles, 4);
-    const int mt = ceil_div(tiles, a.mblocks);
-    a.mblocks = ceil_div(tiles, mt);
-    const dim3 grid(ceil_div(a.pairs, 8) * 8 * a.mblocks);
-    const hipStream_t st = ctx().stream;
-    switch (mt) {
-    case 1: hipLaunchKernelGGL((prefill_gemm_kernel<1, 8, EPI>), grid, dim3(512), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((prefill_gemm_kernel<2, 8, EPI>), grid, dim3(512), 0, st, a); break;
-    case 3: hipLaunchKernelGGL((prefill_gemm_kernel<3, 4, EPI>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((prefill_gemm_kernel<4, 4, EPI>), grid, dim3(256), 0, st, a); break;
-    }
+    const int blocks = token_blocks(M) * ceil_div(N, 256);
+    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    int s = cus / blocks;
+    s = s < groups / 4 ? s : groups / 4;
+    return s < 1 ? 1 : (s < kMaxSplits ? s : kMaxSplits);
+}
+
+template <int MT, int WN, int WK, int EPI>
+void launch_gemm_as(GemmArgs& a, int pairs)
+{
+    a.nblocks = ceil_div(pairs, WN);
+    const dim3 grid(ceil_div(a.nblocks * a.splits, 8) * 8 * a.mblocks);
+    hipLaunchKernelGGL((prefill_gemm_kernel<MT, WN, WK, EPI>), grid, dim3(WN * WK * 64), 0, ctx().stream, a);
+}
+
+// 8 wavefronts in every case, two per SIMD, so that one's vector work runs under the other's products.
+// Four pairs of weight tiles per workgroup read the activations half as often as two; two pairs make
+// twice the workgroups where four would not give every compute unit one.
+template <int EPI>
+int launch_gemm(const char* name, GemmArgs a, int pairs)
+{
+    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    a.mblocks = token_blocks(a.M);
+    if (EPI != EPI_PARTIAL)
+        a.splits = 1;
+    if (a.M <= kTile)
+        launch_gemm_as<1, 2, 4, EPI>(a, pairs);
+    else if (ceil_div(pairs, 4) * a.mblocks * a.splits < cus)
+        launch_gemm_as<2, 2, 4, EPI>(a, pairs);
+    else
+        launch_gemm_as<2, 4, 2, EPI>(a, pairs);
     L2_LAUNCH_CHECK(name);
     return LLAMA2_OK;
 }
@@ -598,7 +702,14 @@ int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
     const size_t vec = up256(static_cast<size_t>(rows) * cfg.dim * 2);
     const size_t hid = up256(static_cast<size_t>(rows) * ceil_div(cfg.hidden_dim, kGroup) * kGroup * 2);
     const size_t rope = static_cast<size_t>(rows) * 128 * sizeof(float);
-    const size_t total = 3 * vec + hid + rope;
+    size_t parts = 0; // the largest [splits][rows][dim] any batch needs
+    for (int m = kTile; m <= rows; m += kTile)
+        for (int k : {cfg.dim, cfg.hidden_dim}) {
+            const size_t n = static_cast<size_t>(residual_splits(m, cfg.dim, ceil_div(k, kGroup))) * m;
+            parts = n > parts ? n : parts;
+        }
+    parts *= static_cast<size_t>(cfg.dim) * sizeof(float);
+    const size_t total = 3 * vec + hid + up256(rope) + parts;
     L2_HIP(hipMalloc(&ws.base, total));
     char* p = static_cast<char*>(ws.base);
     ws.x = reinterpret_cast<uint16_t*>(p);
@@ -606,6 +717,7 @@ int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
     ws.xf = reinterpret_cast<uint16_t*>(p + 2 * vec);
     ws.hf = reinterpret_cast<uint16_t*>(p + 3 * vec);
     ws.rope = reinterpret_cast<float*>(p + 3 * vec + hid);
+    ws.parts = reinterpret_cast<float*>(p + 3 * vec + hid + up256(rope));
     ws.rows = rows;
     // hf beyond hidden_dim is never written and must read as zero
     L2_HIP(hipMemsetAsync(ws.base, 0, total, ctx().stream));
@@ -635,6 +747,8 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
     const int hss = ceil_div(hidden, 128), hws = ceil_div(hidden, 32) * 4, hzs = ceil_div(hss, 8);
     const uint32_t xf_bytes = static_cast<uint32_t>(ws.rows) * ss * kGroup * 2;
     const uint32_t hf_bytes = static_cast<uint32_t>(ws.rows) * hss * kGroup * 2;
+    const int part_rows = ceil_div(M, kTile) * kTile;
+    const int o_splits = residual_splits(M, dim, ss), down_splits = residual_splits(M, dim, hss);
     auto qw = [](const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; };
     hipLaunchKernelGGL(prefill_rope_kernel, dim3(ceil_div(M * 64, 256)), dim3(256), 0, ctx().stream, ws.rope, position,
                        M, c.rope_theta);
@@ -645,7 +759,10 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
         const size_t row = layer_offset + static_cast<size_t>(position) * dim;
         NormArgs n{};
         n.x = ws.x, n.gamma = L.rms_attention, n.xf = ws.xf, n.K = dim, n.eps = 1e-5f;
-        if (i == 0)
+        n.part_rows = part_rows;
+        if (i > 0)
+            n.parts = ws.parts, n.n_parts = down_splits;
+        else
             n.embedding = w.token_embedding_table, n.tokens = s.tokens + position, n.vocab = c.vocab_size;
         L2_TRY(launch_prefill_norm(n, M));
         {
@@ -653,8 +770,8 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
             a.m[0] = qw(L.query), a.m[1] = qw(L.key), a.m[2] = qw(L.value);
             a.out[0] = ws.q, a.out[1] = s.key_cache + row, a.out[2] = s.value_cache + row;
             a.xf = ws.xf, a.xf_bytes = xf_bytes, a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M;
-            a.pairs = 3 * (dim / 64), a.rope = ws.rope;
-            L2_TRY(launch_gemm<EPI_QKV>("prefill qkv", a));
+            a.rope = ws.rope;
+            L2_TRY(launch_gemm<EPI_QKV>("prefill qkv", a, 3 * (dim / 64)));
         }
         if (i == c.n_layers - 1)
             break; // the batch's tokens leave nothing but their cache rows
@@ -667,24 +784,24 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
         }
         {
             GemmArgs a{};
-            a.m[0] = qw(L.output), a.out[0] = ws.x, a.xf = ws.xf, a.xf_bytes = xf_bytes;
-            a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M, a.pairs = dim / 64;
-            L2_TRY(launch_gemm<EPI_RESIDUAL>("prefill o-proj", a));
+            a.m[0] = qw(L.output), a.parts = ws.parts, a.part_rows = part_rows, a.splits = o_splits, a.xf = ws.xf, a.xf_bytes = xf_bytes;
+            a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M;
+            L2_TRY(launch_gemm<EPI_PARTIAL>("prefill o-proj", a, dim / 64));
         }
-        n.gamma = L.rms_feed_forward, n.embedding = nullptr;
+        n.gamma = L.rms_feed_forward, n.embedding = nullptr, n.parts = ws.parts, n.n_parts = o_splits;
         L2_TRY(launch_prefill_norm(n, M));
         {
             GemmArgs a{};
             a.m[0] = qw(L.gate), a.m[1] = qw(L.up), a.out[0] = ws.hf, a.xf = ws.xf, a.xf_bytes = xf_bytes;
-            a.groups = ss, a.N = hidden, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M, a.pairs = ceil_div(hidden, kTile);
+            a.groups = ss, a.N = hidden, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M;
             a.out_groups = hss;
-            L2_TRY(launch_gemm<EPI_SWIGLU>("prefill swiglu", a));
+            L2_TRY(launch_gemm<EPI_SWIGLU>("prefill swiglu", a, ceil_div(hidden, kTile)));
         }
         {
             GemmArgs a{};
-            a.m[0] = qw(L.down), a.out[0] = ws.x, a.xf = ws.hf, a.xf_bytes = hf_bytes;
-            a.groups = hss, a.N = dim, a.ws = hws, a.ss = hss, a.zs = hzs, a.M = M, a.pairs = dim / 64;
-            L2_TRY(launch_gemm<EPI_RESIDUAL>("prefill down-proj", a));
+            a.m[0] = qw(L.down), a.parts = ws.parts, a.part_rows = part_rows, a.splits = down_splits, a.xf = ws.hf, a.xf_bytes = hf_bytes;
+            a.groups = hss, a.N = dim, a.ws = hws, a.ss = hss, a.zs = hzs, a.M = M;
+            L2_TRY(launch_gemm<EPI_PARTIAL>("prefill down-proj", a, dim / 64));
         }
     }
     return LLAMA2_OK;

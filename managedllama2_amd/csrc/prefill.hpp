@@ -18,6 +18,7 @@ struct PrefillWorkspace {
     uint16_t* q = nullptr;    // rotated queries, [rows][dim]
     uint16_t* xf = nullptr;   // normalised input / attention output in fragment order
     uint16_t* hf = nullptr;   // SwiGLU output in fragment order
+    float* parts = nullptr;   // fp32 sums of the residual products over pieces of K
     float* rope = nullptr;    // (cos, sin) of 64 angles per row
     void* base = nullptr;     // the one allocation behind all of them
     int rows = 0;             // capacity, a multiple of 32

@@ -138,7 +138,7 @@ struct GemmArgs {
     const uint16_t* xf;
     uint32_t xf_bytes;
     int groups, N, ws, ss, zs; // N: rows of one tensor
-    int M, mblocks, nblocks, splits;
+    int M, mblocks, pairs, nblocks, splits; // pairs of weight tiles, and blocks of them
     uint16_t* out[3]; // QKV: q, key-cache rows, value-cache rows of this batch; SWIGLU: hf
     float* parts;     // PARTIAL: [splits][part_rows][N]
     int part_rows;
@@ -178,23 +178,43 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, int voff, 
                  : "memory", "m0");
 }
 
+// The same from an address per lane: 16 bytes to `lds` + 16 lane, 4 bytes to `lds` + 4 lane.
+__device__ __forceinline__ void load_to_lds_x4(const void* p, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(p) : "memory", "m0");
+}
+__device__ __forceinline__ void load_to_lds_x1(const void* p, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(p) : "memory", "m0");
+}
+
+// s_waitcnt vmcnt(n), the other counters free
+constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }
+
 // A workgroup owns MT token tiles and WN pairs of weight tiles of 32 rows; the two tiles of a pair hold
 // results that belong together (the two halves of a RoPE pair, gate and up, or neighbours) and stay in one
-// wavefront.  WK wavefronts share the groups of K and add up through LDS at the end; the launch may split
-// K further (EPI_PARTIAL).
+// wavefront.  A step covers WK consecutive groups of K, one per wavefront of a pair; they add up through LDS at
+// the end.  The launch may split K further (EPI_PARTIAL).
 //
-// What bounds it: a wavefront's MT x 16 products of a group take MT x 512 cycles of its matrix core, the
-// dequantisation and the scaling about half as many of its vector unit.  Everything the next group needs has to
-// arrive meanwhile, and loads return in order, so a fragment requested behind a weight from HBM waits
-// for that weight.  Hence the activations go to LDS (each fragment once per workgroup instead of once
-// per wavefront) a whole group ahead, the weights to registers two groups ahead, and there is one wait
-// per group.
+// What bounds it: the products of a group take MT x 512 cycles of a wavefront's matrix core, the
+// dequantisation and the scaling about as many of its vector unit.  The other limit is the rate at which a compute
+// unit looks up addresses: one per cycle and 64 contiguous bytes.  A lane that reads its own row's
+// weights, zero points and scales costs 64 lookups per load, 8 loads per wavefront and step, and made the
+// lookups the slowest part (61 % busy against 28 % of the matrix cores).  So everything comes through LDS,
+// requested in the order of memory: a weight row's 64 WK bytes by neighbouring lanes, a row's
+// scales and zero points of a step once for all WK groups.  Weights are requested two steps ahead (their slot is free
+// as soon as they are in registers, hence the barrier after the read), activations one.
 template <int MT, int WN, int WK, int EPI>
 __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(GemmArgs a)
 {
-    constexpr int kStage = WK * MT * kBlockBytes;
+    constexpr int kStage = WK * MT * kBlockBytes;    // activations of a step
+    constexpr int kWRow = WK * 64;                   // bytes of a weight row per step
+    constexpr int kWStage = WN * 2 * kTile * kWRow;  // weights of a step
+    constexpr int kSStage = WN * 64 * 16, kZStage = WN * 64 * 4;
+    constexpr int kWAt = 2 * kStage, kSAt = kWAt + 2 * kWStage, kZAt = kSAt + 2 * kSStage, kAll = kZAt + 2 * kZStage;
     constexpr int kRed = WK * WN * 2 * 16 * 64 * 4;
-    __shared__ __align__(1024) char lds[2 * kStage > kRed ? 2 * kStage : kRed];
+    static_assert(kAll <= 160 * 1024, "LDS of a compute unit");
+    __shared__ __align__(1024) char lds[kAll > kRed ? kAll : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wn = wave % WN, wk = wave / WN;
     const int h = lane >> 5, l31 = lane & 31;
@@ -204,65 +224,77 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
     const int unit = (slot / a.mblocks) * 8 + (blockIdx.x & 7), mb = slot % a.mblocks;
     if (unit >= a.nblocks * a.splits)
         return;
-    const int nb = unit / a.splits, split = unit - nb * a.splits, pair = nb * WN + wn;
-    int t0, t1, r0, r1; // tensors and first rows of the two tiles
-    if (EPI == EPI_QKV) {
-        const int per = a.N >> 6, t = pair / per, r = pair - t * per;
-        t0 = t1 = t;
-        r0 = (r >> 1) * kRopeHeadSize + (r & 1) * kTile;
-        r1 = r0 + 64;
-    } else if (EPI == EPI_SWIGLU) {
-        t0 = 0, t1 = 1;
-        r0 = r1 = pair * kTile;
-    } else {
-        t0 = t1 = 0;
-        r0 = pair * 2 * kTile;
-        r1 = r0 + kTile;
-    }
+    const int nb = unit / a.splits, split = unit - nb * a.splits;
+    // tensor and first row of tile t of a pair; the last block may have pairs to spare, which repeat the last one
+    auto tile_of = [&](int pair, int t, int& tensor, int& row) {
+        pair = pair < a.pairs ? pair : a.pairs - 1;
+        if (EPI == EPI_QKV) {
+            const int per = a.N >> 6, r = pair % per;
+            tensor = pair / per;
+            row = (r >> 1) * kRopeHeadSize + (r & 1) * kTile + t * 64;
+        } else if (EPI == EPI_SWIGLU) {
+            tensor = t;
+            row = pair * kTile;
+        } else {
+            tensor = 0;
+            row = (pair * 2 + t) * kTile;
+        }
+    };
+    auto rsrc_of = [](const void* p, uint32_t bytes) {
+        const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+        return u32x4{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))),
+                     static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))), bytes, 0x00020000u};
+    };
+    const bool mine = nb * WN + wn < a.pairs;
+    int t0, t1, r0, r1;
+    tile_of(nb * WN + wn, 0, t0, r0);
+    tile_of(nb * WN + wn, 1, t1, r1);
     const int row0 = r0 + l31 < a.N ? r0 + l31 : a.N - 1, row1 = r1 + l31 < a.N ? r1 + l31 : a.N - 1;
-
-    // Reads past the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet
-    // zeros of the input.
-    const QW q0 = a.m[t0], q1 = a.m[t1];
-    const uint32_t wbytes = static_cast<uint32_t>(a.N) * a.ws * 4, zbytes = static_cast<uint32_t>(a.N) * a.zs * 4,
-                   sbytes = static_cast<uint32_t>(a.N) * a.ss * 2;
-    const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(uniform_ptr(q0.w), wbytes), rw1 = make_rsrc(uniform_ptr(q1.w), wbytes),
-                                 rz0 = make_rsrc(uniform_ptr(q0.z), zbytes), rz1 = make_rsrc(uniform_ptr(q1.z), zbytes),
-                                 rs0 = make_rsrc(uniform_ptr(q0.s), sbytes), rs1 = make_rsrc(uniform_ptr(q1.s), sbytes);
-    const unsigned long long xp = reinterpret_cast<unsigned long long>(a.xf);
-    const u32x4 rx = {static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(xp))),
-                      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(xp >> 32))), a.xf_bytes,
-                      0x00020000u};
-    const int wo0 = row0 * a.ws * 4 + h * 32, wo1 = row1 * a.ws * 4 + h * 32;
-    const int zo0 = row0 * a.zs * 4, zo1 = row1 * a.zs * 4, so0 = row0 * a.ss * 2, so1 = row1 * a.ss * 2;
     const int mt0 = mb * MT, last_tile = (a.M - 1) / kTile;
-    const int g_begin = a.groups * split / a.splits, g_end = a.groups * (split + 1) / a.splits;
+    // pieces of K begin at a multiple of 4 groups, so the groups of a step share a word of zero points
+    const int g_begin = (a.groups * split / a.splits) & ~3;
+    const int g_end = split + 1 == a.splits ? a.groups : (a.groups * (split + 1) / a.splits) & ~3;
     const int steps = (g_end - g_begin + WK - 1) / WK;
-    auto group_of = [&](int step) { // a group that does not exist is loaded as the last one and not used
-        const int g = g_begin + step * WK + wk;
-        return g < g_end ? g : g_end - 1;
-    };
-
-    struct Raw {
-        u32x4 w[2][2];
-        uint32_t z[2];
-        uint16_t s[2];
-    };
-    constexpr int kRawLoads = 8;
-    auto load_raw = [&](Raw& r, int g) {
-        r.w[0][0] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0, g * 64, 0);
-        r.w[0][1] = __builtin_amdgcn_raw_buffer_load_b128(rw0, wo0 + 16, g * 64, 0);
-        r.w[1][0] = __builtin_amdgcn_raw_buffer_load_b128(rw1, wo1, g * 64, 0);
-        r.w[1][1] = __builtin_amdgcn_raw_buffer_load_b128(rw1, wo1 + 16, g * 64, 0);
-        r.z[0] = __builtin_amdgcn_raw_buffer_load_b32(rz0, zo0, (g >> 3) * 4, 0);
-        r.z[1] = __builtin_amdgcn_raw_buffer_load_b32(rz1, zo1, (g >> 3) * 4, 0);
-        r.s[0] = __builtin_amdgcn_raw_buffer_load_b16(rs0, so0, g * 2, 0);
-        r.s[1] = __builtin_amdgcn_raw_buffer_load_b16(rs1, so1, g * 2, 0);
+    auto base_of = [&](int step) { // first group; a step that does not exist is loaded as the last one and not used
+        return g_begin + (step < steps ? step : steps - 1) * WK;
     };
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         static_cast<int>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)));
-    auto load_x = [&](int step) { // this wavefront's share of the fragments of its WK group
-        const int g = group_of(step);
+
+    // Weights: this wavefront fetches 4 KB of the step, RPI rows per load.  Piece c of 16 bytes of row r lies in slot
+    // c ^ (r & 7) of the row, so the 8 rows that an LDS read takes at a time meet all banks.  Reads past
+    // the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet zeros of the input.
+    constexpr int LPR = WK * 4, RPI = 64 / LPR;
+    const int wr0 = wave * 4 * RPI; // first row of the block this wavefront fetches
+    int wt, wrow;
+    tile_of(nb * WN + wr0 / 64, (wr0 / kTile) & 1, wt, wrow);
+    wrow += (wr0 & (kTile - 1));
+    const u32x4 rw = rsrc_of(wt == 0 ? a.m[0].w : (wt == 1 ? a.m[1].w : a.m[2].w), static_cast<uint32_t>(a.N) * a.ws * 4);
+    int wvoff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = i * RPI + lane / LPR, row = wrow + r < a.N ? wrow + r : a.N - 1;
+        wvoff[i] = row * a.ws * 4 + ((lane % LPR) ^ ((wr0 + r) & 7)) * 16;
+    }
+    // Scales and zero points of the pair's 64 rows, a lane's row in tile h: 16 bytes that hold the scales of
+    // the step's groups, and the word with their zero points.  Scales need not be aligned to more than their 2 bytes:
+    // offsets count from the word that holds the first one, and the 16 bytes begin at a word and end with the
+    // word that holds the last one.
+    const int szrow = h ? row1 : row0;
+    const QW q0 = a.m[t0], q1 = a.m[t1], qz = h ? q1 : q0;
+    const int al0 = static_cast<int>(reinterpret_cast<uintptr_t>(q0.s) & 2), al1 = static_cast<int>(reinterpret_cast<uintptr_t>(q1.s) & 2);
+    const int alz = h ? al1 : al0;
+    auto scale_at = [&](int al, int row, int g) { return al + (row * a.ss + g) * 2; };
+    auto scale_base = [&](int al, int row, int g) {
+        const int b = scale_at(al, row, g) & ~3, last = ((al + a.N * a.ss * 2 + 3) & ~3) - 16;
+        return b < last ? b : last;
+    };
+    const u32x4 rx = rsrc_of(a.xf, a.xf_bytes);
+
+    constexpr int kWLoads = 4;
+    auto load_x = [&](int step) { // this wavefront's share of the fragments of its group
+        int g = base_of(step) + wk;
+        g = g < g_end ? g : g_end - 1;
         const uint32_t dst = lds_base + (step & 1) * kStage + wk * MT * kBlockBytes;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -275,6 +307,25 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
             }
         }
     };
+    // Scales by the wavefronts of the step's first group, zero points by those of the second.  Whole addresses per
+    // lane: the two tiles may belong to two tensors.  All of them lie inside their tensors.
+    auto load_sz = [&](int step, int g) {
+        const uint32_t slot_at = step & 1;
+        if (wk == 0)
+            load_to_lds_x4(reinterpret_cast<const char*>(qz.s) - alz + scale_base(alz, szrow, g),
+                           lds_base + kSAt + slot_at * kSStage + wn * 1024);
+        else if (wk == 1)
+            load_to_lds_x1(qz.z + static_cast<size_t>(szrow) * a.zs + (g >> 3),
+                           lds_base + kZAt + slot_at * kZStage + wn * 256);
+    };
+    auto load_w = [&](int step) {
+        const int g = base_of(step);
+        const uint32_t dst = lds_base + kWAt + (step & 1) * kWStage + wr0 * kWRow;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            load_to_lds(rw, dst + i * kFragBytes, wvoff[i], g * 64);
+        load_sz(step, g);
+    };
 
     f16v_t acc[MT][2];
 #pragma unroll
@@ -285,36 +336,51 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
             for (int i = 0; i < 16; ++i)
                 acc[mt][t][i] = 0.0f;
 
-    Raw cur, next;
-    load_raw(cur, group_of(0));
+    load_w(0);
     load_x(0);
-    load_raw(next, group_of(1));
-    static_assert(kRawLoads == 8, "the waits below");
-    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    load_w(1);
+    // wk < 2 fetch scales or zero points as well
+    auto wait_for_all_but_the_next_weights = [&] {
+        if (WK == 2 || wk < 2)
+            __builtin_amdgcn_s_waitcnt(wait_vm(kWLoads + 1));
+        else
+            __builtin_amdgcn_s_waitcnt(wait_vm(kWLoads));
+    };
+    asm volatile("" ::: "memory");
+    wait_for_all_but_the_next_weights();
     __syncthreads();
     for (int step = 0; step < steps; ++step) {
-        const int g = g_begin + step * WK + wk;
-        h8_t wf[2][8];
-        float sc[2];
-        const int zsh = (group_of(step) & 7) * 4;
+        const int gb = g_begin + step * WK, g = gb + wk;
+        u32x4 raw[2][2];
+        float z[2], sc[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const float z = static_cast<float>((cur.z[t] >> zsh) & 0xFu);
-            const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
-            const h2_t zlo = {lo, lo}, zhi = {hi, hi};
+            const int r = wn * 64 + t * kTile + l31;
+            const char* wrow_at = lds + kWAt + (step & 1) * kWStage + r * kWRow;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                wf[t][j] = dequant(cur.w[t][j >> 2][j & 3], zlo, zhi);
-            sc[t] = half_bits_to_float(cur.s[t]);
+            for (int i = 0; i < 2; ++i)
+                raw[t][i] = *reinterpret_cast<const u32x4*>(wrow_at + ((wk * 4 + h * 2 + i) ^ (l31 & 7)) * 16);
+            const int row = t ? row1 : row0;
+            const int al = t ? al1 : al0, s_at = scale_at(al, row, g) - scale_base(al, row, gb);
+            sc[t] = half_bits_to_float(
+                *reinterpret_cast<const uint16_t*>(lds + kSAt + (step & 1) * kSStage + r * 16 + (s_at & 15)));
+            z[t] = static_cast<float>(
+                (*reinterpret_cast<const uint32_t*>(lds + kZAt + (step & 1) * kZStage + r * 4) >> ((g & 7) * 4)) & 0xFu);
         }
-        // the weights are taken before anything new is requested: the compiler's own wait for them counts
-        // the loads it knows, and would otherwise wait for the fragments as well
-        __builtin_amdgcn_sched_barrier(0);
-        cur = next;
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the step's weights are in registers ...
+        __syncthreads();                    // ... of every wavefront, their slot is free
         load_x(step + 1);
-        load_raw(next, group_of(step + 2));
-        __builtin_amdgcn_sched_barrier(0);
+        load_w(step + 2);
         if (g < g_end) {
+            h8_t wf[2][8];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const _Float16 lo = static_cast<_Float16>(1024.0f + z[t]), hi = static_cast<_Float16>(-64.0f - z[t]);
+                const h2_t zlo = {lo, lo}, zhi = {hi, hi};
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    wf[t][j] = dequant(raw[t][j >> 2][j & 3], zlo, zhi);
+            }
             const char* xs = lds + (step & 1) * kStage + wk * MT * kBlockBytes + lane * 16;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
@@ -332,8 +398,9 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
                 }
             }
         }
-        // the fragments of the next step are there, only its successor's weights are still on their way
-        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        // the next step's fragments and weights are there, only its successor's weights are still on their way
+        asm volatile("" ::: "memory");
+        wait_for_all_but_the_next_weights();
         __syncthreads();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing may still write LDS
@@ -362,7 +429,7 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
                 v1 += *red_at(w, 1, i);
             }
             const int m = (mt0 + mt) * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (m >= a.M)
+            if (m >= a.M || !mine)
                 continue;
             if (EPI == EPI_QKV) {
                 // q and k are rounded to fp16 before RoPE reads them (native/rope_kernel.cu:14-26)
@@ -413,14 +480,15 @@ static int residual_splits(int M, int N, int groups)
 template <int MT, int WN, int WK, int EPI>
 void launch_gemm_as(GemmArgs& a, int pairs)
 {
+    a.pairs = pairs;
     a.nblocks = ceil_div(pairs, WN);
     const dim3 grid(ceil_div(a.nblocks * a.splits, 8) * 8 * a.mblocks);
     hipLaunchKernelGGL((prefill_gemm_kernel<MT, WN, WK, EPI>), grid, dim3(WN * WK * 64), 0, ctx().stream, a);
 }
 
 // 8 wavefronts in every case, two per SIMD, so that one's vector work runs under the other's products.
-// Four pairs of weight tiles per workgroup read the activations half as often as two; two pairs make
-// twice the workgroups where four would not give every compute unit one.
+// Blocks of 64 tokens and 256 weight rows; of 32 and 128 where there is one token tile or the large ones would occupy less
+// than half of the compute units (13B, 74 tokens: 51 us for SwiGLU on 216 large blocks, 60 on small ones).
 template <int EPI>
 int launch_gemm(const char* name, GemmArgs a, int pairs)
 {
@@ -428,11 +496,10 @@ int launch_gemm(const char* name, GemmArgs a, int pairs)
     a.mblocks = token_blocks(a.M);
     if (EPI != EPI_PARTIAL)
         a.splits = 1;
-    if (a.M <= kTile)
+    if (a.M <= kTile || ceil_div(pairs, 4) * a.mblocks * a.splits < cus / 2) {
+        a.mblocks = ceil_div(a.M, kTile);
         launch_gemm_as<1, 2, 4, EPI>(a, pairs);
-    else if (ceil_div(pairs, 4) * a.mblocks * a.splits < cus)
-        launch_gemm_as<2, 2, 4, EPI>(a, pairs);
-    else
+    } else
         launch_gemm_as<2, 4, 2, EPI>(a, pairs);
     L2_LAUNCH_CHECK(name);
     return LLAMA2_OK;

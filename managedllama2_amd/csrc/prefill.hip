@@ -12,12 +12,13 @@
 // the group's scale applied in fp32, fp32 sums over the groups; scores rounded to fp16, softmax
 // statistics and probabilities in fp32.  The order of the sums is not that of the decode step.
 //
-// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 21.0 ms;
-// 13B, 74 tokens behind 600 rows: 151 -> 11 ms.
+// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.5 ms;
+// 13B, 74 tokens behind 600 rows: 151 -> 9 ms.
 #include "int4_kernels.hpp"
 #include "prefill.hpp"
 
 #include <cmath>
+#include <type_traits>
 
 namespace l2 {
 
@@ -178,11 +179,7 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, int voff, 
                  : "memory", "m0");
 }
 
-// The same from an address per lane: 16 bytes to `lds` + 16 lane, 4 bytes to `lds` + 4 lane.
-__device__ __forceinline__ void load_to_lds_x4(const void* p, uint32_t lds)
-{
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(p) : "memory", "m0");
-}
+// The same from an address per lane, 4 bytes to `lds` + 4 lane.
 __device__ __forceinline__ void load_to_lds_x1(const void* p, uint32_t lds)
 {
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(p) : "memory", "m0");
@@ -192,31 +189,32 @@ __device__ __forceinline__ void load_to_lds_x1(const void* p, uint32_t lds)
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }
 
 // A workgroup owns MT token tiles and WN pairs of weight tiles of 32 rows; the two tiles of a pair hold
-// results that belong together (the two halves of a RoPE pair, gate and up, or neighbours) and stay in one
-// wavefront.  A step covers WK consecutive groups of K, one per wavefront of a pair; they add up through LDS at
-// the end.  The launch may split K further (EPI_PARTIAL).
+// results that belong together (the two halves of a RoPE pair, gate and up, or neighbours).  8 wavefronts: one per
+// weight tile and group, a step covers WK consecutive groups of K.  At the end the WK sums add up, and the tiles
+// of a pair meet, through LDS.  The launch may split K further (EPI_PARTIAL).
 //
-// What bounds it: the products of a group take MT x 512 cycles of a wavefront's matrix core, the
-// dequantisation and the scaling about as many of its vector unit.  The other limit is the rate at which a compute
-// unit looks up addresses: one per cycle and 64 contiguous bytes.  A lane that reads its own row's
-// weights, zero points and scales costs 64 lookups per load, 8 loads per wavefront and step, and made the
-// lookups the slowest part (61 % busy against 28 % of the matrix cores).  So everything comes through LDS,
-// requested in the order of memory: a weight row's 64 WK bytes by neighbouring lanes, a row's
-// scales and zero points of a step once for all WK groups.  Weights are requested two steps ahead (their slot is free
-// as soon as they are in registers, hence the barrier after the read), activations one.
+// What bounds it: a group costs a wavefront MT x 256 cycles of its matrix core (two wavefronts share one), about 400 of
+// its vector unit to unpack the weights and MT x 100 to scale the sums.  The rest has to stay out of the way:
+// - A compute unit looks up one cache address per cycle and 64 contiguous bytes.  A lane that reads its own row's
+//   weights costs 64 lookups per load (65 % busy against 28 % of the matrix cores, when it was done so).  Everything
+//   comes through LDS, requested in the order of memory; LDS delivers 256 bytes per cycle where 16 neighbouring
+//   lanes meet all banks, hence the swizzle of the weight rows.
+// - One barrier per step, LDS for three: activations are requested two steps ahead, weights three, because
+//   they are unpacked into registers a step ahead, each fragment under the last products that need its predecessor.
 template <int MT, int WN, int WK, int EPI>
-__global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(GemmArgs a)
+__global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
 {
-    constexpr int kStage = WK * MT * kBlockBytes;    // activations of a step
-    constexpr int kWRow = WK * 64;                   // bytes of a weight row per step
-    constexpr int kWStage = WN * 2 * kTile * kWRow;  // weights of a step
-    constexpr int kSStage = WN * 64 * 16, kZStage = WN * 64 * 4;
-    constexpr int kWAt = 2 * kStage, kSAt = kWAt + 2 * kWStage, kZAt = kSAt + 2 * kSStage, kAll = kZAt + 2 * kZStage;
-    constexpr int kRed = WK * WN * 2 * 16 * 64 * 4;
+    static_assert(WN * WK == 4, "8 wavefronts");
+    constexpr int kXStage = WK * MT * kBlockBytes;  // activations of a step
+    constexpr int kWRow = WK * 64;                  // bytes of a weight row per step
+    constexpr int kWStage = WN * 2 * kTile * kWRow; // weights of a step
+    constexpr int kZStage = 8 * 256;                // a word with the scale and one with the zero point per row and group
+    constexpr int kWAt = 3 * kXStage, kZAt = kWAt + 3 * kWStage, kAll = kZAt + 3 * kZStage;
+    constexpr int kRed = 8 * 16 * 64 * 4;
     static_assert(kAll <= 160 * 1024, "LDS of a compute unit");
     __shared__ __align__(1024) char lds[kAll > kRed ? kAll : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wn = wave % WN, wk = wave / WN;
+    const int t = wave & 1, wn = (wave >> 1) % WN, wk = (wave >> 1) / WN;
     const int h = lane >> 5, l31 = lane & 31;
     // The token blocks of one block of weights run on one XCD, next to each other in time: its L2
     // serves the weights to all but the first.
@@ -225,203 +223,188 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
     if (unit >= a.nblocks * a.splits)
         return;
     const int nb = unit / a.splits, split = unit - nb * a.splits;
-    // tensor and first row of tile t of a pair; the last block may have pairs to spare, which repeat the last one
-    auto tile_of = [&](int pair, int t, int& tensor, int& row) {
+    // tensor and first row of a tile; the last block may have pairs to spare, which repeat the last one
+    auto tile_of = [&](int pair, int tile, int& tensor, int& row) {
         pair = pair < a.pairs ? pair : a.pairs - 1;
         if (EPI == EPI_QKV) {
             const int per = a.N >> 6, r = pair % per;
             tensor = pair / per;
-            row = (r >> 1) * kRopeHeadSize + (r & 1) * kTile + t * 64;
+            row = (r >> 1) * kRopeHeadSize + (r & 1) * kTile + tile * 64;
         } else if (EPI == EPI_SWIGLU) {
-            tensor = t;
+            tensor = tile;
             row = pair * kTile;
         } else {
             tensor = 0;
-            row = (pair * 2 + t) * kTile;
+            row = (pair * 2 + tile) * kTile;
         }
     };
+    auto tensor_of = [&](int i) { return i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]); };
     auto rsrc_of = [](const void* p, uint32_t bytes) {
         const unsigned long long v = reinterpret_cast<unsigned long long>(p);
         return u32x4{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))),
                      static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))), bytes, 0x00020000u};
     };
-    const bool mine = nb * WN + wn < a.pairs;
-    int t0, t1, r0, r1;
-    tile_of(nb * WN + wn, 0, t0, r0);
-    tile_of(nb * WN + wn, 1, t1, r1);
-    const int row0 = r0 + l31 < a.N ? r0 + l31 : a.N - 1, row1 = r1 + l31 < a.N ? r1 + l31 : a.N - 1;
     const int mt0 = mb * MT, last_tile = (a.M - 1) / kTile;
-    // pieces of K begin at a multiple of 4 groups, so the groups of a step share a word of zero points
-    const int g_begin = (a.groups * split / a.splits) & ~3;
-    const int g_end = split + 1 == a.splits ? a.groups : (a.groups * (split + 1) / a.splits) & ~3;
+    const int g_begin = a.groups * split / a.splits, g_end = a.groups * (split + 1) / a.splits;
     const int steps = (g_end - g_begin + WK - 1) / WK;
-    auto base_of = [&](int step) { // first group; a step that does not exist is loaded as the last one and not used
-        return g_begin + (step < steps ? step : steps - 1) * WK;
+    // what does not exist is loaded as the last one that does, and not used
+    auto base_of = [&](int step) { return g_begin + (step < steps ? step : steps - 1) * WK; };
+    auto group_of = [&](int step) {
+        const int g = g_begin + step * WK + wk;
+        return g < g_end ? g : g_end - 1;
     };
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane(
         static_cast<int>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)lds)));
 
-    // Weights: this wavefront fetches 4 KB of the step, RPI rows per load.  Piece c of 16 bytes of row r lies in slot
-    // c ^ (r & 7) of the row, so the 8 rows that an LDS read takes at a time meet all banks.  Reads past
-    // the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet zeros of the input.
-    constexpr int LPR = WK * 4, RPI = 64 / LPR;
-    const int wr0 = wave * 4 * RPI; // first row of the block this wavefront fetches
-    int wt, wrow;
-    tile_of(nb * WN + wr0 / 64, (wr0 / kTile) & 1, wt, wrow);
-    wrow += (wr0 & (kTile - 1));
-    const u32x4 rw = rsrc_of(wt == 0 ? a.m[0].w : (wt == 1 ? a.m[1].w : a.m[2].w), static_cast<uint32_t>(a.N) * a.ws * 4);
-    int wvoff[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int r = i * RPI + lane / LPR, row = wrow + r < a.N ? wrow + r : a.N - 1;
-        wvoff[i] = row * a.ws * 4 + ((lane % LPR) ^ ((wr0 + r) & 7)) * 16;
-    }
-    // Scales and zero points of the pair's 64 rows, a lane's row in tile h: 16 bytes that hold the scales of
-    // the step's groups, and the word with their zero points.  Scales need not be aligned to more than their 2 bytes:
-    // offsets count from the word that holds the first one, and the 16 bytes begin at a word and end with the
-    // word that holds the last one.
-    const int szrow = h ? row1 : row0;
-    const QW q0 = a.m[t0], q1 = a.m[t1], qz = h ? q1 : q0;
-    const int al0 = static_cast<int>(reinterpret_cast<uintptr_t>(q0.s) & 2), al1 = static_cast<int>(reinterpret_cast<uintptr_t>(q1.s) & 2);
-    const int alz = h ? al1 : al0;
-    auto scale_at = [&](int al, int row, int g) { return al + (row * a.ss + g) * 2; };
-    auto scale_base = [&](int al, int row, int g) {
-        const int b = scale_at(al, row, g) & ~3, last = ((al + a.N * a.ss * 2 + 3) & ~3) - 16;
-        return b < last ? b : last;
-    };
+    // Activations: the fragments of this wavefront's group are shared by its 2 WN wavefronts.
     const u32x4 rx = rsrc_of(a.xf, a.xf_bytes);
-
-    constexpr int kWLoads = 4;
-    auto load_x = [&](int step) { // this wavefront's share of the fragments of its group
-        int g = base_of(step) + wk;
-        g = g < g_end ? g : g_end - 1;
-        const uint32_t dst = lds_base + (step & 1) * kStage + wk * MT * kBlockBytes;
+    constexpr int kXPer = 8 / (2 * WN);
+    auto load_x = [&](int step, int at) {
+        const int g = group_of(step);
+        const uint32_t dst = lds_base + at * kXStage + wk * MT * kBlockBytes;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int tile = mt0 + mt <= last_tile ? mt0 + mt : last_tile; // the last block may have tiles to spare
 #pragma unroll
-            for (int j = 0; j < 8 / WN; ++j) {
-                const int f = wn * (8 / WN) + j;
+            for (int j = 0; j < kXPer; ++j) {
+                const int f = (wave % (2 * WN)) * kXPer + j;
                 load_to_lds(rx, dst + mt * kBlockBytes + f * kFragBytes, lane * 16,
                             (tile * a.groups + g) * kBlockBytes + f * kFragBytes);
             }
         }
     };
-    // Scales by the wavefronts of the step's first group, zero points by those of the second.  Whole addresses per
-    // lane: the two tiles may belong to two tensors.  All of them lie inside their tensors.
-    auto load_sz = [&](int step, int g) {
-        const uint32_t slot_at = step & 1;
-        if (wk == 0)
-            load_to_lds_x4(reinterpret_cast<const char*>(qz.s) - alz + scale_base(alz, szrow, g),
-                           lds_base + kSAt + slot_at * kSStage + wn * 1024);
-        else if (wk == 1)
-            load_to_lds_x1(qz.z + static_cast<size_t>(szrow) * a.zs + (g >> 3),
-                           lds_base + kZAt + slot_at * kZStage + wn * 256);
-    };
-    auto load_w = [&](int step) {
-        const int g = base_of(step);
-        const uint32_t dst = lds_base + kWAt + (step & 1) * kWStage + wr0 * kWRow;
+    // Weights: this wavefront fetches 2 KB of the step, RPI rows per load.  Piece c of 16 bytes of row r lies in
+    // place c ^ swizzle(r) of the row: 16 neighbouring rows put the same piece into 16 different 16-byte columns.
+    // Reads past the end of a tensor return 0; those past the end of a row (K not a multiple of 128) meet
+    // zeros of the input.
+    constexpr int LPR = WK * 4, RPI = 64 / LPR;
+    auto swizzle = [](int r) { return (r / (256 / kWRow)) & (LPR - 1); };
+    const int wr0 = wave * 2 * RPI; // first row of the block this wavefront fetches
+    int wt, wrow;
+    tile_of(nb * WN + wr0 / 64, (wr0 / kTile) & 1, wt, wrow);
+    wrow += wr0 & (kTile - 1);
+    const u32x4 rw = rsrc_of(tensor_of(wt).w, static_cast<uint32_t>(a.N) * a.ws * 4);
+    int wvoff[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            load_to_lds(rw, dst + i * kFragBytes, wvoff[i], g * 64);
-        load_sz(step, g);
+    for (int i = 0; i < 2; ++i) {
+        const int r = i * RPI + lane / LPR, row = wrow + r < a.N ? wrow + r : a.N - 1;
+        wvoff[i] = row * a.ws * 4 + ((lane % LPR) ^ swizzle(wr0 + r)) * 16;
+    }
+    // Scales and zero points of this wavefront's tile and group, by the two halves of the lanes.  Scales need not be
+    // aligned to more than their 2 bytes: the word that holds one is fetched.
+    int tensor, r0;
+    tile_of(nb * WN + wn, t, tensor, r0);
+    const int row = r0 + l31 < a.N ? r0 + l31 : a.N - 1;
+    const QW q = tensor_of(tensor);
+    const int s_odd = static_cast<int>(reinterpret_cast<uintptr_t>(q.s) & 2) + row * a.ss * 2; // from the first word
+    const char* zs_base = h ? reinterpret_cast<const char*>(q.z + static_cast<size_t>(row) * a.zs)
+                            : reinterpret_cast<const char*>(reinterpret_cast<uintptr_t>(q.s) & ~static_cast<uintptr_t>(2));
+    auto load_w = [&](int step, int at) {
+        const int gb = base_of(step), g = group_of(step);
+        const uint32_t dst = lds_base + kWAt + at * kWStage + wr0 * kWRow;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            load_to_lds(rw, dst + i * kFragBytes, wvoff[i], gb * 64);
+        load_to_lds_x1(zs_base + (h ? (g >> 3) * 4 : (s_odd + 2 * g) & ~3), lds_base + kZAt + at * kZStage + wave * 256);
     };
 
-    f16v_t acc[MT][2];
+    f16v_t acc[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
+        acc[mt] = f16v_t{};
+    u32x4 raw[2];
+    h8_t wf[8]; // the current group's weights, n - z in fp16
+    h2_t zlo, zhi;
+    float sc = 0.0f, sc_next = 0.0f;
+    auto read_w = [&](int step, int at) {
+        const int r = (wn * 2 + t) * kTile + l31, g = group_of(step);
+        const char* from = lds + kWAt + at * kWStage + r * kWRow;
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                acc[mt][t][i] = 0.0f;
-
-    load_w(0);
-    load_x(0);
-    load_w(1);
-    // wk < 2 fetch scales or zero points as well
-    auto wait_for_all_but_the_next_weights = [&] {
-        if (WK == 2 || wk < 2)
-            __builtin_amdgcn_s_waitcnt(wait_vm(kWLoads + 1));
-        else
-            __builtin_amdgcn_s_waitcnt(wait_vm(kWLoads));
+        for (int i = 0; i < 2; ++i)
+            raw[i] = *reinterpret_cast<const u32x4*>(from + ((wk * 4 + h * 2 + i) ^ swizzle(r)) * 16);
+        const char* sz = lds + kZAt + at * kZStage + wave * 256 + l31 * 4;
+        sc_next = half_bits_to_float(*reinterpret_cast<const uint16_t*>(sz + ((s_odd + 2 * g) & 2)));
+        const float z = static_cast<float>((*reinterpret_cast<const uint32_t*>(sz + 128) >> ((g & 7) * 4)) & 0xFu);
+        const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
+        zlo = h2_t{lo, lo}, zhi = h2_t{hi, hi};
     };
-    asm volatile("" ::: "memory");
-    wait_for_all_but_the_next_weights();
+    constexpr int kLoads = MT * kXPer + 3; // of a step
+    auto wait_all_but = [](auto n) {
+        __builtin_amdgcn_s_waitcnt(wait_vm(decltype(n)::value));
+        asm volatile("" ::: "memory");
+    };
+    load_w(0, 0);
+    load_x(0, 0);
+    load_w(1, 1);
+    load_x(1, 1);
+    load_w(2, 2);
+    wait_all_but(std::integral_constant<int, 2 * kLoads>{});
     __syncthreads();
+    read_w(0, 0);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        wf[j] = dequant(raw[j >> 2][j & 3], zlo, zhi);
+    int s0 = 0, s1 = 1, s2 = 2; // LDS of this step, the next and the one after it
     for (int step = 0; step < steps; ++step) {
-        const int gb = g_begin + step * WK, g = gb + wk;
-        u32x4 raw[2][2];
-        float z[2], sc[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int r = wn * 64 + t * kTile + l31;
-            const char* wrow_at = lds + kWAt + (step & 1) * kWStage + r * kWRow;
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                raw[t][i] = *reinterpret_cast<const u32x4*>(wrow_at + ((wk * 4 + h * 2 + i) ^ (l31 & 7)) * 16);
-            const int row = t ? row1 : row0;
-            const int al = t ? al1 : al0, s_at = scale_at(al, row, g) - scale_base(al, row, gb);
-            sc[t] = half_bits_to_float(
-                *reinterpret_cast<const uint16_t*>(lds + kSAt + (step & 1) * kSStage + r * 16 + (s_at & 15)));
-            z[t] = static_cast<float>(
-                (*reinterpret_cast<const uint32_t*>(lds + kZAt + (step & 1) * kZStage + r * 4) >> ((g & 7) * 4)) & 0xFu);
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): the step's weights are in registers ...
-        __syncthreads();                    // ... of every wavefront, their slot is free
-        load_x(step + 1);
-        load_w(step + 2);
-        if (g < g_end) {
-            h8_t wf[2][8];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const _Float16 lo = static_cast<_Float16>(1024.0f + z[t]), hi = static_cast<_Float16>(-64.0f - z[t]);
-                const h2_t zlo = {lo, lo}, zhi = {hi, hi};
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    wf[t][j] = dequant(raw[t][j >> 2][j & 3], zlo, zhi);
-            }
-            const char* xs = lds + (step & 1) * kStage + wk * MT * kBlockBytes + lane * 16;
+        // this step's activations and the next one's weights; every wavefront is through with the step before
+        wait_all_but(std::integral_constant<int, kLoads>{});
+        __syncthreads();
+        load_x(step + 2, s2);
+        load_w(step + 3, s0);
+        sc = sc_next;
+        read_w(step + 1, s1);
+        if (g_begin + step * WK + wk < g_end) {
+            const char* xs = lds + s0 * kXStage + wk * MT * kBlockBytes + lane * 16;
+            f16v_t p[MT];
+            h8_t xa[2][MT];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                f16v_t p0 = {}, p1 = {};
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const h8_t xa = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes + j * kFragBytes);
-                    p0 = mfma(xa, wf[0][j], p0);
-                    p1 = mfma(xa, wf[1][j], p1);
-                }
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    acc[mt][0][i] = __builtin_fmaf(p0[i], sc[0], acc[mt][0][i]);
-                    acc[mt][1][i] = __builtin_fmaf(p1[i], sc[1], acc[mt][1][i]);
-                }
+                p[mt] = f16v_t{};
+                xa[0][mt] = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes);
             }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (j + 1 < 8) {
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt)
+                        xa[(j + 1) & 1][mt] = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes + (j + 1) * kFragBytes);
+                }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    p[mt] = mfma(xa[j & 1][mt], wf[j], p[mt]);
+                wf[j] = dequant(raw[j >> 2][j & 3], zlo, zhi);
+                __builtin_amdgcn_sched_barrier(0x2); // vector arithmetic alone may move
+            }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    acc[mt][i] = __builtin_fmaf(p[mt][i], sc, acc[mt][i]);
         }
-        // the next step's fragments and weights are there, only its successor's weights are still on their way
-        asm volatile("" ::: "memory");
-        wait_for_all_but_the_next_weights();
-        __syncthreads();
+        const int s = s0;
+        s0 = s1, s1 = s2, s2 = s;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing may still write LDS
     __syncthreads();
 
-    constexpr int SHARE = 16 / WK; // accumulator registers a wavefront adds up per tile
+    constexpr int SHARE = 16 / (2 * WK); // registers of both tiles that a wavefront adds up
+    const bool mine = nb * WN + wn < a.pairs;
+    int tensor0, row_a, row_b;
+    tile_of(nb * WN + wn, 1, tensor0, row_b);
+    tile_of(nb * WN + wn, 0, tensor0, row_a);
     float* red = reinterpret_cast<float*>(lds);
-    auto red_at = [&](int w, int t, int i) { return red + (((w * WN + wn) * 2 + t) * 16 + i) * 64 + lane; };
+    auto red_at = [&](int w, int tile, int i) { return red + (((w * WN + wn) * 2 + tile) * 16 + i) * 64 + lane; };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         if (mt)
             __syncthreads();
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                *red_at(wk, t, i) = acc[mt][t][i];
+        for (int i = 0; i < 16; ++i)
+            *red_at(wk, t, i) = acc[mt][i];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < SHARE; ++u) {
-            const int i = wk * SHARE + u;
+            const int i = (wk * 2 + t) * SHARE + u;
             float v0 = 0.0f, v1 = 0.0f;
 #pragma unroll
             for (int w = 0; w < WK; ++w) {
@@ -434,20 +417,20 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
             if (EPI == EPI_QKV) {
                 // q and k are rounded to fp16 before RoPE reads them (native/rope_kernel.cu:14-26)
                 uint16_t b0 = float_to_half_bits(v0), b1 = float_to_half_bits(v1);
-                if (t0 < 2) {
-                    const int idx = (r0 & 63) + l31;
+                if (tensor0 < 2) {
+                    const int idx = (row_a & 63) + l31;
                     const float* cs = a.rope + (static_cast<size_t>(m) * 64 + idx) * 2;
                     rope_rotate(b0, b1, half_bits_to_float(b0), half_bits_to_float(b1), cs[0], cs[1]);
                 }
-                uint16_t* o = a.out[t0] + static_cast<size_t>(m) * a.N;
-                o[r0 + l31] = b0;
-                o[r1 + l31] = b1;
+                uint16_t* o = a.out[tensor0] + static_cast<size_t>(m) * a.N;
+                o[row_a + l31] = b0;
+                o[row_b + l31] = b1;
             } else if (EPI == EPI_PARTIAL) {
                 float* o = a.parts + (static_cast<size_t>(split) * a.part_rows + m) * a.N;
-                o[r0 + l31] = v0;
-                o[r1 + l31] = v1;
+                o[row_a + l31] = v0;
+                o[row_b + l31] = v1;
             } else {
-                const int n = r0 + l31;
+                const int n = row_a + l31;
                 if (n < a.N) {
                     float v = v0;
                     v *= 1.0f / (1.0f + expf(-v)); // native/mat_vec_kernel.cu:219-221
@@ -461,46 +444,70 @@ __global__ __launch_bounds__(WN* WK * 64, WN* WK / 4) void prefill_gemm_kernel(G
     }
 }
 
-// Two token tiles per workgroup (one for batches of one tile).
-static int token_blocks(int M) { return M <= kTile ? 1 : ceil_div(M, 2 * kTile); }
+// How a product is cut up: MT token tiles and WN pairs of weight tiles per workgroup, WK groups per step, and
+// pieces of K per launch.
+struct GemmShape {
+    int mt, wn, splits;
+};
 
 constexpr int kMaxSplits = 8;
 
-// Pieces of K of a residual product: as many as it takes to give every compute unit a workgroup, each
-// with at least 4 groups.
-static int residual_splits(int M, int N, int groups)
+// The cheapest of the shapes that fit into LDS, by an estimate in cycles: workgroups run one per compute unit in
+// rounds of equal length, a round is its steps plus filling and draining the pipeline, and every piece of K
+// beyond the first costs the norm that adds them up another reading (about 1024 values per cycle).
+// A step measured 2900 cycles with two token tiles (7B SwiGLU, 511 rows: 3 rounds of 32 steps in 121 us) and
+// 5000 with four (QKV: one round of 32 steps in 72 us); the others lie on the same line; several groups per step
+// (more activations per result) add 400 (two tiles, 7B QKV, 511 rows: 3 rounds of 16 steps in 78 us; 13B, 74 rows:
+// one of 20 in 31).  What the choice gives, against blocks of 64 tokens by 256 weight rows for every size: 7B, 511 rows, QKV 86 -> 76 us (192 workgroups in one round
+// instead of 384 in two), down-proj 66 -> 54; 13B, 74 rows, QKV 42 -> 32.
+static GemmShape gemm_shape(int tiles, int pairs, int groups, bool may_split)
 {
-    const int blocks = token_blocks(M) * ceil_div(N, 256);
+    static constexpr int kStepCycles[5] = {0, 1900, 2900, 3950, 5000};
+    static constexpr int kFixed = 8000, kWideStep = 400;
     const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    int s = cus / blocks;
-    s = s < groups / 4 ? s : groups / 4;
-    return s < 1 ? 1 : (s < kMaxSplits ? s : kMaxSplits);
+    GemmShape best{};
+    long long least = -1;
+    for (int wn = 4; wn >= 1; wn /= 2)
+        for (int mt = wn; mt >= 1; --mt)
+            for (int splits = 1; splits <= (may_split ? kMaxSplits : 1) && (splits == 1 || splits * 4 <= groups); ++splits) {
+                const int wk = 4 / wn;
+                const long long units = static_cast<long long>(ceil_div(tiles, mt)) * ceil_div(pairs, wn) * splits;
+                const int steps = ceil_div(ceil_div(groups, splits), wk);
+                const long long step = kStepCycles[mt] + (wk > 1 ? kWideStep : 0);
+                const long long cost = (units + cus - 1) / cus * (steps * step + kFixed) +
+                                       static_cast<long long>(splits - 1) * tiles * kTile * pairs * 64 / 1024;
+                if (least < 0 || cost < least)
+                    least = cost, best = GemmShape{mt, wn, splits};
+            }
+    return best;
 }
 
-template <int MT, int WN, int WK, int EPI>
-void launch_gemm_as(GemmArgs& a, int pairs)
+static GemmShape residual_shape(int M, int N, int groups) { return gemm_shape(ceil_div(M, kTile), N / 64, groups, true); }
+
+template <int MT, int WN, int EPI>
+void launch_gemm_as(GemmArgs& a)
 {
-    a.pairs = pairs;
-    a.nblocks = ceil_div(pairs, WN);
+    a.mblocks = ceil_div(a.M, MT * kTile);
+    a.nblocks = ceil_div(a.pairs, WN);
     const dim3 grid(ceil_div(a.nblocks * a.splits, 8) * 8 * a.mblocks);
-    hipLaunchKernelGGL((prefill_gemm_kernel<MT, WN, WK, EPI>), grid, dim3(WN * WK * 64), 0, ctx().stream, a);
+    hipLaunchKernelGGL((prefill_gemm_kernel<MT, WN, 4 / WN, EPI>), grid, dim3(512), 0, ctx().stream, a);
 }
 
-// 8 wavefronts in every case, two per SIMD, so that one's vector work runs under the other's products.
-// Blocks of 64 tokens and 256 weight rows; of 32 and 128 where there is one token tile or the large ones would occupy less
-// than half of the compute units (13B, 74 tokens: 51 us for SwiGLU on 216 large blocks, 60 on small ones).
 template <int EPI>
 int launch_gemm(const char* name, GemmArgs a, int pairs)
 {
-    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
-    a.mblocks = token_blocks(a.M);
-    if (EPI != EPI_PARTIAL)
-        a.splits = 1;
-    if (a.M <= kTile || ceil_div(pairs, 4) * a.mblocks * a.splits < cus / 2) {
-        a.mblocks = ceil_div(a.M, kTile);
-        launch_gemm_as<1, 2, 4, EPI>(a, pairs);
-    } else
-        launch_gemm_as<2, 4, 2, EPI>(a, pairs);
+    const GemmShape s = gemm_shape(ceil_div(a.M, kTile), pairs, a.groups, EPI == EPI_PARTIAL);
+    a.pairs = pairs;
+    a.splits = s.splits;
+    switch (s.wn * 10 + s.mt) {
+    case 44: launch_gemm_as<4, 4, EPI>(a); break;
+    case 43: launch_gemm_as<3, 4, EPI>(a); break;
+    case 42: launch_gemm_as<2, 4, EPI>(a); break;
+    case 41: launch_gemm_as<1, 4, EPI>(a); break;
+    case 22: launch_gemm_as<2, 2, EPI>(a); break;
+    case 21: launch_gemm_as<1, 2, EPI>(a); break;
+    default: launch_gemm_as<1, 1, EPI>(a); break;
+    }
     L2_LAUNCH_CHECK(name);
     return LLAMA2_OK;
 }
@@ -772,7 +779,7 @@ int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
     size_t parts = 0; // the largest [splits][rows][dim] any batch needs
     for (int m = kTile; m <= rows; m += kTile)
         for (int k : {cfg.dim, cfg.hidden_dim}) {
-            const size_t n = static_cast<size_t>(residual_splits(m, cfg.dim, ceil_div(k, kGroup))) * m;
+            const size_t n = static_cast<size_t>(residual_shape(m, cfg.dim, ceil_div(k, kGroup)).splits) * m;
             parts = n > parts ? n : parts;
         }
     parts *= static_cast<size_t>(cfg.dim) * sizeof(float);
@@ -815,7 +822,7 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
     const uint32_t xf_bytes = static_cast<uint32_t>(ws.rows) * ss * kGroup * 2;
     const uint32_t hf_bytes = static_cast<uint32_t>(ws.rows) * hss * kGroup * 2;
     const int part_rows = ceil_div(M, kTile) * kTile;
-    const int o_splits = residual_splits(M, dim, ss), down_splits = residual_splits(M, dim, hss);
+    const int o_splits = residual_shape(M, dim, ss).splits, down_splits = residual_shape(M, dim, hss).splits;
     auto qw = [](const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; };
     hipLaunchKernelGGL(prefill_rope_kernel, dim3(ceil_div(M * 64, 256)), dim3(256), 0, ctx().stream, ws.rope, position,
                        M, c.rope_theta);
@@ -851,7 +858,7 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
         }
         {
             GemmArgs a{};
-            a.m[0] = qw(L.output), a.parts = ws.parts, a.part_rows = part_rows, a.splits = o_splits, a.xf = ws.xf, a.xf_bytes = xf_bytes;
+            a.m[0] = qw(L.output), a.parts = ws.parts, a.part_rows = part_rows, a.xf = ws.xf, a.xf_bytes = xf_bytes;
             a.groups = ss, a.N = dim, a.ws = wsz, a.ss = ss, a.zs = zs, a.M = M;
             L2_TRY(launch_gemm<EPI_PARTIAL>("prefill o-proj", a, dim / 64));
         }
@@ -866,7 +873,7 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
         }
         {
             GemmArgs a{};
-            a.m[0] = qw(L.down), a.parts = ws.parts, a.part_rows = part_rows, a.splits = down_splits, a.xf = ws.hf, a.xf_bytes = hf_bytes;
+            a.m[0] = qw(L.down), a.parts = ws.parts, a.part_rows = part_rows, a.xf = ws.hf, a.xf_bytes = hf_bytes;
             a.groups = hss, a.N = dim, a.ws = hws, a.ss = hss, a.zs = hzs, a.M = M;
             L2_TRY(launch_gemm<EPI_PARTIAL>("prefill down-proj", a, dim / 64));
         }

@@ -142,3 +142,26 @@ def test_captured_prompt_replays():
         t.Forward(51, 52)  # the decoder's own path between the replays
     capi.call("llama2_graph_destroy", g)
     t.close()
+
+
+# Widths at which the products take the larger blocks: 1 to 4 token tiles and 1, 2 or 4 pairs of weight tiles per
+# workgroup, K in up to 4 pieces; the pairs of a width that is an odd multiple of 128 do not fill the last block
+@pytest.mark.parametrize("dim,hidden,known", [(1408, 328, 131), (2176, 648, 301), (2176, 648, 601), (1408, 328, 1004),
+                                              (2176, 648, 1004)])
+def test_wide_prompt_blocks(dim, hidden, known):
+    cfg = config(dim, hidden, 2, known + 1)
+    model = synth.random_model(cfg, seed=65, rms_random=True)
+    prompt = synth.rng_for(805, known).integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run", t._decoder, 0, known, known)
+    for g, w in zip(caches(t, cfg, known), caches(ref, cfg, known)):
+        for layer in range(cfg["n_layers"]):
+            want = w[layer].astype(np.float64)
+            # two orders of the same fp32 sums, each rounded to fp16 (2^-11) between the modules
+            assert np.linalg.norm(g[layer] - want) <= 4e-3 * np.linalg.norm(want), layer
+            assert_close_normwise(g[layer].ravel(), want.ravel(), "cache", TOL)
+    assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
+    for tr in (t, ref):
+        tr.close()

@@ -431,7 +431,7 @@ float llama2_sampler_coin(unsigned long long seed, int position);
  * positions below n_prompt keep their prompt token, as Transformer.Generate
  * does, src/Transformer.cs:96-104).  Does not stop on token < 3.  A fused
  * decoder sends all but the last of the known tokens through the layers in
- * batches when there are at least 16 of them: the same cache rows up to the
+ * batches when those are at least 8: the same cache rows up to the
  * order of the fp32 sums. */
 int llama2_decode_run(llama2_decoder* decoder, int position, int steps, int n_prompt);
 /* The same loop with the stochastic sampler: the token at next_position p is

@@ -9,9 +9,12 @@
 namespace l2 {
 
 constexpr int kPrefillMaxRows = 1024; // tokens per batch; longer prompts go through in batches of equal size
-// Fewer known tokens take the decode step one by one: up to half of a matrix tile would be padding, and the
-// short prompts keep the decode step's sums bit for bit.
-constexpr int kPrefillMinRows = 16;
+// Fewer known tokens take the decode step one by one.  A batch of one token tile costs about as much as three
+// steps and the same for 8 rows as for 32.  8 rows and the step after them, against 9 steps: 7B 3.37 ms (9.32),
+// behind 600 rows 4.70 (10.28), behind 3500 rows 11.1 (12.9); 13B 5.54 (16.8); a 2-layer model of width 256
+// 0.11 (0.42).  Below that the gain shrinks and is gone behind a long history, and prompts of a few tokens keep
+// the decode step's sums bit for bit.
+constexpr int kPrefillMinRows = 8;
 
 struct PrefillWorkspace {
     uint16_t* x = nullptr;    // residual stream, [rows][dim]

@@ -1,7 +1,7 @@
 """The batched prompt of the device-resident loop (prefill.hip) against the fp64 oracle, token by token.
 
-llama2_decode_run sends all but the last of the known tokens through the layers in batches when there are
-at least 16 of them; their only results are rows of the key and value caches, which every later step
+llama2_decode_run sends all but the last of the known tokens through the layers in batches when those are
+at least 8; their only results are rows of the key and value caches, which every later step
 attends, so the caches and the first logits are compared.  Both paths round the same quantities to fp16 and
 sum in fp32, in other orders, so over a whole cache (thousands of values) their 2-norm distances from the
 oracle are two samples of the same error: the batch may be 1.5 times as far off as single steps, plus a tenth
@@ -70,6 +70,29 @@ def test_prompt_fills_the_caches(oracle, dim, hidden, known):
     token = int(t.runstate.tokens.to_host(1, known)[0])
     assert token == int(np.argmax(t.runstate.logits.to_host()))
     assert np.array_equal(t.runstate.tokens.to_host(known), prompt)
+    for tr in (t, ref):
+        tr.close()
+
+
+# The smallest batches: most of the one token tile is padding.  One known token fewer goes step by step, bit for bit.
+@pytest.mark.parametrize("dim,hidden", [(128, 136), (384, 1000), (2176, 648)])
+def test_shortest_batches(dim, hidden):
+    cfg = config(dim, hidden, 2, 20)
+    model = synth.random_model(cfg, seed=66, rms_random=True)
+    prompt = synth.rng_for(806, dim).integers(3, 512, 16).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    for known in (8, 9, 12, 15, 16):
+        t.runstate.tokens.copy_to_device(prompt)
+        capi.call("llama2_decode_run", t._decoder, 0, known, known)
+        for g, w in zip(caches(t, cfg, known), caches(ref, cfg, known)):
+            if known == 8:
+                assert np.array_equal(g.view(np.uint16), w.view(np.uint16))
+            for layer in range(cfg["n_layers"]):
+                want = w[layer].astype(np.float64)
+                # as in test_wide_prompt_blocks
+                assert np.linalg.norm(g[layer] - want) <= 4e-3 * np.linalg.norm(want), (known, layer)
+    assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
     for tr in (t, ref):
         tr.close()
 

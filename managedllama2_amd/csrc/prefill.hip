@@ -518,7 +518,8 @@ struct PrefillAttnArgs {
     const uint16_t* kcache;
     const uint16_t* vcache; // layer base, rows of `dim`
     uint16_t* xf;
-    int position, M, dim, n_heads;
+    float* parts; // SPLIT: [splits][n_heads][part_rows][128] sums, then (maximum, sum) of every row
+    int position, M, dim, n_heads, splits, part_rows;
     float scale;
 };
 
@@ -556,7 +557,13 @@ __device__ __forceinline__ void one_by_one(f16v_t (&o)[4], h8_t hi, h8_t lo, con
 // timesteps of ONE query and its probabilities are already the second operand of the product with the
 // transposed values.  Probabilities keep fp32's precision: each is scaled by 2^14 and split into two fp16
 // numbers that go through the matrix cores one after the other (22 bits; below 2^-17 an absolute 2^-39).
-template <int NW>
+//
+// What bounds it: a pass of 64 timesteps is a chain (LDS filled, scores, maximum, probabilities, output) of 4 us
+// when its compute unit holds little else, and a tile walks all its passes.  SPLIT: gridDim.z workgroups share the
+// passes of a tile, and prefill_attn_merge_kernel adds up their fp32 sums, which lie in the L2 in between.
+// 7B, whole prompt in front of the first token, unsplit -> split: 75 tokens behind 3500 rows 12.9 -> 6.8 ms, behind
+// 600 rows 6.57 -> 5.75; 9 tokens behind 3500 rows 11.1 -> 4.7; 512 tokens 11.8 -> 11.6.
+template <int NW, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a)
 {
     __shared__ __align__(16) char ks[kAttnT * kKStride];
@@ -609,8 +616,12 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
                     rv, ((tb + 4 * u + r) * a.dim + head * kRopeHeadSize + (e & 15) * 8) * 2, 0, 0);
         }
     };
-    request(0);
-    for (int tb = 0; tb < t_end; tb += kAttnT) {
+    const int passes = (t_end + kAttnT - 1) / kAttnT;
+    const int t_first = SPLIT ? passes * static_cast<int>(blockIdx.z) / a.splits * kAttnT : 0;
+    const int t_last = SPLIT ? passes * (static_cast<int>(blockIdx.z) + 1) / a.splits * kAttnT : passes * kAttnT;
+    if (t_first < t_last)
+        request(t_first);
+    for (int tb = t_first; tb < t_last; tb += kAttnT) {
         __syncthreads(); // the previous pass has been read
 #pragma unroll
         for (int i = 0; i < KP; ++i) {
@@ -632,7 +643,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
             }
         }
         __syncthreads();
-        if (tb + kAttnT < t_end)
+        if (tb + kAttnT < t_last)
             request(tb + kAttnT);
         if (tb > wave_limit)
             continue; // this tile attends nothing here (the barriers are the same for all wavefronts)
@@ -672,8 +683,11 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
                 bm = fmaxf(bm, s[tt][i]);
             }
         bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
-        const float nm = fmaxf(mx, bm); // finite: timestep 0 is in the first pass
-        const float alpha = expf(mx - nm);
+        const float nm = fmaxf(mx, bm);
+        // a query may attend none of a SPLIT's timesteps so far: its probabilities are 0, not NaN (otherwise
+        // timestep 0 is in the first pass)
+        const float base = SPLIT && nm == -INFINITY ? 0.0f : nm;
+        const float alpha = expf(mx - base);
         mx = nm;
         sum *= alpha;
 #pragma unroll
@@ -688,7 +702,7 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
                 h8_t hi, lo;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const float p = expf(s[tt][8 * j + i] - mx);
+                    const float p = expf(s[tt][8 * j + i] - base);
                     sum += p;
                     const float ps = p * kProbScale;
                     hi[i] = static_cast<_Float16>(ps);
@@ -711,6 +725,20 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
     const float inv = 1.0f / kProbScale;
     if (tile * kTile >= a.M) // the whole wavefront
         return;
+    if constexpr (SPLIT) {
+        const size_t row = (static_cast<size_t>(blockIdx.z) * a.n_heads + head) * a.part_rows + m;
+        float* out = a.parts + row * kRopeHeadSize + 4 * hl;
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                *reinterpret_cast<float4*>(out + d * 32 + 8 * k) =
+                    float4{o[d][4 * k] * inv, o[d][4 * k + 1] * inv, o[d][4 * k + 2] * inv, o[d][4 * k + 3] * inv};
+        float* stats = a.parts + static_cast<size_t>(a.splits) * a.n_heads * a.part_rows * kRopeHeadSize;
+        if (hl == 0)
+            *reinterpret_cast<float2*>(stats + row * 2) = float2{mx, sum};
+        return;
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d)
 #pragma unroll
@@ -739,17 +767,87 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
         }
 }
 
-int launch_prefill_attn(const PrefillAttnArgs& a)
+// Adds up the pieces of a split attention, 16 lanes of 8 outputs per row and head.
+__global__ __launch_bounds__(256) void prefill_attn_merge_kernel(PrefillAttnArgs a)
 {
-    const int tiles = ceil_div(a.M, kTile);
-    const hipStream_t st = ctx().stream;
-    if (ceil_div(tiles, 4) * a.n_heads >= ctx().num_cus)
-        hipLaunchKernelGGL((prefill_attn_kernel<4>), dim3(ceil_div(tiles, 4), a.n_heads), dim3(256), 0, st, a);
-    else if (ceil_div(tiles, 2) * a.n_heads >= ctx().num_cus)
-        hipLaunchKernelGGL((prefill_attn_kernel<2>), dim3(ceil_div(tiles, 2), a.n_heads), dim3(128), 0, st, a);
+    const int m = blockIdx.x * 16 + (threadIdx.x >> 4), head = blockIdx.y, k = (threadIdx.x & 15) * 8;
+    if (m >= a.M)
+        return;
+    const size_t step = static_cast<size_t>(a.n_heads) * a.part_rows, row = static_cast<size_t>(head) * a.part_rows + m;
+    const float2* stats = reinterpret_cast<const float2*>(a.parts + a.splits * step * kRopeHeadSize) + row;
+    float mx = -INFINITY;
+    for (int i = 0; i < a.splits; ++i)
+        mx = fmaxf(mx, stats[i * step].x);
+    float o[8] = {}, sum = 0.0f;
+    for (int i = 0; i < a.splits; ++i) { // in order: deterministic
+        const float2 st = stats[i * step];
+        const float w = st.x == -INFINITY ? 0.0f : expf(st.x - mx); // a piece the row does not attend
+        const float4* p = reinterpret_cast<const float4*>(a.parts + (i * step + row) * kRopeHeadSize + k);
+        const float4 p0 = p[0], p1 = p[1];
+        sum = fmaf(w, st.y, sum);
+        o[0] = fmaf(w, p0.x, o[0]), o[1] = fmaf(w, p0.y, o[1]), o[2] = fmaf(w, p0.z, o[2]), o[3] = fmaf(w, p0.w, o[3]);
+        o[4] = fmaf(w, p1.x, o[4]), o[5] = fmaf(w, p1.y, o[5]), o[6] = fmaf(w, p1.z, o[6]), o[7] = fmaf(w, p1.w, o[7]);
+    }
+    u32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        v[e] = static_cast<uint32_t>(float_to_half_bits(o[2 * e] / sum)) |
+               static_cast<uint32_t>(float_to_half_bits(o[2 * e + 1] / sum)) << 16;
+    *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(a.xf) + frag_offset(m, head * kRopeHeadSize + k, a.n_heads)) =
+        frag_order(v);
+}
+
+struct PrefillAttnShape {
+    int waves, splits;
+};
+
+constexpr int kMaxAttnSplits = 32;
+
+// Tiles share key and value rows (waves) as long as every compute unit has a workgroup.  Passes are split until there
+// are 4 wavefronts per compute unit; more only costs the merge (7B: 512 tokens, 1024 wavefronts 11.62 ms, 2048
+// 11.91; 1003 tokens, 1024 wavefronts 19.3, 2048 19.6; 400 behind 3500 rows, 416 wavefronts 18.7, 832 15.0).
+// A piece may be a single pass: 20 tokens behind 200 rows 3.55 ms, with two passes at least 3.65, unsplit 3.89.
+static PrefillAttnShape prefill_attn_shape(int M, int rows, int n_heads)
+{
+    const int tiles = ceil_div(M, kTile), passes = ceil_div(rows, kAttnT);
+    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    const int waves = ceil_div(tiles, 4) * n_heads >= cus ? 4 : ceil_div(tiles, 2) * n_heads >= cus ? 2 : 1;
+    int splits = 4 * cus / (tiles * n_heads);
+    splits = splits < passes ? splits : passes;
+    splits = splits < kMaxAttnSplits ? splits : kMaxAttnSplits;
+    return PrefillAttnShape{waves, splits > 1 ? splits : 1};
+}
+
+static size_t attn_part_floats(int M, int splits, int n_heads)
+{
+    return splits > 1 ? static_cast<size_t>(splits) * n_heads * ceil_div(M, kTile) * kTile * (kRopeHeadSize + 2) : 0;
+}
+
+template <int NW>
+static void launch_prefill_attn_as(const PrefillAttnArgs& a)
+{
+    const dim3 grid(ceil_div(ceil_div(a.M, kTile), NW), a.n_heads, a.splits), block(NW * 64);
+    if (a.splits > 1)
+        hipLaunchKernelGGL((prefill_attn_kernel<NW, true>), grid, block, 0, ctx().stream, a);
     else
-        hipLaunchKernelGGL((prefill_attn_kernel<1>), dim3(tiles, a.n_heads), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((prefill_attn_kernel<NW, false>), grid, block, 0, ctx().stream, a);
+}
+
+int launch_prefill_attn(PrefillAttnArgs a)
+{
+    const PrefillAttnShape shape = prefill_attn_shape(a.M, a.position + a.M, a.n_heads);
+    a.splits = shape.splits;
+    a.part_rows = ceil_div(a.M, kTile) * kTile;
+    switch (shape.waves) {
+    case 4: launch_prefill_attn_as<4>(a); break;
+    case 2: launch_prefill_attn_as<2>(a); break;
+    default: launch_prefill_attn_as<1>(a); break;
+    }
     L2_LAUNCH_CHECK("prefill attention");
+    if (a.splits > 1) {
+        hipLaunchKernelGGL(prefill_attn_merge_kernel, dim3(ceil_div(a.M, 16), a.n_heads), dim3(256), 0, ctx().stream, a);
+        L2_LAUNCH_CHECK("prefill attention merge");
+    }
     return LLAMA2_OK;
 }
 
@@ -782,7 +880,12 @@ int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
             const size_t n = static_cast<size_t>(residual_shape(m, cfg.dim, ceil_div(k, kGroup)).splits) * m;
             parts = n > parts ? n : parts;
         }
-    parts *= static_cast<size_t>(cfg.dim) * sizeof(float);
+    parts *= cfg.dim;
+    for (int m = kTile; m <= rows; m += kTile) { // attention's pieces, gone before the next product writes its own
+        const size_t n = attn_part_floats(m, prefill_attn_shape(m, cfg.seq_len, cfg.n_heads).splits, cfg.n_heads);
+        parts = n > parts ? n : parts;
+    }
+    parts *= sizeof(float);
     const size_t total = 3 * vec + hid + up256(rope) + parts;
     L2_HIP(hipMalloc(&ws.base, total));
     char* p = static_cast<char*>(ws.base);
@@ -852,7 +955,7 @@ static int prefill_batch(const PrefillWorkspace& ws, const llama2_config& c, con
         {
             PrefillAttnArgs a{};
             a.q = ws.q, a.kcache = s.key_cache + layer_offset, a.vcache = s.value_cache + layer_offset, a.xf = ws.xf;
-            a.position = position, a.M = M, a.dim = dim, a.n_heads = c.n_heads;
+            a.parts = ws.parts, a.position = position, a.M = M, a.dim = dim, a.n_heads = c.n_heads;
             a.scale = 1.0f / sqrtf(static_cast<float>(kRopeHeadSize));
             L2_TRY(launch_prefill_attn(a));
         }

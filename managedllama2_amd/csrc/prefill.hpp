@@ -10,10 +10,9 @@ namespace l2 {
 
 constexpr int kPrefillMaxRows = 1024; // tokens per batch; longer prompts go through in batches of equal size
 // Fewer known tokens take the decode step one by one.  A batch of one token tile costs about as much as three
-// steps and the same for 8 rows as for 32.  8 rows and the step after them, against 9 steps: 7B 3.37 ms (9.32),
-// behind 600 rows 4.70 (10.28), behind 3500 rows 11.1 (12.9); 13B 5.54 (16.8); a 2-layer model of width 256
-// 0.11 (0.42).  Below that the gain shrinks and is gone behind a long history, and prompts of a few tokens keep
-// the decode step's sums bit for bit.
+// steps and the same for 8 rows as for 32.  8 rows and the step after them, against 9 steps: 7B 3.35 ms (9.32),
+// behind 600 rows 3.7 (10.3), behind 3500 rows 4.7 (12.9); 13B 5.55 (16.8); a 2-layer model of width 256
+// 0.11 (0.42).  Prompts of a few tokens keep the decode step's sums bit for bit.
 constexpr int kPrefillMinRows = 8;
 
 struct PrefillWorkspace {
@@ -21,7 +20,7 @@ struct PrefillWorkspace {
     uint16_t* q = nullptr;    // rotated queries, [rows][dim]
     uint16_t* xf = nullptr;   // normalised input / attention output in fragment order
     uint16_t* hf = nullptr;   // SwiGLU output in fragment order
-    float* parts = nullptr;   // fp32 sums of the residual products over pieces of K
+    float* parts = nullptr;   // fp32 sums of the residual products over pieces of K, of attention over pieces of time
     float* rope = nullptr;    // (cos, sin) of 64 angles per row
     void* base = nullptr;     // the one allocation behind all of them
     int rows = 0;             // capacity, a multiple of 32

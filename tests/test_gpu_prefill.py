@@ -120,6 +120,35 @@ def test_prompt_behind_a_history(first, known):
         tr.close()
 
 
+# Attention's passes shared by several workgroups per tile: as many pieces as passes (1 head), more passes than the
+# 32 pieces, pieces of unequal length, a last piece that the first queries of a tile do not attend at all (128 + 33:
+# timesteps 128 .. 161 in passes 2 and 3 with a tile's edge inside), two tiles per workgroup (16 heads, 1003 rows)
+@pytest.mark.parametrize("dim,hidden,first,known", [(128, 136, 700, 9), (128, 136, 3000, 40), (384, 1000, 175, 33),
+                                                    (384, 1000, 128, 34), (640, 648, 1111, 130), (2048, 328, 0, 1004)])
+def test_attention_in_pieces(dim, hidden, first, known):
+    cfg = config(dim, hidden, 2, first + known + 1)
+    model = synth.random_model(cfg, seed=67)
+    rng = synth.rng_for(807, dim, first)
+    n = cfg["n_layers"] * cfg["seq_len"] * dim
+    history = synth.normal_f16(rng, n), synth.normal_f16(rng, n)
+    prompt = rng.integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, first, history)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.keyCache.copy_to_device(history[0])
+    t.runstate.valueCache.copy_to_device(history[1])
+    t.runstate.tokens.copy_to_device(prompt, first)
+    capi.call("llama2_decode_run", t._decoder, first, known, first + known)
+    for g, w in zip(caches(t, cfg, first + known), caches(ref, cfg, first + known)):
+        assert np.array_equal(g[:, :first].view(np.uint16), w[:, :first].view(np.uint16))
+        for layer in range(cfg["n_layers"]):
+            want = w[layer, first:].astype(np.float64)
+            # as in test_wide_prompt_blocks
+            assert np.linalg.norm(g[layer, first:] - want) <= 4e-3 * np.linalg.norm(want), layer
+    assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
+    for tr in (t, ref):
+        tr.close()
+
+
 def test_overflowing_token_reaches_only_later_positions():
     """One token whose embedding overflows to infinities: the rows of the positions before it stay finite."""
     cfg = config(256, 640, 3, 96)

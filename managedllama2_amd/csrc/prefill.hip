@@ -5,7 +5,7 @@
 // ordinary decode step).  Taken one by one each token reads all the weights, 3.6 GB for Llama-2-7B; here up
 // to kPrefillMaxRows tokens share one reading and the matrix products run on the matrix cores:
 //   norm (+ embedding) | QKV + RoPE + cache rows | causal attention | o-proj + residual | norm |
-//   SwiGLU | down-proj + residual: 7 launches per layer and batch.
+//   SwiGLU | down-proj + residual: 7 launches per layer and batch, 8 where attention is split.
 //
 // Arithmetic, module by module as in the decode step: fp16 between the modules, exact integer weights
 // (n - z) in fp16, fp32 sums of their products with the fp16 inputs over a quantisation group of 128,
@@ -13,7 +13,7 @@
 // statistics and probabilities in fp32.  The order of the sums is not that of the decode step.
 //
 // Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.5 ms;
-// 13B, 74 tokens behind 600 rows: 151 -> 9 ms.
+// 13B, 74 tokens behind 600 rows: 151 -> 7 ms.
 #include "int4_kernels.hpp"
 #include "prefill.hpp"
 

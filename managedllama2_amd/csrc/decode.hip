@@ -770,10 +770,10 @@ int launch_step(llama2_decoder* d, int kind, int position)
 // after it is that of a decode step.  Advances position and steps past the batch.
 int run_prompt(llama2_decoder* d, int& position, int& steps, int n_prompt)
 {
-    const long long known = static_cast<long long>(n_prompt) - position;
-    const int batch = static_cast<int>(known < steps ? known : steps) - 1;
-    if (batch < kPrefillMinRows)
+    const long long known = static_cast<long long>(n_prompt) - position; // any n_prompt, also INT_MIN
+    if (known <= kPrefillMinRows || steps <= kPrefillMinRows)
         return LLAMA2_OK;
+    const int batch = static_cast<int>(known < steps ? known : steps) - 1;
     L2_TRY(prefill_run(d->prefill, d->cfg, d->layers.data(), d->w, d->s, position, batch));
     position += batch;
     steps -= batch;

@@ -149,6 +149,27 @@ def test_attention_in_pieces(dim, hidden, first, known):
         tr.close()
 
 
+# No known token whatever a negative n_prompt's distance from the position, all of them with the largest.
+@pytest.mark.parametrize("run", ["llama2_decode_run", "llama2_decode_run_sampled"])
+@pytest.mark.parametrize("first", [0, 1, 20])
+def test_extreme_prompt_lengths(run, first):
+    cfg = config(256, 640, 2, first + 21)
+    model = synth.random_model(cfg, seed=68)
+    prompt = synth.rng_for(808).integers(3, 512, cfg["seq_len"]).astype(np.int32)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    sampling = (0.5, 0.9, 7) if run.endswith("sampled") else ()
+    got = {}
+    for n_prompt in (0, -1, -2**31, -2**31 + first, -2**31 + 30, 2**31 - 1):
+        t.runstate.tokens.copy_to_device(prompt)
+        capi.call(run, t._decoder, first, 20, n_prompt, *sampling)
+        got[n_prompt] = t.runstate.tokens.to_host(first + 21)
+    assert np.array_equal(got[2**31 - 1], prompt)
+    assert not np.array_equal(got[0], prompt) and np.array_equal(got[0][:first + 1], prompt[:first + 1])
+    for n_prompt in (-1, -2**31, -2**31 + first, -2**31 + 30):
+        assert np.array_equal(got[n_prompt], got[0]), n_prompt
+    t.close()
+
+
 def test_overflowing_token_reaches_only_later_positions():
     """One token whose embedding overflows to infinities: the rows of the positions before it stay finite."""
     cfg = config(256, 640, 3, 96)

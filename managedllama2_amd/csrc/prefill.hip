@@ -686,9 +686,9 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
             }
         bm = fmaxf(bm, __shfl_xor(bm, 32, 64));
         const float nm = fmaxf(mx, bm);
-        // a query may attend none of a SPLIT's timesteps so far: its probabilities are 0, not NaN (otherwise
-        // timestep 0 is in the first pass)
-        const float base = SPLIT && nm == -INFINITY ? 0.0f : nm;
+        // no score above -infinity so far (a SPLIT whose timesteps the query does not attend, or scores below
+        // fp16's range): probabilities are 0, not NaN; if none follows, the quotient by their sum is NaN
+        const float base = nm == -INFINITY ? 0.0f : nm;
         const float alpha = expf(mx - base);
         mx = nm;
         sum *= alpha;

@@ -149,6 +149,43 @@ def test_attention_in_pieces(dim, hidden, first, known):
         tr.close()
 
 
+# Scores below fp16's range round to -infinity and get no weight, also where a whole pass of 64 timesteps has no
+# other: 17 heads x 1003 rows go unsplit, 3 heads x 40 rows in one piece per pass.
+@pytest.mark.parametrize("dim,known", [(2176, 1004), (384, 41)])
+def test_scores_below_the_range_of_fp16(oracle, dim, known):
+    first, heads = 64, dim // 128
+    cfg = config(dim, 328, 2, first + known + 1)
+    model = synth.random_model(cfg, seed=69)
+    W, Z, S = model["layers"][0]["q"]
+    model["layers"][0]["q"] = W, Z, S * np.float16(4)
+    token = 9
+    x = model["embedding"].reshape(512, dim)[token].astype(np.float64)
+    x = (x / np.sqrt(np.mean(x * x) + 1e-5)).astype(np.float16)
+    q = oracle.f64_matvec_int4(x, *model["layers"][0]["q"], dim, dim).reshape(heads, 2, 64)
+    # keys opposite to the query in the 14 slowest pairs of RoPE, which turn by less than half a radian either way
+    angle = (first + known / 2) * 10000.0 ** (-np.arange(64) / 64)
+    q = np.stack([q[:, 0] * np.cos(angle) - q[:, 1] * np.sin(angle), q[:, 0] * np.sin(angle) + q[:, 1] * np.cos(angle)], 1)
+    q[:, :, :50] = 0
+    key = np.zeros((2, cfg["seq_len"], dim), np.float16)
+    key[0, :first] = (-60000.0 * q / np.abs(q).max()).reshape(dim)
+    lowest = np.sum(q * q, (1, 2)) * np.cos(0.5) * 60000.0 / np.abs(q).max() / np.sqrt(128)
+    assert np.all(lowest > 70000), lowest.min()
+    value = synth.normal_f16(synth.rng_for(809), key.size)
+    prompt = np.full(known, token, np.int32)
+    ref = step_by_step(cfg, model, prompt, first, (key.ravel(), value))
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.keyCache.copy_to_device(key.ravel())
+    t.runstate.valueCache.copy_to_device(value)
+    t.runstate.tokens.copy_to_device(prompt, first)
+    capi.call("llama2_decode_run", t._decoder, first, known, first + known)
+    for g, w in zip(caches(t, cfg, first + known), caches(ref, cfg, first + known)):
+        assert np.all(np.isfinite(w)) and np.all(np.isfinite(g))
+        want = w[1, first:].astype(np.float64)
+        assert np.linalg.norm(g[1, first:] - want) <= 4e-3 * np.linalg.norm(want)  # as in test_wide_prompt_blocks
+    for tr in (t, ref):
+        tr.close()
+
+
 # No known token whatever a negative n_prompt's distance from the position, all of them with the largest.
 @pytest.mark.parametrize("run", ["llama2_decode_run", "llama2_decode_run_sampled"])
 @pytest.mark.parametrize("first", [0, 1, 20])

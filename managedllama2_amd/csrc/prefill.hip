@@ -10,7 +10,7 @@
 // Arithmetic, module by module as in the decode step: fp16 between the modules, exact integer weights
 // (n - z) in fp16, fp32 sums of their products with the fp16 inputs over a quantisation group of 128,
 // the group's scale applied in fp32, fp32 sums over the groups; scores rounded to fp16, softmax
-// statistics and probabilities in fp32.  The order of the sums is not that of the decode step.
+// statistics in fp32, probabilities with all the bits of fp32.  The order of the sums is not that of the decode step.
 //
 // Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.5 ms;
 // 13B, 74 tokens behind 600 rows: 151 -> 7 ms.
@@ -528,13 +528,28 @@ struct PrefillAttnArgs {
 constexpr int kAttnT = 64;        // timesteps per pass
 constexpr int kKStride = 256 + 16; // bytes of a key row in LDS: 8 lanes x 16 bytes of consecutive rows hit all banks
 constexpr int kVStride = 128 + 16; // bytes of a row of 64 timesteps of one output element
-constexpr float kProbScale = 16384.0f;
+constexpr float kProbScale = 16384.0f; // 2^14: the largest probability, 1, fits into fp16
+constexpr float kRestScale = 8192.0f;  // 2^13: what rounding to fp16 leaves of a scaled probability, at most 4, too
 
 __device__ __forceinline__ int v_row_offset(int d) { return d * kVStride + (d >> 3) * 16; }
 
+// A probability as fp16 numbers: p = (hi + (mid + lo) / 2^13) / 2^14, all 24 bits of it down to 2^-28, below that to
+// the nearest multiple of 2^-51.
+struct ProbParts {
+    h8_t hi, mid, lo;
+    __device__ __forceinline__ void set(int i, float p)
+    {
+        const float ps = p * kProbScale;
+        hi[i] = static_cast<_Float16>(ps);
+        const float rest = (ps - static_cast<float>(hi[i])) * kRestScale;
+        mid[i] = static_cast<_Float16>(rest);
+        lo[i] = static_cast<_Float16>(rest - static_cast<float>(mid[i]));
+    }
+};
+
 // The 16 timesteps t0 .. t0 + 15 of one operand step, one product each, kept only by the queries that
 // attend it (lane half u / 8 holds timestep t0 + u % 8 / 4 * 8 + u / 8 * 4 + u % 4 as element u % 8).
-__device__ __forceinline__ void one_by_one(f16v_t (&o)[4], h8_t hi, h8_t lo, const char* v, int l31, int hl, int t0, int limit)
+__device__ __forceinline__ void one_by_one(f16v_t (&o)[4], const ProbParts& p, const char* v, int l31, int hl, int t0, int limit)
 {
     for (int u = 0; u < 16; ++u) {
         const bool keep = t0 + ((u & 7) >> 2) * 8 + (u >> 3) * 4 + (u & 3) <= limit;
@@ -545,11 +560,12 @@ __device__ __forceinline__ void one_by_one(f16v_t (&o)[4], h8_t hi, h8_t lo, con
             for (int k = 0; k < 4; ++k)
                 w[k] &= hl == (u >> 3) && k == ((u & 7) >> 1) ? ((u & 1) ? 0xFFFF0000u : 0x0000FFFFu) : 0u;
             const h8_t vf = __builtin_bit_cast(h8_t, w);
-            f16v_t c = mfma(vf, hi, f16v_t{});
-            c = mfma(vf, lo, c);
+            const f16v_t c = mfma(vf, p.hi, f16v_t{});
+            f16v_t r = mfma(vf, p.mid, f16v_t{});
+            r = mfma(vf, p.lo, r);
 #pragma unroll
             for (int i = 0; i < 16; ++i)
-                o[d][i] = keep ? o[d][i] + c[i] : o[d][i];
+                o[d][i] = keep ? o[d][i] + __builtin_fmaf(r[i], 1.0f / kRestScale, c[i]) : o[d][i];
         }
     }
 }
@@ -557,8 +573,12 @@ __device__ __forceinline__ void one_by_one(f16v_t (&o)[4], h8_t hi, h8_t lo, con
 // One wavefront per tile of 32 queries of a head, NW tiles per workgroup share the key and value rows in
 // LDS.  Scores are computed transposed (rows: timesteps, columns: queries), so that a lane holds 32
 // timesteps of ONE query and its probabilities are already the second operand of the product with the
-// transposed values.  Probabilities keep fp32's precision: each is scaled by 2^14 and split into two fp16
-// numbers that go through the matrix cores one after the other (22 bits; below 2^-17 an absolute 2^-39).
+// transposed values.  Probabilities keep fp32's precision (ProbParts): three fp16 numbers that go through the
+// matrix cores one after the other, the two small ones, scaled up, into sums of their own for each pass.  Two
+// numbers of 22 bits, with nothing below 2^-39, took the same time (7B, 512 tokens 11.65 ms, three 11.61; 1003 + 24
+// tokens 46.35, 46.46): a pass is bound by its chain, not by the matrix cores.  An infinite value that a query attends may
+// reach its sum as NaN (infinity times a part that is 0): no output can tell, the norm behind it makes
+// NaN of the whole row either way.
 //
 // What bounds it: a pass of 64 timesteps is a chain (LDS filled, scores, maximum, probabilities, output) of 4 us
 // when its compute unit holds little else, and a tile walks all its passes.  SPLIT: gridDim.z workgroups share the
@@ -697,31 +717,36 @@ __global__ __launch_bounds__(NW * 64) void prefill_attn_kernel(PrefillAttnArgs a
 #pragma unroll
             for (int i = 0; i < 16; ++i)
                 o[d][i] *= alpha;
+        ProbParts p[4]; // of the operand steps of 16 timesteps
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                h8_t hi, lo;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float p = expf(s[tt][8 * j + i] - base);
-                    sum += p;
-                    const float ps = p * kProbScale;
-                    hi[i] = static_cast<_Float16>(ps);
-                    lo[i] = static_cast<_Float16>(ps - static_cast<float>(hi[i]));
-                }
-                if (careful) {
-                    one_by_one(o, hi, lo, vs + tt * 64 + hl * 32 + j * 16, l31, hl, tb + tt * 32 + j * 16, limit);
-                    continue;
-                }
-#pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    const h8_t vf =
-                        *reinterpret_cast<const h8_t*>(vs + v_row_offset(d * 32 + l31) + tt * 64 + hl * 32 + j * 16);
-                    o[d] = mfma(vf, hi, o[d]);
-                    o[d] = mfma(vf, lo, o[d]);
-                }
+            for (int i = 0; i < 8; ++i) {
+                const float pr = expf(s[u >> 1][8 * (u & 1) + i] - base);
+                sum += pr;
+                p[u].set(i, pr);
             }
+        auto values = [&](int u) { return vs + (u >> 1) * 64 + hl * 32 + (u & 1) * 16; };
+        if (careful) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                one_by_one(o, p[u], values(u), l31, hl, tb + u * 16, limit);
+            continue;
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            f16v_t r = {};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const h8_t vf = *reinterpret_cast<const h8_t*>(values(u) + v_row_offset(d * 32 + l31));
+                o[d] = mfma(vf, p[u].hi, o[d]);
+                r = mfma(vf, p[u].mid, r);
+                r = mfma(vf, p[u].lo, r);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                o[d][i] = __builtin_fmaf(r[i], 1.0f / kRestScale, o[d][i]);
+        }
     }
     sum += __shfl_xor(sum, 32, 64);
     const float inv = 1.0f / kProbScale;

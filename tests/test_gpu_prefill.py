@@ -186,6 +186,49 @@ def test_scores_below_the_range_of_fp16(oracle, dim, known):
         tr.close()
 
 
+# Probabilities keep fp32's precision however small they are: the first timestep has all the weight and no value, all
+# others are 27.2 lower (p = 2^-39.2) and have values whose sum the residual stream, small itself, feels.  In one piece
+# of the history (128) and in an unsplit launch (2176).
+@pytest.mark.parametrize("dim,first,known", [(128, 64, 9), (2176, 200, 1004)])
+def test_small_probabilities(oracle, dim, first, known):
+    heads = dim // 128
+    cfg = config(dim, 136, 2, first + known + 1)
+    model = synth.random_model(cfg, seed=70)
+    layer, token = model["layers"][0], 9
+    layer["v"] = layer["v"][0], layer["v"][1], np.zeros_like(layer["v"][2])  # the new rows have neither keys
+    layer["k"] = layer["k"][0], layer["k"][1], np.zeros_like(layer["k"][2])  # nor values: scores of 0
+    layer["o"] = layer["o"][0], layer["o"][1], layer["o"][2] * np.float16(8)
+    embedding = model["embedding"].reshape(512, dim)
+    embedding[token] = synth.normal_f16(synth.rng_for(810), dim, 2.0 ** -14)
+    x = embedding[token].astype(np.float64)
+    x = (x / np.sqrt(np.mean(x * x) + 1e-5)).astype(np.float16)
+    q = oracle.f64_matvec_int4(x, *layer["q"], dim, dim).reshape(heads, 2, 64)
+    angle = (first + known / 2) * 10000.0 ** (-np.arange(64) / 64)  # RoPE's slowest pairs turn by 0.12 at most from here
+    q = np.stack([q[:, 0] * np.cos(angle) - q[:, 1] * np.sin(angle), q[:, 0] * np.sin(angle) + q[:, 1] * np.cos(angle)], 1)
+    q[:, :, :58] = 0
+    unit = (q * np.sqrt(128) / np.sum(q * q, (1, 2), keepdims=True)).reshape(dim)  # a score of 1
+    key = np.zeros((2, cfg["seq_len"], dim), np.float16)
+    key[0, 0], key[0, 1:first] = 12 * unit, (12 - 27.2) * unit
+    assert np.all(np.isfinite(key))
+    value = np.zeros_like(key)
+    value[0, 1:first] = 60000.0 * synth.rng_for(811).choice([-1.0, 1.0], dim)
+    prompt = np.full(known, token, np.int32)
+    ref = step_by_step(cfg, model, prompt, first, (key.ravel(), value.ravel()))
+    none = step_by_step(cfg, model, prompt, first, (key.ravel(), np.zeros(key.size, np.float16)))
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.keyCache.copy_to_device(key.ravel())
+    t.runstate.valueCache.copy_to_device(value.ravel())
+    t.runstate.tokens.copy_to_device(prompt, first)
+    capi.call("llama2_decode_run", t._decoder, first, known, first + known)
+    for g, w, z in zip(*(caches(tr, cfg, first + known) for tr in (t, ref, none))):
+        g, w, z = (v[1, first:].astype(np.float64) for v in (g, w, z))
+        assert np.linalg.norm(z - w) >= 0.1 * np.linalg.norm(w)
+        # as in test_wide_prompt_blocks
+        assert np.linalg.norm(g - w) <= 4e-3 * np.linalg.norm(w), np.linalg.norm(g - w) / np.linalg.norm(w)
+    for tr in (t, ref, none):
+        tr.close()
+
+
 # No known token whatever a negative n_prompt's distance from the position, all of them with the largest.
 @pytest.mark.parametrize("run", ["llama2_decode_run", "llama2_decode_run_sampled"])
 @pytest.mark.parametrize("first", [0, 1, 20])
@@ -224,6 +267,31 @@ def test_overflowing_token_reaches_only_later_positions():
         assert np.array_equal(np.isfinite(g), np.isfinite(w))
         assert np.all(np.isfinite(g[:, :bad])) and not np.any(np.isfinite(g[1:, bad:]))
         assert_close_normwise(g[:, :bad].ravel(), w[:, :bad].ravel().astype(np.float64), "cache", TOL)
+    for tr in (t, ref):
+        tr.close()
+
+
+def test_infinite_values_in_the_history():
+    """Attended infinite values: the same rows of the caches end up infinite or NaN as in single steps."""
+    first, known = 70, 33
+    cfg = config(256, 640, 3, first + known + 1)
+    model = synth.random_model(cfg, seed=71)
+    rng = synth.rng_for(812)
+    shape = 3, cfg["seq_len"], 256
+    key, value = (synth.normal_f16(rng, int(np.prod(shape))).reshape(shape) for _ in range(2))
+    value[1, 3, 5], value[1, 40, 130] = np.inf, -np.inf  # in layer 1, one per head
+    prompt = rng.integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, first, (key.ravel(), value.ravel()))
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.keyCache.copy_to_device(key.ravel())
+    t.runstate.valueCache.copy_to_device(value.ravel())
+    t.runstate.tokens.copy_to_device(prompt, first)
+    capi.call("llama2_decode_run", t._decoder, first, known, first + known)
+    for g, w in zip(caches(t, cfg, first + known), caches(ref, cfg, first + known)):
+        for same in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(same(g), same(w)), same
+        assert np.all(np.isnan(g[2, first:])) and np.all(np.isfinite(g[:2, first:]))
+        assert_close_normwise(g[:2, first:].ravel(), w[:2, first:].ravel().astype(np.float64), "cache", TOL)
     for tr in (t, ref):
         tr.close()
 

@@ -399,7 +399,11 @@ typedef struct llama2_decoder llama2_decoder;
 /* Binds a config, a weight set and a run state (all borrowed, all must outlive
  * the decoder) to the per-step launch sequence of Transformer.Forward
  * (src/Transformer.cs:158-190).  GQA is rejected like the reference does
- * (src/Transformer.cs:53-56). */
+ * (src/Transformer.cs:53-56).  A fused decoder keeps a workspace for known
+ * tokens in batches (llama2_decode_run): 78 MiB for Llama-2-7B, 145 MiB for 13B
+ * with contexts of 1024 rows or more, at most half of the memory that is free
+ * and at most LLAMA2_PREFILL_MIB (an environment variable); with less the
+ * batches get smaller, with nothing all tokens go step by step. */
 int llama2_decode_create(llama2_decoder** decoder, const llama2_config* config,
                          const llama2_transformer_weights* weights,
                          const llama2_run_state* state, int mode);

@@ -771,7 +771,7 @@ int launch_step(llama2_decoder* d, int kind, int position)
 int run_prompt(llama2_decoder* d, int& position, int& steps, int n_prompt)
 {
     const long long known = static_cast<long long>(n_prompt) - position; // any n_prompt, also INT_MIN
-    if (known <= kPrefillMinRows || steps <= kPrefillMinRows)
+    if (known <= kPrefillMinRows || steps <= kPrefillMinRows || d->prefill.rows == 0)
         return LLAMA2_OK;
     const int batch = static_cast<int>(known < steps ? known : steps) - 1;
     L2_TRY(prefill_run(d->prefill, d->cfg, d->layers.data(), d->w, d->s, position, batch));
@@ -979,10 +979,6 @@ int llama2_decode_create(llama2_decoder** decoder, const llama2_config* config,
             release(d);
             return hip_fail(e, "llama2_decode_create: scratch allocation");
         }
-        if (const int rc = prefill_create(d->prefill, c)) {
-            release(d);
-            return rc;
-        }
         if (variant >= 0) {
             const int rc = persist_setup(d);
             if (rc != LLAMA2_OK) {
@@ -1011,6 +1007,10 @@ int llama2_decode_create(llama2_decoder** decoder, const llama2_config* config,
                 release(d);
                 return rc;
             }
+        }
+        if (const int rc = prefill_create(d->prefill, c)) { // last: it makes do with the memory that is left
+            release(d);
+            return rc;
         }
     }
     *decoder = d;

@@ -18,6 +18,7 @@
 #include "prefill.hpp"
 
 #include <cmath>
+#include <cstdlib>
 #include <type_traits>
 
 namespace l2 {
@@ -895,12 +896,17 @@ int launch_prefill_norm(const NormArgs& a, int M)
 
 static size_t up256(size_t n) { return (n + 255) / 256 * 256; }
 
-int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
+struct PrefillSizes {
+    size_t vec, hid, rope, parts;
+    size_t total() const { return 3 * vec + hid + rope + parts; }
+};
+
+static PrefillSizes prefill_sizes(const llama2_config& cfg, int rows)
 {
-    const int rows = ceil_div(cfg.seq_len < kPrefillMaxRows ? cfg.seq_len : kPrefillMaxRows, kTile) * kTile;
-    const size_t vec = up256(static_cast<size_t>(rows) * cfg.dim * 2);
-    const size_t hid = up256(static_cast<size_t>(rows) * ceil_div(cfg.hidden_dim, kGroup) * kGroup * 2);
-    const size_t rope = static_cast<size_t>(rows) * 128 * sizeof(float);
+    PrefillSizes z;
+    z.vec = up256(static_cast<size_t>(rows) * cfg.dim * 2);
+    z.hid = up256(static_cast<size_t>(rows) * ceil_div(cfg.hidden_dim, kGroup) * kGroup * 2);
+    z.rope = up256(static_cast<size_t>(rows) * 128 * sizeof(float));
     size_t parts = 0; // the largest [splits][rows][dim] any batch needs
     for (int m = kTile; m <= rows; m += kTile)
         for (int k : {cfg.dim, cfg.hidden_dim}) {
@@ -912,19 +918,48 @@ int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
         const size_t n = attn_part_floats(m, prefill_attn_shape(m, cfg.seq_len, cfg.n_heads).splits, cfg.n_heads);
         parts = n > parts ? n : parts;
     }
-    parts *= sizeof(float);
-    const size_t total = 3 * vec + hid + up256(rope) + parts;
-    L2_HIP(hipMalloc(&ws.base, total));
+    z.parts = parts * sizeof(float);
+    return z;
+}
+
+int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg)
+{
+    // A host may have given nearly all of the memory to its caches (the reference's run state leaves 8 MiB): at
+    // most half of what is free is taken, with smaller batches where that is too little, and without any room
+    // the decoder goes step by step.
+    size_t limit = 0, total_memory = 0;
+    L2_HIP(hipMemGetInfo(&limit, &total_memory));
+    limit /= 2;
+    if (const char* mib = getenv("LLAMA2_PREFILL_MIB")) {
+        const size_t wanted = static_cast<size_t>(strtoull(mib, nullptr, 10)) << 20;
+        limit = wanted < limit ? wanted : limit;
+    }
+    int rows = ceil_div(cfg.seq_len < kPrefillMaxRows ? cfg.seq_len : kPrefillMaxRows, kTile) * kTile;
+    PrefillSizes z{};
+    for (;; rows = ceil_div(rows / 2, kTile) * kTile) {
+        z = prefill_sizes(cfg, rows);
+        if (z.total() <= limit) {
+            const hipError_t e = hipMalloc(&ws.base, z.total());
+            if (e == hipSuccess)
+                break;
+            if (e != hipErrorOutOfMemory)
+                return hip_fail(e, "prefill workspace");
+            (void)hipGetLastError();
+            ws.base = nullptr;
+        }
+        if (rows == kTile)
+            return LLAMA2_OK;
+    }
     char* p = static_cast<char*>(ws.base);
     ws.x = reinterpret_cast<uint16_t*>(p);
-    ws.q = reinterpret_cast<uint16_t*>(p + vec);
-    ws.xf = reinterpret_cast<uint16_t*>(p + 2 * vec);
-    ws.hf = reinterpret_cast<uint16_t*>(p + 3 * vec);
-    ws.rope = reinterpret_cast<float*>(p + 3 * vec + hid);
-    ws.parts = reinterpret_cast<float*>(p + 3 * vec + hid + up256(rope));
+    ws.q = reinterpret_cast<uint16_t*>(p + z.vec);
+    ws.xf = reinterpret_cast<uint16_t*>(p + 2 * z.vec);
+    ws.hf = reinterpret_cast<uint16_t*>(p + 3 * z.vec);
+    ws.rope = reinterpret_cast<float*>(p + 3 * z.vec + z.hid);
+    ws.parts = reinterpret_cast<float*>(p + 3 * z.vec + z.hid + z.rope);
     ws.rows = rows;
     // hf beyond hidden_dim is never written and must read as zero
-    L2_HIP(hipMemsetAsync(ws.base, 0, total, ctx().stream));
+    L2_HIP(hipMemsetAsync(ws.base, 0, z.total(), ctx().stream));
     L2_HIP(hipStreamSynchronize(ctx().stream));
     return LLAMA2_OK;
 }

@@ -23,10 +23,11 @@ struct PrefillWorkspace {
     float* parts = nullptr;   // fp32 sums of the residual products over pieces of K, of attention over pieces of time
     float* rope = nullptr;    // (cos, sin) of 64 angles per row
     void* base = nullptr;     // the one allocation behind all of them
-    int rows = 0;             // capacity, a multiple of 32
+    int rows = 0;             // capacity, a multiple of 32; 0: no workspace, every token is a step
 };
 
-// Sizes `ws` for batches of up to min(seq_len, kPrefillMaxRows) tokens and allocates it.
+// Sizes `ws` for batches of up to min(seq_len, kPrefillMaxRows) tokens and allocates it (7B 78 MiB, 13B 145 MiB for
+// 1024 rows); for fewer, or none, where memory is short.
 int prefill_create(PrefillWorkspace& ws, const llama2_config& cfg);
 void prefill_destroy(PrefillWorkspace& ws);
 // The layers of Transformer.Forward for the `count` tokens at positions position .. position + count - 1,

@@ -296,6 +296,28 @@ def test_infinite_values_in_the_history():
         tr.close()
 
 
+# Where memory is short the workspace shrinks (here to 128 and 64 rows), and without one the loop goes step by
+# step as it does for short prompts, bit for bit; the decoder is never refused.
+@pytest.mark.parametrize("mib", [None, "2", "1", "0"])
+def test_short_of_memory(mib, monkeypatch):
+    cfg = config(256, 640, 2, 420)
+    model = synth.random_model(cfg, seed=72)
+    prompt = synth.rng_for(813).integers(3, 512, 401).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    if mib is not None:
+        monkeypatch.setenv("LLAMA2_PREFILL_MIB", mib)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run", t._decoder, 0, 401, 401)
+    for g, w in zip(caches(t, cfg, 401), caches(ref, cfg, 401)):
+        assert np.array_equal(g.view(np.uint16), w.view(np.uint16)) == (mib == "0")
+        for layer in range(2):
+            want = w[layer].astype(np.float64)
+            assert np.linalg.norm(g[layer] - want) <= 4e-3 * np.linalg.norm(want), layer  # as in test_wide_prompt_blocks
+    for tr in (t, ref):
+        tr.close()
+
+
 def test_captured_prompt_replays():
     """The whole prompt as a graph of the caller's: every replay gives the caches of the eager call."""
     cfg = config(256, 640, 2, 64)

@@ -31,6 +31,12 @@ def caches(t, cfg, n):
     return [b.to_host().reshape(shape)[:, :n] for b in (t.runstate.keyCache, t.runstate.valueCache)]
 
 
+def clear_caches(t):
+    """Every row NaN: what a run does not write cannot pass for what it should have written."""
+    for b in (t.runstate.keyCache, t.runstate.valueCache):
+        b.copy_to_device(np.full(b.size, np.nan, np.float16))
+
+
 def step_by_step(cfg, model, prompt, first, history=None):
     """The same positions through single steps (what the loop did for fewer known tokens)."""
     t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
@@ -84,6 +90,7 @@ def test_shortest_batches(dim, hidden):
     t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
     for known in (8, 9, 12, 15, 16):
         t.runstate.tokens.copy_to_device(prompt)
+        clear_caches(t)
         capi.call("llama2_decode_run", t._decoder, 0, known, known)
         for g, w in zip(caches(t, cfg, known), caches(ref, cfg, known)):
             if known == 8:
@@ -344,8 +351,8 @@ def test_captured_prompt_replays():
     t.close()
 
 
-# Widths at which the products take the larger blocks: 1 to 4 token tiles and 1, 2 or 4 pairs of weight tiles per
-# workgroup, K in up to 4 pieces; the pairs of a width that is an odd multiple of 128 do not fill the last block
+# Widths at which some of the products take the larger blocks, K in up to 4 pieces; the pairs of a width that is an odd
+# multiple of 128 do not fill the last block
 @pytest.mark.parametrize("dim,hidden,known", [(1408, 328, 131), (2176, 648, 301), (2176, 648, 601), (1408, 328, 1004),
                                               (2176, 648, 1004)])
 def test_wide_prompt_blocks(dim, hidden, known):
@@ -365,3 +372,93 @@ def test_wide_prompt_blocks(dim, hidden, known):
     assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
     for tr in (t, ref):
         tr.close()
+
+
+# The widths of 7B and 13B, two layers deep (the last one leaves its attention and MLP out).  On 256 compute units the
+# prompt lengths reach, in token tiles x pairs of weight tiles per workgroup:
+#   QKV         11 12 14 22 24 34 44 (7B: 11, 51, 151, 76, 251, 385, 512 tokens)
+#   SwiGLU      12 22 24 34 44 (11, 51, 76, 151, 251)
+#   o-, down-proj  11 14 22 24 34 44, K in 1 to 8 pieces (1x4: 13B, 75)
+#   attention   1, 2 and 4 tiles per workgroup (11, 512, 1004), 1 to 4 pieces (11, 76, 151, 251)
+@pytest.mark.parametrize("widths,lengths", [(synth.LLAMA2_7B, (11, 51, 76, 151, 251, 385, 512, 1004)),
+                                            (synth.LLAMA2_13B, (75, 321, 1004))])
+def test_model_widths(widths, lengths):
+    cfg = dict(widths, n_layers=2, vocab_size=512, seq_len=max(lengths))
+    model = synth.random_model(cfg, seed=73, rms_random=True)
+    for layer in model["layers"]:
+        # scores of ordinary size: with the scales as drawn they reach hundreds, where ONE fp16 rounding of a score
+        # moves its probability by a quarter and single rows say nothing
+        for name in ("q", "k"):
+            layer[name] = layer[name][:2] + (layer[name][2] * np.float16(0.25),)
+    prompt = synth.rng_for(814).integers(3, 512, max(lengths)).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    want = [v.astype(np.float64) for v in caches(ref, cfg, max(lengths))]
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    for known in lengths:
+        t.runstate.tokens.copy_to_device(prompt)
+        clear_caches(t)
+        capi.call("llama2_decode_run", t._decoder, 0, known, known)
+        for name, g, w in zip("kv", caches(t, cfg, known), want):
+            for layer in range(2):
+                d = g[layer].astype(np.float64) - w[layer, :known]
+                # the whole as in test_wide_prompt_blocks; a row by itself (a misplaced tile) by the 7 roundings to fp16
+                # between a layer's rows and the next one's, each off by 2^-11 at most, doubled on the way by the MLP
+                rows = np.linalg.norm(d, axis=1) / np.linalg.norm(w[layer, :known], axis=1)
+                print(known, name, layer, "%.2e, worst row %.2e" % (np.sqrt(np.mean(rows * rows)), rows.max()))
+                assert np.linalg.norm(d) <= 4e-3 * np.linalg.norm(w[layer, :known]), (known, name, layer)
+                assert rows.max() <= 14 * 2.0 ** -11, (known, name, layer, int(rows.argmax()), rows.max())
+    assert_close_normwise(t.runstate.logits.to_host(), ref.runstate.logits.to_host().astype(np.float64), "logits", TOL)
+    for tr in (t, ref):
+        tr.close()
+
+
+# The other loops that batch their prompt: sampling, and the persistent step (same bits as the launch sequence behind
+# the same batch).
+def test_sampled_run_behind_a_batch():
+    cfg, known, steps, seed = config(256, 640, 2, 64), 41, 60, 99
+    model = synth.random_model(cfg, seed=74)
+    prompt = synth.rng_for(815).integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+    clear_caches(t)
+    t.runstate.tokens.copy_to_device(prompt)
+    capi.call("llama2_decode_run_sampled", t._decoder, 0, steps, known, 0.7, 0.9, seed)
+    for g, w in zip(caches(t, cfg, known), caches(ref, cfg, known)):
+        for layer in range(cfg["n_layers"]):
+            want = w[layer].astype(np.float64)
+            assert np.linalg.norm(g[layer] - want) <= 4e-3 * np.linalg.norm(want), layer  # as in test_wide_prompt_blocks
+    tokens = t.runstate.tokens.to_host(steps + 1)
+    assert np.array_equal(tokens[:known], prompt) and len(set(tokens[known:].tolist())) > 4
+    token = C.c_int()
+    for pos in range(known - 1, steps):  # the steps behind the batch again, one by one, with the same coins
+        t.Forward(pos, pos + 1)
+        coin = float(capi.load().llama2_sampler_coin(seed, pos + 1))
+        capi.call("llama2_decode_sample_top_p", t._decoder, pos + 1, 1, 0.7, 0.9, coin, C.byref(token))
+        assert token.value == tokens[pos + 1], pos
+    for tr in (t, ref):
+        tr.close()
+
+
+def test_persistent_run_behind_a_batch():
+    cfg, known, steps = config(256, 640, 2, 64), 41, 60
+    model = synth.random_model(cfg, seed=75)
+    prompt = synth.rng_for(816).integers(3, 512, known).astype(np.int32)
+    ref = step_by_step(cfg, model, prompt, 0)
+    got = []
+    for mode in (capi.DECODE_FUSED | capi.DECODE_PERSISTENT, FUSED_GRAPH | capi.DECODE_PERSISTENT, FUSED_GRAPH):
+        t = Transformer(dict(cfg), model, mode=mode)
+        clear_caches(t)
+        t.runstate.tokens.copy_to_device(prompt)
+        capi.call("llama2_decode_run", t._decoder, 0, steps, known)
+        capi.call("llama2_decode_check", t._decoder)
+        got.append([v.view(np.uint16) for v in caches(t, cfg, steps)] + [t.runstate.tokens.to_host(steps + 1)])
+        t.close()
+    for g, w in zip(got[2], caches(ref, cfg, known)):
+        for layer in range(cfg["n_layers"]):
+            want = w[layer].astype(np.float64)
+            d = g.view(np.float16)[layer, :known] - want
+            assert np.linalg.norm(d) <= 4e-3 * np.linalg.norm(want), layer  # as in test_wide_prompt_blocks
+    for other in got[:2]:
+        for a, b in zip(other, got[2]):
+            assert np.array_equal(a, b)
+    ref.close()

@@ -11,9 +11,9 @@ hipGraph so the host's per-call cost never bounds what the GPU does.
 
 Prints ONE JSON line: whole-job HBM GB/s over the algorithmic bytes of the
 mat-vec set (`value`), the roofline record of the dominant kernel (fused
-SwiGLU), the single 4096x4096 mat-vec and the 13B layer set
-(configs[2]), decode attention GB/s at 512/2048/4096 rows, full greedy decode
-tokens/s (128-token prompt + 256 generated tokens), and the reference's
+SwiGLU), the single 4096x4096 mat-vec and the 13B layer set,
+decode attention GB/s at 512/2048/4096 rows, greedy decode (generated
+tokens/s, prompt and run times of 128 + 256 tokens), and the reference's
 single-threaded C# CPU path (restated in C) timed beside it.
 
 Every timed figure comes from at least 100 graph replays after warm-up (HIP
@@ -102,7 +102,7 @@ def main():
     zs, ss, ws = (lambda t: (t[2], t[1], t[0]))(synth.qweight_sizes(dim))
     hzs, hss, hws = (lambda t: (t[2], t[1], t[0]))(synth.qweight_sizes(hidden))
 
-    # ---- the random-init 7B model (configs[4] distributions), generated layer by layer
+    # ---- the random-init 7B model, generated layer by layer
     t0 = time.time()
     rng = synth.rng_for(1, 7)
     first_layer = []
@@ -224,7 +224,7 @@ def main():
         "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "int4 weights x f16 activations, f32 accumulate", "data": "synthetic",
-        "config": {"workload": "configs[1]: 7B layer mat-vec set (QKV, o+res, SwiGLU, down+res), "
+        "config": {"workload": "7B layer mat-vec set (QKV, o+res, SwiGLU, down+res), "
                                "%d distinct layers cycled (cold HBM)" % n_layers,
                    "dim": dim, "hidden_dim": hidden, "algorithmic_bytes_per_step": sizes["total"]},
     }
@@ -277,7 +277,7 @@ def main():
         result["per_kernel"] = per_kernel
 
     if "cfg0" in legs:
-        # configs[0]: ONE int4 mat-vec 4096 x 4096 (plain, and with the residual epilogue), cycled over the
+        # ONE int4 mat-vec 4096 x 4096 (plain, and with the residual epilogue), cycled over the
         # model's 128 distinct q / k / v / o tensors (1.1 GB: cold HBM).  8 732 672 algorithmic bytes
         # (+ 8 192 for the residual read); floor at 8 TB/s: 1.09 us.
         tensors = [w for L in layers for w in (L.queryWeight, L.keyWeight, L.valueWeight, L.outputWeight)]
@@ -294,11 +294,11 @@ def main():
                           "floor_us_at_8TBps": round(nbytes / 8e6, 3)}
             log("  cfg0 %-9s %6.2f us  %6.0f GB/s (%.1f%% of peak; floor %.2f us)" %
                 (name, us, nbytes / us / 1e3, 100 * nbytes / us / 1e3 / HBM_PEAK_GBPS, nbytes / 8e6))
-        cfg0["workload"] = "configs[0]: single AWQ int4 mat-vec K = N = 4096, %d distinct tensors cycled" % len(tensors)
+        cfg0["workload"] = "single AWQ int4 mat-vec K = N = 4096, %d distinct tensors cycled" % len(tensors)
         result["cfg0"] = cfg0
 
     if "cfg2" in legs:
-        # configs[2]: the Llama-2-13B layer mat-vec set (dim 5120, hidden 13824; 14 padded zero words per
+        # the Llama-2-13B layer mat-vec set (dim 5120, hidden 13824; 14 padded zero words per
         # down-proj row) over 4 distinct layers (660 MB: cold HBM).  164 960 256 algorithmic bytes; floor 20.6 us.
         d13, h13, n13 = synth.LLAMA2_13B["dim"], synth.LLAMA2_13B["hidden_dim"], 4
         s13 = synth.layer_matvec_set_bytes(d13, h13)
@@ -330,7 +330,7 @@ def main():
         def dn13(L):
             capi.call("llama2_mat_vec_residual_int4", x13.ptr, hbuf13.ptr, *p3(L["down"]), h13, d13, hz13, hq13, hw13)
 
-        cfg2 = {"workload": "configs[2]: 13B layer mat-vec set, %d distinct layers cycled" % n13,
+        cfg2 = {"workload": "13B layer mat-vec set, %d distinct layers cycled" % n13,
                 "algorithmic_bytes_per_step": s13["total"], "floor_us_at_8TBps": round(s13["total"] / 8e6, 2)}
         graph = capture(lambda i: [f(L13[i % n13]) for f in (qkv13, o13, sw13, dn13)], n13)
         us, spread, replays = measure(graph, n13, replays=4 * MIN_REPLAYS)
@@ -371,7 +371,7 @@ def main():
         dst.free()
 
     if "attn" in legs:
-        # configs[3]: decode attention over the fp16 KV cache, 32 heads x 128, RoPE at pos = S on the
+        # decode attention over the fp16 KV cache, 32 heads x 128, RoPE at pos = S on the
         # newest row, scores, softmax, weighted value sum; cycled over the 32 layers' cache slices
         rs = model.runstate
         seq_cap = model.config.seq_len
@@ -460,19 +460,22 @@ def main():
         capi.call("llama2_decode_destroy", dec)
 
     if "decode" in legs:
-        # 128 seeded prompt tokens, 256 greedy tokens, every step on the device
+        # 128 seeded prompt tokens, 256 greedy tokens, every step on the device.  The prompt's tokens share one
+        # reading of the weights (in batches), so the rates are those of the generated tokens, each of which
+        # reads all of them; the prompt alone and the whole run are times.
         n_prompt, n_gen = 128, 256
         steps = n_prompt + n_gen - 1
         prompt = synth.rng_for(5).integers(3, cfg["vocab_size"], n_prompt).astype(np.int32)
         model.runstate.tokens.copy_to_device(prompt)
-        capi.call("llama2_decode_run", model._decoder, 0, 16, n_prompt)  # warm-up
+        capi.call("llama2_decode_run", model._decoder, 0, n_prompt + 8, n_prompt)  # warm-up
         capi.call("llama2_sync")
         ev.start()
         capi.call("llama2_decode_run", model._decoder, 0, steps, n_prompt)
         ms = ev.stop_ms()
         toks = model.runstate.tokens.to_host(n_prompt + n_gen)
-        tok_s = steps / (ms * 1e-3)
-        # the generated tokens alone: each reads all the weights, the prompt's tokens share one reading
+        ev.start()
+        capi.call("llama2_decode_run", model._decoder, 0, n_prompt, n_prompt)
+        prompt_ms = ev.stop_ms()
         n_steps = steps - n_prompt
         ev.start()
         capi.call("llama2_decode_run", model._decoder, n_prompt, n_steps, n_prompt)
@@ -481,10 +484,9 @@ def main():
         kv_avg = 2 * n_layers * (n_prompt + 1 + steps) / 2 * dim * 2
         bytes_tok = (n_layers * (sizes["total"] - 126_000 + 2 * 2 * dim) + 2 * cfg["vocab_size"] * dim
                      + 2 * dim + 2 * dim + kv_avg)
-        result["decode"] = {"tokens_per_s": round(tok_s, 1), "ms_per_token": round(ms / steps, 4),
-                            "forward_steps": steps, "prompt": n_prompt, "generated": n_gen,
-                            "mode": args.decode_mode,
-                            "generation_tokens_per_s": round(gen_s, 1),
+        result["decode"] = {"tokens_per_s": round(gen_s, 1), "ms_per_token": round(gen_ms / n_steps, 4),
+                            "generation_steps": n_steps, "prompt": n_prompt, "generated": n_gen,
+                            "run_ms": round(ms, 3), "prompt_ms": round(prompt_ms, 3), "mode": args.decode_mode,
                             "GBps": round(bytes_tok * gen_s / 1e9, 1),
                             "pct_of_hbm_peak": round(100 * bytes_tok * gen_s / 1e9 / HBM_PEAK_GBPS, 2),
                             "bandwidth_bound_tokens_per_s": round(HBM_PEAK_GBPS * 1e9 / bytes_tok, 1),
@@ -506,8 +508,8 @@ def main():
         host_tok_s = n_host / (time.perf_counter() - t1)
         result["decode"]["host_loop_tokens_per_s"] = round(host_tok_s, 1)
         log("decode, host loop with one read-back per token: %.1f tok/s" % host_tok_s)
-        log("decode: %.1f tok/s with the prompt, generation %.1f tok/s (%.0f GB/s = %.1f%% of peak; ceiling %.0f tok/s)" %
-            (tok_s, gen_s, bytes_tok * gen_s / 1e9, 100 * bytes_tok * gen_s / 1e9 / HBM_PEAK_GBPS,
+        log("decode: %.2f ms, of it the prompt %.2f ms; generation %.1f tok/s (%.0f GB/s = %.1f%% of peak; ceiling %.0f tok/s)" %
+            (ms, prompt_ms, gen_s, bytes_tok * gen_s / 1e9, 100 * bytes_tok * gen_s / 1e9 / HBM_PEAK_GBPS,
              HBM_PEAK_GBPS * 1e9 / bytes_tok))
 
     if "sampler" in legs:
@@ -544,10 +546,11 @@ def main():
         steps = n_prompt + n_gen - 1
         prompt = synth.rng_for(5).integers(3, vocab, n_prompt).astype(np.int32)
         model.runstate.tokens.copy_to_device(prompt)
-        capi.call("llama2_decode_run_sampled", model._decoder, 0, 16, n_prompt, temp, top_p, 1)  # warm-up
+        capi.call("llama2_decode_run_sampled", model._decoder, 0, n_prompt, n_prompt, temp, top_p, 1)  # warm-up
         capi.call("llama2_sync")
+        steps -= n_prompt  # the generated tokens, as in the greedy leg
         ev.start()
-        capi.call("llama2_decode_run_sampled", model._decoder, 0, steps, n_prompt, temp, top_p, 1)
+        capi.call("llama2_decode_run_sampled", model._decoder, n_prompt, steps, n_prompt, temp, top_p, 1)
         ms = ev.stop_ms()
         sampler["decode_tokens_per_s"] = round(steps / (ms * 1e-3), 1)
         sampler["decode_ms_per_token"] = round(ms / steps, 4)
@@ -557,7 +560,7 @@ def main():
             sp, coins = model.sampler, np.random.default_rng(7)
             sp.temperature, sp.topP, sp.random = temp, top_p, coins.random
             t1 = time.perf_counter()
-            n_host = sum(1 for _ in model.Generate(prompt, steps, stop_on_special=False))
+            n_host = sum(1 for _ in model.Generate(prompt, n_prompt + steps, stop_on_special=False))
             sampler["host_loop_tokens_per_s"] = round(n_host / (time.perf_counter() - t1), 1)
             sp.temperature = 0.0
         result["sampler"] = sampler

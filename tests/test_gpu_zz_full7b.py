@@ -1,4 +1,4 @@
-"""full Llama-2-7B-shape greedy decode with random-init weights --
+"""Full Llama-2-7B-shape greedy decode with random-init weights --
 32 layers, dim 4096, 32 heads, FFN 11008, int4 g128 linear layers, fp16
 embedding / classifier over a 32000 vocabulary, 128 seeded prompt tokens
 followed by 256 argmax tokens, every step on the device (hipGraph replay).

@@ -10,7 +10,8 @@
 //     zero without any lane predication);
 //   * a wavefront owns a span of consecutive rows, all wavefronts resident at once, the row
 //     sequence fully unrolled with the next row's loads in flight while the current one is
-//     reduced (int4_matvec_span_kernel: every shape the decoder and the benches launch); the
+//     reduced (int4_matvec_span_kernel: every launch of the 7B shapes, and of the 13B ones all but
+//     the decode step's QKV launch, whose wavefronts of one row do not fit at once: 12.2 us there); the
 //     two older kernels (persistent wavefronts that stride over the rows, one row or a block of
 //     rows per item) take the launches it refuses;
 //   * the input vector is staged once per workgroup in LDS, pre-permuted to

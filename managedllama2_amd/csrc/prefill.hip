@@ -12,7 +12,7 @@
 // the group's scale applied in fp32, fp32 sums over the groups; scores rounded to fp16, softmax
 // statistics in fp32, probabilities with all the bits of fp32.  The order of the sums is not that of the decode step.
 //
-// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.5 ms;
+// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.3 ms;
 // 13B, 74 tokens behind 600 rows: 151 -> 7 ms.
 #include "int4_kernels.hpp"
 #include "prefill.hpp"
@@ -197,9 +197,11 @@ constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }
 // of a pair meet, through LDS.  The launch may split K further (EPI_PARTIAL).
 //
 // What bounds it: a group costs a wavefront MT x 256 cycles of its matrix core (two wavefronts share one), about 400 of
-// its vector unit to unpack the weights and MT x 100 to scale the sums.  The rest has to stay out of the way:
+// its vector unit to unpack the weights and MT x 100 to scale the sums, and the two units hardly overlap: over the
+// SwiGLU launch of 511 rows of 7B (135 us) the matrix cores are busy 32 %, the vector units 38 % of the time, without an LDS
+// bank conflict.  The rest has to stay out of the way:
 // - A compute unit looks up one cache address per cycle and 64 contiguous bytes.  A lane that reads its own row's
-//   weights costs 64 lookups per load (65 % busy against 28 % of the matrix cores, when it was done so).  Everything
+//   weights costs 64 lookups per load (13.2 ms instead of 11.9 for the 512-token prompt).  Everything
 //   comes through LDS, requested in the order of memory; LDS delivers 256 bytes per cycle where 16 neighbouring
 //   lanes meet all banks, hence the swizzle of the weight rows.
 // - One barrier per step, LDS for three: activations are requested two steps ahead, weights three, because
@@ -458,11 +460,14 @@ constexpr int kMaxSplits = 8;
 // The cheapest of the shapes that fit into LDS, by an estimate in cycles: workgroups run one per compute unit in
 // rounds of equal length, a round is its steps plus filling and draining the pipeline, and every piece of K
 // beyond the first costs the norm that adds them up another reading (about 1024 values per cycle).
-// A step measured 2900 cycles with two token tiles (7B SwiGLU, 511 rows: 3 rounds of 32 steps in 121 us) and
-// 5000 with four (QKV: one round of 32 steps in 72 us); the others lie on the same line; several groups per step
-// (more activations per result) add 400 (two tiles, 7B QKV, 511 rows: 3 rounds of 16 steps in 78 us; 13B, 74 rows:
-// one of 20 in 31).  What the choice gives, against blocks of 64 tokens by 256 weight rows for every size: 7B, 511 rows, QKV 86 -> 76 us (192 workgroups in one round
-// instead of 384 in two), down-proj 66 -> 54; 13B, 74 rows, QKV 42 -> 32.
+// Cycles of a step at 2.4 GHz in launches of 20 steps and more, tiles 1 / 2 / 3 / 4: 2300 .. 2400 / 2900 .. 3100 /
+// 3900 .. 4400 / 4650 .. 5400, which the table follows but for one tile; several groups per step (more activations per
+// result) add 200 .. 600.  Of 68 launches of 7B and 13B with 32 to 1003 rows those with pieces of 16 steps or more take 0.93 to
+// 1.25 times the estimate, those with fewer 1.2 to 1.75 times: filling the pipeline and storing the sums of the pieces.
+// The estimate does not see that each of the 8 XCDs gets whole blocks of weights, so that some may need one more round
+// (13B, 1003 rows, o-proj: 20 blocks x 11, 33 workgroups on 32 compute units, 123 us instead of 69).  What the choice
+// gives, against blocks of 64 tokens by 256 weight rows for every size: 7B, 511 rows, QKV 86 -> 76 us (192 workgroups
+// in one round instead of 384 in two), down-proj 66 -> 54; 13B, 74 rows, QKV 42 -> 32.
 static GemmShape gemm_shape(int tiles, int pairs, int groups, bool may_split)
 {
     static constexpr int kStepCycles[5] = {0, 1900, 2900, 3950, 5000};

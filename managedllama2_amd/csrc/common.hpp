@@ -16,6 +16,8 @@ namespace l2 {
 // ------------------------------------------------------------------ host side
 constexpr int kMaxRetiredPartials = 32;
 
+struct SamplerScratch;
+
 struct Context {
     bool ready = false;
     int device = -1;
@@ -38,9 +40,7 @@ struct Context {
     int n_retired_partials = 0;
     // per-head arrival counters of llama2_multi_head_attention (zero between launches)
     unsigned* attn_counters = nullptr;
-    // second buffer of the sampler's radix sort (LLAMA2_MAX_SAMPLER_SIZE keys and payloads)
-    uint16_t* sort_keys = nullptr;
-    int* sort_values = nullptr;
+    SamplerScratch* sampler = nullptr; // between the sampler's launches (sampler_kernels.hpp)
 };
 
 constexpr int kMaxAttnHeads = 1024;
@@ -51,7 +51,7 @@ int hip_fail(hipError_t e, const char* what);
 int ensure_attn_partials(size_t bytes);
 // Device address of llama2_vec_mat_static's scratch array on `device` (current), asked for once at llama2_init.
 int resolve_vec_mat_static_scratch(int device);
-// Sampler.Sample's stochastic branch in one launch (sampler.hip).  token_only: the caller reads the
+// Sampler.Sample's stochastic branch (sampler.hip).  token_only: the caller reads the
 // token alone, so the sort may stop at the head of the distribution that holds top_p of the mass.
 int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, float temperature, float top_p, float coin,
                   int* result, int pos, bool token_only);

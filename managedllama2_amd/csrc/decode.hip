@@ -359,15 +359,6 @@ void launch_attn(const AttnShape& shape, int n_heads, const AttnArgs& a)
 // angles, so the 32 QKV launches of a step do not each call powf/cosf/sinf.
 constexpr size_t kStateBytes = kStateInts * sizeof(int) + kRopeHeadSize * sizeof(float);
 
-__device__ __forceinline__ void write_rope_table(int* state, int i, int pos, float theta)
-{
-    float c, s;
-    rope_cos_sin(c, s, i, kRopeHeadSize, pos, theta);
-    float* tab = reinterpret_cast<float*>(state + kStateInts);
-    tab[2 * i] = c;
-    tab[2 * i + 1] = s;
-}
-
 __global__ void set_state_kernel(int* state, int pos, int n_prompt, int advance, int n_slots, float theta)
 {
     if (threadIdx.x == 0) {
@@ -404,55 +395,6 @@ __global__ __launch_bounds__(1024) void argmax_step_kernel(const uint16_t* x, in
         if (advance0)
             state[0] = pos0 + 1;
     }
-}
-
-// Sampler.Sample's stochastic branch (src/Sampler.cs:48-67) against the device
-// state: the token at pos+1 is drawn with the coin of (seed, pos+1) iff
-// pos+1 >= n_prompt; then the position advances like in argmax_step_kernel.
-struct SampleStepArgs {
-    uint16_t* logits;
-    int* indices;
-    int size;
-    int* tokens;
-    int* state;
-    uint16_t* keys2; // second buffer of the global-memory sort (vocabularies beyond kSortLdsItems)
-    int* values2;
-    float temperature, top_p;
-    unsigned long long seed;
-    float theta;
-};
-
-template <bool LDS_SORT>
-__device__ __forceinline__ void sample_step(const SampleStepArgs& a, SamplerLds& lds, SortLds* buf)
-{
-    const int pos0 = a.state[0], n_prompt = a.state[1], advance0 = a.state[2], n_slots = a.state[3];
-    if (advance0 && threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
-        write_rope_table(a.state, threadIdx.x - 64, pos0 + 1, a.theta); // for the next step
-    if (pos0 + 1 >= n_prompt && pos0 + 1 < n_slots) { // uniform over the workgroup
-        const float coin = sampler_coin(a.seed, pos0 + 1);
-        const int token = sample_dev<LDS_SORT ? 4 : 8, LDS_SORT, true>(a.logits, a.indices, a.size, a.temperature, a.top_p,
-                                                                 coin, a.keys2, a.values2, lds, buf);
-        if (threadIdx.x == 0)
-            a.tokens[pos0 + 1] = token;
-    }
-    __syncthreads(); // every thread has read the state
-    if (threadIdx.x == 0) {
-        if (advance0)
-            a.state[0] = pos0 + 1;
-    }
-}
-
-__global__ __launch_bounds__(kSampBlock) void sample_step_kernel(SampleStepArgs a)
-{
-    __shared__ SamplerLds lds;
-    __shared__ SortLds buf;
-    sample_step<true>(a, lds, &buf);
-}
-
-__global__ __launch_bounds__(kSampBlock) void sample_step_big_kernel(SampleStepArgs a)
-{
-    __shared__ SamplerLds lds;
-    sample_step<false>(a, lds, nullptr);
 }
 
 } // namespace l2
@@ -664,16 +606,16 @@ int launch_argmax_step(llama2_decoder* d)
     return LLAMA2_OK;
 }
 
+// Sampler.Sample's stochastic branch (src/Sampler.cs:48-67) against the device
+// state: the token at pos+1 is drawn with the coin of (seed, pos+1) iff
+// pos+1 >= n_prompt; then the position advances like in argmax_step_kernel.
 int launch_sample_step(llama2_decoder* d, float temperature, float top_p, unsigned long long seed)
 {
-    SampleStepArgs a{d->s.logits, d->s.indices, d->cfg.vocab_size, d->s.tokens, d->state, ctx().sort_keys,
-                     ctx().sort_values, temperature, top_p, seed, d->cfg.rope_theta};
-    if (a.size <= kSortLdsItems)
-        hipLaunchKernelGGL(sample_step_kernel, dim3(1), dim3(kSampBlock), 0, ctx().stream, a);
-    else
-        hipLaunchKernelGGL(sample_step_big_kernel, dim3(1), dim3(kSampBlock), 0, ctx().stream, a);
-    L2_LAUNCH_CHECK("sample_step_kernel");
-    return LLAMA2_OK;
+    SampleArgs a{};
+    a.logits = d->s.logits, a.indices = d->s.indices, a.size = d->cfg.vocab_size;
+    a.temperature = temperature, a.top_p = top_p, a.head = 1;
+    a.state = d->state, a.tokens = d->s.tokens, a.seed = seed, a.theta = d->cfg.rope_theta;
+    return sample_enqueue("sampled step", a);
 }
 
 int check_sampling(const char* fn, const llama2_decoder* d, float temperature)

@@ -26,6 +26,18 @@ constexpr int kSpareTokenSlot = 4;
 constexpr int kStateSerial = 5;   // counts persistent steps (bumped right before each, by nothing else): their hand-over tags derive from it
 constexpr int kStateError = 6;    // set by the persistent step when a bounded wait gave up
 
+#if defined(__HIPCC__)
+// Entry i of the (cos, sin) table of a position's RoPE angles behind the state's ints.
+__device__ __forceinline__ void write_rope_table(int* state, int i, int pos, float theta)
+{
+    float c, s;
+    rope_cos_sin(c, s, i, kRopeHeadSize, pos, theta);
+    float* tab = reinterpret_cast<float*>(state + kStateInts);
+    tab[2 * i] = c;
+    tab[2 * i + 1] = s;
+}
+#endif
+
 struct PersistLayer { // one per layer, in device memory
     QW q, k, v, o, gate, up, down;
     const uint16_t* rms_att;

@@ -1,7 +1,7 @@
 // Runtime half of the C ABI: device context, memory, stream, events, errors.
 // Replaces what the reference gets from ManagedCuda (CudaContext,
 // CudaDeviceVariable<T>; src/Module.cs:7-26, src/RunState.cs:27-53).
-#include "common.hpp"
+#include "sampler_kernels.hpp"
 
 #include <cstdio>
 #include <cstdlib>
@@ -106,8 +106,7 @@ int llama2_init(int device)
     L2_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.attn_counters), kMaxAttnHeads * sizeof(unsigned)));
     L2_HIP(hipMemset(c.attn_counters, 0, kMaxAttnHeads * sizeof(unsigned)));
-    L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.sort_keys), LLAMA2_MAX_SAMPLER_SIZE * sizeof(uint16_t)));
-    L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.sort_values), LLAMA2_MAX_SAMPLER_SIZE * sizeof(int)));
+    L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.sampler), sizeof(SamplerScratch)));
     c.device = device;
     if (int rc = resolve_vec_mat_static_scratch(device)) {
         c.device = -1;
@@ -139,12 +138,9 @@ int llama2_shutdown(void)
     if (c.attn_counters)
         L2_HIP(hipFree(c.attn_counters));
     c.attn_counters = nullptr;
-    if (c.sort_keys)
-        L2_HIP(hipFree(c.sort_keys));
-    c.sort_keys = nullptr;
-    if (c.sort_values)
-        L2_HIP(hipFree(c.sort_values));
-    c.sort_values = nullptr;
+    if (c.sampler)
+        L2_HIP(hipFree(c.sampler));
+    c.sampler = nullptr;
     L2_HIP(hipStreamDestroy(c.stream));
     c.stream = nullptr;
     c.ready = false;

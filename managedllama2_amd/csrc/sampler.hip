@@ -1,79 +1,75 @@
 // The stochastic sampler's modules (src/SoftmaxLogits.cs, Sort.cs,
 // CumulativeSum.cs, SampleTopP.cs; kernels native/softmax_logits_kernel.cu,
 // sort_kernel.cu, cumulative_sum_kernel.cu, sample_top_p_kernel.cu) and the
-// whole stochastic branch of Sampler.Sample (src/Sampler.cs:48-67) as one launch.
-// Every kernel is one 1024-thread workgroup, like the reference's.
+// whole stochastic branch of Sampler.Sample (src/Sampler.cs:48-67).
 #include "sampler_kernels.hpp"
 
 namespace l2 {
-
-template <int CH>
-__global__ __launch_bounds__(kSampBlock) void softmax_logits_kernel(uint16_t* logits, int size, float temperature,
-                                                                    int* indices)
-{
-    __shared__ SamplerLds lds;
-    softmax_logits_dev<CH>(logits, size, temperature, indices, lds);
-}
-
-template <int CH>
-__global__ __launch_bounds__(kSampBlock) void sort_kernel(uint16_t* keys, int* values, int size, uint16_t* keys2,
-                                                          int* values2)
-{
-    __shared__ SamplerLds lds;
-    sort_dev<CH>(keys, values, size, keys2, values2, lds);
-}
-
-__global__ __launch_bounds__(kSampBlock) void sort_lds_kernel(uint16_t* keys, int* values, int size)
-{
-    __shared__ SamplerLds lds;
-    __shared__ SortLds buf;
-    sort_lds_dev<false>(keys, values, size, lds, buf);
-}
-
-template <int CH>
-__global__ __launch_bounds__(kSampBlock) void cumulative_sum_kernel(uint16_t* values, int size)
-{
-    __shared__ SamplerLds lds;
-    cumulative_sum_dev<CH>(values, size, lds);
-}
-
-template <int CH>
-__global__ __launch_bounds__(kSampBlock) void sample_top_p_kernel(const uint16_t* logits, const int* indices, int size,
-                                                                  float threshold, int* result, int pos)
-{
-    __shared__ SamplerLds lds;
-    const int token = sample_top_p_dev<CH>(logits, indices, size, threshold, lds);
-    if (threadIdx.x == 0)
-        result[pos] = token;
-}
-
-template <bool HEAD_ONLY>
-__global__ __launch_bounds__(kSampBlock) void sample_kernel(uint16_t* logits, int* indices, int size, float temperature,
-                                                            float top_p, float coin, int* result, int pos)
-{
-    __shared__ SamplerLds lds;
-    __shared__ SortLds buf;
-    const int token =
-        sample_dev<4, true, HEAD_ONLY>(logits, indices, size, temperature, top_p, coin, nullptr, nullptr, lds, &buf);
-    if (threadIdx.x == 0)
-        result[pos] = token;
-}
-
-__global__ __launch_bounds__(kSampBlock) void sample_big_kernel(uint16_t* logits, int* indices, int size,
-                                                                float temperature, float top_p, float coin, int* result,
-                                                                int pos, uint16_t* keys2, int* values2)
-{
-    __shared__ SamplerLds lds;
-    const int token = sample_dev<8, false>(logits, indices, size, temperature, top_p, coin, keys2, values2, lds, nullptr);
-    if (threadIdx.x == 0)
-        result[pos] = token;
-}
 
 int check_sampler_size(const char* fn, int size)
 {
     L2_CHECK(size > 0, "%s: size=%d must be positive", fn, size);
     if (size > LLAMA2_MAX_SAMPLER_SIZE)
         return fail(LLAMA2_ERR_UNSUPPORTED, "%s: size=%d exceeds %d", fn, size, LLAMA2_MAX_SAMPLER_SIZE);
+    return LLAMA2_OK;
+}
+
+int check_temperature(const char* fn, float temperature)
+{
+    L2_CHECK(temperature > 0.0f, "%s: temperature=%g must be positive (temperature 0 is the argmax branch)", fn,
+             static_cast<double>(temperature));
+    return LLAMA2_OK;
+}
+
+static void launch_exp(const SampleArgs& a)
+{
+    const dim3 grid(kSampBlock / kExpShare + (a.state ? 1 : 0));
+    if (sampler_chunks(a.size) == 4)
+        hipLaunchKernelGGL(sampler_exp_kernel<4>, grid, dim3(kExpThreads), 0, ctx().stream, a);
+    else
+        hipLaunchKernelGGL(sampler_exp_kernel<8>, grid, dim3(kExpThreads), 0, ctx().stream, a);
+}
+
+static void launch_rank(const SampleArgs& a, uint16_t* keys, int* values, bool identity)
+{
+    const int tiles = ceil_div(a.size, kSampTile);
+    const dim3 grid(tiles * (kSampTile / kSampRun));
+    if (tiles <= kSampTiles / 2)
+        hipLaunchKernelGGL(sampler_rank_kernel<kSampTiles / 2>, grid, dim3(kSampBlock), 0, ctx().stream, a, keys, values,
+                           identity ? 1 : 0);
+    else
+        hipLaunchKernelGGL(sampler_rank_kernel<kSampTiles>, grid, dim3(kSampBlock), 0, ctx().stream, a, keys, values,
+                           identity ? 1 : 0);
+}
+
+template <bool PICK>
+static void launch_pick(const SampleArgs& a, const uint16_t* in, bool in_place)
+{
+    const int ch = sampler_chunks(a.size);
+    const dim3 grid(in_place ? 1 : ceil_div(a.size, 64 * 8 * ch));
+    if (ch == 4)
+        hipLaunchKernelGGL((sampler_pick_kernel<4, PICK>), grid, dim3(kSampBlock), 0, ctx().stream, a, in);
+    else
+        hipLaunchKernelGGL((sampler_pick_kernel<8, PICK>), grid, dim3(kSampBlock), 0, ctx().stream, a, in);
+}
+
+int sample_enqueue(const char* name, const SampleArgs& args)
+{
+    SampleArgs a = args;
+    SamplerScratch* s = ctx().sampler;
+    a.s = s;
+    if (!sample_sorts(a.top_p))
+        a.head = -1;
+    else if (a.size > kSampHeadItems)
+        a.head = 0;
+    launch_exp(a);
+    hipLaunchKernelGGL(sampler_tile_kernel<TILE_EXPS>, dim3(ceil_div(a.size, kSampTile)), dim3(kTileThreads), 0,
+                       ctx().stream, a, static_cast<const uint16_t*>(nullptr), static_cast<const int*>(nullptr),
+                       a.head < 0 ? s->keys : a.head > 0 ? a.logits : nullptr);
+    if (a.head >= 0)
+        launch_rank(a, s->keys, a.indices, true);
+    launch_pick<true>(a, s->keys, false);
+    L2_LAUNCH_CHECK(name);
     return LLAMA2_OK;
 }
 
@@ -88,15 +84,6 @@ using namespace l2;
             return rc_;       \
     } while (0)
 
-// 8-element chunks per thread: 4 cover 32768 elements, 8 cover 65536
-#define L2_SAMPLER_LAUNCH(kernel, size, ...)                                                                   \
-    do {                                                                                                       \
-        if ((size) <= 4 * 8 * kSampBlock)                                                                      \
-            hipLaunchKernelGGL(kernel<4>, dim3(1), dim3(kSampBlock), 0, ctx().stream, __VA_ARGS__);            \
-        else                                                                                                   \
-            hipLaunchKernelGGL(kernel<8>, dim3(1), dim3(kSampBlock), 0, ctx().stream, __VA_ARGS__);            \
-    } while (0)
-
 extern "C" {
 
 int llama2_softmax_logits(llama2_half* logits, int size, float temperature, int* indices)
@@ -105,10 +92,13 @@ int llama2_softmax_logits(llama2_half* logits, int size, float temperature, int*
     const char* fn = "llama2_softmax_logits";
     L2_CHECK(logits && indices, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
-    L2_CHECK(temperature > 0.0f, "%s: temperature=%g must be positive (temperature 0 is the argmax branch)", fn,
-             static_cast<double>(temperature));
+    L2_TRY(check_temperature(fn, temperature));
     L2_CHECK(aligned(logits, 16) && aligned(indices, 16), "%s: logits and indices must be 16-byte aligned", fn);
-    L2_SAMPLER_LAUNCH(softmax_logits_kernel, size, logits, size, temperature, indices);
+    SampleArgs a{};
+    a.logits = logits, a.indices = indices, a.size = size, a.temperature = temperature, a.s = ctx().sampler, a.head = -1;
+    launch_exp(a);
+    hipLaunchKernelGGL(sampler_tile_kernel<TILE_EXPS>, dim3(ceil_div(size, kSampTile)), dim3(kTileThreads), 0, ctx().stream,
+                       a, static_cast<const uint16_t*>(nullptr), static_cast<const int*>(nullptr), logits);
     L2_LAUNCH_CHECK(fn);
     return LLAMA2_OK;
 }
@@ -120,10 +110,11 @@ int llama2_sort(llama2_half* keys, int* values, int size)
     L2_CHECK(keys && values, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
     L2_CHECK(aligned(keys, 16) && aligned(values, 16), "%s: keys and values must be 16-byte aligned", fn);
-    if (size <= kSortLdsItems)
-        hipLaunchKernelGGL(sort_lds_kernel, dim3(1), dim3(kSampBlock), 0, ctx().stream, keys, values, size);
-    else
-        L2_SAMPLER_LAUNCH(sort_kernel, size, keys, values, size, ctx().sort_keys, ctx().sort_values);
+    SampleArgs a{};
+    a.size = size, a.s = ctx().sampler;
+    hipLaunchKernelGGL(sampler_tile_kernel<TILE_KEYS>, dim3(ceil_div(size, kSampTile)), dim3(kTileThreads), 0, ctx().stream,
+                       a, keys, values, static_cast<uint16_t*>(nullptr));
+    launch_rank(a, keys, values, false);
     L2_LAUNCH_CHECK(fn);
     return LLAMA2_OK;
 }
@@ -135,7 +126,9 @@ int llama2_cumulative_sum(llama2_half* values, int size)
     L2_CHECK(values, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
     L2_CHECK(aligned(values, 16), "%s: values must be 16-byte aligned", fn);
-    L2_SAMPLER_LAUNCH(cumulative_sum_kernel, size, values, size);
+    SampleArgs a{};
+    a.logits = values, a.size = size;
+    launch_pick<false>(a, values, true);
     L2_LAUNCH_CHECK(fn);
     return LLAMA2_OK;
 }
@@ -148,7 +141,12 @@ int llama2_sample_top_p(const llama2_half* logits, const int* indices, int size,
     L2_TRY(check_sampler_size(fn, size));
     L2_CHECK(pos >= 0, "%s: pos=%d is negative", fn, pos);
     L2_CHECK(aligned(logits, 16), "%s: logits must be 16-byte aligned", fn);
-    L2_SAMPLER_LAUNCH(sample_top_p_kernel, size, logits, indices, size, threshold, result, pos);
+    if (sampler_chunks(size) == 4)
+        hipLaunchKernelGGL(sample_top_p_kernel<4>, dim3(1), dim3(kSampBlock), 0, ctx().stream, logits, indices, size,
+                           threshold, result, pos);
+    else
+        hipLaunchKernelGGL(sample_top_p_kernel<8>, dim3(1), dim3(kSampBlock), 0, ctx().stream, logits, indices, size,
+                           threshold, result, pos);
     L2_LAUNCH_CHECK(fn);
     return LLAMA2_OK;
 }
@@ -169,21 +167,14 @@ int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, floa
 {
     L2_CHECK(logits && indices && result, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
-    L2_CHECK(temperature > 0.0f, "%s: temperature=%g must be positive (temperature 0 is the argmax branch)", fn,
-             static_cast<double>(temperature));
+    L2_TRY(check_temperature(fn, temperature));
     L2_CHECK(pos >= 0, "%s: pos=%d is negative", fn, pos);
     L2_CHECK(aligned(logits, 16) && aligned(indices, 16), "%s: logits and indices must be 16-byte aligned", fn);
-    if (size <= kSortLdsItems && token_only)
-        hipLaunchKernelGGL(sample_kernel<true>, dim3(1), dim3(kSampBlock), 0, ctx().stream, logits, indices, size,
-                           temperature, top_p, coin, result, pos);
-    else if (size <= kSortLdsItems)
-        hipLaunchKernelGGL(sample_kernel<false>, dim3(1), dim3(kSampBlock), 0, ctx().stream, logits, indices, size,
-                           temperature, top_p, coin, result, pos);
-    else
-        hipLaunchKernelGGL(sample_big_kernel, dim3(1), dim3(kSampBlock), 0, ctx().stream, logits, indices, size,
-                           temperature, top_p, coin, result, pos, ctx().sort_keys, ctx().sort_values);
-    L2_LAUNCH_CHECK(fn);
-    return LLAMA2_OK;
+    SampleArgs a{};
+    a.logits = logits, a.indices = indices, a.size = size;
+    a.temperature = temperature, a.top_p = top_p, a.coin = coin, a.result = result, a.pos = pos;
+    a.head = token_only ? 1 : 0;
+    return sample_enqueue(fn, a);
 }
 
 } // namespace l2

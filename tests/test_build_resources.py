@@ -1,8 +1,7 @@
 """Register allocation of the built kernels.  A kernel whose private (scratch) memory grows into
 kilobytes per lane still computes the right thing, so no parity test notices, but every launch
-then pays for a scratch allocation of its own (measured: 1.7 ms instead of 70 us for the
-one-launch sampler).  The sampler's phases are non-inlined calls precisely to keep the register
-allocator from spilling; this compiles every translation unit of the library and reads the
+then pays for a scratch allocation of its own (measured on an earlier, one-launch sampler: 1.7 ms
+instead of 70 us).  This compiles every translation unit of the library and reads the
 compiler's own resource report.
 
 The same compile also yields the device assembly, which must hold no packed fp32 arithmetic

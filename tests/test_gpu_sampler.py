@@ -252,3 +252,51 @@ class TestSample:
         for i in range(n):
             counts[fused_sample(logits, T, 1.0, (i + 0.5) / n)[0]] += 1
         assert np.max(np.abs(counts / n - p)) < 5e-3
+
+
+class TestTileEdges:
+    """The sort works on tiles of 1024 keys that are placed among each other in runs of 128, the exponentials and the
+    prefix sums on 32 values per thread up to 32768 keys and 64 beyond: sizes around those."""
+    SIZES = [127, 128, 129, 1023, 1024, 1025, 2047, 2049, 32255, 32256, 32257, 32767, 65535]
+
+    @pytest.mark.parametrize("size", SIZES)
+    @pytest.mark.parametrize("keys", ["few", "equal", "falling", "rising", "special"])
+    def test_sort(self, oracle, size, keys):
+        rng = synth.rng_for(951, size)
+        if keys == "few":  # every key many times, in every tile
+            k = rng.integers(-3, 4, size).astype(np.float16)
+        elif keys == "equal":
+            k = np.full(size, 0.25, np.float16)
+        elif keys == "special":
+            bits = np.array([0x0000, 0x8000, 0x7C00, 0xFC00, 0xFBFF, 0x7BFF, 0x0001, 0x8001, 0x3C00], np.uint16)
+            k = bits[rng.integers(0, bits.size, size)].view(np.float16)
+        else:
+            k = np.sort(synth.normal_f16(rng, size, 3.0))[::-1 if keys == "falling" else 1]
+        v = rng.integers(-2 ** 31, 2 ** 31 - 1, size).astype(np.int32)
+        got, values = Sort(np.ascontiguousarray(k), v)
+        want, wvalues = oracle.ref_sort(np.ascontiguousarray(k), v)
+        assert np.array_equal(got.view(np.uint16), want.view(np.uint16)) and np.array_equal(values, wvalues)
+
+    @pytest.mark.parametrize("size", SIZES)
+    def test_sample(self, oracle, size):
+        rng = synth.rng_for(952, size)
+        logits = synth.normal_f16(rng, size, 3.0)
+        logits[rng.integers(0, size, size // 4)] = -np.inf  # masked tokens
+        for top_p in (0.9, 1.0):
+            t1, cdf1, idx1 = fused_sample(logits, 0.7, top_p, 0.61)
+            t2, cdf2, idx2 = module_sample(logits, 0.7, top_p, 0.61)
+            assert t1 == t2 and np.array_equal(idx1, idx2)
+            assert np.array_equal(cdf1.view(np.uint16), cdf2.view(np.uint16))
+            assert t1 == oracle.ref_sample_top_p(cdf1, idx1, float(np.float32(0.61) * np.float32(top_p)))
+            assert logits[t1] > -np.inf
+
+    @pytest.mark.parametrize("size", [1000, 32000, 65536])
+    def test_infinite_logits_and_temperatures(self, size):
+        x = synth.normal_f16(synth.rng_for(953, size), size, 2.0)
+        flat, _ = SoftmaxLogits(x, float("inf"))  # every quotient is 0
+        assert np.all(flat == np.float16(1.0 / size))
+        x[size // 2] = np.inf
+        got, _ = SoftmaxLogits(x, 0.5)
+        assert np.all(np.isnan(got))  # exp(inf - inf), as in the reference
+        got, _ = SoftmaxLogits(np.full(size, -np.inf, np.float16), 0.5)
+        assert np.all(np.isnan(got))

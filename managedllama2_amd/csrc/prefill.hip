@@ -12,7 +12,7 @@
 // the group's scale applied in fp32, fp32 sums over the groups; scores rounded to fp16, softmax
 // statistics in fp32, probabilities with all the bits of fp32.  The order of the sums is not that of the decode step.
 //
-// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 11.3 ms;
+// Measured, Llama-2-7B: 512 prompt tokens one by one 560 ms, 511 in one batch and the last as a step 10.7 ms;
 // 13B, 74 tokens behind 600 rows: 151 -> 7 ms.
 #include "int4_kernels.hpp"
 #include "prefill.hpp"
@@ -20,6 +20,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 namespace l2 {
 
@@ -148,19 +149,16 @@ struct GemmArgs {
     const float* rope;
 };
 
-// 8 nibbles of a word as fp16 n - z, exact: n sits in the mantissa of 1024 + n (bits 0-3 of a half) or
+// Pair k of the 8 nibbles of a word as fp16 n - z, exact: n sits in the mantissa of 1024 + n (bits 0-3 of a half) or
 // 1024 + 16 n (bits 4-7).
-__device__ __forceinline__ h8_t dequant(uint32_t w, h2_t zlo /* 1024 + z */, h2_t zhi /* -(64 + z) */)
+__device__ __forceinline__ uint32_t dequant_pair(uint32_t w, int k, h2_t zlo /* 1024 + z */, h2_t zhi /* -(64 + z) */)
 {
     const h2_t sixteenth = {static_cast<_Float16>(0.0625f), static_cast<_Float16>(0.0625f)};
-    const uint32_t w8 = w >> 8;
     uint32_t magic = 0x64006400u; // in a vector register: (w & mask) | magic is one instruction then
     asm("" : "+v"(magic));
-    const h2_t a = as_h2((w & 0x000F000Fu) | magic) - zlo;
-    const h2_t b = __builtin_elementwise_fma(as_h2((w & 0x00F000F0u) | magic), sixteenth, zhi);
-    const h2_t c = as_h2((w8 & 0x000F000Fu) | magic) - zlo;
-    const h2_t d = __builtin_elementwise_fma(as_h2((w8 & 0x00F000F0u) | magic), sixteenth, zhi);
-    return h8_t{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+    const uint32_t v = k >= 2 ? w >> 8 : w;
+    return k & 1 ? as_u32(__builtin_elementwise_fma(as_h2((v & 0x00F000F0u) | magic), sixteenth, zhi))
+                 : as_u32(as_h2((v & 0x000F000Fu) | magic) - zlo);
 }
 
 __device__ __forceinline__ f16v_t mfma(h8_t a, h8_t b, f16v_t c)
@@ -191,21 +189,35 @@ __device__ __forceinline__ void load_to_lds_x1(const void* p, uint32_t lds)
 // s_waitcnt vmcnt(n), the other counters free
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }
 
+template <int N, typename F>
+__device__ __forceinline__ void static_for(const F& f) // f(0) .. f(N - 1), the index as a constant
+{
+    [&]<int... I>(std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+    (std::make_integer_sequence<int, N>{});
+}
+
 // A workgroup owns MT token tiles and WN pairs of weight tiles of 32 rows; the two tiles of a pair hold
 // results that belong together (the two halves of a RoPE pair, gate and up, or neighbours).  8 wavefronts: one per
 // weight tile and group, a step covers WK consecutive groups of K.  At the end the WK sums add up, and the tiles
 // of a pair meet, through LDS.  The launch may split K further (EPI_PARTIAL).
 //
-// What bounds it: a group costs a wavefront MT x 256 cycles of its matrix core (two wavefronts share one), about 400 of
-// its vector unit to unpack the weights and MT x 100 to scale the sums, and the two units hardly overlap: over the
-// SwiGLU launch of 511 rows of 7B (135 us) the matrix cores are busy 32 %, the vector units 38 % of the time, without an LDS
-// bank conflict.  The rest has to stay out of the way:
+// What bounds it: the power the matrix cores take.  A step of four tiles is 1024 cycles of matrix products per wavefront, two
+// wavefronts to a SIMD, and takes 2990; the clock falls from 2.4 to 1.6 .. 2.0 GHz while it lasts (a loop of
+// nothing but these products on random numbers, with their LDS reads, runs at 1.8).  7B, 511 rows, QKV: 1.08 PFLOP/s over the
+// steps, where a library product of 8192^3 reaches 1.16.  What is left is the 3.5 us to the first step and 4 us behind the
+// last, and rounds of workgroups that do not fill the card.  So the vector work and the loads stay out of the way:
+// - Vector work runs beside the matrix products only where it stands between them (5 instructions for one product
+//   of 32 cycles cost nothing, 8 cost 12 cycles); left to the compiler the unpacking and the scaled sums came after the
+//   products of their step, 5000 cycles for four tiles.
 // - A compute unit looks up one cache address per cycle and 64 contiguous bytes.  A lane that reads its own row's
 //   weights costs 64 lookups per load (13.2 ms instead of 11.9 for the 512-token prompt).  Everything
 //   comes through LDS, requested in the order of memory; LDS delivers 256 bytes per cycle where 16 neighbouring
 //   lanes meet all banks, hence the swizzle of the weight rows.
 // - One barrier per step, LDS for three: activations are requested two steps ahead, weights three, because
-//   they are unpacked into registers a step ahead, each fragment under the last products that need its predecessor.
+//   they are unpacked into registers a step ahead.
+// - Results leave in pieces of 16 bytes after one exchange of all tiles through LDS, their RoPE angles requested
+//   before it: stored as they lie in the registers, 2 bytes per lane and tile by tile, they took 25 us of the 72 of QKV.
+// 7B, 511 rows: QKV 76 -> 62 us; the whole 512-token prompt 11.25 -> 10.75 ms.
 template <int MT, int WN, int WK, int EPI>
 __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
 {
@@ -215,7 +227,8 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
     constexpr int kWStage = WN * 2 * kTile * kWRow; // weights of a step
     constexpr int kZStage = 8 * 256;                // a word with the scale and one with the zero point per row and group
     constexpr int kWAt = 3 * kXStage, kZAt = kWAt + 3 * kWStage, kAll = kZAt + 3 * kZStage;
-    constexpr int kRed = 8 * 16 * 64 * 4;
+    constexpr int kRedRow = kTile + 4, kRed = 8 * MT * kTile * kRedRow * 4;
+    static_assert(kRed <= 160 * 1024, "LDS of a compute unit");
     static_assert(kAll <= 160 * 1024, "LDS of a compute unit");
     __shared__ __align__(1024) char lds[kAll > kRed ? kAll : kRed];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -313,23 +326,35 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
         load_to_lds_x1(zs_base + (h ? (g >> 3) * 4 : (s_odd + 2 * g) & ~3), lds_base + kZAt + at * kZStage + wave * 256);
     };
 
-    f16v_t acc[MT];
+    // The products of a step are one sequence, tile by tile and fragment by fragment; every product is a slot that also
+    // holds a share of the vector work, pinned there by scheduling fences: the activations of three slots later, the
+    // next step's weights, and the scaled sum of the tile before (whose last product needs two slots to finish).
+    constexpr int N = MT * 8, kAhead = 3, kRing = kAhead + 1, kFirstPair = 3;
+    f16v_t acc[MT], p[2];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
         acc[mt] = f16v_t{};
+    p[0] = p[1] = f16v_t{};
     u32x4 raw[2];
-    h8_t wf[8]; // the current group's weights, n - z in fp16
+    u32x4 wf[2][8]; // weights of this step's group and of the next one's, n - z in fp16
     h2_t zlo, zhi;
-    float sc = 0.0f, sc_next = 0.0f;
-    auto read_w = [&](int step, int at) {
+    float sc = 0.0f, sc_next = 0.0f, sc_pending = 0.0f; // scales of this group, the next, and of the sums still in p
+    uint32_t zword;
+    uint16_t sbits;
+    auto read_w = [&](int step, int at) { // what it reads is used later than the slots before
         const int r = (wn * 2 + t) * kTile + l31, g = group_of(step);
         const char* from = lds + kWAt + at * kWStage + r * kWRow;
+        const char* sz = lds + kZAt + at * kZStage + wave * 256 + l31 * 4;
+        sbits = *reinterpret_cast<const uint16_t*>(sz + ((s_odd + 2 * g) & 2));
+        zword = *reinterpret_cast<const uint32_t*>(sz + 128);
 #pragma unroll
         for (int i = 0; i < 2; ++i)
             raw[i] = *reinterpret_cast<const u32x4*>(from + ((wk * 4 + h * 2 + i) ^ swizzle(r)) * 16);
-        const char* sz = lds + kZAt + at * kZStage + wave * 256 + l31 * 4;
-        sc_next = half_bits_to_float(*reinterpret_cast<const uint16_t*>(sz + ((s_odd + 2 * g) & 2)));
-        const float z = static_cast<float>((*reinterpret_cast<const uint32_t*>(sz + 128) >> ((g & 7) * 4)) & 0xFu);
+    };
+    auto unpack_sz = [&](int step) {
+        sc_next = half_bits_to_float(sbits);
+        asm("" : "+v"(sc_next)); // a float from here on: the multiply-adds take it as one
+        const float z = static_cast<float>((zword >> ((group_of(step) & 7) * 4)) & 0xFu);
         const _Float16 lo = static_cast<_Float16>(1024.0f + z), hi = static_cast<_Float16>(-64.0f - z);
         zlo = h2_t{lo, lo}, zhi = h2_t{hi, hi};
     };
@@ -346,104 +371,156 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
     wait_all_but(std::integral_constant<int, 2 * kLoads>{});
     __syncthreads();
     read_w(0, 0);
+    unpack_sz(0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-        wf[j] = dequant(raw[j >> 2][j & 3], zlo, zhi);
+    for (int k = 0; k < 32; ++k)
+        wf[0][k >> 2][k & 3] = dequant_pair(raw[k >> 4][(k >> 2) & 3], k & 3, zlo, zhi);
     int s0 = 0, s1 = 1, s2 = 2; // LDS of this step, the next and the one after it
-    for (int step = 0; step < steps; ++step) {
+    auto flush = [&](int tile, int sum, int from, int to) { // results from .. to - 1 of p[sum] into a tile's sums
+#pragma unroll
+        for (int i = from; i < to; ++i)
+            acc[tile][i] = __builtin_fmaf(p[sum][i], sc_pending, acc[tile][i]);
+    };
+    auto body = [&](auto parity, int step) {
+        constexpr int P = decltype(parity)::value;
+        constexpr int kFirst = P * MT & 1; // the sums' register of the first tile; the other one holds the last tile before
         // this step's activations and the next one's weights; every wavefront is through with the step before
         wait_all_but(std::integral_constant<int, kLoads>{});
         __syncthreads();
+        const char* xs = lds + s0 * kXStage + wk * MT * kBlockBytes + lane * 16;
+        h8_t xa[kRing];
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+            xa[i] = *reinterpret_cast<const h8_t*>(xs + (i >> 3) * kBlockBytes + (i & 7) * kFragBytes);
+        read_w(step + 1, s1);
         load_x(step + 2, s2);
         load_w(step + 3, s0);
         sc = sc_next;
-        read_w(step + 1, s1);
-        if (g_begin + step * WK + wk < g_end) {
-            const char* xs = lds + s0 * kXStage + wk * MT * kBlockBytes + lane * 16;
-            f16v_t p[MT];
-            h8_t xa[2][MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) {
-                p[mt] = f16v_t{};
-                xa[0][mt] = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (j + 1 < 8) {
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        xa[(j + 1) & 1][mt] = *reinterpret_cast<const h8_t*>(xs + mt * kBlockBytes + (j + 1) * kFragBytes);
+        if (WK == 1 || g_begin + step * WK + wk < g_end) {
+            static_for<N>([&](auto slot) {
+                constexpr int i = decltype(slot)::value, mt = i >> 3, j = i & 7;
+                if constexpr (i + kAhead < N) {
+                    constexpr int n = i + kAhead;
+                    xa[n % kRing] = *reinterpret_cast<const h8_t*>(xs + (n >> 3) * kBlockBytes + (n & 7) * kFragBytes);
                 }
+                f16v_t& q = p[(kFirst + mt) & 1];
+                q = mfma(xa[i % kRing], __builtin_bit_cast(h8_t, wf[P][j]), j == 0 ? f16v_t{} : q);
+                if (i == 2)
+                    unpack_sz(step + 1);
+                if constexpr (j >= 2) // 16 results over the slots 2 .. 7
+                    flush(mt == 0 ? MT - 1 : mt - 1, (kFirst + mt + 1) & 1, (j - 2) * 8 / 3, (j - 1) * 8 / 3);
+                if (j == 7)
+                    sc_pending = sc;
+                if constexpr (i >= kFirstPair) {
+                    constexpr int from = (i - kFirstPair) * 32 / (N - kFirstPair), to = (i - kFirstPair + 1) * 32 / (N - kFirstPair);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    p[mt] = mfma(xa[j & 1][mt], wf[j], p[mt]);
-                wf[j] = dequant(raw[j >> 2][j & 3], zlo, zhi);
-                __builtin_amdgcn_sched_barrier(0x2); // vector arithmetic alone may move
-            }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int i = 0; i < 16; ++i)
-                    acc[mt][i] = __builtin_fmaf(p[mt][i], sc, acc[mt][i]);
+                    for (int k = from; k < to; ++k)
+                        wf[P ^ 1][k >> 2][k & 3] = dequant_pair(raw[k >> 4][(k >> 2) & 3], k & 3, zlo, zhi);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else { // the last step of a piece that has no group for this wavefront
+            flush(MT - 1, (kFirst + 1) & 1, 0, 16);
+            sc_pending = 0.0f;
+            p[0] = p[1] = f16v_t{};
         }
         const int s = s0;
         s0 = s1, s1 = s2, s2 = s;
+    };
+    int step = 0;
+    for (; step + 1 < steps; step += 2) {
+        body(std::integral_constant<int, 0>{}, step);
+        body(std::integral_constant<int, 1>{}, step + 1);
+    }
+    if (step < steps) {
+        body(std::integral_constant<int, 0>{}, step);
+        flush(MT - 1, (MT - 1) & 1, 0, 16);
+    } else {
+        flush(MT - 1, (2 * MT - 1) & 1, 0, 16);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing may still write LDS
     __syncthreads();
 
-    constexpr int SHARE = 16 / (2 * WK); // registers of both tiles that a wavefront adds up
+    // Rows of 32 results lie kRedRow floats apart; a thread takes 8 neighbours of both tiles of the pair.
     const bool mine = nb * WN + wn < a.pairs;
     int tensor0, row_a, row_b;
     tile_of(nb * WN + wn, 1, tensor0, row_b);
     tile_of(nb * WN + wn, 0, tensor0, row_a);
-    float* red = reinterpret_cast<float*>(lds);
-    auto red_at = [&](int w, int tile, int i) { return red + (((w * WN + wn) * 2 + tile) * 16 + i) * 64 + lane; };
+    constexpr int kPasses = (MT + WK - 1) / WK; // 128 WK threads for MT x 128 such pieces
+    const int piece = (wk * 2 + t) * 64 + lane;
+    auto row_of = [&](int pass) { return (piece + pass * 128 * WK) >> 2; };
+    const int n8 = (piece & 3) * 8;
+    float4 angles[EPI == EPI_QKV ? kPasses : 1][4];
+    if (EPI == EPI_QKV && tensor0 < 2) { // requested together, before the results are exchanged
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        if (mt)
-            __syncthreads();
+        for (int pass = 0; pass < kPasses; ++pass) {
+            const int m = mt0 * kTile + row_of(pass);
+            const float* cs = a.rope + (static_cast<size_t>(m < a.M ? m : a.M - 1) * 64 + (row_a & 63) + n8) * 2;
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                angles[pass][k] = reinterpret_cast<const float4*>(cs)[k];
+        }
+    }
+    float* red = reinterpret_cast<float*>(lds);
+    auto red_at = [&](int w, int tile, int row) { return red + (((w * WN + wn) * 2 + tile) * MT * kTile + row) * kRedRow; };
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-            *red_at(wk, t, i) = acc[mt][i];
-        __syncthreads();
+            red_at(wk, t, mt * kTile + 8 * (i >> 2) + 4 * h + (i & 3))[l31] = acc[mt][i];
+    __syncthreads();
 #pragma unroll
-        for (int u = 0; u < SHARE; ++u) {
-            const int i = (wk * 2 + t) * SHARE + u;
-            float v0 = 0.0f, v1 = 0.0f;
+    for (int pass = 0; pass < kPasses; ++pass) {
+        const int row = row_of(pass), m = mt0 * kTile + row;
+        if (row >= MT * kTile || m >= a.M || !mine)
+            continue;
+        float v0[8] = {}, v1[8] = {};
 #pragma unroll
-            for (int w = 0; w < WK; ++w) {
-                v0 += *red_at(w, 0, i);
-                v1 += *red_at(w, 1, i);
+        for (int w = 0; w < WK; ++w)
+#pragma unroll
+            for (int k = 0; k < 8; k += 4) {
+                const float4 r0 = *reinterpret_cast<const float4*>(red_at(w, 0, row) + n8 + k);
+                const float4 r1 = *reinterpret_cast<const float4*>(red_at(w, 1, row) + n8 + k);
+                v0[k] += r0.x, v0[k + 1] += r0.y, v0[k + 2] += r0.z, v0[k + 3] += r0.w;
+                v1[k] += r1.x, v1[k + 1] += r1.y, v1[k + 2] += r1.z, v1[k + 3] += r1.w;
             }
-            const int m = (mt0 + mt) * kTile + 8 * (i >> 2) + 4 * h + (i & 3);
-            if (m >= a.M || !mine)
-                continue;
-            if (EPI == EPI_QKV) {
-                // q and k are rounded to fp16 before RoPE reads them (native/rope_kernel.cu:14-26)
-                uint16_t b0 = float_to_half_bits(v0), b1 = float_to_half_bits(v1);
+        if (EPI == EPI_QKV) {
+            // q and k are rounded to fp16 before RoPE reads them (native/rope_kernel.cu:14-26)
+            u32x4 oa, ob;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                uint16_t b0 = float_to_half_bits(v0[k]), b1 = float_to_half_bits(v1[k]);
                 if (tensor0 < 2) {
-                    const int idx = (row_a & 63) + l31;
-                    const float* cs = a.rope + (static_cast<size_t>(m) * 64 + idx) * 2;
-                    rope_rotate(b0, b1, half_bits_to_float(b0), half_bits_to_float(b1), cs[0], cs[1]);
+                    const float4 cs = angles[pass][k >> 1];
+                    rope_rotate(b0, b1, half_bits_to_float(b0), half_bits_to_float(b1), k & 1 ? cs.z : cs.x,
+                                k & 1 ? cs.w : cs.y);
                 }
-                uint16_t* o = a.out[tensor0] + static_cast<size_t>(m) * a.N;
-                o[row_a + l31] = b0;
-                o[row_b + l31] = b1;
-            } else if (EPI == EPI_PARTIAL) {
-                float* o = a.parts + (static_cast<size_t>(split) * a.part_rows + m) * a.N;
-                o[row_a + l31] = v0;
-                o[row_b + l31] = v1;
-            } else {
-                const int n = row_a + l31;
-                if (n < a.N) {
-                    float v = v0;
+                oa[k >> 1] = k & 1 ? oa[k >> 1] | static_cast<uint32_t>(b0) << 16 : b0;
+                ob[k >> 1] = k & 1 ? ob[k >> 1] | static_cast<uint32_t>(b1) << 16 : b1;
+            }
+            uint16_t* o = a.out[tensor0] + static_cast<size_t>(m) * a.N + n8;
+            *reinterpret_cast<u32x4*>(o + row_a) = oa;
+            *reinterpret_cast<u32x4*>(o + row_b) = ob;
+        } else if (EPI == EPI_PARTIAL) {
+            float* o = a.parts + (static_cast<size_t>(split) * a.part_rows + m) * a.N + n8;
+#pragma unroll
+            for (int k = 0; k < 8; k += 4) {
+                *reinterpret_cast<float4*>(o + row_a + k) = make_float4(v0[k], v0[k + 1], v0[k + 2], v0[k + 3]);
+                *reinterpret_cast<float4*>(o + row_b + k) = make_float4(v1[k], v1[k + 1], v1[k + 2], v1[k + 3]);
+            }
+        } else {
+            const int n = row_a + n8; // N is a multiple of 8
+            if (n < a.N) {
+                u32x4 o;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    float v = v0[k];
                     v *= 1.0f / (1.0f + expf(-v)); // native/mat_vec_kernel.cu:219-221
-                    v *= v1;
-                    const int e = n & 7;
-                    *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(a.out[0]) + frag_offset(m, n, a.out_groups) +
-                                                 2 * ((e & 3) * 2 + (e >> 2))) = float_to_half_bits(v);
+                    v *= v1[k];
+                    const uint32_t bits = float_to_half_bits(v);
+                    o[k >> 1] = k & 1 ? o[k >> 1] | bits << 16 : bits;
                 }
+                *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(a.out[0]) + frag_offset(m, n, a.out_groups)) = frag_order(o);
             }
         }
     }

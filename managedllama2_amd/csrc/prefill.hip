@@ -96,25 +96,40 @@ __global__ __launch_bounds__(256) void prefill_norm_kernel(NormArgs a)
     p.load(src, a.K);
     g.load(a.gamma, a.K);
     if (a.parts) {
+        // Four pieces are requested together: one after the other each waited for the one before (511 rows, four
+        // pieces: 10.5 us, together 9.8; 74 rows of 13B with six 7.2 and 6.0).
+        constexpr int kTogether = 4;
+        float sum[PIECES][8] = {};
+        for (int t0 = 0; t0 < a.n_parts; t0 += kTogether) {
+            u32x4 q[kTogether][PIECES][2];
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) {
-            const int k = (threadIdx.x + i * 256) * 8;
-            if (k >= a.K)
-                continue;
-            float sum[8] = {};
-            for (int t = 0; t < a.n_parts; ++t) {
-                const float* q = a.parts + (static_cast<size_t>(t) * a.part_rows + m) * a.K + k;
+            for (int u = 0; u < kTogether; ++u) {
+                // behind the last piece a buffer of no length, which reads as zero and moves no data
+                const bool have = t0 + u < a.n_parts;
+                const __amdgpu_buffer_rsrc_t r =
+                    make_rsrc(a.parts + (static_cast<size_t>(have ? t0 + u : 0) * a.part_rows + m) * a.K, have ? a.K * 4 : 0);
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    sum[e] += q[e];
+                for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        q[u][i][e] = __builtin_amdgcn_raw_buffer_load_b128(r, (threadIdx.x + i * 256) * 32 + e * 16, 0, 0);
             }
+#pragma unroll
+            for (int u = 0; u < kTogether; ++u)
+#pragma unroll
+                for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        sum[i][e] += __uint_as_float(q[u][i][e >> 2][e & 3]);
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const h2_t x = as_h2(p.v[i][e]);
-                p.v[i][e] = static_cast<uint32_t>(float_to_half_bits(sum[2 * e] + static_cast<float>(x[0]))) |
-                            static_cast<uint32_t>(float_to_half_bits(sum[2 * e + 1] + static_cast<float>(x[1]))) << 16;
+                p.v[i][e] = static_cast<uint32_t>(float_to_half_bits(sum[i][2 * e] + static_cast<float>(x[0]))) |
+                            static_cast<uint32_t>(float_to_half_bits(sum[i][2 * e + 1] + static_cast<float>(x[1]))) << 16;
             }
-        }
     }
     if (a.embedding || a.parts) {
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(row, a.K * 2);
@@ -534,33 +549,31 @@ struct GemmShape {
 
 constexpr int kMaxSplits = 8;
 
-// The cheapest of the shapes that fit into LDS, by an estimate in cycles: workgroups run one per compute unit in
-// rounds of equal length, a round is its steps plus filling and draining the pipeline, and every piece of K
-// beyond the first costs the norm that adds them up another reading (about 1024 values per cycle).
-// Cycles of a step at 2.4 GHz in launches of 20 steps and more, tiles 1 / 2 / 3 / 4: 2300 .. 2400 / 2900 .. 3100 /
-// 3900 .. 4400 / 4650 .. 5400, which the table follows but for one tile; several groups per step (more activations per
-// result) add 200 .. 600.  Of 68 launches of 7B and 13B with 32 to 1003 rows those with pieces of 16 steps or more take 0.93 to
-// 1.25 times the estimate, those with fewer 1.2 to 1.75 times: filling the pipeline and storing the sums of the pieces.
-// The estimate does not see that each of the 8 XCDs gets whole blocks of weights, so that some may need one more round
-// (13B, 1003 rows, o-proj: 20 blocks x 11, 33 workgroups on 32 compute units, 123 us instead of 69).  What the choice
-// gives, against blocks of 64 tokens by 256 weight rows for every size: 7B, 511 rows, QKV 86 -> 76 us (192 workgroups
-// in one round instead of 384 in two), down-proj 66 -> 54; 13B, 74 rows, QKV 42 -> 32.
+// The cheapest of the shapes that fit into LDS, by an estimate in ns that was fitted to the times of 700 launches of 7B and
+// 13B (all shapes, 32 to 1003 rows): a launch takes 4.3 us, every round of workgroups (one per compute unit) 3.1 us to fill
+// and drain and its steps; the last round's steps go faster the fewer compute units it has, because the clock follows the
+// power that the matrix cores take.  Blocks of weights go to the 8 XCDs in turn, so the rounds are those of the XCD with the
+// most blocks.  A piece of K is written and read once more at about 4.5 TB/s.  Over those launches the shapes
+// picked take 0.8 % more than the best ones of each size together; with the XCDs and the clock left out 3.4 % (13B, 1003
+// rows, o-proj: 20 blocks of 11, 33 workgroups on 32 compute units, 131 us instead of 89).
 static GemmShape gemm_shape(int tiles, int pairs, int groups, bool may_split)
 {
-    static constexpr int kStepCycles[5] = {0, 1900, 2900, 3950, 5000};
-    static constexpr int kFixed = 8000, kWideStep = 400;
-    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
+    static constexpr int kStepNs[5] = {0, 900, 1330, 1710, 2070}; // by token tiles, one group of K
+    static constexpr int kLaunchNs = 4300, kRoundNs = 3100, kXcds = 8;
+    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256, per_xcd = cus >= kXcds ? cus / kXcds : 1;
     GemmShape best{};
     long long least = -1;
     for (int wn = 4; wn >= 1; wn /= 2)
         for (int mt = wn; mt >= 1; --mt)
             for (int splits = 1; splits <= (may_split ? kMaxSplits : 1) && (splits == 1 || splits * 4 <= groups); ++splits) {
                 const int wk = 4 / wn;
-                const long long units = static_cast<long long>(ceil_div(tiles, mt)) * ceil_div(pairs, wn) * splits;
-                const int steps = ceil_div(ceil_div(groups, splits), wk);
-                const long long step = kStepCycles[mt] + (wk > 1 ? kWideStep : 0);
-                const long long cost = (units + cus - 1) / cus * (steps * step + kFixed) +
-                                       static_cast<long long>(splits - 1) * tiles * kTile * pairs * 64 / 1024;
+                const int units = ceil_div(ceil_div(pairs, wn) * splits, kXcds) * ceil_div(tiles, mt); // of one XCD
+                const int rounds = ceil_div(units, per_xcd), last = units - (rounds - 1) * per_xcd;
+                const long long steps = ceil_div(ceil_div(groups, splits), wk);
+                const long long step = kStepNs[mt] * (wk > 1 ? 107 : 100) / 100;
+                const long long cost = kLaunchNs + kRoundNs * rounds +
+                                       steps * step * ((rounds - 1) * 10 * per_xcd + 6 * per_xcd + 4 * last) / (10 * per_xcd) +
+                                       (may_split ? static_cast<long long>(splits) * tiles * kTile * pairs * 64 * 4 / 4500 : 0);
                 if (least < 0 || cost < least)
                     least = cost, best = GemmShape{mt, wn, splits};
             }

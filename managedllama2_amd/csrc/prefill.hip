@@ -204,11 +204,10 @@ __device__ __forceinline__ void load_to_lds_x1(const void* p, uint32_t lds)
 // s_waitcnt vmcnt(n), the other counters free
 constexpr int wait_vm(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }
 
-template <int N, typename F>
-__device__ __forceinline__ void static_for(const F& f) // f(0) .. f(N - 1), the index as a constant
+template <typename F, int... I>
+__device__ __forceinline__ void static_for(const F& f, std::integer_sequence<int, I...>) // f(0), f(1) ... with constant indices
 {
-    [&]<int... I>(std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-    (std::make_integer_sequence<int, N>{});
+    (f(std::integral_constant<int, I>{}), ...);
 }
 
 // A workgroup owns MT token tiles and WN pairs of weight tiles of 32 rows; the two tiles of a pair hold
@@ -412,7 +411,7 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
         load_w(step + 3, s0);
         sc = sc_next;
         if (WK == 1 || g_begin + step * WK + wk < g_end) {
-            static_for<N>([&](auto slot) {
+            static_for([&](auto slot) {
                 constexpr int i = decltype(slot)::value, mt = i >> 3, j = i & 7;
                 if constexpr (i + kAhead < N) {
                     constexpr int n = i + kAhead;
@@ -433,7 +432,7 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
                         wf[P ^ 1][k >> 2][k & 3] = dequant_pair(raw[k >> 4][(k >> 2) & 3], k & 3, zlo, zhi);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-            });
+            }, std::make_integer_sequence<int, N>{});
         } else { // the last step of a piece that has no group for this wavefront
             flush(MT - 1, (kFirst + 1) & 1, 0, 16);
             sc_pending = 0.0f;

@@ -10,8 +10,7 @@
 //     zero without any lane predication);
 //   * a wavefront owns a span of consecutive rows, all wavefronts resident at once, the row
 //     sequence fully unrolled with the next row's loads in flight while the current one is
-//     reduced (int4_matvec_span_kernel: every launch of the 7B shapes, and of the 13B ones all but
-//     the decode step's QKV launch, whose wavefronts of one row do not fit at once: 12.2 us there); the
+//     reduced (int4_matvec_span_kernel: every launch of the 7B and 13B shapes); the
 //     two older kernels (persistent wavefronts that stride over the rows, one row or a block of
 //     rows per item) take the launches it refuses;
 //   * the input vector is staged once per workgroup in LDS, pre-permuted to
@@ -698,8 +697,13 @@ struct SpanPlan {
 // Scale words (pairs of fp16) a lane fetches per tensor: ROWS rows of at most 16 J scales each.
 constexpr int span_scale_words(int J, int ROWS) { return (ROWS * 16 * J + 127) / 128; }
 
+// QKV + RoPE: wavefronts per SIMD that the registers have to leave room for.  Its N / 8 workgroups of one row per
+// wavefront are all there at once with 3 to a compute unit where dim is 4097 .. 6144; left alone the compiler requests all rows
+// ahead and takes 124 registers, two workgroups.  13B: 12.0 us by wavefronts that stride over the rows, 11.2 like this.
+constexpr int span_waves_per_simd(int J, int MODE) { return MODE == QKV_ROPE && J == 3 ? 6 : 1; }
+
 template <int J, int MODE, int STAGE, int TN, int WAVES, int ROWS>
-__global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a, SpanPlan plan)
+__global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4_matvec_span_kernel(Int4Args a, SpanPlan plan)
 {
     static_assert(MODE != QKV_ROPE || (WAVES == 8 && ROWS == 1 && TN == 3), "RoPE pairs: 8 wavefronts, one row each");
     constexpr int SD = span_scale_words(J, ROWS);

@@ -151,6 +151,7 @@ constexpr int DPP_ROW_HALF_MIRROR = 0x141; // lane i <- lane 7-i within 8
 constexpr int DPP_ROW_MIRROR = 0x140;      // lane i <- lane 15-i within 16
 constexpr int DPP_ROW_BCAST15 = 0x142;     // lane 15 of each row -> next row
 constexpr int DPP_ROW_BCAST31 = 0x143;     // lane 31 -> rows 2,3
+constexpr int DPP_ROW_NEWBCAST = 0x150;    // + i: lane i of each row of 16 -> the whole row
 
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ float dpp_f32(float v)
@@ -167,6 +168,16 @@ __device__ __forceinline__ float row16_sum(float v)
     v += dpp_f32<DPP_QUAD_XOR2>(v);
     v += dpp_f32<DPP_ROW_HALF_MIRROR>(v);
     v += dpp_f32<DPP_ROW_MIRROR>(v);
+    return v;
+}
+
+// Largest value of each 16-lane row, in every lane of it.
+__device__ __forceinline__ float row16_max(float v)
+{
+    v = fmaxf(v, dpp_f32<DPP_QUAD_XOR1>(v));
+    v = fmaxf(v, dpp_f32<DPP_QUAD_XOR2>(v));
+    v = fmaxf(v, dpp_f32<DPP_ROW_HALF_MIRROR>(v));
+    v = fmaxf(v, dpp_f32<DPP_ROW_MIRROR>(v));
     return v;
 }
 

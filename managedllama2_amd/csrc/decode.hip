@@ -94,14 +94,14 @@ inline AttnShape attn_shape(int index, int seq_len)
 }
 
 struct AttnArgs;
-void launch_attn(const AttnShape& shape, int n_heads, const AttnArgs& a);
+void launch_attn(const AttnShape& shape, int n_heads, const AttnArgs& a, bool parts = false);
 
 struct AttnArgs {
     const uint16_t* q;
     const uint16_t* kcache; // layer base, rows of `dim` halfs
     const uint16_t* vcache;
     uint16_t* out; // [n_heads * 128]
-    float* part;   // [n_heads][max_splits][kPartStride]
+    float* part;   // [n_heads][max_splits][kPartStride]; ATTN_PARTS: [max_splits][dim], then [max_splits][n_heads][2]
     unsigned* counters; // [n_heads], zero between launches
     const int* pos_ptr; // device-resident position, or null: attend `seq` rows
     int seq;
@@ -142,9 +142,16 @@ __device__ __forceinline__ u32x4 rope_lane8(u32x4 mine, int l16, const float* ta
     return r;
 }
 
-template <int WAVES, bool ROPE>
+enum AttnKind {
+    ATTN_OUT,   // the output, merged by the last workgroup of a head
+    ATTN_ROPE,  // the same, with the rotation of the query and the newest key inside
+    ATTN_PARTS, // the blocks' results as they are: the o-projection merges them (launch_o_merge)
+};
+
+template <int WAVES, AttnKind KIND>
 __global__ __launch_bounds__(WAVES * 64) void fused_attn_kernel(AttnArgs a)
 {
+    constexpr bool ROPE = KIND == ATTN_ROPE;
     constexpr int GROUPS = WAVES * 4;   // 16-lane groups, one timestep each per pass
     constexpr int SPLIT_T = GROUPS * 8; // timesteps per workgroup
     __shared__ float sc[SPLIT_T];
@@ -248,6 +255,16 @@ __global__ __launch_bounds__(WAVES * 64) void fused_attn_kernel(AttnArgs a)
         for (int g = 0; g < WAVES; ++g)
             val += red[g][threadIdx.x];
     }
+    if constexpr (KIND == ATTN_PARTS) {
+        if (threadIdx.x < kRopeHeadSize)
+            a.part[static_cast<size_t>(split) * a.dim + h * kRopeHeadSize + threadIdx.x] = val;
+        if (threadIdx.x == 0) {
+            float* stats = a.part + static_cast<size_t>(a.max_splits) * a.dim + (split * gridDim.y + h) * 2;
+            stats[0] = m;
+            stats[1] = l;
+        }
+        return;
+    }
     uint16_t* out = a.out + static_cast<size_t>(h) * kRopeHeadSize;
     if (nsplit == 1) {
         if (threadIdx.x < kRopeHeadSize)
@@ -330,14 +347,18 @@ template <int WAVES>
 static void launch_attn_waves(const dim3 grid, const AttnArgs& a)
 {
     if (a.q_rw)
-        hipLaunchKernelGGL((fused_attn_kernel<WAVES, true>), grid, dim3(WAVES * 64), 0, ctx().stream, a);
+        hipLaunchKernelGGL((fused_attn_kernel<WAVES, ATTN_ROPE>), grid, dim3(WAVES * 64), 0, ctx().stream, a);
     else
-        hipLaunchKernelGGL((fused_attn_kernel<WAVES, false>), grid, dim3(WAVES * 64), 0, ctx().stream, a);
+        hipLaunchKernelGGL((fused_attn_kernel<WAVES, ATTN_OUT>), grid, dim3(WAVES * 64), 0, ctx().stream, a);
 }
 
-void launch_attn(const AttnShape& shape, int n_heads, const AttnArgs& a)
+void launch_attn(const AttnShape& shape, int n_heads, const AttnArgs& a, bool parts)
 {
     const dim3 grid(shape.splits, n_heads);
+    if (parts) { // blocks of 128 rows
+        hipLaunchKernelGGL((fused_attn_kernel<kSmallWaves, ATTN_PARTS>), grid, dim3(kSmallWaves * 64), 0, ctx().stream, a);
+        return;
+    }
     switch (shape.waves) {
     case 2: launch_attn_waves<2>(grid, a); break;
     case 4: launch_attn_waves<4>(grid, a); break;
@@ -564,20 +585,25 @@ int forward_fused(llama2_decoder* d, int shape)
             a.rope_table = reinterpret_cast<const float*>(d->state + kStateInts);
             L2_TRY((launch_int4<QKV_ROPE, STAGE_RMSNORM>("fused qkv", a)));
         }
+        Int4Args o{}; // :177
+        o.m[0] = qw(L.output), o.out[0] = s.x, o.x = s.xb;
+        o.K = dim, o.N = dim, o.ws = ws, o.ss = ss, o.zs = zs, o.n_tensors = 1;
+        o.parts = d->attn_part, o.pos_ptr = d->state, o.block_shift = ceil_log2(as.waves * 32);
+        const bool merge = as.waves == kSmallWaves && launch_o_merge(o, as.splits, false);
         {
             AttnArgs a{}; // :175 (MultiHeadAttention :150-156)
             a.q = s.q, a.kcache = s.key_cache + layer_offset, a.vcache = s.value_cache + layer_offset, a.out = s.xb;
             a.part = d->attn_part, a.counters = d->counters, a.pos_ptr = d->state;
             a.dim = dim, a.max_splits = as.splits;
             a.scale = 1.0f / sqrtf(static_cast<float>(d->head_size));
-            launch_attn(as, c.n_heads, a);
+            launch_attn(as, c.n_heads, a, merge);
             L2_LAUNCH_CHECK("fused attention");
         }
-        {
-            Int4Args a{}; // :177
-            a.m[0] = qw(L.output), a.out[0] = s.x, a.x = s.xb;
-            a.K = dim, a.N = dim, a.ws = ws, a.ss = ss, a.zs = zs, a.n_tensors = 1;
-            L2_TRY((launch_int4<RESIDUAL, STAGE_X>("fused o-proj", a)));
+        if (merge) {
+            launch_o_merge(o, as.splits, true);
+            L2_LAUNCH_CHECK("fused o-proj");
+        } else {
+            L2_TRY((launch_int4<RESIDUAL, STAGE_X>("fused o-proj", o)));
         }
         {
             Int4Args a{}; // :179 + :181

@@ -47,7 +47,10 @@ enum Mode {
 enum Stage {
     STAGE_X = 0,       // x as given
     STAGE_RMSNORM = 1, // half(rms * gamma * x), x = a.x or (layer 0) the embedding row of tokens[*pos]
+    STAGE_MERGE = 2,   // the attention output, merged from the results of up to kMergeBlocks blocks of timesteps per head
+                       // (span kernel only)
 };
+constexpr int kMergeBlocks = 2;
 
 constexpr int kRopeHeadSize = 128; // QKV_ROPE assumes head_size 128 (pairs i, i+64)
 
@@ -70,6 +73,10 @@ struct Int4Args {
     int kv_dim;
     float theta;
     const float* rope_table; // (cos, sin) of the step's position for i < 64, or null: computed here from theta
+    // STAGE_MERGE: the sums [kMergeBlocks][K], then (maximum, sum) [kMergeBlocks][head]; a block is 2^block_shift timesteps,
+    // those up to *pos_ptr count
+    const float* parts;
+    int block_shift;
 };
 
 constexpr int kAuxStream = 2; // "nt": weights are touched once
@@ -121,27 +128,31 @@ __device__ __forceinline__ u32x4 staged_order(const u32x4 v, int word)
     return o;
 }
 
+// Piece e (8 inputs) into the LDS image; neighbouring lanes hold neighbouring pieces.
+template <int J>
+__device__ __forceinline__ void commit_piece(u32x4* xs, float* sx, const u32x4 v, int e)
+{
+    xs[(e & 3) * (J * 64) + (e >> 2)] = staged_order(v, e & 3);
+    const h2_t one = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
+    float s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        s = __builtin_amdgcn_fdot2(as_h2(v[k]), one, s, false);
+    s += dpp_f32<DPP_QUAD_XOR1>(s); // the 4 words of a chunk sit in one quad of lanes
+    s += dpp_f32<DPP_QUAD_XOR2>(s);
+    if ((e & 3) == 0)
+        sx[e >> 2] = s;
+}
+
 // One thread's pieces of the input into the LDS image; `tid` < 256.
 template <int J>
 __device__ __forceinline__ void commit_pieces_t(u32x4* xs, float* sx, const VecPieces<J>& p, int tid)
 {
-    constexpr int JC = J * 64;
 #pragma unroll
-    for (int i = 0; i < J; ++i) { // JC*4 pieces over 256 threads = J per thread
-        const int e = tid + i * 256;
-        const u32x4 v = p.v[i];
-        xs[(e & 3) * JC + (e >> 2)] = staged_order(v, e & 3);
-        const h2_t one = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
-        float s = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            s = __builtin_amdgcn_fdot2(as_h2(v[k]), one, s, false);
-        s += dpp_f32<DPP_QUAD_XOR1>(s); // the 4 words of a chunk sit in one quad of lanes
-        s += dpp_f32<DPP_QUAD_XOR2>(s);
-        if ((e & 3) == 0)
-            sx[e >> 2] = s;
-    }
+    for (int i = 0; i < J; ++i) // 256 J pieces over 256 threads = J per thread
+        commit_piece<J>(xs, sx, p.v[i], tid + i * 256);
 }
+
 
 template <int J>
 __device__ __forceinline__ void commit_pieces(u32x4* xs, float* sx, const VecPieces<J>& p)
@@ -763,8 +774,9 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
     // vector load and taken into a scalar register only where it is used.  Vector loads return in order
     // and are waited for by count; read where it is used (`a.pos_ptr[0]` after the first row's requests)
     // it made the wavefront wait for that whole row before the input could be staged.
+    constexpr int MB = STAGE == STAGE_MERGE ? kMergeBlocks : 0;
     uint32_t pos_bits = 0;
-    if (MODE == QKV_ROPE)
+    if (MODE == QKV_ROPE || MB > 0)
         pos_bits = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(a.pos_ptr, a.pos_ptr ? 4 : 0), 0, 0, 0);
     auto position = [&]() -> int {
         asm volatile("" : "+v"(pos_bits)); // stays where it is written
@@ -779,7 +791,24 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
         token = token < 0 ? 0 : (token >= a.vocab ? a.vocab - 1 : token); // never read outside the table
         xsrc = a.embedding + static_cast<size_t>(token) * a.K;
     }
-    if (stager) {
+    // Merging the blocks of attention: a thread takes 8 of a head's 128 elements, 16 neighbours a head, and lane i of the 16
+    // block i's statistics.  Everything is requested before the number of blocks is known.
+    u32x4 pv[MB > 0 ? MB : 1][2];
+    uint32_t part_max = 0, part_sum = 0;
+    if constexpr (MB > 0) {
+        constexpr int kNowhere = 1 << 30; // behind the end of the buffer: reads as zero
+        const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.parts, (a.K + a.K / kRopeHeadSize * 2) * MB * 4);
+        const int at = ((lane & 15) * (a.K / kRopeHeadSize) + static_cast<int>(threadIdx.x >> 4)) * 8 + a.K * MB * 4;
+        const bool have = static_cast<int>(threadIdx.x) * 8 < a.K;
+        part_max = __builtin_amdgcn_raw_buffer_load_b32(rp, have && (lane & 15) < MB ? at : kNowhere, 0, 0);
+        part_sum = __builtin_amdgcn_raw_buffer_load_b32(rp, have && (lane & 15) < MB ? at + 4 : kNowhere, 0, 0);
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                pv[b][e] = __builtin_amdgcn_raw_buffer_load_b128(
+                    rp, have ? (b * a.K + static_cast<int>(threadIdx.x) * 8 + e * 4) * 4 : kNowhere, 0, 0);
+    } else if (stager) {
         xp.load(xsrc, a.K);
         if (STAGE == STAGE_RMSNORM)
             gp.load(a.gamma, a.K);
@@ -837,8 +866,33 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
         if (stager)
             xp.scale(rms, gp);
     }
-    if (stager)
+    if constexpr (MB > 0) {
+        // the merge at the end of fused_attn_kernel, value by value
+        const int blocks = (position() >> a.block_shift) + 1, l16 = lane & 15;
+        const float m = l16 < blocks ? __uint_as_float(part_max) : -INFINITY;
+        const float largest = row16_max(m); // by all lanes: a lane that is switched off gives its neighbours nothing
+        const float w = l16 < blocks ? expf(m - largest) : 0.0f;
+        const float sum = row16_sum(l16 < blocks ? w * __uint_as_float(part_sum) : 0.0f);
+        float o[8] = {};
+        const float wb[kMergeBlocks] = {dpp_f32<DPP_ROW_NEWBCAST>(w), dpp_f32<DPP_ROW_NEWBCAST + 1>(w)};
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const uint32_t v = b < blocks ? pv[b][k >> 2][k & 3] : 0u; // a block that is not there has left nothing
+                o[k] = fmaf(wb[b], __uint_as_float(v), o[k]);
+            }
+        u32x4 x = {};
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            x[k >> 1] |= static_cast<uint32_t>(float_to_half_bits(o[k] / sum)) << (16 * (k & 1));
+        if (static_cast<int>(threadIdx.x) * 8 >= a.K)
+            x = u32x4{};
+        for (int e = threadIdx.x; e < J * 256; e += WAVES * 64, x = u32x4{}) // the threads cover K, the rest is zero
+            commit_piece<J>(xs, sx, x, e);
+    } else if (stager) {
         commit_pieces_t<J>(xs, sx, xp, threadIdx.x);
+    }
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
 #pragma unroll
@@ -1027,7 +1081,7 @@ inline int resident_waves()
 // The span kernel for this launch, if the shape suits it: scales readable 4 bytes at a time, and
 // all wavefronts resident at once with ROWS rows each.
 template <int J, int MODE, int STAGE, int TN, int WAVES, int ROWS>
-inline bool try_span(const Int4Args& a)
+inline bool try_span(const Int4Args& a, bool launch = true)
 {
     constexpr auto kernel = int4_matvec_span_kernel<J, MODE, STAGE, TN, WAVES, ROWS>;
     SpanPlan plan{};
@@ -1043,19 +1097,26 @@ inline bool try_span(const Int4Args& a)
     }
     if (plan.grid * WAVES > resident_waves<kernel, WAVES * 64>())
         return false;
-    hipLaunchKernelGGL(kernel, dim3(plan.grid), dim3(WAVES * 64), 0, ctx().stream, a, plan);
+    if (launch)
+        hipLaunchKernelGGL(kernel, dim3(plan.grid), dim3(WAVES * 64), 0, ctx().stream, a, plan);
+    return true;
+}
+
+inline bool span_allowed(const Int4Args& a, int tensors)
+{
+    if (ctx().int4_no_span || ctx().int4_narrow || ctx().int4_blocks || (a.ss & 1))
+        return false;
+    for (int t = 0; t < tensors; ++t)
+        if (!aligned(a.m[t].s, 4))
+            return false;
     return true;
 }
 
 template <int J, int MODE, int STAGE>
 inline bool launch_span(const Int4Args& a)
 {
-    if (ctx().int4_no_span || ctx().int4_narrow || ctx().int4_blocks || (a.ss & 1))
+    if (!span_allowed(a, MODE == SWIGLU ? 2 : a.n_tensors))
         return false;
-    const int tn = MODE == SWIGLU ? 2 : a.n_tensors;
-    for (int t = 0; t < tn; ++t)
-        if (!aligned(a.m[t].s, 4))
-            return false;
     // Rows per wavefront and wavefronts per workgroup as measured on the 7B / 13B shapes: one row per
     // wavefront where that many wavefronts fit, three for the SwiGLU pair of tensors.
     if constexpr (MODE == QKV_ROPE) {
@@ -1104,6 +1165,23 @@ inline void launch_j(const Int4Args& a, int max_waves)
 // Number of chunk-columns a lane holds per row for a K-input tensor.
 inline int chunk_columns(int ws) { return ceil_div(ws / 4, 64); }
 constexpr int kMaxChunkColumns = 8; // K <= 16384 on the unrolled kernels
+
+// The o-projection that merges the blocks of attention while it stages its input, if there is one for the shape
+// (launch: false only asks).  Every workgroup reads the results of all blocks, so there is one of 16 wavefronts per
+// compute unit.  What the hand-over inside the attention launch costs (2.1 us) is what two blocks gain, less 0.6 us
+// of staging: 7B at 130 .. 250 rows 1108 -> 1084 us per token.  Four blocks gain 0.1 % (1114.9 us for 1117), eight lose 3 %
+// (1180 for 1146 at 700 rows), and so does 13B's o-projection, whose 20 rows per compute unit fit no such workgroup,
+// with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.
+inline bool launch_o_merge(const Int4Args& a, int blocks, bool launch)
+{
+    if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || !span_allowed(a, 1))
+        return false;
+    switch (ceil_div(a.ws / 4, 64)) {
+    case 1: return try_span<1, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    case 2: return try_span<2, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    default: return false;
+    }
+}
 
 // Wavefronts kept resident per launch: 16 per CU while a lane holds up to 3
 // chunks of a row (20 for the three-tensor QKV launch of single rows), 8 per CU

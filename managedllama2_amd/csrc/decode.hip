@@ -240,8 +240,8 @@ __global__ __launch_bounds__(WAVES * 64) void fused_attn_kernel(AttnArgs a)
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) { // the 4 groups of a wavefront, then the wavefronts through LDS
-        o[k] += __shfl_xor(o[k], 16, 64);
-        o[k] += __shfl_xor(o[k], 32, 64);
+        o[k] = add_xor16(o[k]);
+        o[k] = add_xor32(o[k]);
     }
     if (lane < 16) {
 #pragma unroll

@@ -233,9 +233,6 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
 }
 
-constexpr int DPP_QUAD_XOR3 = 0x1B;  // quad_perm:[3,2,1,0]
-constexpr int DPP_ROW_ROR8 = 0x128;  // lane i <- lane (i + 8) % 16
-
 template <int MASK>
 __device__ __forceinline__ uint32_t lane_xor(uint32_t v)
 {

@@ -17,6 +17,7 @@ namespace l2 {
 constexpr int kMaxRetiredPartials = 32;
 
 struct SamplerScratch;
+struct HostStep;
 
 struct Context {
     bool ready = false;
@@ -41,6 +42,8 @@ struct Context {
     // per-head arrival counters of llama2_multi_head_attention (zero between launches)
     unsigned* attn_counters = nullptr;
     SamplerScratch* sampler = nullptr; // between the sampler's launches (sampler_kernels.hpp)
+    // Pinned: where a kernel leaves the token that the call behind it returns (a copy of 4 bytes is a launch of 4.3 us)
+    int* host_token = nullptr;
 };
 
 constexpr int kMaxAttnHeads = 1024;
@@ -54,7 +57,7 @@ int resolve_vec_mat_static_scratch(int device);
 // Sampler.Sample's stochastic branch (sampler.hip).  token_only: the caller reads the
 // token alone, so the sort may stop at the head of the distribution that holds top_p of the mass.
 int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, float temperature, float top_p, float coin,
-                  int* result, int pos, bool token_only);
+                  int* result, int pos, bool token_only, const HostStep* host = nullptr);
 
 // HIP's current device is a per-thread setting: a host thread other than the one that called
 // llama2_init (a thread-pool worker of the managed host, say) is bound to the library's device on

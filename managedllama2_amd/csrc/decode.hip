@@ -398,6 +398,23 @@ __global__ void bump_serial_kernel(int* state)
         state[kStateSerial] = state[kStateSerial] + 1;
 }
 
+// Argmax for a host that reads the token back (src/Sampler.cs:44-47,69): tokens[pos] = argmax(logits) if write_token,
+// else the token that is there; the next position's step state on the way.
+__global__ __launch_bounds__(1024) void argmax_host_kernel(const uint16_t* x, int size, int* tokens, int pos, int write_token,
+                                                           HostStep host)
+{
+    __shared__ float sv[16];
+    __shared__ int si[16];
+    if (threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
+        write_host_step_state(host, threadIdx.x - 64);
+    const int best = block1024_argmax(x, size, sv, si);
+    if (threadIdx.x == 0) {
+        if (write_token)
+            tokens[pos] = best;
+        write_host_token(host, write_token ? best : tokens[pos]);
+    }
+}
+
 // Sampler.Sample greedy branch (src/Sampler.cs:44-47) against the device state:
 // tokens[pos+1] = argmax(logits) iff pos+1 >= n_prompt; lowest index wins ties.
 __global__ __launch_bounds__(1024) void argmax_step_kernel(const uint16_t* x, int size, int* tokens, int* state,
@@ -440,6 +457,8 @@ struct llama2_decoder {
     hipGraphExec_t graphs[kGraphKinds][l2::kAttnShapes + 1] = {};
     float sampled_temperature = 0.0f, sampled_top_p = 0.0f;
     unsigned long long sampled_seed = 0;
+    int ready_position = -1; // position whose state a host's sampling call left on the device, or -1
+    bool replayed = false;   // a call was captured: replays may set the state at any time
     // persistent step (LLAMA2_DECODE_PERSISTENT): kernel variant, per-layer pointer table and
     // hand-over buffers on the device, and the launch arguments
     int persist_variant = -1;
@@ -674,6 +693,35 @@ int set_state(llama2_decoder* d, int pos, int n_prompt, int advance)
     hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, ctx().stream, d->state, pos, n_prompt, advance,
                        d->cfg.seq_len, d->cfg.rope_theta);
     L2_LAUNCH_CHECK("set_state_kernel");
+    return LLAMA2_OK;
+}
+
+// The state of a step that a host asked for by position; nothing to do where the sampling of the token before left it.
+int set_host_state(llama2_decoder* d, int pos)
+{
+    if (ctx().capturing)
+        d->replayed = true; // a replay sets the state without a call here
+    if (d->ready_position == pos && !d->replayed)
+        return LLAMA2_OK;
+    d->ready_position = -1;
+    return set_state(d, pos, INT_MAX, 0);
+}
+
+// What the sampling kernel of a host's own loop does on the way.
+HostStep host_step(llama2_decoder* d, int next_position)
+{
+    HostStep h{};
+    h.token = ctx().host_token;
+    if ((d->mode & LLAMA2_DECODE_FUSED) && next_position < d->cfg.seq_len)
+        h.state = d->state, h.next = next_position, h.n_slots = d->cfg.seq_len, h.theta = d->cfg.rope_theta;
+    return h;
+}
+
+int take_host_token(llama2_decoder* d, const HostStep& h, int* token)
+{
+    L2_HIP(hipStreamSynchronize(ctx().stream));
+    *token = *static_cast<volatile int*>(ctx().host_token);
+    d->ready_position = h.state ? h.next : -1;
     return LLAMA2_OK;
 }
 
@@ -1010,7 +1058,7 @@ int llama2_decode_forward(llama2_decoder* d, int position, int next_position)
              next_position, position + 1);
     if (!(d->mode & LLAMA2_DECODE_FUSED))
         return forward_modules(d, position, next_position);
-    L2_TRY(set_state(d, position, INT_MAX, 0));
+    L2_TRY(set_host_state(d, position));
     return launch_step(d, llama2_decoder::kGraphForward, position);
 }
 
@@ -1023,8 +1071,12 @@ int llama2_decode_sample(llama2_decoder* d, int next_position, int generate_toke
     const TokenSlot slot = token_slot(d, next_position);
     L2_CHECK(slot.tokens == d->s.tokens || generate_token,
              "llama2_decode_sample: next_position=%d is past the last token of the context", next_position);
-    L2_TRY(llama2_argmax(d->s.logits, d->cfg.vocab_size, slot.tokens, slot.index, generate_token));
-    L2_TRY(llama2_memcpy_d2h(token, slot.tokens, static_cast<size_t>(slot.index) * sizeof(int), sizeof(int)));
+    L2_CHECK(!ctx().capturing, "llama2_decode_sample: not allowed during graph capture");
+    const HostStep h = host_step(d, next_position);
+    hipLaunchKernelGGL(argmax_host_kernel, dim3(1), dim3(1024), 0, ctx().stream, d->s.logits, d->cfg.vocab_size, slot.tokens,
+                       slot.index, generate_token, h);
+    L2_LAUNCH_CHECK("argmax_host_kernel");
+    L2_TRY(take_host_token(d, h, token));
     return persist_status(d, "llama2_decode_sample");
 }
 
@@ -1039,9 +1091,11 @@ int llama2_decode_sample_top_p(llama2_decoder* d, int next_position, int generat
     L2_CHECK(next_position >= 0 && next_position <= d->cfg.seq_len, "%s: next_position=%d", fn, next_position);
     L2_TRY(check_sampling(fn, d, temperature));
     const TokenSlot slot = token_slot(d, next_position);
+    L2_CHECK(!ctx().capturing, "%s: not allowed during graph capture", fn);
+    const HostStep h = host_step(d, next_position);
     L2_TRY(sample_launch(fn, d->s.logits, d->s.indices, d->cfg.vocab_size, temperature, top_p, coin, slot.tokens,
-                         slot.index, true)); // :50-66
-    L2_TRY(llama2_memcpy_d2h(token, slot.tokens, static_cast<size_t>(slot.index) * sizeof(int), sizeof(int))); // :69
+                         slot.index, true, &h)); // :50-66
+    L2_TRY(take_host_token(d, h, token)); // :69
     return persist_status(d, fn);
 }
 
@@ -1083,6 +1137,8 @@ int llama2_decode_run_sampled(llama2_decoder* d, int position, int steps, int n_
         }
         d->sampled_temperature = temperature, d->sampled_top_p = top_p, d->sampled_seed = seed;
     }
+    d->ready_position = -1;
+    d->replayed |= ctx().capturing;
     L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)
@@ -1104,6 +1160,8 @@ int llama2_decode_run(llama2_decoder* d, int position, int steps, int n_prompt)
         }
         return LLAMA2_OK;
     }
+    d->ready_position = -1;
+    d->replayed |= ctx().capturing;
     L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)

@@ -38,6 +38,35 @@ __device__ __forceinline__ void write_rope_table(int* state, int i, int pos, flo
 }
 #endif
 
+#if defined(__HIPCC__)
+// What a host that drives the loop itself has done for it by the kernel that samples: the token in pinned memory, and the
+// state of the next position's step (set_state_kernel's with n_prompt INT_MAX and no advance).
+struct HostStep {
+    int* token;  // or null
+    int* state;  // or null
+    int next, n_slots;
+    float theta;
+};
+__device__ __forceinline__ void write_host_step_state(const HostStep& h, int thread)
+{
+    if (!h.state)
+        return;
+    if (thread == 0) {
+        h.state[kStatePos] = h.next;
+        h.state[kStatePrompt] = 0x7FFFFFFF;
+        h.state[kStateAdvance] = 0;
+        h.state[kStateSlots] = h.n_slots;
+    }
+    if (thread < kRopeHeadSize / 2)
+        write_rope_table(h.state, thread, h.next, h.theta);
+}
+__device__ __forceinline__ void write_host_token(const HostStep& h, int token)
+{
+    if (h.token)
+        __hip_atomic_store(h.token, token, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+#endif
+
 struct PersistLayer { // one per layer, in device memory
     QW q, k, v, o, gate, up, down;
     const uint16_t* rms_att;

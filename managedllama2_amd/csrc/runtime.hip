@@ -107,6 +107,7 @@ int llama2_init(int device)
     L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.attn_counters), kMaxAttnHeads * sizeof(unsigned)));
     L2_HIP(hipMemset(c.attn_counters, 0, kMaxAttnHeads * sizeof(unsigned)));
     L2_HIP(hipMalloc(reinterpret_cast<void**>(&c.sampler), sizeof(SamplerScratch)));
+    L2_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.host_token), sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     c.device = device;
     if (int rc = resolve_vec_mat_static_scratch(device)) {
         c.device = -1;
@@ -141,6 +142,9 @@ int llama2_shutdown(void)
     if (c.sampler)
         L2_HIP(hipFree(c.sampler));
     c.sampler = nullptr;
+    if (c.host_token)
+        L2_HIP(hipHostFree(c.host_token));
+    c.host_token = nullptr;
     L2_HIP(hipStreamDestroy(c.stream));
     c.stream = nullptr;
     c.ready = false;

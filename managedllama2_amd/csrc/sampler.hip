@@ -23,7 +23,7 @@ int check_temperature(const char* fn, float temperature)
 
 static void launch_exp(const SampleArgs& a)
 {
-    const dim3 grid(kSampBlock / kExpShare + (a.state ? 1 : 0));
+    const dim3 grid(kSampBlock / kExpShare + (a.state || a.host.state ? 1 : 0));
     if (sampler_chunks(a.size) == 4)
         hipLaunchKernelGGL(sampler_exp_kernel<4>, grid, dim3(kExpThreads), 0, ctx().stream, a);
     else
@@ -163,7 +163,7 @@ int llama2_sample(llama2_half* logits, int* indices, int size, float temperature
 namespace l2 {
 
 int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, float temperature, float top_p, float coin,
-                  int* result, int pos, bool token_only)
+                  int* result, int pos, bool token_only, const HostStep* host)
 {
     L2_CHECK(logits && indices && result, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
@@ -174,6 +174,8 @@ int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, floa
     a.logits = logits, a.indices = indices, a.size = size;
     a.temperature = temperature, a.top_p = top_p, a.coin = coin, a.result = result, a.pos = pos;
     a.head = token_only ? 1 : 0;
+    if (host)
+        a.host = *host;
     return sample_enqueue(fn, a);
 }
 

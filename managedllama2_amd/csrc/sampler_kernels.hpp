@@ -68,6 +68,7 @@ struct SampleArgs {
     int* tokens;
     unsigned long long seed;
     float theta;
+    HostStep host; // a host's own loop
 };
 
 // Queues the four launches (three without a sort); checks nothing.
@@ -141,6 +142,10 @@ __global__ __launch_bounds__(kExpThreads) void sampler_exp_kernel(SampleArgs a)
     __shared__ float red[kExpThreads / 64];
     __shared__ float val[kExpShare][N + 4];
     if (blockIdx.x == kSampBlock / kExpShare) { // one more workgroup in a decode step
+        if (!a.state) {
+            write_host_step_state(a.host, threadIdx.x);
+            return;
+        }
         const int next = a.state[kStatePos] + 1;
         if (threadIdx.x == 0) {
             a.s->go = next >= a.state[kStatePrompt] && next < a.state[kStateSlots];
@@ -678,7 +683,9 @@ __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, 
     for (int w = 1; w < kSampWaves; ++w)
         best = first_hit[w] < best ? first_hit[w] : best;
     if (!a.state) {
-        a.result[a.pos] = a.indices[best];
+        const int token = a.indices[best];
+        a.result[a.pos] = token;
+        write_host_token(a.host, token);
         return;
     }
     const int next = a.state[kStatePos] + 1;

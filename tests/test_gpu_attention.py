@@ -204,3 +204,30 @@ def test_rejects_unsupported():
     assert capi.raw("llama2_multi_head_attention", out.ptr, dq.ptr, dk.ptr, dv.ptr, 64, 512, 4, 0.125, 8) == capi.ERR_UNSUPPORTED
     assert capi.raw("llama2_multi_head_attention", out.ptr, dq.ptr, dk.ptr, dv.ptr, HS, 512, 4, 0.1, 5) == capi.ERR_INVALID_ARGUMENT
     assert capi.raw("llama2_multi_head_attention", out.ptr, dq.ptr, dk.ptr, dv.ptr, HS, 512, 0, 0.1, 4) == capi.ERR_INVALID_ARGUMENT
+
+
+# Beyond 1024 rows every wavefront keeps the softmax statistics of its own 32 rows (8 wavefronts a block up to 16384 rows,
+# 16 beyond): a last block with rows for one wavefront alone, for part of one, for all but one; and rows whose scores lie
+# below fp16's range (-infinity, no weight) filling a wavefront's share, a whole block, and the first block.
+@pytest.mark.parametrize("seq", [1025, 1031, 1056, 1057, 1279, 1280, 1281, 2304, 16384, 16385, 16900])
+def test_statistics_per_wavefront(oracle, seq):
+    dim, heads = 256, 2
+    q, k, v = inputs(711, dim, seq)
+    got = fused(q, k, v, dim, heads, seq)
+    assert_close_up_to_ties(got, oracle_chain(oracle, q, k, v, dim, heads, seq, True), "attention %d/%d/%d" % (dim, heads, seq))
+
+
+@pytest.mark.parametrize("masked", [(32, 64), (256, 512), (0, 256), (0, 1300), (1024, 1301)])
+def test_wavefronts_and_blocks_without_weight(masked):
+    dim, heads, seq = 256, 2, 1301
+    q, k, v = inputs(712, dim, seq)
+    q = np.abs(q) + np.float16(1)
+    k = k.reshape(seq, dim)
+    k[masked[0]:masked[1]] = np.float16(-60000)  # scores below -65504
+    v = v.reshape(seq, dim)
+    v[masked[0]:masked[1]] = np.float16(60000)   # no weight, however large
+    got = fused(q, k.ravel(), v.ravel(), dim, heads, seq)
+    rest = np.r_[0:masked[0], masked[1]:seq]
+    want = fused(q, k[rest].ravel(), v[rest].ravel(), dim, heads, rest.size)
+    assert np.all(np.isfinite(got))
+    assert_close_normwise(got, want, "rows %s without weight" % (masked,))  # the same sums in other blocks

@@ -51,7 +51,8 @@ typedef uint16_t llama2_half;
 /* Largest softmax row, as in the reference (native/softmax_kernel.cu:5). */
 #define LLAMA2_MAX_SOFTMAX_SIZE 8192
 /* Largest `size` of the sampler modules (softmax_logits, sort, cumulative_sum,
- * sample_top_p): one 1024-thread workgroup holds the whole vector. */
+ * sample_top_p): the 1024 partial sums, whose order is that of one
+ * workgroup, take up to 64 elements each; positions and ranks are 16 bits. */
 #define LLAMA2_MAX_SAMPLER_SIZE 65536
 
 /* ---------------------------------------------------------------- runtime */

@@ -893,9 +893,9 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
     } else if (stager) {
         commit_pieces_t<J>(xs, sx, xp, threadIdx.x);
     }
-    // Scales and zero words lie in a piece of LDS of the wavefront's own.  Rows of up to 4096 inputs: written behind the barrier,
-    // which then waits for nothing but the input (7B step at 20 / 260 / 4000 rows 1024 -> 1022, 1100 -> 1098, 1447 -> 1442 us); longer rows, with fewer wavefronts to wait
-    // for, lose 0.2 % by it.
+    // Scales and zero words lie in a piece of LDS of the wavefront's own.  Rows of up to 4096 inputs: written behind the
+    // barrier, which then waits for nothing but the input (7B step at 20 / 260 / 4000 rows 1024 -> 1022, 1100 -> 1098,
+    // 1447 -> 1442 us); longer rows, with fewer wavefronts to wait for, lose 0.2 % by it.
     auto keep_meta = [&]() {
 #pragma unroll
         for (int t = 0; t < TN; ++t) {

@@ -33,14 +33,15 @@ namespace l2 {
 // (up to 16 loads of 16 bytes per lane; rows outside the block are out of the
 // buffer's range and cost no traffic), 16 lanes share one timestep, scores are
 // rounded to fp16 like the reference's `attention` buffer, softmax statistics
-// are per block and the blocks of a head are merged by whichever workgroup
-// finishes last (fixed merge order: deterministic).
+// are per block or wavefront (below) and the blocks of a head are merged by
+// whichever workgroup finishes last (fixed merge order: deterministic), or, two
+// blocks of a decode step, by the o-projection (launch_o_merge).
 //
 // One compute unit pulls only a few tens of GB/s, so a short sequence wants
 // many small blocks (4 wavefronts, 128 rows); the exchange between workgroups
 // costs about 3 us whatever their number, and a long sequence wants fewer
-// merges.  Measured on 32 heads (one launch, RoPE inside), 64 / 128 / 256 / 512
-// rows per block: 512 rows 7.4 / 7.3 / 8.8 / 11.0 us, 2048 rows 17.7 / 12.1 /
+// merges.  Measured on 32 heads (one launch, RoPE inside; with the choice made
+// here 6.9 / 11.2 / 17.3 us since), 64 / 128 / 256 / 512 rows per block: 512 rows 7.4 / 7.3 / 8.8 / 11.0 us, 2048 rows 17.7 / 12.1 /
 // 11.4 / 15.5 us, 4096 rows 31.2 / 21.5 / 17.3 / 19.4 us: 128-row blocks up to
 // 1024 rows, 256-row blocks (8 wavefronts) beyond.  Dispatching workgroups
 // that find nothing to do is not free: a grid sized for the whole context costs
@@ -48,12 +49,13 @@ namespace l2 {
 // device, but the host always knows an upper bound for it, so it picks the
 // launch shape (block size, number of blocks) from a short list by that bound.
 // Blocks of 256 and 512 rows keep the softmax statistics per wavefront: nothing waits for the keys of the other
-// wavefronts, there is one barrier instead of two, and every exponential is taken once instead of once per wavefront.  Registers
-// for 24 wavefronts per compute unit, all 16 loads of a lane requested before the first is used.  32 heads without RoPE, 1100 / 2048
-// / 4096 / 8192 rows: 8.7 / 10.8 / 17.0 / 29.0 -> 8.1 / 10.2 / 16.5 / 28.7 us (16.6 / 29.4 with 16 wavefronts per compute unit).
+// wavefronts, there is one barrier instead of two, and every exponential is taken once instead of once per
+// wavefront.  Registers for 24 wavefronts per compute unit, all 16 loads of a lane requested before the first is
+// used.  32 heads without RoPE, 1100 / 2048 / 4096 / 8192 rows: 8.7 / 10.8 / 17.0 / 29.0 -> 8.1 / 10.2 / 16.5 /
+// 28.7 us (16.6 / 29.4 for the last two with 16 wavefronts per compute unit).
 // Blocks of 128 rows share their sums bit for bit with the persistent step and keep the statistics of the block.
 // Measured in the decode loop: one 256-row block of 8 wavefronts for 129 .. 256 rows
-// is as fast as two 128-row blocks and a merge, two 256-row blocks for 257 .. 512 rows
+// is as fast as two 128-row blocks that merge in the launch, two 256-row blocks for 257 .. 512 rows
 // lose 1.2 % against four 128-row blocks.
 constexpr int kAttnWaves = 16;
 constexpr int kSplitT = 32 * kAttnWaves; // 512: only for contexts beyond 64 blocks of 256 rows
@@ -450,9 +452,10 @@ __global__ __launch_bounds__(1024) void argmax_host_kernel(const uint16_t* x, in
 {
     __shared__ float sv[16];
     __shared__ int si[16];
-    if (threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
-        write_host_step_state(host, threadIdx.x - 64);
-    const int best = block1024_argmax(x, size, sv, si);
+    const int best = block1024_argmax(x, size, sv, si, [&]() {
+        if (threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
+            write_host_step_state(host, threadIdx.x - 64);
+    });
     if (threadIdx.x == 0) {
         if (write_token)
             tokens[pos] = best;
@@ -469,9 +472,10 @@ __global__ __launch_bounds__(1024) void argmax_step_kernel(const uint16_t* x, in
     __shared__ int si[16];
     // read by every thread before thread 0 updates the position (one 16-byte scalar load)
     const int pos0 = state[0], n_prompt = state[1], advance0 = state[2], n_slots = state[3];
-    if (advance0 && threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
-        write_rope_table(state, threadIdx.x - 64, pos0 + 1, theta); // for the next step
-    const int best = block1024_argmax(x, size, sv, si);
+    const int best = block1024_argmax(x, size, sv, si, [&]() {
+        if (advance0 && threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
+            write_rope_table(state, threadIdx.x - 64, pos0 + 1, theta); // for the next step
+    });
     if (threadIdx.x == 0) {
         if (pos0 + 1 >= n_prompt && pos0 + 1 < n_slots)
             tokens[pos0 + 1] = best;

@@ -176,6 +176,23 @@ class TestArgmax:
                 capi.call("llama2_argmax", d2.ptr + 2 * off, n, result.ptr, 0, 1)
                 assert int(result[0]) == n - 1, (n, off)
 
+    @pytest.mark.parametrize("n", [1, 8, 1001, 8191, 32767, 32768, 32776, 65539, 100003])
+    def test_lowest_index_of_the_largest_value(self, n):
+        # up to 32768 elements are held in registers, the rest is read again; a NaN never wins, minus infinity
+        # does if there is nothing else, and 0 is the answer where there is nothing at all
+        rng = synth.rng_for(335 + n)
+        few = f16(rng.integers(-2, 3, n))  # many equal values, in every wavefront
+        some_nan = few.copy()
+        some_nan[rng.random(n) < 0.5] = np.nan
+        late = np.full(n, -np.inf, np.float16)
+        late[n // 2:] = np.float16(-65504)
+        for x in (few, some_nan, late, np.full(n, -np.inf, np.float16), np.full(n, np.nan, np.float16),
+                  np.where(np.arange(n) < n - 1, np.float16(np.nan), np.float16(-np.inf)).astype(np.float16),
+                  np.where(np.arange(n) % 2 == 0, np.float16(-0.0), np.float16(0.0)).astype(np.float16)):
+            real = np.flatnonzero(~np.isnan(x))
+            want = int(real[np.argmax(x[real])]) if real.size else 0
+            assert self.Argmax(x, n) == want, (n, want)
+
     def test_write_token_flag_and_position(self):
         rng = synth.rng_for(333)
         x = f16(rng.random(100))

@@ -166,14 +166,29 @@ __device__ __forceinline__ float dpp_f32(float v)
         float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, false));
 }
 
-// Sum over each 16-lane row; every lane of the row ends with the row total.
-__device__ __forceinline__ float row16_sum(float v)
+// Sum over each 16-lane row, the sums of neighbouring lanes in front of it; every lane of the row ends with a total.
+__device__ __forceinline__ float row16_sum_of_pairs(float v)
 {
-    v += dpp_f32<DPP_QUAD_XOR1>(v);
     v += dpp_f32<DPP_QUAD_XOR2>(v);
     v += dpp_f32<DPP_ROW_HALF_MIRROR>(v);
     v += dpp_f32<DPP_ROW_MIRROR>(v);
     return v;
+}
+
+// Sum over each 16-lane row; every lane of the row ends with the row total.
+__device__ __forceinline__ float row16_sum(float v)
+{
+    v += dpp_f32<DPP_QUAD_XOR1>(v);
+    return row16_sum_of_pairs(v);
+}
+
+// Denominator of merged blocks of timesteps: sum of w * l over each 16-lane row, block i in lane i; the total is that of
+// the row's first lane.  The fused multiply-add of the first level is written out: left to the compiler it came and went
+// with the code around it, and the three kernels that merge (attention, o-projection, persistent step) owe each other
+// the same bits.
+__device__ __forceinline__ float row16_dot(float w, float l)
+{
+    return row16_sum_of_pairs(__builtin_fmaf(w, l, dpp_f32<DPP_QUAD_XOR1>(w * l)));
 }
 
 // Largest value of each 16-lane row, in every lane of it.
@@ -186,14 +201,20 @@ __device__ __forceinline__ float row16_max(float v)
     return v;
 }
 
-// Sum over the 64-lane wavefront, returned in every lane (as a scalar).
-__device__ __forceinline__ float wave_sum(float v)
+// Sum of the four row totals (lane 15 of each row), returned in every lane (as a scalar).
+__device__ __forceinline__ float wave_sum_of_rows(float v)
 {
-    v = row16_sum(v);
     v += dpp_f32<DPP_ROW_BCAST15, 0xA>(v);
     v += dpp_f32<DPP_ROW_BCAST31, 0xC>(v);
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
+
+// Sum over the 64-lane wavefront, returned in every lane (as a scalar).
+__device__ __forceinline__ float wave_sum(float v) { return wave_sum_of_rows(row16_sum(v)); }
+
+// The denominator of up to 64 blocks; up to 16 blocks it has the bits of row16_dot's first lane (lanes 0 and 15 of a
+// row add up the same terms in the same order, and the other rows are zero).
+__device__ __forceinline__ float wave_dot(float w, float l) { return wave_sum_of_rows(row16_dot(w, l)); }
 
 // Largest value of the 64-lane wavefront, in every lane; all lanes take part.  By row operations and lane reads: six
 // shuffles are six round trips through LDS (softmax of 300 scores 3.28 -> 3.08 us, a decode step of 7B at 700 rows

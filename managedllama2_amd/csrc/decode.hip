@@ -367,7 +367,7 @@ __global__ __launch_bounds__(WAVES * 64, KIND != ATTN_ROPE && WAVES == kMidWaves
         const float M = wave_max(have ? mi : -INFINITY);
         const float w = have ? expf(mi - M) : 0.0f;
         wsh[threadIdx.x] = w;
-        const float L = wave_sum(w * li);
+        const float L = wave_dot(w, li);
         if (threadIdx.x == 0)
             lsh[0] = L;
     }

@@ -475,7 +475,7 @@ __global__ __launch_bounds__(kPThreads) void decode_persist_kernel(PersistArgs a
                 const float M = wave_max(mi);
                 const float w = have ? expf(mi - M) : 0.0f;
                 mrg_w[lane] = w;
-                const float Lm = wave_sum(w * li);
+                const float Lm = wave_dot(w, li);
                 if (lane == 0)
                     mrg_l = Lm;
             }

@@ -867,12 +867,12 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
             xp.scale(rms, gp);
     }
     if constexpr (MB > 0) {
-        // the merge at the end of fused_attn_kernel, value by value
+        // the merge at the end of fused_attn_kernel, in the same arithmetic
         const int blocks = (position() >> a.block_shift) + 1, l16 = lane & 15;
         const float m = l16 < blocks ? __uint_as_float(part_max) : -INFINITY;
         const float largest = row16_max(m); // by all lanes: a lane that is switched off gives its neighbours nothing
         const float w = l16 < blocks ? expf(m - largest) : 0.0f;
-        const float sum = row16_sum(l16 < blocks ? w * __uint_as_float(part_sum) : 0.0f);
+        const float sum = dpp_f32<DPP_ROW_NEWBCAST>(row16_dot(w, l16 < blocks ? __uint_as_float(part_sum) : 0.0f));
         float o[8] = {};
         const float wb[kMergeBlocks] = {dpp_f32<DPP_ROW_NEWBCAST>(w), dpp_f32<DPP_ROW_NEWBCAST + 1>(w)};
 #pragma unroll

@@ -59,7 +59,10 @@ typedef uint16_t llama2_half;
 
 /* new CudaContext(deviceID): src/Transformer.cs:48-49.  Idempotent per device. */
 int llama2_init(int device);
-/* Releases the stream and internal scratch.  Caller-owned buffers stay valid. */
+/* Releases the stream and internal scratch.  Caller-owned buffers and decoders
+ * stay valid and work again after the next llama2_init on the same device; graphs
+ * that the caller captured from modules with scratch (llama2_vec_mat,
+ * llama2_multi_head_attention, the sampler modules) hold its address and do not. */
 int llama2_shutdown(void);
 /* Text of the calling thread's last error ("" if none).  Never NULL. */
 const char* llama2_last_error(void);

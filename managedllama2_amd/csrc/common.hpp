@@ -41,7 +41,7 @@ struct Context {
     int n_retired_partials = 0;
     // per-head arrival counters of llama2_multi_head_attention (zero between launches)
     unsigned* attn_counters = nullptr;
-    SamplerScratch* sampler = nullptr; // between the sampler's launches (sampler_kernels.hpp)
+    SamplerScratch* sampler = nullptr; // between the sampler modules' launches (sampler_kernels.hpp)
     // Pinned: where a kernel leaves the token that the call behind it returns (a copy of 4 bytes is a launch of 4.3 us)
     int* host_token = nullptr;
 };
@@ -56,8 +56,8 @@ int ensure_attn_partials(size_t bytes);
 int resolve_vec_mat_static_scratch(int device);
 // Sampler.Sample's stochastic branch (sampler.hip).  token_only: the caller reads the
 // token alone, so the sort may stop at the head of the distribution that holds top_p of the mass.
-int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, float temperature, float top_p, float coin,
-                  int* result, int pos, bool token_only, const HostStep* host = nullptr);
+int sample_launch(const char* fn, SamplerScratch* scratch, uint16_t* logits, int* indices, int size, float temperature,
+                  float top_p, float coin, int* result, int pos, bool token_only, const HostStep* host = nullptr);
 
 // HIP's current device is a per-thread setting: a host thread other than the one that called
 // llama2_init (a thread-pool worker of the managed host, say) is bound to the library's device on

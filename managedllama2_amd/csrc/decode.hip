@@ -494,6 +494,9 @@ struct llama2_decoder {
     int mode;
     int kv_dim;
     int head_size;
+    // between the sampler's launches (run states with an indices buffer); the decoder's own, because captured steps keep
+    // its address and must replay for as long as the decoder lives, also after a llama2_shutdown and llama2_init
+    l2::SamplerScratch* sampler = nullptr;
     // fused path
     int* state = nullptr;
     float* attn_part = nullptr;
@@ -707,7 +710,7 @@ int launch_sample_step(llama2_decoder* d, float temperature, float top_p, unsign
 {
     SampleArgs a{};
     a.logits = d->s.logits, a.indices = d->s.indices, a.size = d->cfg.vocab_size;
-    a.temperature = temperature, a.top_p = top_p, a.head = 1;
+    a.temperature = temperature, a.top_p = top_p, a.head = 1, a.s = d->sampler;
     a.state = d->state, a.tokens = d->s.tokens, a.seed = seed, a.theta = d->cfg.rope_theta;
     return sample_enqueue("sampled step", a);
 }
@@ -854,6 +857,8 @@ void release(llama2_decoder* d)
                 (void)hipGraphExecDestroy(g);
     if (d->state)
         (void)hipFree(d->state);
+    if (d->sampler)
+        (void)hipFree(d->sampler);
     if (d->persist_layers)
         (void)hipFree(d->persist_layers);
     if (d->persist_scratch)
@@ -1024,6 +1029,8 @@ int llama2_decode_create(llama2_decoder** decoder, const llama2_config* config,
         hipError_t e = hipMalloc(reinterpret_cast<void**>(&d->state), kStateBytes);
         if (e == hipSuccess)
             e = hipMemsetAsync(d->state, 0, kStateBytes, ctx().stream);
+        if (e == hipSuccess && state->indices && c.vocab_size <= LLAMA2_MAX_SAMPLER_SIZE)
+            e = hipMalloc(reinterpret_cast<void**>(&d->sampler), sizeof(SamplerScratch));
         if (e == hipSuccess)
             e = hipStreamSynchronize(ctx().stream);
         if (e != hipSuccess) {
@@ -1142,8 +1149,8 @@ int llama2_decode_sample_top_p(llama2_decoder* d, int next_position, int generat
     const TokenSlot slot = token_slot(d, next_position);
     L2_CHECK(!ctx().capturing, "%s: not allowed during graph capture", fn);
     const HostStep h = host_step(d, next_position);
-    L2_TRY(sample_launch(fn, d->s.logits, d->s.indices, d->cfg.vocab_size, temperature, top_p, coin, slot.tokens,
-                         slot.index, true, &h)); // :50-66
+    L2_TRY(sample_launch(fn, d->sampler, d->s.logits, d->s.indices, d->cfg.vocab_size, temperature, top_p, coin,
+                         slot.tokens, slot.index, true, &h)); // :50-66
     L2_TRY(take_host_token(d, h, token)); // :69
     return persist_status(d, fn);
 }
@@ -1165,7 +1172,7 @@ int llama2_decode_run_sampled(llama2_decoder* d, int position, int steps, int n_
         for (int pos = position; pos < position + steps; ++pos) {
             L2_TRY(forward_modules(d, pos, pos + 1));
             if (pos + 1 >= n_prompt && pos + 1 < d->cfg.seq_len) // the token after the last row has no slot
-                L2_TRY(sample_launch(fn, d->s.logits, d->s.indices, d->cfg.vocab_size, temperature, top_p,
+                L2_TRY(sample_launch(fn, d->sampler, d->s.logits, d->s.indices, d->cfg.vocab_size, temperature, top_p,
                                      sampler_coin(seed, pos + 1), d->s.tokens, pos + 1, true));
         }
         return LLAMA2_OK;

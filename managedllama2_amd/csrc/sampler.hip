@@ -56,8 +56,7 @@ static void launch_pick(const SampleArgs& a, const uint16_t* in, bool in_place)
 int sample_enqueue(const char* name, const SampleArgs& args)
 {
     SampleArgs a = args;
-    SamplerScratch* s = ctx().sampler;
-    a.s = s;
+    SamplerScratch* s = a.s;
     if (!sample_sorts(a.top_p))
         a.head = -1;
     else if (a.size > kSampHeadItems)
@@ -155,15 +154,16 @@ int llama2_sample(llama2_half* logits, int* indices, int size, float temperature
                   int* result, int pos)
 {
     L2_REQUIRE_INIT();
-    return sample_launch("llama2_sample", logits, indices, size, temperature, top_p, coin, result, pos, false);
+    return sample_launch("llama2_sample", ctx().sampler, logits, indices, size, temperature, top_p, coin, result, pos,
+                         false);
 }
 
 } // extern "C"
 
 namespace l2 {
 
-int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, float temperature, float top_p, float coin,
-                  int* result, int pos, bool token_only, const HostStep* host)
+int sample_launch(const char* fn, SamplerScratch* scratch, uint16_t* logits, int* indices, int size, float temperature,
+                  float top_p, float coin, int* result, int pos, bool token_only, const HostStep* host)
 {
     L2_CHECK(logits && indices && result, "%s: null pointer", fn);
     L2_TRY(check_sampler_size(fn, size));
@@ -171,7 +171,7 @@ int sample_launch(const char* fn, uint16_t* logits, int* indices, int size, floa
     L2_CHECK(pos >= 0, "%s: pos=%d is negative", fn, pos);
     L2_CHECK(aligned(logits, 16) && aligned(indices, 16), "%s: logits and indices must be 16-byte aligned", fn);
     SampleArgs a{};
-    a.logits = logits, a.indices = indices, a.size = size;
+    a.logits = logits, a.indices = indices, a.size = size, a.s = scratch;
     a.temperature = temperature, a.top_p = top_p, a.coin = coin, a.result = result, a.pos = pos;
     a.head = token_only ? 1 : 0;
     if (host)

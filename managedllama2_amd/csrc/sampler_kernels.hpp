@@ -35,7 +35,7 @@ constexpr int kSampHeadItems = 32256;
 // 8-element chunks per thread of the 1024 whose sums the results are: 4 up to 32768 elements, 8 up to 65536
 inline int sampler_chunks(int size) { return size <= 4 * 8 * kSampBlock ? 4 : 8; }
 
-// Device memory between the launches; one per library, all launches are in order on its stream.
+// Device memory between the launches, which are in order on the library's stream: one for the modules, and one per decoder.
 struct SamplerScratch {
     uint16_t exps[LLAMA2_MAX_SAMPLER_SIZE];  // half(exp(l - max))
     uint16_t keys[LLAMA2_MAX_SAMPLER_SIZE];  // probabilities in the order that the prefix sums take them

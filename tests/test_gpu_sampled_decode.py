@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from managedllama2_amd import capi, hostlib, modelfile, synth
+from managedllama2_amd.device import DeviceVariable
 from managedllama2_amd.transformer import Transformer
 
 pytestmark = pytest.mark.gpu
@@ -130,6 +131,29 @@ def test_graph_replays_of_the_sampling_step_are_stable():
         runs.append(list(t.runstate.tokens.to_host(26)))
         capi.call("llama2_memset", t.runstate.logits.ptr, 0, 16)
     assert runs[0] == runs[1] == runs[2]
+    t.close()
+
+
+@pytest.mark.parametrize("vocab_size", [1000, 32000, 40000])
+def test_captured_sampling_steps_outlive_a_shutdown(vocab_size):
+    """A decoder's captured steps hold the address of what lies between the sampler's launches.  That memory is the
+    decoder's own: after llama2_shutdown and llama2_init the steps neither read nor write what was allocated since."""
+    cfg = dict(CFG, vocab_size=vocab_size, n_layers=1)
+    model = synth.random_model(cfg, seed=39, rms_random=True)
+    prompt = [int(t) for t in synth.rng_for(606).integers(3, vocab_size, 3)]
+    t = Transformer(dict(cfg), model, mode=FUSED_GRAPH)
+
+    def run():
+        t.runstate.tokens.copy_to_device(np.array(prompt + [0] * 40, np.int32))
+        capi.call("llama2_decode_run_sampled", t._decoder, 0, 25, len(prompt), T, TOP_P, SEED)
+        return list(t.runstate.tokens.to_host(26))
+
+    want = run()
+    capi.call("llama2_shutdown")
+    capi.call("llama2_init", 0)
+    newcomers = [DeviceVariable.from_host(np.full(n // 4, 0x5A5A5A5A, np.uint32)) for n in (1 << 18, 917 << 10, 1 << 20) * 8]
+    assert run() == want
+    assert all((x.to_host() == 0x5A5A5A5A).all() for x in newcomers)
     t.close()
 
 

@@ -510,7 +510,7 @@ struct llama2_decoder {
     float sampled_temperature = 0.0f, sampled_top_p = 0.0f;
     unsigned long long sampled_seed = 0;
     int ready_position = -1; // position whose state a host's sampling call left on the device, or -1
-    bool replayed = false;   // a call was captured: replays may set the state at any time
+    bool replayed = false;   // a call was recorded: replays may set the state at any time
     // persistent step (LLAMA2_DECODE_PERSISTENT): kernel variant, per-layer pointer table and
     // hand-over buffers on the device, and the launch arguments
     int persist_variant = -1;
@@ -748,11 +748,19 @@ int set_state(llama2_decoder* d, int pos, int n_prompt, int advance)
     return LLAMA2_OK;
 }
 
+// The calls are being recorded: between llama2_graph_begin_capture and _end_capture, or by a caller that captures
+// llama2_stream() with the runtime's own calls.
+bool recorded()
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return ctx().capturing || hipStreamIsCapturing(ctx().stream, &status) != hipSuccess ||
+           status != hipStreamCaptureStatusNone;
+}
+
 // The state of a step that a host asked for by position; nothing to do where the sampling of the token before left it.
 int set_host_state(llama2_decoder* d, int pos)
 {
-    if (ctx().capturing)
-        d->replayed = true; // a replay sets the state without a call here
+    d->replayed |= recorded(); // a replay sets the state without a call here
     if (d->ready_position == pos && !d->replayed)
         return LLAMA2_OK;
     d->ready_position = -1;
@@ -1194,7 +1202,7 @@ int llama2_decode_run_sampled(llama2_decoder* d, int position, int steps, int n_
         d->sampled_temperature = temperature, d->sampled_top_p = top_p, d->sampled_seed = seed;
     }
     d->ready_position = -1;
-    d->replayed |= ctx().capturing;
+    d->replayed |= recorded();
     L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)
@@ -1217,7 +1225,7 @@ int llama2_decode_run(llama2_decoder* d, int position, int steps, int n_prompt)
         return LLAMA2_OK;
     }
     d->ready_position = -1;
-    d->replayed |= ctx().capturing;
+    d->replayed |= recorded();
     L2_TRY(run_prompt(d, position, steps, n_prompt));
     L2_TRY(set_state(d, position, n_prompt, 1));
     for (int i = 0; i < steps; ++i)

@@ -1,6 +1,6 @@
 """A host's sampling call leaves the state of the next position's step on the device, so that the forward call for
 that position need not set it.  Every other call in between -- another position, the device-resident loop, a graph the caller
-captured -- has to set it again: each step's logits and cache rows are compared with those of a decoder that never sampled."""
+captured -- has to set it again, and a recorded step sets its own: each step's logits and cache rows are compared with those of a decoder that never sampled."""
 import ctypes as C
 
 import numpy as np
@@ -61,4 +61,47 @@ def test_steps_in_any_order(mode, temperature):
         check(pos)
     capi.call("llama2_graph_destroy", graph)
     for x in (t, ref, other):
+        x.close()
+
+
+@pytest.mark.parametrize("loop", [False, True])
+def test_a_caller_that_captures_the_stream_itself(loop):
+    """llama2_stream() may be captured with the runtime's own calls: what is recorded sets its own state, and the
+    replays count like those of a graph of the library."""
+    model = synth.random_model(CFG, seed=92)
+    t, ref = (Transformer(dict(CFG), model, mode=capi.DECODE_FUSED) for _ in range(2))
+    tokens = synth.rng_for(972).integers(3, 1000, CFG["seq_len"]).astype(np.int32)
+    for x in (t, ref):
+        x.runstate.tokens.copy_to_device(tokens)
+        for pos in range(12):
+            x.Forward(pos, pos + 1)
+    want = {}
+    for pos in (9, 10):
+        ref.Forward(pos, pos + 1)
+        want[pos] = ref.runstate.logits.to_host().view(np.uint16)
+    def logits_are_those_of(pos):
+        return np.array_equal(t.runstate.logits.to_host().view(np.uint16), want[pos])
+
+    lib = capi.load()
+    stream = C.c_void_p(lib.llama2_stream())
+    graph, replay = C.c_void_p(), C.c_void_p()
+
+    t.Forward(9, 10), t.Sample(10, False)  # leaves the state of position 10
+    assert lib.hipStreamBeginCapture(stream, 1) == 0  # of this thread
+    if loop:
+        capi.call("llama2_decode_run", t._decoder, 9, 1, 11)
+    else:
+        capi.call("llama2_decode_forward", t._decoder, 10, 11)
+    assert lib.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert lib.hipGraphInstantiate(C.byref(replay), graph, None, None, 0) == 0
+    for _ in range(3):
+        t.Forward(3, 4), t.Sample(4, False)
+        assert lib.hipGraphLaunch(replay, stream) == 0
+        assert logits_are_those_of(9 if loop else 10)
+        t.Forward(8, 9), t.Sample(9, False)  # leaves the state of position 9 ...
+        assert lib.hipGraphLaunch(replay, stream) == 0  # ... which is gone then
+        t.Forward(9, 10)
+        assert logits_are_those_of(9)
+    assert lib.hipGraphExecDestroy(replay) == 0 and lib.hipGraphDestroy(graph) == 0
+    for x in (t, ref):
         x.close()

@@ -585,6 +585,7 @@ __global__ __launch_bounds__(kSampBlock) void sampler_rank_kernel(SampleArgs a, 
 template <int CH, bool PICK>
 __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, const uint16_t* in)
 {
+    constexpr bool kStaged = PICK || CH > 4;
     __shared__ u32x4 chunk[CH * kSampBlock];
     __shared__ float total[kSampWaves];
     __shared__ int first_hit[kSampWaves];
@@ -608,14 +609,19 @@ __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, 
     int best = size - 1;
     if (go) {
         // 16-byte pieces come in the order of memory; piece p lies at p ^ (p / 16 % CH), where the 16 threads that LDS
-        // serves at a time find theirs, CH apart, in 16 different places
+        // serves at a time find theirs, CH apart, in 16 different places.  Without a pick there is one workgroup, and up to
+        // 32768 values its threads load their own pieces: 32000 values take 4.56 us, through LDS and its barrier 5.00 (1000:
+        // 2.54 and 2.62).  65536 values take 9.4 us like that, for a thread's 8 pieces are 128 bytes apart from the next
+        // one's, and 8.5 through LDS.
+        if (kStaged) {
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int p = threadIdx.x + c * kSampBlock;
-            if (p * 8 < size)
-                chunk[p ^ ((p >> 4) & (CH - 1))] = load_bits8(in, p * 8, size, 0);
+            for (int c = 0; c < CH; ++c) {
+                const int p = threadIdx.x + c * kSampBlock;
+                if (p * 8 < size)
+                    chunk[p ^ ((p >> 4) & (CH - 1))] = load_bits8(in, p * 8, size, 0);
+            }
+            __syncthreads();
         }
-        __syncthreads();
         const int first = threadIdx.x * 8 * CH;
         float f[CH][8];
         float run = 0.0f;
@@ -623,7 +629,7 @@ __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, 
         for (int c = 0; c < CH; ++c) {
             const int p = threadIdx.x * CH + c;
             if (p * 8 < size) {
-                const u32x4 v = chunk[p ^ ((p >> 4) & (CH - 1))];
+                const u32x4 v = kStaged ? chunk[p ^ ((p >> 4) & (CH - 1))] : load_bits8(in, p * 8, size, 0);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     run += half_of(v, k);

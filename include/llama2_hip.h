@@ -291,7 +291,7 @@ int llama2_cumulative_sum(llama2_half* values, int size);
 int llama2_sample_top_p(const llama2_half* logits, const int* indices, int size, float threshold,
                         int* result, int pos);
 
-/* The stochastic branch of Sampler.Sample (src/Sampler.cs:50-66) in one call (four launches):
+/* The stochastic branch of Sampler.Sample (src/Sampler.cs:50-66) in one call (up to four launches):
  * softmax_logits; if 0 < top_p < 1: sort and threshold = coin * top_p, else
  * threshold = coin; cumulative_sum; sample_top_p into result[pos].  logits and
  * indices are overwritten exactly as by the four module calls (same device

@@ -53,8 +53,22 @@ static void launch_pick(const SampleArgs& a, const uint16_t* in, bool in_place)
         hipLaunchKernelGGL((sampler_pick_kernel<8, PICK>), grid, dim3(kSampBlock), 0, ctx().stream, a, in);
 }
 
+template <bool PICK>
+static void launch_one(const SampleArgs& a)
+{
+    if (a.size <= 8 * kSampBlock)
+        hipLaunchKernelGGL((sampler_one_kernel<1, PICK>), dim3(1), dim3(kSampBlock), 0, ctx().stream, a);
+    else
+        hipLaunchKernelGGL((sampler_one_kernel<2, PICK>), dim3(1), dim3(kSampBlock), 0, ctx().stream, a);
+}
+
 int sample_enqueue(const char* name, const SampleArgs& args)
 {
+    if (!sample_sorts(args.top_p) && args.size <= kSampOneItems) {
+        launch_one<true>(args);
+        L2_LAUNCH_CHECK(name);
+        return LLAMA2_OK;
+    }
     SampleArgs a = args;
     SamplerScratch* s = a.s;
     if (!sample_sorts(a.top_p))
@@ -95,6 +109,11 @@ int llama2_softmax_logits(llama2_half* logits, int size, float temperature, int*
     L2_CHECK(aligned(logits, 16) && aligned(indices, 16), "%s: logits and indices must be 16-byte aligned", fn);
     SampleArgs a{};
     a.logits = logits, a.indices = indices, a.size = size, a.temperature = temperature, a.s = ctx().sampler, a.head = -1;
+    if (size <= kSampOneItems) {
+        launch_one<false>(a);
+        L2_LAUNCH_CHECK(fn);
+        return LLAMA2_OK;
+    }
     launch_exp(a);
     hipLaunchKernelGGL(sampler_tile_kernel<TILE_EXPS>, dim3(ceil_div(size, kSampTile)), dim3(kTileThreads), 0, ctx().stream,
                        a, static_cast<const uint16_t*>(nullptr), static_cast<const int*>(nullptr), logits);

@@ -6,6 +6,7 @@
 //   sampler_tile_kernel   the sum, the probabilities, tiles of 1024 of them sorted
 //   sampler_rank_kernel   the place of every item: how many items of each tile sort in front of it
 //   sampler_pick_kernel   prefix sums and the pick
+// A short vector that need not be sorted takes one launch of one workgroup (sampler_one_kernel).
 //
 // What bounds it: nothing but latency; 32000 logits are 64 KB.  The reference's shape, one workgroup of 1024
 // threads for everything, kept one of 256 compute units busy: the two divisions and the exp of every logit took 14 us
@@ -71,7 +72,7 @@ struct SampleArgs {
     HostStep host; // a host's own loop
 };
 
-// Queues the four launches (three without a sort); checks nothing.
+// Queues the four launches (without a sort three, or one); checks nothing.
 int sample_enqueue(const char* name, const SampleArgs& a);
 
 inline bool sample_sorts(float top_p) { return !(top_p <= 0.0f || top_p >= 1.0f); } // src/Sampler.cs:56
@@ -578,10 +579,100 @@ __global__ __launch_bounds__(kSampBlock) void sampler_rank_kernel(SampleArgs a, 
 // ---- 4. prefix sums and the pick -------------------------------------------------------
 // native/cumulative_sum_kernel.cu:8-26: inclusive prefix sums in fp32, each rounded to fp16.  A thread sums its
 // 8 CH consecutive values in order, the thread totals are scanned by doubling within a wavefront and in order over the
-// wavefronts.  Every workgroup scans everything (64 KB from the L2) and stores the share of wavefront blockIdx.x, so
-// that nothing has to be handed from one to the other; in a launch of one workgroup it stores everything and may work
-// in place.  native/sample_top_p_kernel.cu:8-21: the first workgroup finds the first position whose sum reaches the
-// threshold (the last position if none does) of `indices`.
+// wavefronts.  `piece(p)` gives the 16-byte piece p of the values; all = false: the sums of wavefront blockIdx.x alone are
+// stored.  PICK, native/sample_top_p_kernel.cu:8-21: returns a thread's first position whose sum reaches the threshold,
+// or the last position.
+template <int CH, bool PICK, class F>
+__device__ __forceinline__ int prefix_sums(const F& piece, int size, float threshold, bool all, uint16_t* out, float* total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int first = threadIdx.x * 8 * CH;
+    int best = size - 1;
+    float f[CH][8];
+    float run = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int p = threadIdx.x * CH + c;
+        if (p * 8 < size) {
+            const u32x4 v = piece(p);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                run += half_of(v, k);
+                f[c][k] = run;
+            }
+        }
+    }
+    float inc = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const float o = __shfl_up(inc, off, 64);
+        if (lane >= off)
+            inc += o;
+    }
+    if (lane == 63)
+        total[wave] = inc;
+    __syncthreads();
+    float before = 0.0f; // total of the wavefronts in front of this one
+#pragma unroll
+    for (int w = 0; w < kSampWaves; ++w)
+        before += w < wave ? total[w] : 0.0f;
+    before = before + inc - run;
+    // Probabilities are not negative (or all of them are NaN): a thread whose last sum does not reach the threshold
+    // has none that does, so only those that have one look for the first.
+    const bool hit = PICK && blockIdx.x == 0 && first < size &&
+                     half_bits_to_float(float_to_half_bits(before + run)) >= threshold;
+    const bool mine = all || wave == static_cast<int>(blockIdx.x);
+    if (mine || hit) {
+#pragma unroll
+        for (int c = CH - 1; c >= 0; --c) {
+            const int base = first + c * 8;
+            if (base < size) {
+                uint16_t b[8];
+#pragma unroll
+                for (int k = 7; k >= 0; --k) {
+                    b[k] = float_to_half_bits(before + f[c][k]);
+                    if (hit && base + k < size && half_bits_to_float(b[k]) >= threshold)
+                        best = base + k;
+                }
+                if (mine)
+                    store_half8(out, base, size, b);
+            }
+        }
+    }
+    return best;
+}
+
+// The lowest of the threads' positions; where its token goes.  go = false: a decode step that draws none.
+__device__ __forceinline__ void finish_pick(const SampleArgs& a, int best, bool go, int* first_hit)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const int o = __shfl_xor(best, off, 64);
+        best = o < best ? o : best;
+    }
+    if ((threadIdx.x & 63) == 0)
+        first_hit[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    for (int w = 1; w < kSampWaves; ++w)
+        best = first_hit[w] < best ? first_hit[w] : best;
+    if (!a.state) {
+        const int token = a.indices[best];
+        a.result[a.pos] = token;
+        write_host_token(a.host, token);
+        return;
+    }
+    const int next = a.state[kStatePos] + 1;
+    if (go)
+        a.tokens[next] = a.indices[best];
+    if (a.state[kStateAdvance])
+        a.state[kStatePos] = next;
+}
+
+// Every workgroup scans everything (64 KB from the L2) and stores the share of wavefront blockIdx.x, so that nothing has
+// to be handed from one to the other; in a launch of one workgroup it stores everything and may work in place.  The
+// first workgroup picks.
 template <int CH, bool PICK>
 __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, const uint16_t* in)
 {
@@ -589,7 +680,6 @@ __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, 
     __shared__ u32x4 chunk[CH * kSampBlock];
     __shared__ float total[kSampWaves];
     __shared__ int first_hit[kSampWaves];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int size = a.size;
     float threshold = a.coin;
     bool go = true;
@@ -622,83 +712,115 @@ __global__ __launch_bounds__(kSampBlock) void sampler_pick_kernel(SampleArgs a, 
             }
             __syncthreads();
         }
-        const int first = threadIdx.x * 8 * CH;
-        float f[CH][8];
-        float run = 0.0f;
+        best = prefix_sums<CH, PICK>(
+            [&](int p) { return kStaged ? chunk[p ^ ((p >> 4) & (CH - 1))] : load_bits8(in, p * 8, size, 0); }, size,
+            threshold, gridDim.x == 1, a.logits, total);
+    }
+    if (PICK && blockIdx.x == 0)
+        finish_pick(a, best, go, first_hit);
+}
+
+// ---- 1, 2 and 4 in one workgroup ---------------------------------------------------------
+// Without a sort the launches of the others cost more than one compute unit alone takes for a short vector: the
+// probabilities of 1000 / 5000 / 8192 / 11264 logits take 5.8 / 6.6 / 6.7 / 6.5 us in two launches of many workgroups and
+// 2.7 / 4.1 / 4.9 / 6.2 here, with the pick (and 2.5 us for the copy of the logits) 11.1 / 12.6 / 12.7 / 13.2 in three and 6.6 /
+// 8.1 / 8.9 / 11.0 here.  Every 2048 logits more are another wavefront with a second piece on each SIMD and 0.5 us.
+constexpr int kSampOneItems = 11 * 1024;
+
+template <int PIECES, bool PICK> // PIECES: of 8 logits per thread
+__global__ __launch_bounds__(kSampBlock) void sampler_one_kernel(SampleArgs a)
+{
+    constexpr int CH = 4; // pieces per thread of the prefix sums
+    __shared__ u32x4 chunk[PICK ? PIECES * kSampBlock : 1];
+    __shared__ float red[3][kSampWaves];
+    __shared__ int first_hit[kSampWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float threshold = a.coin;
+    bool go = true;
+    if (PICK && a.state) { // read by every thread before the first one changes it, behind the barrier of finish_pick
+        const int next = a.state[kStatePos] + 1;
+        go = next >= a.state[kStatePrompt] && next < a.state[kStateSlots];
+        threshold = sampler_coin(a.seed, next);
+        if (a.state[kStateAdvance] && threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
+            write_rope_table(a.state, threadIdx.x - 64, next, a.theta); // for the next step
+    } else if (PICK && threadIdx.x >= 64) {
+        write_host_step_state(a.host, threadIdx.x - 64);
+    }
+    int best = a.size - 1;
+    if (go) {
+        float f[PIECES][8];
+        uint16_t b[PIECES][8];
+        float m = -INFINITY;
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int p = threadIdx.x * CH + c;
-            if (p * 8 < size) {
-                const u32x4 v = kStaged ? chunk[p ^ ((p >> 4) & (CH - 1))] : load_bits8(in, p * 8, size, 0);
+        for (int c = 0; c < PIECES; ++c) {
+            const int base = (threadIdx.x + c * kSampBlock) * 8;
+            if (base < a.size) {
+                const u32x4 v = load_bits8(a.logits, base, a.size, 0xFC00u);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
-                    run += half_of(v, k);
-                    f[c][k] = run;
+                    f[c][k] = half_bits_to_float(float_to_half_bits(half_of(v, k) / a.temperature));
+                    m = base + k < a.size ? fmaxf(m, f[c][k]) : m;
                 }
             }
         }
-        float inc = run;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float o = __shfl_up(inc, off, 64);
-            if (lane >= off)
-                inc += o;
-        }
-        if (lane == 63)
-            total[wave] = inc;
+        m = wave_max(m);
+        if (lane == 0)
+            red[0][wave] = m;
         __syncthreads();
-        float before = 0.0f; // total of the wavefronts in front of this one
+        m = row16_max(red[0][lane & 15]);
+        float sum = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kSampWaves; ++w)
-            before += w < wave ? total[w] : 0.0f;
-        before = before + inc - run;
-        // Probabilities are not negative (or all of them are NaN): a thread whose last sum does not reach the threshold
-        // has none that does, so only those that have one look for the first.
-        const bool hit = PICK && blockIdx.x == 0 && first < size &&
-                         half_bits_to_float(float_to_half_bits(before + run)) >= threshold;
-        if (gridDim.x == 1 || wave == static_cast<int>(blockIdx.x) || hit) {
+        for (int c = 0; c < PIECES; ++c) {
+            const int base = (threadIdx.x + c * kSampBlock) * 8;
+            if (base < a.size) {
 #pragma unroll
-            for (int c = CH - 1; c >= 0; --c) {
-                const int base = first + c * 8;
-                if (base < size) {
-                    uint16_t b[8];
-#pragma unroll
-                    for (int k = 7; k >= 0; --k) {
-                        b[k] = float_to_half_bits(before + f[c][k]);
-                        if (hit && base + k < size && half_bits_to_float(b[k]) >= threshold)
-                            best = base + k;
-                    }
-                    if (gridDim.x == 1 || wave == static_cast<int>(blockIdx.x))
-                        store_half8(a.logits, base, size, b);
+                for (int k = 0; k < 8; ++k) {
+                    const float e = base + k < a.size ? expf(f[c][k] - m) : 0.0f;
+                    sum += e;
+                    b[c][k] = float_to_half_bits(e);
                 }
             }
         }
-    }
-    if (!PICK || blockIdx.x != 0)
-        return;
+        sum = wave_sum(sum);
+        if (lane == 0)
+            red[1][wave] = sum;
+        __syncthreads();
+        sum = wave_sum(lane < kSampWaves ? red[1][lane] : 0.0f);
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(best, off, 64);
-        best = o < best ? o : best;
+        for (int c = 0; c < PIECES; ++c) {
+            const int p = threadIdx.x + c * kSampBlock, base = p * 8;
+            if (base < a.size) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    b[c][k] = float_to_half_bits(half_bits_to_float(b[c][k]) / sum);
+                if (PICK) {
+                    u32x4 v;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        v[k] = b[c][2 * k] | static_cast<uint32_t>(b[c][2 * k + 1]) << 16;
+                    chunk[p ^ ((p >> 4) & (CH - 1))] = v;
+                } else {
+                    store_half8(a.logits, base, a.size, b[c]);
+                }
+                if (base + 8 <= a.size) {
+                    u32x4* to = reinterpret_cast<u32x4*>(a.indices + base);
+                    const uint32_t i = base;
+                    to[0] = u32x4{i, i + 1, i + 2, i + 3};
+                    to[1] = u32x4{i + 4, i + 5, i + 6, i + 7};
+                } else {
+                    for (int i = base; i < a.size; ++i)
+                        a.indices[i] = i;
+                }
+            }
+        }
+        if (PICK) {
+            __syncthreads();
+            best = prefix_sums<CH, true>([&](int p) { return chunk[p ^ ((p >> 4) & (CH - 1))]; }, a.size, threshold, true,
+                                         a.logits, red[2]);
+        }
     }
-    if (lane == 0)
-        first_hit[wave] = best;
-    __syncthreads();
-    if (threadIdx.x != 0)
-        return;
-    for (int w = 1; w < kSampWaves; ++w)
-        best = first_hit[w] < best ? first_hit[w] : best;
-    if (!a.state) {
-        const int token = a.indices[best];
-        a.result[a.pos] = token;
-        write_host_token(a.host, token);
-        return;
-    }
-    const int next = a.state[kStatePos] + 1;
-    if (go)
-        a.tokens[next] = a.indices[best];
-    if (a.state[kStateAdvance])
-        a.state[kStatePos] = next;
+    if (PICK)
+        finish_pick(a, best, go, first_hit);
 }
 
 // The pick alone, on any values.

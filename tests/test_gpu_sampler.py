@@ -290,6 +290,32 @@ class TestTileEdges:
             assert t1 == oracle.ref_sample_top_p(cdf1, idx1, float(np.float32(0.61) * np.float32(top_p)))
             assert logits[t1] > -np.inf
 
+    @pytest.mark.parametrize("size", [1, 5, 8, 511, 513, 4097, 8192, 8193, 10007, 11264])
+    @pytest.mark.parametrize("temperature", [0.01, 0.7, float("inf")])
+    def test_one_workgroup_equals_many(self, size, temperature):
+        """Up to 11264 logits, and without a sort, one workgroup does it all.  With masked tokens behind them the same
+        logits go through the launches of many workgroups: the same sums, so the same bits."""
+        x = synth.normal_f16(synth.rng_for(954, size), size, 2.0)
+        x[size // 3] = x[-1] = np.float16(-0.0)
+        if np.isfinite(temperature):  # -inf / inf is no number
+            x[size // 2] = -np.inf if size > 5 else x[size // 2]
+            longer = np.concatenate([x, np.full(12000 - size, -np.inf, np.float16)])
+            p, idx = SoftmaxLogits(x, temperature)
+            wp, widx = SoftmaxLogits(longer, temperature)
+            assert np.array_equal(p.view(np.uint16), wp[:size].view(np.uint16)) and np.array_equal(idx, widx[:size])
+            for top_p, coin in ((1.0, 0.0), (0.0, 0.37), (2.0, 0.93), (1.0, 0.9999)):
+                t1, cdf1, idx1 = fused_sample(x, temperature, top_p, coin)
+                t2, cdf2, idx2 = fused_sample(longer, temperature, top_p, coin)
+                # a sum that never reaches the coin picks the last position
+                assert t1 == (t2 if t2 < size else size - 1)
+                assert np.array_equal(cdf1.view(np.uint16), cdf2[:size].view(np.uint16)) and np.array_equal(idx1, idx2[:size])
+        else:
+            p, _ = SoftmaxLogits(x, temperature)
+            assert np.all(p == np.float16(1.0 / size))
+        nothing = np.full(size, np.nan, np.float16)
+        assert np.all(np.isnan(SoftmaxLogits(nothing, temperature)[0]))
+        assert fused_sample(nothing, temperature, 1.0, 0.5)[0] == size - 1
+
     @pytest.mark.parametrize("size", [1000, 32000, 65536])
     def test_infinite_logits_and_temperatures(self, size):
         x = synth.normal_f16(synth.rng_for(953, size), size, 2.0)

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(1024) void argmax_host_kernel(const uint16_t* x, in
                                                            HostStep host)
 {
     __shared__ float sv[16];
-    __shared__ int si[16];
+    __shared__ int si[1];
     const int best = block1024_argmax(x, size, sv, si, [&]() {
         if (threadIdx.x >= 64 && threadIdx.x < 64 + kRopeHeadSize / 2)
             write_host_step_state(host, threadIdx.x - 64);
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(1024) void argmax_step_kernel(const uint16_t* x, in
                                                            float theta)
 {
     __shared__ float sv[16];
-    __shared__ int si[16];
+    __shared__ int si[1];
     // read by every thread before thread 0 updates the position (one 16-byte scalar load)
     const int pos0 = state[0], n_prompt = state[1], advance0 = state[2], n_slots = state[3];
     const int best = block1024_argmax(x, size, sv, si, [&]() {
@@ -581,6 +581,23 @@ int forward_modules(llama2_decoder* d, int position, int next_position)
 }
 
 QW qw(const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; }
+
+// The o-projection that merges the blocks of attention while it stages its input, if there is one for the shape
+// (launch: false only asks).  Every workgroup reads the results of all blocks, so there is one of 16 wavefronts per
+// compute unit.  What the hand-over inside the attention launch costs (2.1 us) is what two blocks gain, less 0.6 us
+// of staging: 7B at 130 .. 250 rows 1108 -> 1084 us per token.  Four blocks gain 0.1 % (1114.9 us for 1117), eight lose 3 %
+// (1180 for 1146 at 700 rows), and so does 13B's o-projection, whose 20 rows per compute unit fit no such workgroup,
+// with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.
+bool launch_o_merge(const Int4Args& a, int blocks, bool launch)
+{
+    if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || !span_allowed(a, 1))
+        return false;
+    switch (ceil_div(a.ws / 4, 64)) {
+    case 1: return try_span<1, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    case 2: return try_span<2, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    default: return false;
+    }
+}
 
 constexpr int kPersistShape = kAttnShapes; // index of the persistent step among the launch shapes
 

@@ -153,7 +153,6 @@ __device__ __forceinline__ void commit_pieces_t(u32x4* xs, float* sx, const VecP
         commit_piece<J>(xs, sx, p.v[i], tid + i * 256);
 }
 
-
 template <int J>
 __device__ __forceinline__ void commit_pieces(u32x4* xs, float* sx, const VecPieces<J>& p)
 {
@@ -1070,8 +1069,8 @@ __global__ __launch_bounds__(256) void int4_matvec_generic_kernel(Int4Args a)
 // Wavefronts of a 256-thread kernel that fit on the GPU at once.  The kernels here are persistent
 // (a wavefront walks over its rows until none is left), so a grid larger than that is not "more
 // parallelism": the workgroups that do not fit start when the first ones are done, a second round
-// that nobody overlaps with (13B QKV: 13.4 us with 20 wavefronts per CU requested and 16 resident,
-// 11.0 us with 16 requested).
+// that nobody overlaps with (13B QKV while it had these kernels: 13.4 us with 20 wavefronts per CU
+// requested and 16 resident, 11.0 us with 16 requested; the span kernel has its launches now).
 template <auto Kernel, int THREADS = 256>
 inline int resident_waves()
 {
@@ -1174,23 +1173,6 @@ inline void launch_j(const Int4Args& a, int max_waves)
 // Number of chunk-columns a lane holds per row for a K-input tensor.
 inline int chunk_columns(int ws) { return ceil_div(ws / 4, 64); }
 constexpr int kMaxChunkColumns = 8; // K <= 16384 on the unrolled kernels
-
-// The o-projection that merges the blocks of attention while it stages its input, if there is one for the shape
-// (launch: false only asks).  Every workgroup reads the results of all blocks, so there is one of 16 wavefronts per
-// compute unit.  What the hand-over inside the attention launch costs (2.1 us) is what two blocks gain, less 0.6 us
-// of staging: 7B at 130 .. 250 rows 1108 -> 1084 us per token.  Four blocks gain 0.1 % (1114.9 us for 1117), eight lose 3 %
-// (1180 for 1146 at 700 rows), and so does 13B's o-projection, whose 20 rows per compute unit fit no such workgroup,
-// with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.
-inline bool launch_o_merge(const Int4Args& a, int blocks, bool launch)
-{
-    if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || !span_allowed(a, 1))
-        return false;
-    switch (ceil_div(a.ws / 4, 64)) {
-    case 1: return try_span<1, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
-    case 2: return try_span<2, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
-    default: return false;
-    }
-}
 
 // Wavefronts kept resident per launch: 16 per CU while a lane holds up to 3
 // chunks of a row (20 for the three-tensor QKV launch of single rows), 8 per CU

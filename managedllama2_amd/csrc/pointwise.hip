@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kBlock) void argmax_kernel(const uint16_t* x, int s
                                                         int write_token)
 {
     __shared__ float sv[kBlockWaves];
-    __shared__ int si[kBlockWaves];
+    __shared__ int si[1];
     const int best = block1024_argmax(x, size, sv, si);
     if (threadIdx.x == 0 && write_token)
         result[pos] = best;

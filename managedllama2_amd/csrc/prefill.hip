@@ -215,11 +215,12 @@ __device__ __forceinline__ void static_for(const F& f, std::integer_sequence<int
 // weight tile and group, a step covers WK consecutive groups of K.  At the end the WK sums add up, and the tiles
 // of a pair meet, through LDS.  The launch may split K further (EPI_PARTIAL).
 //
-// What bounds it: the power the matrix cores take.  A step of four tiles is 1024 cycles of matrix products per wavefront, two
-// wavefronts to a SIMD, and takes 2990; the clock falls from 2.4 to 1.6 .. 2.0 GHz while it lasts (a loop of
-// nothing but these products on random numbers, with their LDS reads, runs at 1.8).  7B, 511 rows, QKV: 1.08 PFLOP/s over the
-// steps, where a library product of 8192^3 reaches 1.16.  What is left is the 3.5 us to the first step and 4 us behind the
-// last, and rounds of workgroups that do not fill the card.  So the vector work and the loads stay out of the way:
+// What bounds it: a step of four tiles is 1024 cycles of matrix products per wavefront, two wavefronts to a SIMD, and takes
+// 2990, so that the matrix cores wait 940 of them (the barrier, LDS, vector work that no product covers); and the clock, which
+// their power brings from 2.4 down to 1.6 .. 2.0 GHz (a loop of nothing but these products on random numbers, with
+// their LDS reads, runs at 1.8 and reaches 1.65 PFLOP/s).  7B, 511 rows, QKV: 1.08 PFLOP/s over the steps; a library product of
+// 8192^3 reaches 1.14.  Around the steps there are 3.5 us to the first and 4 us behind the last one, and rounds of
+// workgroups that do not fill the card.  So the vector work and the loads stay out of the way:
 // - Vector work runs beside the matrix products only where it stands between them (5 instructions for one product
 //   of 32 cycles cost nothing, 8 cost 12 cycles); left to the compiler the unpacking and the scaled sums came after the
 //   products of their step, 5000 cycles for four tiles.

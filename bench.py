@@ -541,7 +541,7 @@ def main():
                                           capi.call("llama2_sort", lg.ptr, idx.ptr, vocab),
                                           capi.call("llama2_cumulative_sum", lg.ptr, vocab),
                                           capi.call("llama2_sample_top_p", lg.ptr, idx.ptr, vocab, 0.45, tok.ptr, 1)))
-        timed("one_launch_us", lambda: capi.call("llama2_sample", lg.ptr, idx.ptr, vocab, temp, top_p, 0.5, tok.ptr, 1))
+        timed("one_call_us", lambda: capi.call("llama2_sample", lg.ptr, idx.ptr, vocab, temp, top_p, 0.5, tok.ptr, 1))
         n_prompt, n_gen = 128, 256
         steps = n_prompt + n_gen - 1
         prompt = synth.rng_for(5).integers(3, vocab, n_prompt).astype(np.int32)
@@ -567,7 +567,7 @@ def main():
         log("sampler (32000 logits, T=0.5, top-p 0.9): softmax %.1f + sort %.1f + cumsum %.1f + pick %.1f us; "
             "four modules %.1f us, one call %.1f us; sampled decode %.1f tok/s (host loop %s)" %
             (sampler["softmax_logits_us"], sampler["sort_us"], sampler["cumulative_sum_us"],
-             sampler["sample_top_p_us"], sampler["four_modules_us"], sampler["one_launch_us"],
+             sampler["sample_top_p_us"], sampler["four_modules_us"], sampler["one_call_us"],
              sampler["decode_tokens_per_s"], sampler.get("host_loop_tokens_per_s")))
 
     if "repack" in legs:

@@ -1,6 +1,6 @@
 """Sampler.Sample with temperature and top-p (src/Sampler.cs:40-70) inside the
 decode loop: the host loop over the four sampler modules, the decoder's
-one-launch sampler, the device-resident sampling loop (eager and hipGraph) and
+sampler in one call, the device-resident sampling loop (eager and hipGraph) and
 the C++ host must all pick the same tokens from the same coins, and agree with
 the CPU oracle teacher-forced on the GPU's history."""
 import ctypes as C
@@ -60,7 +60,7 @@ def test_coin_is_the_oracles(oracle):
 
 
 def test_decoder_sampler_equals_module_sampler():
-    """Host loop over the four sampler modules == decoder's one-launch sampler (the module-by-module
+    """Host loop over the four sampler modules == decoder's sampler in one call (the module-by-module
     forward gives bit-identical logits in both, so every token must agree)."""
     model = synth.random_model(CFG, seed=33, rms_random=True)
     prompt = [int(t) for t in synth.rng_for(601).integers(3, CFG["vocab_size"], 4)]
@@ -101,7 +101,7 @@ def test_device_resident_sampling_loop(mode):
 
 @pytest.mark.parametrize("temperature", [0.05, 0.3, 1.0, 3.0, 30.0])
 def test_device_loop_sorts_only_what_it_needs(temperature):
-    """The decoder's samplers (one launch per token, and the device-resident loop) sort only the head of
+    """The decoder's samplers (one call per token, and the device-resident loop) sort only the head of
     the distribution that holds more than top_p of the mass, and everything when there is no short head;
     the sampler modules sort all 32000 entries.  From peaked (a handful of candidates) to flat (no short
     head) the tokens must be the same."""

@@ -213,7 +213,7 @@ def module_sample(logits, temperature, top_p, coin, pos=1):
 class TestSample:
     @pytest.mark.parametrize("size", [5, 1000, 32000, 40000])
     @pytest.mark.parametrize("top_p", [0.9, 1.0, 0.0, 0.3])
-    def test_one_launch_equals_the_four_modules(self, oracle, size, top_p):
+    def test_one_call_equals_the_four_modules(self, oracle, size, top_p):
         rng = synth.rng_for(941, size)
         logits = synth.normal_f16(rng, size, 2.0)
         for coin in (0.0, 0.37, 0.93, 0.999999):

@@ -695,8 +695,9 @@ __global__ __launch_bounds__(256) void int4_matvec_block_kernel(Int4Args a)
 //     row's requests had become "vector load, wait for everything"; the kernel arguments were
 //     fetched in five dependent round trips; with one row per wavefront the compiler mixed the dot
 //     product into the staging code.  See the comments at those three places below.
-// QKV_ROPE: a workgroup of 8 wavefronts takes rows n .. n + 3 and n + 64 .. n + 67 of a head (of
+// QKV_ROPE, one row per wavefront: a workgroup of 8 takes rows n .. n + 3 and n + 64 .. n + 67 of a head (of
 // q, k and v), the two halves of four RoPE pairs, and exchanges the fp16-rounded results through LDS.
+// Two rows: a wavefront takes the two rows of a pair itself.
 // ---------------------------------------------------------------------------------------------
 
 struct SpanPlan {
@@ -707,15 +708,15 @@ struct SpanPlan {
 // Scale words (pairs of fp16) a lane fetches per tensor: ROWS rows of at most 16 J scales each.
 constexpr int span_scale_words(int J, int ROWS) { return (ROWS * 16 * J + 127) / 128; }
 
-// QKV + RoPE: wavefronts per SIMD that the registers have to leave room for.  Its N / 8 workgroups of one row per
-// wavefront are all there at once with 3 to a compute unit where dim is 4097 .. 6144; left alone the compiler requests all rows
-// ahead and takes 124 registers, two workgroups.  13B: 12.0 us by wavefronts that stride over the rows, 11.2 like this.
-constexpr int span_waves_per_simd(int J, int MODE) { return MODE == QKV_ROPE && J == 3 ? 6 : 1; }
-
 template <int J, int MODE, int STAGE, int TN, int WAVES, int ROWS>
-__global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4_matvec_span_kernel(Int4Args a, SpanPlan plan)
+__global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a, SpanPlan plan)
 {
-    static_assert(MODE != QKV_ROPE || (WAVES == 8 && ROWS == 1 && TN == 3), "RoPE pairs: 8 wavefronts, one row each");
+    // The rows i and i + 64 of a RoPE pair are not neighbours: their scales and zero words are two runs, one to each
+    // half of the lanes.
+    constexpr bool PAIR = MODE == QKV_ROPE && ROWS == 2;
+    static_assert(MODE != QKV_ROPE || (TN == 3 && (PAIR ? J <= 4 : WAVES == 8 && ROWS == 1)),
+                  "RoPE pairs: 8 wavefronts of one row each, or one pair each of rows with at most 64 scales");
+    constexpr int kRowStep = PAIR ? 64 : 1;
     constexpr int SD = span_scale_words(J, ROWS);
     constexpr int JC = J * 64;
     constexpr int Q = ROWS * TN; // row loads per wavefront
@@ -735,7 +736,11 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
         bx = (k >> 4) * 128 + (bx & 7) * 16 + (k & 15);
     }
     int r0, n;
-    if (MODE == QKV_ROPE) { // 16 workgroups per head: rows 4 b .. 4 b + 3 (wavefronts 0-3) and + 64 (wavefronts 4-7)
+    if (PAIR) {
+        const int pair = bx * WAVES + wave;
+        r0 = (pair >> 6) * kRopeHeadSize + (pair & 63);
+        n = r0 < a.N ? 2 : 0;
+    } else if (MODE == QKV_ROPE) { // 16 workgroups per head: rows 4 b .. 4 b + 3 (wavefronts 0-3) and + 64 (wavefronts 4-7)
         r0 = (bx >> 4) * kRopeHeadSize + (bx & 15) * 4 + (wave & 3) + (wave >> 2) * 64;
         n = r0 < a.N ? 1 : 0;
     } else {
@@ -749,7 +754,7 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
     auto load_w = [&](u32x4 (&w)[J], int q) { // q = i TN + t: constants after unrolling
         const int i = q / TN, t = q % TN;
         const __amdgpu_buffer_rsrc_t rw =
-            make_rsrc(uniform_ptr(a.m[t].w + static_cast<size_t>(r0 + i) * a.ws), i < n ? a.ws * 4 : 0);
+            make_rsrc(uniform_ptr(a.m[t].w + static_cast<size_t>(r0 + i * kRowStep) * a.ws), i < n ? a.ws * 4 : 0);
 #pragma unroll
         for (int j = 0; j < J; ++j)
             w[j] = __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16 + j * 1024, 0, kAuxStream);
@@ -816,10 +821,19 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
     if (MODE == QKV_ROPE && a.rope_table && threadIdx.x < kRopeHeadSize)
         rope_entry = a.rope_table[threadIdx.x];
     uint32_t sreg[TN][SD], zreg[TN], res = 0;
+    const int rows_apart = n ? (n - 1) * kRowStep + 1 : 0; // from the first row to behind the last one
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(uniform_ptr(a.m[t].s + static_cast<size_t>(r0) * a.ss), n * a.ss * 2);
-        const __amdgpu_buffer_rsrc_t rz = make_rsrc(uniform_ptr(a.m[t].z + static_cast<size_t>(r0) * a.zs), n * a.zs * 4);
+        const __amdgpu_buffer_rsrc_t rs =
+            make_rsrc(uniform_ptr(a.m[t].s + static_cast<size_t>(r0) * a.ss), rows_apart * a.ss * 2);
+        const __amdgpu_buffer_rsrc_t rz =
+            make_rsrc(uniform_ptr(a.m[t].z + static_cast<size_t>(r0) * a.zs), rows_apart * a.zs * 4);
+        if (PAIR) { // a word behind the end of its row belongs to another row and meets zeros of the input
+            const int row = (lane >> 5) * kRowStep, word = (lane & 31) * 4;
+            sreg[t][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, row * a.ss * 2 + word, 0, 0);
+            zreg[t] = __builtin_amdgcn_raw_buffer_load_b32(rz, row * a.zs * 4 + word, 0, 0);
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < SD; ++k)
             sreg[t][k] = __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4 + k * 256, 0, 0);
@@ -927,8 +941,9 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
             __builtin_amdgcn_sched_barrier(0);
         const int i = q / TN, t = q % TN;
         Frag<J, 1> cur;
-        const uint16_t* sp = reinterpret_cast<const uint16_t*>(&meta_s[wave][t][0]) + i * a.ss + (lane >> 2);
-        const uint32_t* zp = &meta_z[wave][t][0] + i * a.zs + (lane >> 5);
+        const uint16_t* sp =
+            reinterpret_cast<const uint16_t*>(&meta_s[wave][t][0]) + i * (PAIR ? 64 : a.ss) + (lane >> 2);
+        const uint32_t* zp = &meta_z[wave][t][0] + i * (PAIR ? 32 : a.zs) + (lane >> 5);
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             cur.w[0][j] = ring[q & 1][j];
@@ -941,7 +956,24 @@ __global__ __launch_bounds__(WAVES * 64, span_waves_per_simd(J, MODE)) void int4
         outv[t] = lane == i ? s : outv[t];
     }
 
-    if (MODE == QKV_ROPE) {
+    if constexpr (PAIR) {
+        const int pos = position();
+        if (lane < n) { // lane 0 row i, lane 1 row i + 64; the unfused path stores q/k as fp16 and RoPE reads them back
+            const int i = r0 & 63, row = r0 + lane * kRowStep;
+            const float c = rope_tab[2 * i], sn = rope_tab[2 * i + 1];
+            uint16_t rotated[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const float mine = half_bits_to_float(float_to_half_bits(outv[t])), other = dpp_f32<DPP_QUAD_XOR1>(mine);
+                uint16_t b0, b1;
+                rope_rotate(b0, b1, lane ? other : mine, lane ? mine : other, c, sn); // native/rope_kernel.cu:14-26
+                rotated[t] = lane ? b1 : b0;
+            }
+            a.out[0][row] = rotated[0];
+            a.out[1][static_cast<size_t>(pos) * a.kv_dim + row] = rotated[1];
+            a.out[2][static_cast<size_t>(pos) * a.kv_dim + row] = float_to_half_bits(outv[2]);
+        }
+    } else if (MODE == QKV_ROPE) {
         // the unfused path stores q/k as fp16 and RoPE reads them back: keep that rounding
         const float qv = half_bits_to_float(float_to_half_bits(__builtin_bit_cast(
             float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, outv[0])))));
@@ -1096,7 +1128,7 @@ inline bool try_span(const Int4Args& a, bool launch = true)
     if (MODE == QKV_ROPE) {
         if (a.N % kRopeHeadSize)
             return false;
-        plan.grid = a.N / 8;
+        plan.grid = ROWS == 2 ? ceil_div(a.N / 2, WAVES) : a.N / 8;
     } else {
         int waves = ceil_div(a.N, ROWS);
         waves = ceil_div(waves, WAVES * 8) * (WAVES * 8);
@@ -1127,11 +1159,31 @@ inline bool launch_span(const Int4Args& a)
         return false;
     // Rows per wavefront and wavefronts per workgroup as measured on the 7B / 13B shapes: one row per
     // wavefront where that many wavefronts fit, three for the SwiGLU pair of tensors.
+    // Rows of 4097 .. 6144 inputs (J = 3, where the input that a lane holds takes 50 registers) are slower by the compute unit that
+    // has one workgroup more than the others: 13B's QKV had 640 workgroups on 256 compute units.  There one workgroup
+    // per compute unit takes its whole share where that is at most 12 wavefronts of two rows or 8 of seven.
+    const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
     if constexpr (MODE == QKV_ROPE) {
+        // 13B decode step, profiled: 11.6 us (640 workgroups of 8 wavefronts, one row each) -> 10.2
+        if constexpr (J == 3) {
+            if (a.n_tensors == 3 && ceil_div(a.N / 2, 12) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
+                return true;
+        }
         return a.n_tensors == 3 && try_span<J, MODE, STAGE, 3, 8, 1>(a);
     } else if constexpr (MODE == SWIGLU) {
+        // 13824 rows 14.9 us (8 wavefronts of four rows) -> 14.2, 14336 15.0 -> 14.3; three rows keep what they fit: 12288
+        // rows 12.9 us, 13.4 with seven
+        if constexpr (J == 3) {
+            if (ceil_div(a.N, 8 * 3) > 2 * cus && ceil_div(a.N, 8 * 7) <= cus && try_span<J, MODE, STAGE, 2, 8, 7>(a))
+                return true;
+        }
         return try_span<J, MODE, STAGE, 2, 8, 3>(a) || try_span<J, MODE, STAGE, 2, 8, 4>(a);
     } else if constexpr (MODE == PLAIN) {
+        // 4224 / 5120 / 6144 rows 10.2 / 10.7 / 11.2 us (8 wavefronts of two rows) -> 8.6 / 9.3 / 10.4
+        if constexpr (J == 3) {
+            if (a.n_tensors == 3 && ceil_div(a.N, 12 * 2) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
+                return true;
+        }
         if (a.n_tensors == 3)
             return try_span<J, MODE, STAGE, 3, 8, 1>(a) || try_span<J, MODE, STAGE, 3, 8, 2>(a);
         if (a.n_tensors != 1)

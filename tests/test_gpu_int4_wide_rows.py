@@ -1,0 +1,68 @@
+"""The int4 mat-vecs of rows of 4097 .. 6144 inputs, where one workgroup per compute unit takes its whole share of the
+rows: QKV in 12 wavefronts of two rows (with RoPE the two rows of a pair), SwiGLU in 8 of seven.  Sizes at the
+edges of the rule: workgroups full and partly empty, the last size that one workgroup per compute unit holds and the next.
+
+The order in which a row is added up is the same in every int4 kernel, and so are the RMSNorm and the rotation of the fused
+step and of the modules: cache rows, query and single mat-vecs are compared bit for bit, SwiGLU with fp64.
+"""
+import numpy as np
+import pytest
+
+from managedllama2_amd import capi, synth
+from managedllama2_amd.transformer import Transformer
+from gpu_util import assert_close, sizes, up, upq
+
+pytestmark = pytest.mark.gpu
+
+
+def bits(a):
+    return np.asarray(a).view(np.uint16)
+
+
+@pytest.mark.parametrize("heads", [33, 34, 40, 48])
+def test_qkv_rope_pairs_equal_the_modules(heads):
+    dim, seq = 128 * heads, 24
+    cfg = dict(dim=dim, hidden_dim=256, n_layers=1, n_heads=heads, n_kv_heads=heads, vocab_size=64, seq_len=seq,
+               rope_theta=10000.0)
+    model = synth.random_model(cfg, seed=31, rms_random=True)
+    prompt = synth.rng_for(612, heads).integers(3, 64, seq).astype(np.int32)
+    outs = []
+    for mode in (capi.DECODE_MODULES, capi.DECODE_FUSED):
+        t = Transformer(dict(cfg), model, mode=mode)
+        t.runstate.tokens.copy_to_device(prompt)
+        q = []
+        for pos in (0, 1, 7, 8, 23):
+            t.Forward(pos, pos + 1)
+            q.append(t.runstate.q.to_host())
+        outs.append((np.stack(q), t.runstate.keyCache.to_host(), t.runstate.valueCache.to_host()))
+        t.close()
+    for a, b, what in zip(outs[0], outs[1], ("query", "key cache", "value cache")):
+        assert np.array_equal(bits(a), bits(b)), what
+
+
+@pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 1000), (6144, 6), (4352, 24)])
+def test_three_tensors_equal_one_at_a_time(K, N):
+    rng = synth.rng_for(613, K, N)
+    zs, ss, ws = sizes(K)
+    x = up(synth.normal_f16(rng, K))
+    qs = [upq(synth.random_qweight(rng, K, N)) for _ in range(3)]
+    three = [up(np.zeros(N, np.float16)) for _ in range(3)]
+    capi.call("llama2_qkv_mat_vec", *[o.ptr for o in three], x.ptr,
+              *[p for q in qs for p in (q.Weight.ptr, q.Zeros.ptr, q.Scales.ptr)], K, N, zs, ss, ws)
+    for q, got in zip(qs, three):
+        one = up(np.zeros(N, np.float16))
+        capi.call("llama2_mat_vec_int4", one.ptr, x.ptr, q.Weight.ptr, q.Zeros.ptr, q.Scales.ptr, K, N, zs, ss, ws)
+        assert np.array_equal(bits(got.to_host()), bits(one.to_host()))
+
+
+@pytest.mark.parametrize("K,N", [(5120, 12288), (5120, 12296), (4224, 14336), (6144, 14344)])
+def test_swiglu_of_many_rows(oracle, K, N):
+    rng = synth.rng_for(614, K, N)
+    zs, ss, ws = sizes(K)
+    g, u = synth.random_qweight(rng, K, N), synth.random_qweight(rng, K, N)
+    x = synth.normal_f16(rng, K)
+    dg, du, dx, out = upq(g), upq(u), up(x), up(np.zeros(N, np.float16))
+    capi.call("llama2_mat_vec_swiglu", out.ptr, dx.ptr, dg.Weight.ptr, dg.Zeros.ptr, dg.Scales.ptr, du.Weight.ptr,
+              du.Zeros.ptr, du.Scales.ptr, K, N, zs, ss, ws)
+    gv, uv = oracle.f64_matvec_int4(x, *g, K, N), oracle.f64_matvec_int4(x, *u, K, N)
+    assert_close(out.to_host(), gv / (1 + np.exp(-gv)) * uv, "swiglu %dx%d" % (K, N))  # 2e-3: two fp16 roundings

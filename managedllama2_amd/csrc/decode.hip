@@ -669,7 +669,7 @@ int forward_fused(llama2_decoder* d, int shape)
             if (i == 0)
                 a.embedding = d->w.token_embedding_table, a.tokens = s.tokens, a.vocab = c.vocab_size, a.x_out = s.x;
             a.pos_ptr = d->state;
-            a.kv_dim = d->kv_dim, a.theta = c.rope_theta;
+            a.kv_dim = d->kv_dim;
             a.rope_table = reinterpret_cast<const float*>(d->state + kStateInts);
             L2_TRY((launch_int4<QKV_ROPE, STAGE_RMSNORM>("fused qkv", a)));
         }

@@ -71,8 +71,7 @@ struct Int4Args {
     const int* pos_ptr;
     // QKV_ROPE
     int kv_dim;
-    float theta;
-    const float* rope_table; // (cos, sin) of the step's position for i < 64, or null: computed here from theta
+    const float* rope_table; // (cos, sin) of the step's position for i < 64
     // STAGE_MERGE: the sums [kMergeBlocks][K], then (maximum, sum) [kMergeBlocks][head]; a block is 2^block_shift timesteps,
     // those up to *pos_ptr count
     const float* parts;
@@ -267,7 +266,7 @@ __global__ __launch_bounds__(256) void int4_matvec_kernel(Int4Args a)
     // The RoPE table is requested before the weights as well: loads return in order, so a value
     // requested after them would hold up the staging below until the first weights have arrived.
     float rope_entry = 0.0f;
-    if (MODE == QKV_ROPE && a.rope_table && threadIdx.x < kRopeHeadSize)
+    if (MODE == QKV_ROPE && threadIdx.x < kRopeHeadSize)
         rope_entry = a.rope_table[threadIdx.x];
     Frag<J, R> cur;
     uint16_t cur_res = 0;
@@ -277,17 +276,8 @@ __global__ __launch_bounds__(256) void int4_matvec_kernel(Int4Args a)
     // The position lives in device memory: outside layer 0 it is read only here, after the weight
     // loads above were issued.
     const int pos = MODE == QKV_ROPE && a.pos_ptr ? a.pos_ptr[0] : 0;
-    if (MODE == QKV_ROPE) {
-        if (a.rope_table) { // prepared by the kernel that set the position
-            if (threadIdx.x < kRopeHeadSize)
-                rope_tab[threadIdx.x] = rope_entry;
-        } else if (threadIdx.x < kRopeHeadSize / 2) {
-            float c, s;
-            rope_cos_sin(c, s, threadIdx.x, kRopeHeadSize, pos, a.theta);
-            rope_tab[2 * threadIdx.x] = c;
-            rope_tab[2 * threadIdx.x + 1] = s;
-        }
-    }
+    if (MODE == QKV_ROPE && threadIdx.x < kRopeHeadSize)
+        rope_tab[threadIdx.x] = rope_entry;
     if (STAGE == STAGE_RMSNORM) {
         if (a.embedding && blockIdx.x == 0) { // the residual stream starts as the embedding row
             const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.x_out, a.K * 2);
@@ -555,7 +545,7 @@ __global__ __launch_bounds__(256) void int4_matvec_block_kernel(Int4Args a)
     // The RoPE table is requested before the weights as well: loads return in order, so a value
     // requested after them would hold up the staging below until the first weights have arrived.
     float rope_entry = 0.0f;
-    if (MODE == QKV_ROPE && a.rope_table && threadIdx.x < kRopeHeadSize)
+    if (MODE == QKV_ROPE && threadIdx.x < kRopeHeadSize)
         rope_entry = a.rope_table[threadIdx.x];
     asm volatile("" ::: "memory"); // the input stays ahead of the weights in the memory queue
     BFrag<J, G, RB> cur;
@@ -567,17 +557,8 @@ __global__ __launch_bounds__(256) void int4_matvec_block_kernel(Int4Args a)
     // The position lives in device memory: outside layer 0 it is read only here, after the weight
     // loads above were issued.
     const int pos = MODE == QKV_ROPE && a.pos_ptr ? a.pos_ptr[0] : 0;
-    if (MODE == QKV_ROPE) {
-        if (a.rope_table) { // prepared by the kernel that set the position
-            if (threadIdx.x < kRopeHeadSize)
-                rope_tab[threadIdx.x] = rope_entry;
-        } else if (threadIdx.x < kRopeHeadSize / 2) {
-            float c, s;
-            rope_cos_sin(c, s, threadIdx.x, kRopeHeadSize, pos, a.theta);
-            rope_tab[2 * threadIdx.x] = c;
-            rope_tab[2 * threadIdx.x + 1] = s;
-        }
-    }
+    if (MODE == QKV_ROPE && threadIdx.x < kRopeHeadSize)
+        rope_tab[threadIdx.x] = rope_entry;
     if (STAGE == STAGE_RMSNORM) {
         if (a.embedding && blockIdx.x == 0) { // the residual stream starts as the embedding row
             const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.x_out, a.K * 2);
@@ -725,7 +706,6 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
     __shared__ float red4[4];
     __shared__ uint32_t meta_s[WAVES][TN][SD * 64];
     __shared__ uint32_t meta_z[WAVES][TN][64];
-    __shared__ float rope_tab[MODE == QKV_ROPE ? kRopeHeadSize : 2]; // (cos, sin) pairs
     __shared__ float pair_val[MODE == QKV_ROPE ? 2 * WAVES : 2];     // q and k of every wavefront's row
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     // Workgroups go to the 8 XCDs round-robin: within every aligned group of 128 workgroups, give each
@@ -817,9 +797,11 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
         if (STAGE == STAGE_RMSNORM)
             gp.load(a.gamma, a.K);
     }
-    float rope_entry = 0.0f;
-    if (MODE == QKV_ROPE && a.rope_table && threadIdx.x < kRopeHeadSize)
-        rope_entry = a.rope_table[threadIdx.x];
+    // The one entry of the position's RoPE table that the wavefront needs, in every lane: no table in LDS, which the staging
+    // waited for and the epilogue read back (7B QKV + RoPE 7.0 -> 6.7 us back to back).
+    u32x2 angle = {};
+    if (MODE == QKV_ROPE)
+        angle = __builtin_amdgcn_raw_buffer_load_b64(make_rsrc(a.rope_table, kRopeHeadSize * 4), (r0 & 63) * 8, 0, 0);
     uint32_t sreg[TN][SD], zreg[TN], res = 0;
     const int rows_apart = n ? (n - 1) * kRowStep + 1 : 0; // from the first row to behind the last one
 #pragma unroll
@@ -848,20 +830,6 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
     load_w(ring[0], 0);
     asm volatile("" ::: "memory");
 
-    if (MODE == QKV_ROPE) {
-        if (a.rope_table) { // prepared by the kernel that set the position
-            if (threadIdx.x < kRopeHeadSize)
-                rope_tab[threadIdx.x] = rope_entry;
-        } else {
-            const int pos = position(); // all threads: the value is moved from lane 0
-            if (threadIdx.x < kRopeHeadSize / 2) {
-                float c, sn;
-                rope_cos_sin(c, sn, threadIdx.x, kRopeHeadSize, pos, a.theta);
-                rope_tab[2 * threadIdx.x] = c;
-                rope_tab[2 * threadIdx.x + 1] = sn;
-            }
-        }
-    }
     if (STAGE == STAGE_RMSNORM) {
         if (a.embedding && blockIdx.x == 0 && stager) { // the residual stream starts as the embedding row
             const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.x_out, a.K * 2);
@@ -959,8 +927,8 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
     if constexpr (PAIR) {
         const int pos = position();
         if (lane < n) { // lane 0 row i, lane 1 row i + 64; the unfused path stores q/k as fp16 and RoPE reads them back
-            const int i = r0 & 63, row = r0 + lane * kRowStep;
-            const float c = rope_tab[2 * i], sn = rope_tab[2 * i + 1];
+            const int row = r0 + lane * kRowStep;
+            const float c = __uint_as_float(angle[0]), sn = __uint_as_float(angle[1]);
             uint16_t rotated[2];
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
@@ -986,8 +954,8 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
         __syncthreads();
         const int pos = position();
         if (lane == 0 && n) {
-            const int partner = wave ^ 4, i = r0 & 63; // pair index within the head
-            const float c = rope_tab[2 * i], sn = rope_tab[2 * i + 1];
+            const int partner = wave ^ 4;
+            const float c = __uint_as_float(angle[0]), sn = __uint_as_float(angle[1]);
             uint16_t* kdst = a.out[1] + static_cast<size_t>(pos) * a.kv_dim;
             uint16_t* vdst = a.out[TN > 2 ? 2 : 0] + static_cast<size_t>(pos) * a.kv_dim;
             uint16_t b0, b1;

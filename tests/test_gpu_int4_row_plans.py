@@ -1,6 +1,8 @@
-"""The int4 mat-vecs of rows of 4097 .. 6144 inputs, where one workgroup per compute unit takes its whole share of the
-rows: QKV in 12 wavefronts of two rows (with RoPE the two rows of a pair), SwiGLU in 8 of seven.  Sizes at the
-edges of the rule: workgroups full and partly empty, the last size that one workgroup per compute unit holds and the next.
+"""Which rows a wavefront of the int4 mat-vecs takes, at the edges of the rules that decide it.
+
+Rows of 4097 .. 6144 inputs: one workgroup per compute unit takes its whole share of the rows, QKV in 12 wavefronts of two rows
+(with RoPE the two rows of a pair), SwiGLU in 8 of seven.  Workgroups full and partly empty, the last size that one
+workgroup per compute unit holds and the next.
 
 The order in which a row is added up is the same in every int4 kernel, and so are the RMSNorm and the rotation of the fused
 step and of the modules: cache rows, query and single mat-vecs are compared bit for bit, SwiGLU with fp64.
@@ -55,8 +57,11 @@ def test_three_tensors_equal_one_at_a_time(K, N):
         assert np.array_equal(bits(got.to_host()), bits(one.to_host()))
 
 
-@pytest.mark.parametrize("K,N", [(5120, 12288), (5120, 12296), (4224, 14336), (6144, 14344)])
-def test_swiglu_of_many_rows(oracle, K, N):
+# SwiGLU takes one, two or three rows per wavefront as the compute units allow: the edges on 256 of them, then the wide rows.
+@pytest.mark.parametrize("K,N", [(128, 1), (256, 2048), (512, 2049), (256, 4096), (256, 4097), (256, 6144), (384, 6145),
+                                 (256, 8192), (256, 8193), (2304, 1409), (4096, 8187),
+                                 (5120, 12288), (5120, 12296), (4224, 14336), (6144, 14344)])
+def test_swiglu_rows_per_wavefront(oracle, K, N):
     rng = synth.rng_for(614, K, N)
     zs, ss, ws = sizes(K)
     g, u = synth.random_qweight(rng, K, N), synth.random_qweight(rng, K, N)

@@ -157,6 +157,7 @@ struct GemmArgs {
     uint32_t xf_bytes;
     int groups, N, ws, ss, zs; // N: rows of one tensor
     int M, mblocks, pairs, nblocks, splits; // pairs of weight tiles, and blocks of them
+    int first, mblocks2; // blocks of weights of one XCD that meet blocks of MT token tiles (the rest: MT2), and blocks of MT2
     uint16_t* out[3]; // QKV: q, key-cache rows, value-cache rows of this batch; SWIGLU: hf
     float* parts;     // PARTIAL: [splits][part_rows][N]
     int part_rows;
@@ -233,28 +234,29 @@ __device__ __forceinline__ void static_for(const F& f, std::integer_sequence<int
 // - Results leave in pieces of 16 bytes after one exchange of all tiles through LDS, their RoPE angles requested
 //   before it: stored as they lie in the registers, 2 bytes per lane and tile by tile, they took 25 us of the 72 of QKV.
 // 7B, 511 rows: QKV 76 -> 62 us; the whole 512-token prompt 11.25 -> 10.75 ms.
+template <int MT, int WN, int WK>
+struct GemmLds {
+    static constexpr int kXStage = WK * MT * kBlockBytes;  // activations of a step
+    static constexpr int kWRow = WK * 64;                  // bytes of a weight row per step
+    static constexpr int kWStage = WN * 2 * kTile * kWRow; // weights of a step
+    static constexpr int kZStage = 8 * 256;                // a word with the scale and one with the zero point per row and group
+    static constexpr int kWAt = 3 * kXStage, kZAt = kWAt + 3 * kWStage, kAll = kZAt + 3 * kZStage;
+    static constexpr int kRedRow = kTile + 4, kRed = 8 * MT * kTile * kRedRow * 4;
+    static constexpr int kBytes = kAll > kRed ? kAll : kRed;
+    static_assert(kBytes <= 160 * 1024, "LDS of a compute unit");
+};
+
+// Block `unit` of weights (and piece of K) with block `mb` of MT token tiles.
 template <int MT, int WN, int WK, int EPI>
-__global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
+__device__ __forceinline__ void gemm_block(const GemmArgs& a, char* lds, int unit, int mb)
 {
     static_assert(WN * WK == 4, "8 wavefronts");
-    constexpr int kXStage = WK * MT * kBlockBytes;  // activations of a step
-    constexpr int kWRow = WK * 64;                  // bytes of a weight row per step
-    constexpr int kWStage = WN * 2 * kTile * kWRow; // weights of a step
-    constexpr int kZStage = 8 * 256;                // a word with the scale and one with the zero point per row and group
-    constexpr int kWAt = 3 * kXStage, kZAt = kWAt + 3 * kWStage, kAll = kZAt + 3 * kZStage;
-    constexpr int kRedRow = kTile + 4, kRed = 8 * MT * kTile * kRedRow * 4;
-    static_assert(kRed <= 160 * 1024, "LDS of a compute unit");
-    static_assert(kAll <= 160 * 1024, "LDS of a compute unit");
-    __shared__ __align__(1024) char lds[kAll > kRed ? kAll : kRed];
+    using Lds = GemmLds<MT, WN, WK>;
+    constexpr int kXStage = Lds::kXStage, kWRow = Lds::kWRow, kWStage = Lds::kWStage, kZStage = Lds::kZStage;
+    constexpr int kWAt = Lds::kWAt, kZAt = Lds::kZAt, kRedRow = Lds::kRedRow;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t = wave & 1, wn = (wave >> 1) % WN, wk = (wave >> 1) / WN;
     const int h = lane >> 5, l31 = lane & 31;
-    // The token blocks of one block of weights run on one XCD, next to each other in time: its L2
-    // serves the weights to all but the first.
-    const int slot = blockIdx.x >> 3;
-    const int unit = (slot / a.mblocks) * 8 + (blockIdx.x & 7), mb = slot % a.mblocks;
-    if (unit >= a.nblocks * a.splits)
-        return;
     const int nb = unit / a.splits, split = unit - nb * a.splits;
     // tensor and first row of a tile; the last block may have pairs to spare, which repeat the last one
     auto tile_of = [&](int pair, int tile, int& tensor, int& row) {
@@ -271,7 +273,12 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
             row = (pair * 2 + tile) * kTile;
         }
     };
-    auto tensor_of = [&](int i) { return i == 0 ? a.m[0] : (i == 1 ? a.m[1] : a.m[2]); };
+    // by value: a choice among the arguments themselves puts them into scratch memory
+    auto choose = [](int i, auto first, auto second, auto third) { return i == 0 ? first : (i == 1 ? second : third); };
+    auto tensor_of = [&](int i) {
+        return QW{choose(i, a.m[0].w, a.m[1].w, a.m[2].w), choose(i, a.m[0].z, a.m[1].z, a.m[2].z),
+                  choose(i, a.m[0].s, a.m[1].s, a.m[2].s)};
+    };
     auto rsrc_of = [](const void* p, uint32_t bytes) {
         const unsigned long long v = reinterpret_cast<unsigned long long>(p);
         return u32x4{static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))),
@@ -513,7 +520,7 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
                 oa[k >> 1] = k & 1 ? oa[k >> 1] | static_cast<uint32_t>(b0) << 16 : b0;
                 ob[k >> 1] = k & 1 ? ob[k >> 1] | static_cast<uint32_t>(b1) << 16 : b1;
             }
-            uint16_t* o = a.out[tensor0] + static_cast<size_t>(m) * a.N + n8;
+            uint16_t* o = choose(tensor0, a.out[0], a.out[1], a.out[2]) + static_cast<size_t>(m) * a.N + n8;
             *reinterpret_cast<u32x4*>(o + row_a) = oa;
             *reinterpret_cast<u32x4*>(o + row_b) = ob;
         } else if (EPI == EPI_PARTIAL) {
@@ -541,10 +548,36 @@ __global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
     }
 }
 
+// The token blocks of one block of weights run on one XCD, next to each other in time: its L2 serves the weights to all but the
+// first.  With MT2 other than MT the first blocks of weights of every XCD are taken with MT token tiles, in rounds that
+// fill its compute units, the others with MT2: what would be a last round of few workgroups that take as long as the others becomes one of
+// more and shorter ones.
+template <int MT, int MT2, int WN, int WK, int EPI>
+__global__ __launch_bounds__(512, 2) void prefill_gemm_kernel(GemmArgs a)
+{
+    constexpr int kBytes = GemmLds<MT, WN, WK>::kBytes, kBytes2 = GemmLds<MT2, WN, WK>::kBytes;
+    __shared__ __align__(1024) char lds[kBytes > kBytes2 ? kBytes : kBytes2];
+    int slot = blockIdx.x >> 3, mblocks = a.mblocks, row = 0; // row: of 8 blocks of weights, one to an XCD
+    const bool second = MT2 != MT && slot >= a.first * a.mblocks;
+    if (second)
+        slot -= a.first * a.mblocks, mblocks = a.mblocks2, row = a.first;
+    const int unit = (row + slot / mblocks) * 8 + (blockIdx.x & 7), mb = slot % mblocks;
+    if (unit >= a.nblocks * a.splits)
+        return;
+    if constexpr (MT2 != MT) {
+        if (second) {
+            gemm_block<MT2, WN, WK, EPI>(a, lds, unit, mb);
+            return;
+        }
+    }
+    gemm_block<MT, WN, WK, EPI>(a, lds, unit, mb);
+}
+
 // How a product is cut up: MT token tiles and WN pairs of weight tiles per workgroup, WK groups per step, and
 // pieces of K per launch.
 struct GemmShape {
     int mt, wn, splits;
+    int mt2, first; // mt2 other than mt: the first `first` blocks of weights of every XCD with mt token tiles, the rest with mt2
 };
 
 constexpr int kMaxSplits = 8;
@@ -575,20 +608,44 @@ static GemmShape gemm_shape(int tiles, int pairs, int groups, bool may_split)
                                        steps * step * ((rounds - 1) * 10 * per_xcd + 6 * per_xcd + 4 * last) / (10 * per_xcd) +
                                        (may_split ? static_cast<long long>(splits) * tiles * kTile * pairs * 64 * 4 / 4500 : 0);
                 if (least < 0 || cost < least)
-                    least = cost, best = GemmShape{mt, wn, splits};
+                    least = cost, best = GemmShape{mt, wn, splits, mt, 0};
             }
+    if (may_split)
+        return best;
+    // Two heights of workgroup, the higher ones in full rounds.  7B, 511 rows, SwiGLU: 44 workgroups for the 32 compute units of an
+    // XCD; 32 of them and 24 of half the height instead.  The whole prompt, one height -> two: 7B 350 / 512 / 740 / 1004 tokens
+    // 9.33 / 10.92 / 14.98 / 18.31 ms -> 9.15 / 10.60 / 14.78 / 17.97, 13B 310 / 940 / 1004 14.86 / 35.7 / 36.9 -> 14.47 / 34.8 / 36.2.
+    // Where the estimate finds no gain (7B up to 340 rows, 450, 560 .. 690) one height stays.
+    static constexpr int kMixed[][2] = {{4, 3}, {4, 2}, {3, 2}};
+    const int rows = ceil_div(ceil_div(pairs, 4), kXcds);
+    for (const auto& m : kMixed)
+        for (int first = 1; first < rows; ++first) {
+            const int units = first * ceil_div(tiles, m[0]), units2 = (rows - first) * ceil_div(tiles, m[1]);
+            if (units % per_xcd)
+                continue;
+            const int rounds = units / per_xcd, rounds2 = ceil_div(units2, per_xcd), last = units2 - (rounds2 - 1) * per_xcd;
+            const long long cost = kLaunchNs + kRoundNs * (rounds + rounds2) + static_cast<long long>(groups) * rounds * kStepNs[m[0]] +
+                                   static_cast<long long>(groups) * kStepNs[m[1]] *
+                                       ((rounds2 - 1) * 10 * per_xcd + 6 * per_xcd + 4 * last) / (10 * per_xcd);
+            if (cost < least)
+                least = cost, best = GemmShape{m[0], 4, 1, m[1], first};
+        }
     return best;
 }
 
 static GemmShape residual_shape(int M, int N, int groups) { return gemm_shape(ceil_div(M, kTile), N / 64, groups, true); }
 
-template <int MT, int WN, int EPI>
+template <int MT, int WN, int EPI, int MT2 = MT>
 void launch_gemm_as(GemmArgs& a)
 {
     a.mblocks = ceil_div(a.M, MT * kTile);
+    a.mblocks2 = ceil_div(a.M, MT2 * kTile);
     a.nblocks = ceil_div(a.pairs, WN);
-    const dim3 grid(ceil_div(a.nblocks * a.splits, 8) * 8 * a.mblocks);
-    hipLaunchKernelGGL((prefill_gemm_kernel<MT, WN, 4 / WN, EPI>), grid, dim3(512), 0, ctx().stream, a);
+    const int rows = ceil_div(a.nblocks * a.splits, 8);
+    if (MT2 == MT)
+        a.first = rows;
+    const dim3 grid(8 * (a.first * a.mblocks + (rows - a.first) * a.mblocks2));
+    hipLaunchKernelGGL((prefill_gemm_kernel<MT, MT2, WN, 4 / WN, EPI>), grid, dim3(512), 0, ctx().stream, a);
 }
 
 template <int EPI>
@@ -597,6 +654,19 @@ int launch_gemm(const char* name, GemmArgs a, int pairs)
     const GemmShape s = gemm_shape(ceil_div(a.M, kTile), pairs, a.groups, EPI == EPI_PARTIAL);
     a.pairs = pairs;
     a.splits = s.splits;
+    a.first = s.first;
+    if constexpr (EPI != EPI_PARTIAL) {
+        if (s.mt2 != s.mt) {
+            if (s.mt == 4 && s.mt2 == 3)
+                launch_gemm_as<4, 4, EPI, 3>(a);
+            else if (s.mt == 4)
+                launch_gemm_as<4, 4, EPI, 2>(a);
+            else
+                launch_gemm_as<3, 4, EPI, 2>(a);
+            L2_LAUNCH_CHECK(name);
+            return LLAMA2_OK;
+        }
+    }
     switch (s.wn * 10 + s.mt) {
     case 44: launch_gemm_as<4, 4, EPI>(a); break;
     case 43: launch_gemm_as<3, 4, EPI>(a); break;

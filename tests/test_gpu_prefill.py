@@ -412,6 +412,14 @@ def test_model_widths(widths, lengths):
         tr.close()
 
 
+# Products whose workgroups come in two heights, on 256 compute units: 4 and 2 token tiles, 3 and 2, 4 and 3, of SwiGLU and of
+# QKV (dim 4352: QKV 4 and 3); row by row as above.
+@pytest.mark.parametrize("dim,hidden,known", [(1024, 4352, 950), (1024, 5376, 740), (1024, 6400, 950), (2816, 256, 950),
+                                              (3456, 256, 740), (4352, 256, 950)])
+def test_workgroups_of_two_heights(dim, hidden, known):
+    test_model_widths(config(dim, hidden, 2, known), (known,))
+
+
 # The other loops that batch their prompt: sampling, and the persistent step (same bits as the launch sequence behind
 # the same batch).
 def test_sampled_run_behind_a_batch():

@@ -590,11 +590,11 @@ QW qw(const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; }
 // with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.
 bool launch_o_merge(const Int4Args& a, int blocks, bool launch)
 {
-    if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || !span_allowed(a, 1))
+    if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || (a.ss & 1))
         return false;
     switch (ceil_div(a.ws / 4, 64)) {
-    case 1: return try_span<1, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
-    case 2: return try_span<2, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    case 1: return span_allowed<1>(a, 1) && try_span<1, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
+    case 2: return span_allowed<2>(a, 1) && try_span<2, RESIDUAL, STAGE_MERGE, 1, 16, 1>(a, launch);
     default: return false;
     }
 }

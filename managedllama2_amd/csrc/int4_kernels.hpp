@@ -686,8 +686,13 @@ struct SpanPlan {
     int base, rem; // rows per wavefront: base, one more for the first rem wavefronts
 };
 
-// Scale words (pairs of fp16) a lane fetches per tensor: ROWS rows of at most 16 J scales each.
-constexpr int span_scale_words(int J, int ROWS) { return (ROWS * 16 * J + 127) / 128; }
+// Words a lane fetches of the scales per tensor: ROWS rows of at most 16 J of them.  Rows of up to 2048 inputs (J = 1): one scale
+// per lane, read as the 2 bytes that it is, so that a row may begin anywhere and have an odd number of them; else pairs.
+constexpr bool span_single_scales(int J) { return J == 1; }
+constexpr int span_scale_words(int J, int ROWS)
+{
+    return span_single_scales(J) ? (ROWS * 16 + 63) / 64 : (ROWS * 16 * J + 127) / 128;
+}
 
 template <int J, int MODE, int STAGE, int TN, int WAVES, int ROWS>
 __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a, SpanPlan plan)
@@ -818,7 +823,8 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
         }
 #pragma unroll
         for (int k = 0; k < SD; ++k)
-            sreg[t][k] = __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4 + k * 256, 0, 0);
+            sreg[t][k] = span_single_scales(J) ? __builtin_amdgcn_raw_buffer_load_b16(rs, lane * 2 + k * 128, 0, 0)
+                                               : __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4 + k * 256, 0, 0);
         zreg[t] = __builtin_amdgcn_raw_buffer_load_b32(rz, lane * 4, 0, 0);
     }
     if (MODE == RESIDUAL) {
@@ -881,8 +887,12 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
 #pragma unroll
-            for (int k = 0; k < SD; ++k)
-                meta_s[wave][t][lane + 64 * k] = sreg[t][k];
+            for (int k = 0; k < SD; ++k) {
+                if (span_single_scales(J))
+                    reinterpret_cast<uint16_t*>(&meta_s[wave][t][0])[lane + 64 * k] = static_cast<uint16_t>(sreg[t][k]);
+                else
+                    meta_s[wave][t][lane + 64 * k] = sreg[t][k];
+            }
             meta_z[wave][t][lane] = zreg[t];
         }
     };
@@ -1110,20 +1120,23 @@ inline bool try_span(const Int4Args& a, bool launch = true)
     return true;
 }
 
+template <int J>
 inline bool span_allowed(const Int4Args& a, int tensors)
 {
-    if (ctx().int4_no_span || ctx().int4_narrow || ctx().int4_blocks || (a.ss & 1))
+    if (ctx().int4_no_span || ctx().int4_narrow || ctx().int4_blocks)
         return false;
+    if (span_single_scales(J))
+        return true;
     for (int t = 0; t < tensors; ++t)
         if (!aligned(a.m[t].s, 4))
             return false;
-    return true;
+    return (a.ss & 1) == 0;
 }
 
 template <int J, int MODE, int STAGE>
 inline bool launch_span(const Int4Args& a)
 {
-    if (!span_allowed(a, MODE == SWIGLU ? 2 : a.n_tensors))
+    if (!span_allowed<J>(a, MODE == SWIGLU ? 2 : a.n_tensors))
         return false;
     // Rows per wavefront and wavefronts per workgroup as measured on the 7B / 13B shapes: one row per
     // wavefront where that many wavefronts fit, three for the SwiGLU pair of tensors.

@@ -57,6 +57,33 @@ def test_three_tensors_equal_one_at_a_time(K, N):
         assert np.array_equal(bits(got.to_host()), bits(one.to_host()))
 
 
+# Rows of up to 2048 inputs may have an odd number of scales and begin at any of them: scales that lie 2 bytes off a word, odd
+# and even numbers of groups, ragged last groups and rows that do not fill the last wavefront.
+@pytest.mark.parametrize("K,N", [(8, 5), (136, 9), (384, 77), (640, 640), (1408, 512), (1928, 33), (2048, 35)])
+def test_scales_at_any_two_bytes(oracle, K, N):
+    rng = synth.rng_for(615, K, N)
+    zs, ss, ws = sizes(K)
+    qs = [synth.random_qweight(rng, K, N) for _ in range(3)]
+    x, res = synth.normal_f16(rng, K), synth.normal_f16(rng, N)
+    want = [oracle.f64_matvec_int4(x, *q, K, N) for q in qs]
+    dx, results = up(x), []
+    for shift in (0, 1):
+        parts = []
+        for W, Z, S in qs:
+            dev = up(W), up(Z), up(np.concatenate([np.full(shift, np.inf, np.float16), S]))
+            parts.append((dev, (dev[0].ptr, dev[1].ptr, dev[2].ptr + 2 * shift)))
+        ptrs = [p for _, q in parts for p in q]
+        outs = [up(np.zeros(N, np.float16)) for _ in range(4)] + [up(res)]
+        capi.call("llama2_qkv_mat_vec", *[o.ptr for o in outs[:3]], dx.ptr, *ptrs, K, N, zs, ss, ws)
+        capi.call("llama2_mat_vec_swiglu", outs[3].ptr, dx.ptr, *ptrs[:6], K, N, zs, ss, ws)
+        capi.call("llama2_mat_vec_residual_int4", outs[4].ptr, dx.ptr, *ptrs[:3], K, N, zs, ss, ws)
+        results.append([o.to_host() for o in outs])
+        for got, w in zip(results[-1], want + [want[0] / (1 + np.exp(-want[0])) * want[1], want[0] + res.astype(np.float64)]):
+            assert_close(got, w, "any two bytes %dx%d" % (K, N))  # 2e-3: fp16 results of fp32 sums
+    for a, b in zip(*results):
+        assert np.array_equal(bits(a), bits(b))
+
+
 # SwiGLU takes one, two or three rows per wavefront as the compute units allow: the edges on 256 of them, then the wide rows.
 @pytest.mark.parametrize("K,N", [(128, 1), (256, 2048), (512, 2049), (256, 4096), (256, 4097), (256, 6144), (384, 6145),
                                  (256, 8192), (256, 8193), (2304, 1409), (4096, 8187),

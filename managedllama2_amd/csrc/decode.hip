@@ -40,10 +40,8 @@ namespace l2 {
 // One compute unit pulls only a few tens of GB/s, so a short sequence wants
 // many small blocks (4 wavefronts, 128 rows); the exchange between workgroups
 // costs about 3 us whatever their number, and a long sequence wants fewer
-// merges.  Measured on 32 heads (one launch, RoPE inside; with the choice made
-// here 6.9 / 11.2 / 17.3 us since), 64 / 128 / 256 / 512 rows per block: 512 rows 7.4 / 7.3 / 8.8 / 11.0 us, 2048 rows 17.7 / 12.1 /
-// 11.4 / 15.5 us, 4096 rows 31.2 / 21.5 / 17.3 / 19.4 us: 128-row blocks up to
-// 1024 rows, 256-row blocks (8 wavefronts) beyond.  Dispatching workgroups
+// merges: 128-row blocks up to 1536 rows, 256-row blocks (8 wavefronts) beyond, measured below.  8 blocks of 512 rows are
+// 0.8 us faster than 16 of 256 at 3980 rows of 32 heads back to back, and 0.9 us slower in the decode step.  Dispatching workgroups
 // that find nothing to do is not free: a grid sized for the whole context costs
 // several microseconds per launch at short lengths.  The position lives on the
 // device, but the host always knows an upper bound for it, so it picks the
@@ -67,16 +65,19 @@ constexpr int kMaxSplits = 64; // one lane per block in the merge
 constexpr int kPartStride = kRopeHeadSize + 2; // 128 partial outputs, block max, block sum
 
 inline int attn_max_splits(int seq_len) { return ceil_div(seq_len, kSplitT); }
-constexpr int kSmallBlockMaxSeq = 1024;                   // 128-row blocks up to this length,
+// Measured back to back, 32 and 40 heads, 128 / 256 rows per block: 1030 rows 8.4 / 8.7 and 10.1 / 11.3 us, 1280 9.0 / 9.7 and
+// 10.5 / 12.3, 1536 9.9 / 9.8 and 11.3 / 12.4, 1700 10.3 / 9.9 and 12.0 / 12.4, 2048 11.3 / 10.5 and 13.2 / 12.8.
+constexpr int kSmallBlockMaxSeq = 1536;                   // 128-row blocks up to this length,
 constexpr int kMidBlockMaxSeq = kMaxSplits * kMidSplitT;  // 256-row blocks up to this one (16384), 512-row blocks beyond
 
-// Launch shapes of the decode step: 1, 2, 4, 8 blocks of 128 rows; 8, 16, 32, 64 blocks
+// Launch shapes of the decode step: 1, 2, 4, 8, 16 blocks of 128 rows; 8, 16, 32, 64 blocks
 // of 256 rows; 512-row blocks over the whole context.
 constexpr int ceil_log2(int v) { return v <= 1 ? 0 : 1 + ceil_log2((v + 1) / 2); }
-constexpr int kSmallShapes = ceil_log2(kSmallBlockMaxSeq / kSmallSplitT) + 1;             // 4
-constexpr int kMidFirstLog = ceil_log2(kSmallBlockMaxSeq / kMidSplitT) + 1;               // 3: 8 blocks
-constexpr int kMidShapes = ceil_log2(kMaxSplits) - kMidFirstLog + 1;                      // 4
+constexpr int kSmallShapes = ceil_log2(kSmallBlockMaxSeq / kSmallSplitT) + 1; // 5
+constexpr int kMidFirstLog = 3;                                                        // 8 blocks
+constexpr int kMidShapes = ceil_log2(kMaxSplits) - kMidFirstLog + 1;                   // 4
 constexpr int kAttnShapes = kSmallShapes + kMidShapes + 1;
+static_assert((kMidSplitT << kMidFirstLog) >= kSmallBlockMaxSeq, "the first shape of 256-row blocks goes on from there");
 struct AttnShape {
     int waves;
     int splits;
@@ -232,17 +233,19 @@ __global__ __launch_bounds__(WAVES * 64, KIND != ATTN_ROPE && WAVES == kMidWaves
         for (int k = 0; k < SPLIT_T / 64; ++k)
             m = fmaxf(m, sc[lane + 64 * k]);
         m = wave_max(m);
-#pragma unroll
-        for (int k = 0; k < SPLIT_T / 64; ++k)
-            l += expf(sc[lane + 64 * k] - m);
-        l = wave_sum(l);
     } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             m = fmaxf(m, s[i]);
         m = wave_max(m);
     }
-    const float base = kByWave && m == -INFINITY ? 0.0f : m; // a wavefront may have no attended timestep at all
+    const float base = m == -INFINITY ? 0.0f : m; // no attended timestep of the wavefront, or of the block, may have a finite score
+    if constexpr (!kByWave) {
+#pragma unroll
+        for (int k = 0; k < SPLIT_T / 64; ++k)
+            l += expf(sc[lane + 64 * k] - base);
+        l = wave_sum(l);
+    }
     float o[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k)
@@ -345,19 +348,23 @@ __global__ __launch_bounds__(WAVES * 64, KIND != ATTN_ROPE && WAVES == kMidWaves
     }
     // Merge the blocks of this head.  The partials are read with agent-scope
     // buffer loads (they were written by other workgroups of this launch); a read
-    // beyond the last block returns 0, so the loads are unconditional, and the
-    // first eight blocks' outputs are requested before the weights are known.
+    // beyond the last block returns 0.
     const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.part + static_cast<size_t>(h) * a.max_splits * kPartStride,
                                                 static_cast<uint32_t>(nsplit) * kPartStride * sizeof(float));
     float* wsh = sc;         // per-block weights exp(m_i - M)   (nsplit <= kMaxSplits <= SPLIT_T)
     float* lsh = &red[0][0]; // the merged denominator
     const int j = threadIdx.x & (kRopeHeadSize - 1);
-    float v[8] = {};
-    if (threadIdx.x < kRopeHeadSize) {
+    float v[2][8] = {}; // this round of 8 blocks and the next, both requested before the weights are known
+    auto request = [&](float (&o)[8], int from) {
 #pragma unroll
         for (int u = 0; u < 8; ++u)
-            v[u] = __builtin_bit_cast(float,
-                                      __builtin_amdgcn_raw_buffer_load_b32(rp, (u * kPartStride + j) * 4, 0, kAuxAgent));
+            o[u] = __builtin_bit_cast(
+                float, __builtin_amdgcn_raw_buffer_load_b32(rp, ((from + u) * kPartStride + j) * 4, 0, kAuxAgent));
+    };
+    if (threadIdx.x < kRopeHeadSize) {
+        request(v[0], 0);
+        if (nsplit > 8) // 16 blocks, 2100 .. 3980 rows: 0.25 us less than one round after the other, both unasked 0.2 more with 8
+            request(v[1], 8);
     }
     if (threadIdx.x < 64) { // one wavefront: block i in lane i
         const int off = (threadIdx.x * kPartStride + kRopeHeadSize) * 4;
@@ -377,14 +384,15 @@ __global__ __launch_bounds__(WAVES * 64, KIND != ATTN_ROPE && WAVES == kMidWaves
         for (int i0 = 0;;) { // block order is fixed: deterministic
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                O = fmaf(i0 + u < nsplit ? wsh[i0 + u] : 0.0f, v[u], O);
+                O = fmaf(i0 + u < nsplit ? wsh[i0 + u] : 0.0f, v[0][u], O);
             i0 += 8;
             if (i0 >= nsplit)
                 break;
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                v[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                                                     rp, ((i0 + u) * kPartStride + j) * 4, 0, kAuxAgent));
+                v[0][u] = v[1][u];
+            if (i0 + 8 < nsplit)
+                request(v[1], i0 + 8);
         }
         out[threadIdx.x] = float_to_half_bits(O / lsh[0]);
     }

@@ -217,6 +217,32 @@ def test_statistics_per_wavefront(oracle, seq):
     assert_close_up_to_ties(got, oracle_chain(oracle, q, k, v, dim, heads, seq, True), "attention %d/%d/%d" % (dim, heads, seq))
 
 
+# The lengths at which the block size changes, and 9, 12, 16 and 33 blocks, whose results the merge requests in rounds of 8.
+@pytest.mark.parametrize("heads,seq", [(2, 1025), (2, 1408), (2, 1536), (2, 1537), (3, 2048), (2, 2049), (2, 4096), (33, 3400),
+                                       (2, 8193)])
+def test_block_sizes_by_length(oracle, heads, seq):
+    dim = 128 * heads
+    q, k, v = inputs(713, dim, seq)
+    got = fused(q, k, v, dim, heads, seq)
+    assert_close_up_to_ties(got, oracle_chain(oracle, q, k, v, dim, heads, seq, True), "attention %d/%d/%d" % (dim, heads, seq))
+
+
+# The same below 1024 rows: a block of 128 without any weight.
+@pytest.mark.parametrize("seq,masked", [(600, (128, 256)), (200, (128, 200)), (1500, (1408, 1500))])
+def test_short_blocks_without_weight(seq, masked):
+    dim, heads = 256, 2
+    q, k, v = inputs(714, dim, seq)
+    q = np.abs(q) + np.float16(1)
+    k = k.reshape(seq, dim)
+    k[masked[0]:masked[1]] = np.float16(-60000)
+    v = v.reshape(seq, dim)
+    v[masked[0]:masked[1]] = np.float16(60000)
+    rest = np.r_[0:masked[0], masked[1]:seq]
+    got, want = fused(q, k.ravel(), v.ravel(), dim, heads, seq), fused(q, k[rest].ravel(), v[rest].ravel(), dim, heads, rest.size)
+    assert np.all(np.isfinite(got))
+    assert_close_normwise(got, want, "rows %s without weight" % (masked,))
+
+
 @pytest.mark.parametrize("masked", [(32, 64), (256, 512), (0, 256), (0, 1300), (1024, 1301)])
 def test_wavefronts_and_blocks_without_weight(masked):
     dim, heads, seq = 256, 2, 1301

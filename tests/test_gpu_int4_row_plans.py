@@ -57,6 +57,24 @@ def test_three_tensors_equal_one_at_a_time(K, N):
         assert np.array_equal(bits(got.to_host()), bits(one.to_host()))
 
 
+# A single tensor of 3841 .. 4096 rows and 2049 .. 4096 inputs goes in workgroups of 16 wavefronts, the rows around that in fours:
+# a row's result does not depend on how many there are.
+@pytest.mark.parametrize("K", [2056, 4096])
+def test_rows_that_fill_one_workgroup_per_compute_unit(K):
+    rng = synth.rng_for(616, K)
+    zs, ss, ws = sizes(K)
+    x, q = up(synth.normal_f16(rng, K)), upq(synth.random_qweight(rng, K, 4104))
+    res = synth.normal_f16(rng, 4104)
+    outs = {}
+    for N in (3840, 3841, 4095, 4096, 4104):
+        plain, residual = up(np.zeros(N, np.float16)), up(res[:N].copy())
+        capi.call("llama2_mat_vec_int4", plain.ptr, x.ptr, q.Weight.ptr, q.Zeros.ptr, q.Scales.ptr, K, N, zs, ss, ws)
+        capi.call("llama2_mat_vec_residual_int4", residual.ptr, x.ptr, q.Weight.ptr, q.Zeros.ptr, q.Scales.ptr, K, N, zs, ss, ws)
+        outs[N] = bits(plain.to_host()), bits(residual.to_host())
+    for N, (plain, residual) in outs.items():
+        assert np.array_equal(plain, outs[4104][0][:N]) and np.array_equal(residual, outs[4104][1][:N]), N
+
+
 # Rows of up to 2048 inputs may have an odd number of scales and begin at any of them: scales that lie 2 bytes off a word, odd
 # and even numbers of groups, ragged last groups and rows that do not fill the last wavefront.
 @pytest.mark.parametrize("K,N", [(8, 5), (136, 9), (384, 77), (640, 640), (1408, 512), (1928, 33), (2048, 35)])

@@ -1159,18 +1159,22 @@ inline bool launch_span(const Int4Args& a)
                 return true;
         }
         // As few rows one after the other as one workgroup per compute unit allows, up to three: K 1024, 1408 / 4096 rows 4.6 /
-        // 4.7 us (three) -> 3.3 / 4.1, K 4096 6.1 / 6.5 -> 3.9 / 5.6, K 8192 7.7 / 8.5 -> 5.5 / 8.3.  Up to 8192 rows two
-        // workgroups with two rows each rather than one and a third with three: K 4096 9.3 us -> 7.9, K 8192 15.8 -> 13.8.
-        const int per_row = ceil_div(a.N, 8); // workgroups of 8 wavefronts with one row each
-        if (per_row <= cus && try_span<J, MODE, STAGE, 2, 8, 1>(a))
-            return true;
-        if ((per_row <= 2 * cus || (per_row > 3 * cus && per_row <= 4 * cus)) && try_span<J, MODE, STAGE, 2, 8, 2>(a))
-            return true;
+        // 4.7 us (three) -> 3.3 / 4.1, K 4096 6.1 / 6.5 -> 3.9 / 5.6, K 5120 6.6 / 6.9 -> 4.7 / 6.2.  Up to 8192 rows two
+        // workgroups with two rows each rather than one and a third with three: K 4096 9.3 us -> 7.9, K 5120 11.4 -> 9.3.
+        // (K 8192, 4096 rows: 8.1 with three and 8.3 with two.)
+        if constexpr (J <= 3) {
+            const int per_row = ceil_div(a.N, 8); // workgroups of 8 wavefronts with one row each
+            if (per_row <= cus && try_span<J, MODE, STAGE, 2, 8, 1>(a))
+                return true;
+            if ((per_row <= 2 * cus || (per_row > 3 * cus && per_row <= 4 * cus)) && try_span<J, MODE, STAGE, 2, 8, 2>(a))
+                return true;
+        }
         return try_span<J, MODE, STAGE, 2, 8, 3>(a) || try_span<J, MODE, STAGE, 2, 8, 4>(a);
     } else if constexpr (MODE == PLAIN) {
-        // 4224 / 5120 / 6144 rows 10.2 / 10.7 / 11.2 us (8 wavefronts of two rows) -> 8.6 / 9.3 / 10.4
+        // 4224 / 5120 / 6144 rows 10.2 / 10.7 / 11.2 us (8 wavefronts of two rows) -> 8.6 / 9.3 / 10.4; up to 4096 rows two
+        // workgroups per compute unit hold 8 wavefronts of one row: 2048 / 4096 rows 6.1 / 8.3 us, 8.2 / 8.6 with 12 of two
         if constexpr (J == 3) {
-            if (a.n_tensors == 3 && ceil_div(a.N, 12 * 2) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
+            if (a.n_tensors == 3 && a.N > 16 * cus && ceil_div(a.N, 12 * 2) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
                 return true;
         }
         if (a.n_tensors == 3)

@@ -42,7 +42,7 @@ def test_qkv_rope_pairs_equal_the_modules(heads):
         assert np.array_equal(bits(a), bits(b)), what
 
 
-@pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 1000), (6144, 6), (4352, 24)])
+@pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 4096), (6144, 4097), (4352, 24)])
 def test_three_tensors_equal_one_at_a_time(K, N):
     rng = synth.rng_for(613, K, N)
     zs, ss, ws = sizes(K)

@@ -410,9 +410,10 @@ __global__ __launch_bounds__(kPThreads) void decode_persist_kernel(PersistArgs a
                 for (int k = 0; k < kPBlockRows / 64; ++k)
                     m = fmaxf(m, sc[q4][lane + 64 * k]);
                 m = wave_max(m);
+                const float base = m == -INFINITY ? 0.0f : m; // as fused_attn_kernel: a block may have no finite score, and no weight then
 #pragma unroll
                 for (int k = 0; k < kPBlockRows / 64; ++k)
-                    lsum += expf(sc[q4][lane + 64 * k] - m);
+                    lsum += expf(sc[q4][lane + 64 * k] - base);
                 lsum = wave_sum(lsum);
                 float o[8];
 #pragma unroll
@@ -420,7 +421,7 @@ __global__ __launch_bounds__(kPThreads) void decode_persist_kernel(PersistArgs a
                     o[k] = 0.0f;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const float p = expf(s[i] - m); // 0 for masked timesteps
+                    const float p = expf(s[i] - base); // 0 for masked timesteps
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
                         const h2_t v2 = as_h2(vv[i][k]);

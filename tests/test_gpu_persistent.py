@@ -110,6 +110,38 @@ def test_persistent_step_with_long_history(oracle, pos):
         assert_close_normwise(outs[1][0], want, "logits at pos %d" % pos, 1e-2)
 
 
+# A block of 128 rows whose scores all lie below fp16's range (-infinity) has no weight, in the three places that merge blocks:
+# the o-projection (two blocks), the attention launch (more) and the persistent step.
+@pytest.mark.parametrize("pos,masked", [(200, (0, 128)), (300, (128, 256)), (300, (0, 256)), (1000, (384, 512))])
+def test_blocks_without_weight(pos, masked):
+    cfg = dict(HS128, n_layers=1, seq_len=pos + 1)
+    dim, heads = cfg["dim"], cfg["n_heads"]
+    model = synth.random_model(cfg, seed=13, rms_random=True)
+    rng = synth.rng_for(411, pos)
+    kc = synth.normal_f16(rng, (pos + 1) * dim).reshape(pos + 1, dim)
+    vc = synth.normal_f16(rng, (pos + 1) * dim).reshape(pos + 1, dim)
+
+    def step(mode):
+        t = Transformer(dict(cfg), model, mode=mode)
+        t.runstate.keyCache.copy_to_device(kc)
+        t.runstate.valueCache.copy_to_device(vc)
+        t.runstate.tokens.copy_to_device(np.array([17], np.int32), pos)
+        t.Forward(pos, pos + 1)
+        check_ok(t)
+        logits, q = t.runstate.logits.to_host(), t.runstate.q.to_host()
+        t.close()
+        return logits, q
+
+    q = step(FUSED)[1]  # rotated; it does not depend on the history
+    assert np.abs(q.astype(np.float64)).reshape(heads, 128).sum(axis=1).min() * 60000 / np.sqrt(128) > 2 * 65520
+    kc[masked[0]:masked[1]] = np.where(q < 0, 60000, -60000)
+    vc[masked[0]:masked[1]] = np.float16(60000)  # no weight, however large
+    fused, persistent, modules = step(FUSED)[0], step(PERSIST)[0], step(capi.DECODE_MODULES)[0]
+    assert np.all(np.isfinite(fused)) and np.all(np.isfinite(persistent))
+    assert np.array_equal(bits(fused), bits(persistent))
+    assert_close_normwise(fused, modules.astype(np.float64), "logits behind rows without weight", 1e-2)
+
+
 @pytest.mark.parametrize("mode", [PERSIST, PERSIST_GRAPH])
 def test_persistent_device_resident_loop(mode):
     """llama2_decode_run: 260 steps without the host, crossing from one to two

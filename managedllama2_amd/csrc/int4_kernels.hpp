@@ -79,6 +79,7 @@ struct Int4Args {
 };
 
 constexpr int kAuxStream = 2; // "nt": weights are touched once
+constexpr int kNowhere = 1 << 30; // a byte behind the end of any buffer it is used with: reads as zero
 
 template <int J, int R>
 struct Frag { // what one lane holds of R rows: J chunks each + its group's zero word and scale
@@ -785,7 +786,6 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
     u32x4 pv[MB > 0 ? MB : 1][2];
     uint32_t part_max = 0, part_sum = 0;
     if constexpr (MB > 0) {
-        constexpr int kNowhere = 1 << 30; // behind the end of the buffer: reads as zero
         const __amdgpu_buffer_rsrc_t rp = make_rsrc(a.parts, (a.K + a.K / kRopeHeadSize * 2) * MB * 4);
         const int at = ((lane & 15) * (a.K / kRopeHeadSize) + static_cast<int>(threadIdx.x >> 4)) * 8 + a.K * MB * 4;
         const bool have = static_cast<int>(threadIdx.x) * 8 < a.K;
@@ -808,6 +808,14 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
     if (MODE == QKV_ROPE)
         angle = __builtin_amdgcn_raw_buffer_load_b64(make_rsrc(a.rope_table, kRopeHeadSize * 4), (r0 & 63) * 8, 0, 0);
     uint32_t sreg[TN][SD], zreg[TN], res = 0;
+    // Several rows: the scales of all of them are one run, and lanes behind the end of a row (whose share of the input is 0) read the
+    // next row's.  An infinite or NaN scale would reach the row before its own that way.  Spread: each row has 16 J places,
+    // those behind its end are read from nowhere.  Rows of up to 2048 inputs and launches of three tensors: QKV 5120 x 5120 9.3 us
+    // with and without, SwiGLU of an odd number of groups 0.05 .. 0.15 us (1920 x 11008 6.19 -> 6.28), small models' steps the same.
+    // SwiGLU and single tensors of longer rows keep the run and so expect finite scales: spread, the compiler
+    // orders SwiGLU's loads otherwise, and 7B's step takes 1.0 % longer, 13B's 1.6 (masked in registers instead 1.0 and 1.5).
+    constexpr bool kSpread = ROWS > 1 && !PAIR && (J == 1 || TN == 3);
+    constexpr int kUnit = span_single_scales(J) ? 2 : 4; // bytes
     const int rows_apart = n ? (n - 1) * kRowStep + 1 : 0; // from the first row to behind the last one
 #pragma unroll
     for (int t = 0; t < TN; ++t) {
@@ -815,16 +823,23 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
             make_rsrc(uniform_ptr(a.m[t].s + static_cast<size_t>(r0) * a.ss), rows_apart * a.ss * 2);
         const __amdgpu_buffer_rsrc_t rz =
             make_rsrc(uniform_ptr(a.m[t].z + static_cast<size_t>(r0) * a.zs), rows_apart * a.zs * 4);
-        if (PAIR) { // a word behind the end of its row belongs to another row and meets zeros of the input
+        if (PAIR) { // a zero word behind the end of its row belongs to another row and meets zeros of the input
             const int row = (lane >> 5) * kRowStep, word = (lane & 31) * 4;
-            sreg[t][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, row * a.ss * 2 + word, 0, 0);
+            // such a scale may be infinite: read from nowhere instead
+            sreg[t][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, word < a.ss * 2 ? row * a.ss * 2 + word : kNowhere, 0, 0);
             zreg[t] = __builtin_amdgcn_raw_buffer_load_b32(rz, row * a.zs * 4 + word, 0, 0);
             continue;
         }
 #pragma unroll
-        for (int k = 0; k < SD; ++k)
-            sreg[t][k] = span_single_scales(J) ? __builtin_amdgcn_raw_buffer_load_b16(rs, lane * 2 + k * 128, 0, 0)
-                                               : __builtin_amdgcn_raw_buffer_load_b32(rs, lane * 4 + k * 256, 0, 0);
+        for (int k = 0; k < SD; ++k) {
+            int at = (lane + 64 * k) * kUnit;
+            if (kSpread) {
+                const int row = static_cast<unsigned>(at) / (32 * J), byte = static_cast<unsigned>(at) % (32 * J);
+                at = byte < a.ss * 2 ? row * a.ss * 2 + byte : kNowhere;
+            }
+            sreg[t][k] = span_single_scales(J) ? __builtin_amdgcn_raw_buffer_load_b16(rs, at, 0, 0)
+                                               : __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+        }
         zreg[t] = __builtin_amdgcn_raw_buffer_load_b32(rz, lane * 4, 0, 0);
     }
     if (MODE == RESIDUAL) {
@@ -920,7 +935,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4_matvec_span_kernel(Int4Args a
         const int i = q / TN, t = q % TN;
         Frag<J, 1> cur;
         const uint16_t* sp =
-            reinterpret_cast<const uint16_t*>(&meta_s[wave][t][0]) + i * (PAIR ? 64 : a.ss) + (lane >> 2);
+            reinterpret_cast<const uint16_t*>(&meta_s[wave][t][0]) + i * (PAIR ? 64 : kSpread ? 16 * J : a.ss) + (lane >> 2);
         const uint32_t* zp = &meta_z[wave][t][0] + i * (PAIR ? 32 : a.zs) + (lane >> 5);
 #pragma unroll
         for (int j = 0; j < J; ++j) {

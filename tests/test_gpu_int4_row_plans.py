@@ -42,6 +42,73 @@ def test_qkv_rope_pairs_equal_the_modules(heads):
         assert np.array_equal(bits(a), bits(b)), what
 
 
+# An infinite scale spoils its own row and no other, also where a wavefront takes several rows and the one in front has lanes
+# without inputs: rows of up to 2048 inputs, three tensors of longer ones, and SwiGLU of longer ones with one row per wavefront.
+# Odd and even numbers of groups; one, two, three and four rows of SwiGLU, one and two of the others.
+@pytest.mark.parametrize("K,N", [(136, 96), (384, 77), (384, 4100), (640, 8200), (1408, 6100), (1920, 8204), (512, 13000),
+                                 (2304, 2048), (4224, 1500), (4224, 4300), (5120, 5120), (5120, 6144)])
+def test_infinite_scale_stays_in_its_row(K, N):
+    rng = synth.rng_for(617, K, N)
+    zs, ss, ws = sizes(K)
+    x, res = up(synth.normal_f16(rng, K)), synth.normal_f16(rng, N)
+    qs = [synth.random_qweight(rng, K, N) for _ in range(3)]
+    rows = np.arange(1, N, 11)  # comes to every place among a wavefront's rows
+    spoilt = []
+    for i, (W, Z, S) in enumerate(qs):
+        S = S.copy().reshape(N, ss)
+        S[rows, rng.integers(0, ss, rows.size) if i else 0] = np.inf
+        spoilt.append((W, Z, S.ravel()))
+
+    def run(tensors):
+        dev = [upq(q) for q in tensors]
+        ptrs = [p for q in dev for p in (q.Weight.ptr, q.Zeros.ptr, q.Scales.ptr)]
+        outs = dict((name, up(np.zeros(N, np.float16))) for name in "qkv")
+        capi.call("llama2_qkv_mat_vec", *[o.ptr for o in outs.values()], x.ptr, *ptrs, K, N, zs, ss, ws)
+        if K <= 2048 or N <= 2048:
+            outs["swiglu"] = up(np.zeros(N, np.float16))
+            capi.call("llama2_mat_vec_swiglu", outs["swiglu"].ptr, x.ptr, *ptrs[:6], K, N, zs, ss, ws)
+        if K <= 2048:
+            outs["plain"], outs["residual"] = up(np.zeros(N, np.float16)), up(res)
+            capi.call("llama2_mat_vec_int4", outs["plain"].ptr, x.ptr, *ptrs[:3], K, N, zs, ss, ws)
+            capi.call("llama2_mat_vec_residual_int4", outs["residual"].ptr, x.ptr, *ptrs[:3], K, N, zs, ss, ws)
+        return dict((name, o.to_host()) for name, o in outs.items())
+
+    others = np.setdiff1d(np.arange(N), rows)
+    clean, got = run(qs), run(spoilt)
+    for what in clean:
+        assert np.array_equal(bits(got[what][others]), bits(clean[what][others])), what
+        if what != "swiglu":  # a gate of -infinity gives 0 times the up row
+            assert not np.any(np.isfinite(got[what][rows])), what
+
+
+# An infinite scale of one row spoils that row and the one it is rotated with, and nothing else.
+@pytest.mark.parametrize("heads", [3, 34, 40])
+def test_qkv_rope_infinite_scale_stays_in_its_pair(heads):
+    dim = 128 * heads
+    cfg = dict(dim=dim, hidden_dim=256, n_layers=1, n_heads=heads, n_kv_heads=heads, vocab_size=64, seq_len=16,
+               rope_theta=10000.0)
+    model = synth.random_model(cfg, seed=32, rms_random=True)
+    ss, outs = synth.qweight_sizes(dim)[1], []
+    rows = np.arange(0, dim, 41)
+    for spoil in (False, True):
+        if spoil:
+            for i, name in enumerate(("q", "k", "v")):
+                W, Z, S = model["layers"][0][name]
+                S = S.copy().reshape(dim, ss)
+                S[rows, i] = np.inf
+                model["layers"][0][name] = W, Z, S.ravel()
+        t = Transformer(dict(cfg), model, mode=capi.DECODE_FUSED)
+        t.runstate.tokens.copy_to_device(np.array([5] * 16, np.int32))
+        t.Forward(9, 10)
+        outs.append([t.runstate.q.to_host(), t.runstate.keyCache.to_host(dim, 9 * dim), t.runstate.valueCache.to_host(dim, 9 * dim)])
+        t.close()
+    for what, clean, got in zip(("query", "key", "value"), *outs):
+        touched = rows if what == "value" else np.union1d(rows, rows ^ 64)
+        others = np.setdiff1d(np.arange(dim), touched)
+        assert np.array_equal(bits(got[others]), bits(clean[others])), what
+        assert not np.any(np.isfinite(got[rows])), what
+
+
 @pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 4096), (6144, 4097), (4352, 24)])
 def test_three_tensors_equal_one_at_a_time(K, N):
     rng = synth.rng_for(613, K, N)

@@ -1135,17 +1135,20 @@ inline bool try_span(const Int4Args& a, bool launch = true)
     return true;
 }
 
+inline bool scales_in_pairs(const Int4Args& a, int tensors)
+{
+    for (int t = 0; t < tensors; ++t)
+        if (!aligned(a.m[t].s, 4))
+            return false;
+    return (a.ss & 1) == 0;
+}
+
 template <int J>
 inline bool span_allowed(const Int4Args& a, int tensors)
 {
     if (ctx().int4_no_span || ctx().int4_narrow || ctx().int4_blocks)
         return false;
-    if (span_single_scales(J))
-        return true;
-    for (int t = 0; t < tensors; ++t)
-        if (!aligned(a.m[t].s, 4))
-            return false;
-    return (a.ss & 1) == 0;
+    return span_single_scales(J) || scales_in_pairs(a, tensors);
 }
 
 template <int J, int MODE, int STAGE>
@@ -1191,6 +1194,13 @@ inline bool launch_span(const Int4Args& a)
         if constexpr (J == 3) {
             if (a.n_tensors == 3 && a.N > 16 * cus && ceil_div(a.N, 12 * 2) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
                 return true;
+        }
+        // Scales that can only be read one by one: with fewer than four rows of each tensor per compute unit a wavefront per row
+        // (int4_matvec_kernel) beats one that takes its row of all three: K 384, 256 / 512 rows 2.72 / 2.84 us for 2.87 / 2.89, K 1920
+        // 3.03 / 3.24 for 3.32 / 3.45; 1024 rows 3.50 both, 1920 rows 3.99 for 3.67.
+        if constexpr (span_single_scales(J)) {
+            if (a.n_tensors == 3 && a.N < 4 * cus && !scales_in_pairs(a, 3))
+                return false;
         }
         if (a.n_tensors == 3)
             return try_span<J, MODE, STAGE, 3, 8, 1>(a) || try_span<J, MODE, STAGE, 3, 8, 2>(a);

@@ -109,7 +109,9 @@ def test_qkv_rope_infinite_scale_stays_in_its_pair(heads):
         assert not np.any(np.isfinite(got[rows])), what
 
 
-@pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 4096), (6144, 4097), (4352, 24)])
+# (the last three: an odd number of groups below, at and above four rows per compute unit)
+@pytest.mark.parametrize("K,N", [(5120, 5120), (5120, 6144), (5120, 6152), (4224, 4096), (6144, 4097), (4352, 24), (384, 1023),
+                                 (1920, 1024), (640, 1025)])
 def test_three_tensors_equal_one_at_a_time(K, N):
     rng = synth.rng_for(613, K, N)
     zs, ss, ws = sizes(K)

@@ -412,8 +412,8 @@ def test_model_widths(widths, lengths):
         tr.close()
 
 
-# Products whose workgroups come in two heights, on 256 compute units: 4 and 2 token tiles, 3 and 2, 4 and 3, of SwiGLU and of
-# QKV (dim 4352: QKV 4 and 3); row by row as above.
+# Products around the sizes at which workgroups come in two heights, on 256 compute units: 3 and 2 token tiles, 4 and 3, of SwiGLU and of
+# QKV (dim 4352: QKV 4 and 3; 4352 hidden and dim 2816 keep one height); row by row as above.
 @pytest.mark.parametrize("dim,hidden,known", [(1024, 4352, 950), (1024, 5376, 740), (1024, 6400, 950), (2816, 256, 950),
                                               (3456, 256, 740), (4352, 256, 950)])
 def test_workgroups_of_two_heights(dim, hidden, known):

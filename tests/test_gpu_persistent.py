@@ -67,13 +67,14 @@ def test_persistent_equals_fused_bit_for_bit():
             assert np.array_equal(bits(a), bits(b)), "%s differ between the launch sequence and the persistent step" % what
 
 
-@pytest.mark.parametrize("pos", [127, 128, 511, 512, 1100, 3071, 3072, 3100])
+@pytest.mark.parametrize("pos", [127, 128, 511, 512, 1023, 1024, 1100, 1535, 1536, 2047, 3071, 3072, 3100])
 def test_persistent_step_with_long_history(oracle, pos):
-    """1, 2, 4, 5, 9 and 24 attention blocks of 128 rows; from 3072 rows on the decoder falls
-    back to the launch sequence for the step.  Up to 1024 attended rows the launch sequence uses
+    """1, 2, 4, 5, 8, 9, 12, 13, 16 and 24 attention blocks of 128 rows; from 3072 rows on the decoder falls
+    back to the launch sequence for the step.  Up to 1536 attended rows the launch sequence uses
     128-row blocks as well and the two agree bit for bit; beyond, the launch sequence merges
     256-row blocks (a different, equally valid grouping of the same sums), and the comparison is
-    norm-wise at the per-module tolerance."""
+    norm-wise at the per-module tolerance.  The launch sequence as captured graphs agrees with itself on both sides
+    of every change of its launch shape."""
     cfg = dict(HS128, seq_len=max(1200, pos + 40))
     dim, L, S = cfg["dim"], cfg["n_layers"], cfg["seq_len"]
     model = synth.random_model(cfg, seed=11, rms_random=True)
@@ -82,7 +83,7 @@ def test_persistent_step_with_long_history(oracle, pos):
     vc = synth.normal_f16(rng, L * S * dim)
     token = np.array([17], np.int32)
     outs = []
-    for mode in (FUSED, PERSIST, PERSIST_GRAPH):
+    for mode in (FUSED, PERSIST, PERSIST_GRAPH, FUSED | capi.DECODE_GRAPH):
         t = Transformer(dict(cfg), model, mode=mode)
         t.runstate.keyCache.copy_to_device(kc)
         t.runstate.valueCache.copy_to_device(vc)
@@ -93,9 +94,10 @@ def test_persistent_step_with_long_history(oracle, pos):
         vrow = t.runstate.valueCache.to_host(dim, (L - 1) * S * dim + pos * dim)
         outs.append((t.runstate.logits.to_host(), row, vrow))
         t.close()
-    same_blocks = pos + 1 <= 1024 or pos + 1 > 3072
-    for a, b, what in zip(outs[1], outs[2], ("logits", "k row", "v row")):  # persistent: eager == graph replay
-        assert np.array_equal(bits(a), bits(b)), "%s at pos %d" % (what, pos)
+    same_blocks = pos + 1 <= 1536 or pos + 1 > 3072
+    for eager, graph in ((outs[1], outs[2]), (outs[0], outs[3])):
+        for a, b, what in zip(eager, graph, ("logits", "k row", "v row")):
+            assert np.array_equal(bits(a), bits(b)), "%s at pos %d" % (what, pos)
     for a, b, what in zip(outs[0], outs[1], ("logits", "k row", "v row")):
         if same_blocks:
             assert np.array_equal(bits(a), bits(b)), "%s at pos %d" % (what, pos)

@@ -206,10 +206,11 @@ def test_rejects_unsupported():
     assert capi.raw("llama2_multi_head_attention", out.ptr, dq.ptr, dk.ptr, dv.ptr, HS, 512, 0, 0.1, 4) == capi.ERR_INVALID_ARGUMENT
 
 
-# Beyond 1024 rows every wavefront keeps the softmax statistics of its own 32 rows (8 wavefronts a block up to 16384 rows,
-# 16 beyond): a last block with rows for one wavefront alone, for part of one, for all but one; and rows whose scores lie
-# below fp16's range (-infinity, no weight) filling a wavefront's share, a whole block, and the first block.
-@pytest.mark.parametrize("seq", [1025, 1031, 1056, 1057, 1279, 1280, 1281, 2304, 16384, 16385, 16900])
+# Beyond 1536 rows every wavefront keeps the softmax statistics of its own 32 rows (8 wavefronts a block up to 16384 rows,
+# 16 beyond): a last block with rows for one wavefront alone, for part of one, for all but one; and (last two tests) rows whose
+# scores lie below fp16's range (-infinity, no weight) filling a wavefront's share, a whole block, and the first block.
+@pytest.mark.parametrize("seq", [1025, 1031, 1056, 1057, 1279, 1280, 1281, 1537, 1543, 1568, 1569, 1760, 1761, 1792, 1793, 2304,
+                                 16384, 16385, 16900])
 def test_statistics_per_wavefront(oracle, seq):
     dim, heads = 256, 2
     q, k, v = inputs(711, dim, seq)
@@ -227,7 +228,7 @@ def test_block_sizes_by_length(oracle, heads, seq):
     assert_close_up_to_ties(got, oracle_chain(oracle, q, k, v, dim, heads, seq, True), "attention %d/%d/%d" % (dim, heads, seq))
 
 
-# The same below 1024 rows: a block of 128 without any weight.
+# Up to 1536 rows: a block of 128 without any weight.
 @pytest.mark.parametrize("seq,masked", [(600, (128, 256)), (200, (128, 200)), (1500, (1408, 1500))])
 def test_short_blocks_without_weight(seq, masked):
     dim, heads = 256, 2
@@ -243,9 +244,8 @@ def test_short_blocks_without_weight(seq, masked):
     assert_close_normwise(got, want, "rows %s without weight" % (masked,))
 
 
-@pytest.mark.parametrize("masked", [(32, 64), (256, 512), (0, 256), (0, 1300), (1024, 1301)])
-def test_wavefronts_and_blocks_without_weight(masked):
-    dim, heads, seq = 256, 2, 1301
+def without_weight(seq, masked):
+    dim, heads = 256, 2
     q, k, v = inputs(712, dim, seq)
     q = np.abs(q) + np.float16(1)
     k = k.reshape(seq, dim)
@@ -257,3 +257,16 @@ def test_wavefronts_and_blocks_without_weight(masked):
     want = fused(q, k[rest].ravel(), v[rest].ravel(), dim, heads, rest.size)
     assert np.all(np.isfinite(got))
     assert_close_normwise(got, want, "rows %s without weight" % (masked,))  # the same sums in other blocks
+
+
+@pytest.mark.parametrize("masked", [(32, 64), (256, 512), (0, 256), (0, 1300), (1024, 1301)])
+def test_wavefronts_and_blocks_without_weight(masked):
+    without_weight(1301, masked)
+
+
+# 9 blocks of 8 wavefronts, then 34 of 16
+@pytest.mark.parametrize("seq,masked", [(2301, (32, 64)), (2301, (256, 512)), (2301, (0, 256)), (2301, (0, 2300)), (2301, (2048, 2301)),
+                                        (2301, (300, 2200)), (17000, (32, 64)), (17000, (512, 1024)), (17000, (0, 16896)),
+                                        (17000, (16896, 17000))])
+def test_wavefronts_without_weight_keeping_their_own_statistics(seq, masked):
+    without_weight(seq, masked)

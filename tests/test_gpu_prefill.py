@@ -420,6 +420,30 @@ def test_workgroups_of_two_heights(dim, hidden, known):
     test_model_widths(config(dim, hidden, 2, known), (known,))
 
 
+# A row's sums do not depend on how many rows are with it, as long as a step takes one group of K and K comes in the same pieces: the
+# same rows in a batch whose QKV or SwiGLU has workgroups of two heights and in one that has one height, bit for
+# bit.  (product, dim, hidden, rows with two heights, rows with one); tests/test_prompt_product_shapes.py holds them to that.
+TWO_HEIGHTS = [("qkv", 2816, 256, 991, 960), ("qkv", 3456, 256, 750, 800), ("qkv", 4352, 256, 930, 890),
+               ("swiglu", 2304, 4224, 992, 920), ("swiglu", 2304, 6272, 915, 990), ("swiglu", 3200, 5248, 700, 670)]
+
+
+@pytest.mark.parametrize("product,dim,hidden,two,one", TWO_HEIGHTS)
+def test_two_heights_equal_one_bit_for_bit(product, dim, hidden, two, one):
+    layers = 1 if product == "qkv" else 2  # the last layer ends with its cache rows
+    cfg = config(dim, hidden, layers, max(two, one) + 1)
+    model = synth.random_model(cfg, seed=77, rms_random=True)
+    prompt = synth.rng_for(817, dim).integers(3, 512, max(two, one) + 1).astype(np.int32)
+    t, got = Transformer(dict(cfg), model, mode=FUSED_GRAPH), []
+    for rows in (two, one):
+        t.runstate.tokens.copy_to_device(prompt)
+        clear_caches(t)
+        capi.call("llama2_decode_run", t._decoder, 0, rows + 1, rows + 1)
+        got.append(caches(t, cfg, min(two, one)))
+    for name, a, b in zip("kv", *got):
+        assert np.all(np.isfinite(a)) and np.array_equal(a.view(np.uint16), b.view(np.uint16)), name
+    t.close()
+
+
 # The other loops that batch their prompt: sampling, and the persistent step (same bits as the launch sequence behind
 # the same batch).
 def test_sampled_run_behind_a_batch():

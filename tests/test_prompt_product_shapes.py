@@ -8,6 +8,7 @@ import subprocess
 import pytest
 
 from managedllama2_amd import synth
+from test_gpu_prefill import TWO_HEIGHTS
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "managedllama2_amd", "csrc")
 SOURCE = """
@@ -65,3 +66,21 @@ def test_two_heights_of_the_model_widths(shape):
     two = [rows for rows in range(32, 1025, 32) if len(set(heights(swiglu(shape, dim, hidden, rows)))) > 1]
     assert two == [320, 416, 448, 480, 928, 960, 992, 1024]
     assert all(len(set(heights(qkv(shape, dim, rows)))) == 1 for rows in range(32, 1025, 32))
+
+
+@pytest.mark.parametrize("product,dim,hidden,two,one", TWO_HEIGHTS)
+def test_compared_batches_differ_in_the_heights_alone(shape, product, dim, hidden, two, one):
+    a, b = ((qkv(shape, dim, r) if product == "qkv" else swiglu(shape, dim, hidden, r)) for r in (two, one))
+    assert a[0] != a[3] and b[0] == b[3] and a[1] == b[1] == 4  # one group of K per step on both sides
+    if product == "swiglu":
+        for K in (dim, hidden):  # o- and down-projection: groups per step and pieces of K
+            assert shape(two, dim // 64, K, True)[1:3] == shape(one, dim // 64, K, True)[1:3]
+        for rows in (two, one):  # attention in one piece: at most 4 workgroups per compute unit
+            assert 4 * 256 // (-(-rows // 32) * (dim // 128)) <= 1
+            # and the other product of the layer has the same groups per step
+            assert qkv(shape, dim, rows)[1] == 4
+
+
+def test_all_pairs_of_heights_are_compared(shape):
+    assert {(p, heights(qkv(shape, d, r) if p == "qkv" else swiglu(shape, d, h, r))) for p, d, h, r, _ in TWO_HEIGHTS} == {
+        (p, pair) for p in ("qkv", "swiglu") for pair in ((4, 3), (4, 2), (3, 2))}

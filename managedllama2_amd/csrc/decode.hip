@@ -595,7 +595,9 @@ QW qw(const llama2_qweight& q) { return QW{q.weight, q.zeros, q.scales}; }
 // compute unit.  What the hand-over inside the attention launch costs (2.1 us) is what two blocks gain, less 0.6 us
 // of staging: 7B at 130 .. 250 rows 1108 -> 1084 us per token.  Four blocks gain 0.1 % (1114.9 us for 1117), eight lose 3 %
 // (1180 for 1146 at 700 rows), and so does 13B's o-projection, whose 20 rows per compute unit fit no such workgroup,
-// with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.
+// with any (10 wavefronts of two rows: 1888 us for 1892): they merge in the attention launch.  So do odd numbers of groups (3, 5,
+// .. 15 heads), though the kernel for up to 2048 inputs reads their scales by now: steps of 8 layers at 130 .. 250 rows would take
+// 0.2 .. 2.8 % less (15 heads 157 -> 154 us).
 bool launch_o_merge(const Int4Args& a, int blocks, bool launch)
 {
     if (blocks != kMergeBlocks || a.K % kRopeHeadSize || a.K != a.N || (a.ss & 1))

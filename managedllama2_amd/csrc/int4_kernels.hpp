@@ -1163,12 +1163,12 @@ inline bool launch_span(const Int4Args& a)
     // per compute unit takes its whole share where that is at most 12 wavefronts of two rows or 8 of seven.
     const int cus = ctx().num_cus > 0 ? ctx().num_cus : 256;
     if constexpr (MODE == QKV_ROPE) {
-        // 13B decode step, profiled: 11.6 us (640 workgroups of 8 wavefronts, one row each) -> 10.2
-        if constexpr (J == 3) {
-            if (a.n_tensors == 3 && ceil_div(a.N / 2, 12) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a))
-                return true;
-        }
-        return a.n_tensors == 3 && try_span<J, MODE, STAGE, 3, 8, 1>(a);
+        // 13B decode step, profiled: 11.6 us (640 workgroups of 8 wavefronts, one row each) -> 10.2.  Rows that are too many for
+        // that are too many for one per wavefront as well (16 resident wavefronts per compute unit).
+        if constexpr (J == 3)
+            return a.n_tensors == 3 && ceil_div(a.N / 2, 12) <= cus && try_span<J, MODE, STAGE, 3, 12, 2>(a);
+        else
+            return a.n_tensors == 3 && try_span<J, MODE, STAGE, 3, 8, 1>(a);
     } else if constexpr (MODE == SWIGLU) {
         // 13824 rows 14.9 us (8 wavefronts of four rows) -> 14.2, 14336 15.0 -> 14.3; three rows keep what they fit: 12288
         // rows 12.9 us, 13.4 with seven

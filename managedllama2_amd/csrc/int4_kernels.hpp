@@ -1210,7 +1210,9 @@ inline bool launch_span(const Int4Args& a)
     if constexpr (MODE == PLAIN || MODE == RESIDUAL) {
         // One tensor whose rows fill one workgroup of 16 wavefronts on every compute unit: a quarter of the staging, and nobody waits
         // for a second workgroup.  4096 rows of 4096 / 2560 inputs 3.87 / 3.61 us (4 wavefronts) -> 3.77 / 3.44, in the step of 7B behind
-        // 255 rows 0.3 %; 3072 rows, which leave compute units empty, are 3.46 with 4 wavefronts and 3.69 with 16.
+        // 255 rows 0.3 %; 3072 rows, which leave compute units empty, are 3.46 with 4 wavefronts and 3.69 with 16.  2304 .. 4096 inputs by
+        // 3841 .. 4096 rows all take 2 .. 8 % less.  J = 1 would take 1 .. 6 % less (512 x 4096 2.79 -> 2.69), not taken so far; J = 3
+        // up to 9 % more (5120 x 4096 4.30 -> 4.48).
         if constexpr (J == 2) {
             if (a.n_tensors == 1 && a.N > 15 * cus && a.N <= 16 * cus && try_span<J, MODE, STAGE, 1, 16, 1>(a))
                 return true;

@@ -378,6 +378,7 @@ def test_wide_prompt_blocks(dim, hidden, known):
 # prompt lengths reach, in token tiles x pairs of weight tiles per workgroup:
 #   QKV         11 12 14 22 24 34 44 (7B: 11, 51, 151, 76, 251, 385, 512 tokens)
 #   SwiGLU      12 22 24 34 44 (11, 51, 76, 151, 251)
+#   two heights SwiGLU 34 and 24 (385; 13B 321), 44 and 24 (512; 13B 1004), QKV 44 and 24 (1004)
 #   o-, down-proj  11 14 22 24 34 44, K in 1 to 8 pieces (1x4: 13B, 75)
 #   attention   1, 2 and 4 tiles per workgroup (11, 512, 1004), 1 to 4 pieces (11, 76, 151, 251)
 @pytest.mark.parametrize("widths,lengths", [(synth.LLAMA2_7B, (11, 51, 76, 151, 251, 385, 512, 1004)),
